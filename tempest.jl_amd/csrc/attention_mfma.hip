@@ -870,6 +870,7 @@ bool mfma_attention_takes(const th_attention_desc* d) {
 
 int build_attention_mfma_fwd(const th_attention_desc* d, th_launch** out) {
   if (int r = check_mfma(d, false)) return r;
+  if (decode_attention_takes(d)) return build_attention_decode_fwd(d, 16, false, out);
   switch (d->head_dim) {
     case 64: return fwd_launch<64>(d, out);
     case 128: return fwd_launch<128>(d, out);

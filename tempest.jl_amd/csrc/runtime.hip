@@ -64,7 +64,13 @@ void point_workspace(th_launch* l) {
 
 int ensure_workspace(th_launch* l) {
   if (l->ws_bytes == 0 || l->ws) return TH_OK;
-  if (int r = device_alloc(l->ws_bytes, &l->ws)) return r;
+  // A caller may be recording its stream: an allocation is no part of what
+  // it records, and is allowed there in the relaxed mode only.
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  TH_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  const int r = device_alloc(l->ws_bytes, &l->ws);
+  TH_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  if (r) return r;
   l->ws_owned = true;
   point_workspace(l);
   return TH_OK;
