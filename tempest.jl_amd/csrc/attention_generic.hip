@@ -499,6 +499,7 @@ namespace th {
 int build_attention_general_fwd(const th_attention_desc* d, th_launch** out) {
   if (int r = check(d, false)) return r;
   if (decode_attention_takes(d)) return build_attention_decode_fwd(d, 4, true, out);
+  if (masked_attention_takes(d)) return build_attention_masked_fwd(d, out);
   const bool f32 = (d->flags & TH_ATTN_F32) != 0;
   const int dp = padded_dim(d->head_dim);
   const void* fn = f32 ? fwd_kernel<true>(dp) : fwd_kernel<false>(dp);
@@ -523,6 +524,7 @@ int build_attention_general_fwd(const th_attention_desc* d, th_launch** out) {
 
 int build_attention_general_bwd(const th_attention_desc* d, th_launch** out) {
   if (int r = check(d, true)) return r;
+  if (masked_attention_takes(d)) return build_attention_masked_bwd(d, out);
   const bool f32 = (d->flags & TH_ATTN_F32) != 0;
   const int dp = padded_dim(d->head_dim);
   GenArgs a = args_of(d);

@@ -26,6 +26,17 @@
 // Masks: keys past the keys' length and, causal, keys after the query
 // (key <= query, positions from 0) weigh 0; queries past the sequence are
 // computed on zeros and not stored.
+// Device-held masks (M; bf16 at d = 64 and 128, which the general kernels'
+// vector ALUs ran before): a first key per query and a key count per sequence.
+// A forward or dQ workgroup starts at its queries' least first key, a dK/dV
+// workgroup finds the span of queries that see any of its keys, so packed
+// documents cost their own pairs and not the sequence's; blocks are not
+// paired with their mirror (the work follows the documents), the last ones,
+// the longest without documents, go first.  The general kernels hold P and dS
+// in fp32, so here each is hi + lo in bf16 (2^-17 relative) and takes two
+// products, on operands that are bf16 already.  Rows may start at any element.
+// B2 H12 S2048 d64 in documents of about 256, forward + backward: 5981 us on
+// the general kernels, 190 here.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -70,11 +81,45 @@ struct MArgs {
   int32_t nsplit, span;
   float* part;
   float* part_ml;
+  const int32_t* starts;   // M only: (positions, batch), 1-based, or null
+  const int32_t* lengths;  // M only: (batch), or null
 };
+
+// Global rows of M's arrays start at any element.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+typedef u32x2 u32x2_any __attribute__((aligned(2)));
+
+// The keys of sequence b (M: lengths[b] clamped to the keys' extent).
+template <bool M>
+__device__ __forceinline__ int keys_of(const MArgs& p, int b) {
+  if constexpr (M)
+    if (p.lengths) return min(max(p.lengths[b], 0), p.kv_seq);
+  return p.kv_seq;
+}
+
+// The first key query j < seq of sequence b sees.
+__device__ __forceinline__ int first_of(const MArgs& p, int j, int b) {
+  return p.starts ? p.starts[(int64_t)j + (int64_t)p.seq * b] - 1 : 0;
+}
+
+// The least of x over the workgroup's 256 threads, through four ints of LDS;
+// a barrier on both sides.
+__device__ __forceinline__ int least(int x, int* at) {
+#pragma unroll
+  for (int i = 1; i < 64; i *= 2) x = min(x, __shfl_xor(x, i, 64));
+  __syncthreads();
+  if (threadIdx.x % 64 == 0) at[threadIdx.x / 64] = x;
+  __syncthreads();
+  return min(min(at[0], at[1]), min(at[2], at[3]));
+}
 
 __device__ __forceinline__ float bf16_float(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+// What pack2 rounded away of each.
+__device__ __forceinline__ uint32_t rest2(float a, float b, uint32_t packed) {
+  return pack2(a - __uint_as_float(packed << 16), b - __uint_as_float(packed & 0xffff0000u));
 }
 // The value lane l ^ 32 holds.
 __device__ __forceinline__ float other_half(float x) {
@@ -118,7 +163,7 @@ __device__ __forceinline__ void row_operand(const uint16_t* row, bool live, bf16
   const int lane = threadIdx.x % 64;
 #pragma unroll
   for (int ks = 0; ks < D / 16; ++ks)
-    f[ks] = live ? *reinterpret_cast<const bf16x8*>(row + 16 * ks + 8 * (lane / 32)) : bf16x8{};
+    f[ks] = live ? (bf16x8)(u32x4) * reinterpret_cast<const u32x4_any*>(row + 16 * ks + 8 * (lane / 32)) : bf16x8{};
 }
 
 // A 64-position tile of an operand staged through registers: thread t holds
@@ -132,7 +177,7 @@ struct Stage {
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int c = threadIdx.x + 256 * i, row = c / kChunks, col = c % kChunks;
-      r[i] = row0 + row < limit ? *reinterpret_cast<const u32x4*>(base + (int64_t)(row0 + row) * ss + 8 * col)
+      r[i] = row0 + row < limit ? (u32x4) * reinterpret_cast<const u32x4_any*>(base + (int64_t)(row0 + row) * ss + 8 * col)
                                 : u32x4{0, 0, 0, 0};
     }
   }
@@ -159,7 +204,7 @@ __device__ __forceinline__ int block_of(int pass, int x, int nb) { return pass =
 // Keys [k_lo, k_hi) of query block qb: all of them (split < 0), or part
 // `split` of the sweep, which leaves its unnormalised O' and (m, l) for the
 // combining kernel.
-template <int D>
+template <int D, bool M>
 __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const int b, const int split) {
   constexpr int NS = D / 16, NB = D / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
@@ -177,16 +222,24 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
   for (int i = 0; i < NB; ++i) o[i] = f32x16{};
   float m = -INFINITY, l = 0.0f;
   const float c = p.scale * kLog2e;
-  const int qlast = min(qb * 128 + 127, p.seq - 1);
-  const int kend = p.causal ? min(p.kv_seq, qlast + 1) : p.kv_seq;
-  const int k_lo = split < 0 ? 0 : split * p.span, k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
+  const int nk = keys_of<M>(p, b), qlast = min(qb * 128 + 127, p.seq - 1);
+  const int kend = p.causal ? min(nk, qlast + 1) : nk;
+  int k_lo = split < 0 ? 0 : split * p.span, first = 0;
+  if constexpr (M) {
+    // The sweep starts at the block's least first key, a wave's share of it at the wave's.
+    if (p.starts) {
+      first = query < p.seq ? first_of(p, query, b) : 0x7fffffff;
+      k_lo = max(0, min(least(first, reinterpret_cast<int*>(lds + 4 * kTile<D>)), nk)) / 64 * 64;
+    }
+  }
+  const int k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
   const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
   Stage<D> sk, sv;
   auto K = [&](int s) { return lds + 2 * s * kTile<D>; };
   auto V = [&](int s) { return lds + (2 * s + 1) * kTile<D>; };
   if (nsteps > 0) {
-    sk.load(kbase, p.k_ss, k_lo, p.kv_seq);
-    sv.load(vbase, p.k_ss, k_lo, p.kv_seq);
+    sk.load(kbase, p.k_ss, k_lo, nk);
+    sv.load(vbase, p.k_ss, k_lo, nk);
     sk.store(K(0));
     sv.store(V(0));
   }
@@ -194,8 +247,8 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
   for (int j = 0; j < nsteps; ++j) {
     const int cur = j & 1, k0 = k_lo + 64 * j;
     if (j + 1 < nsteps) {
-      sk.load(kbase, p.k_ss, k0 + 64, p.kv_seq);
-      sv.load(vbase, p.k_ss, k0 + 64, p.kv_seq);
+      sk.load(kbase, p.k_ss, k0 + 64, nk);
+      sv.load(vbase, p.k_ss, k0 + 64, nk);
     }
     // S' (64 keys x 32 queries): keys 32 kb + 8 (i / 4) + 4 lh + i % 4 in register i.
     f32x16 s[2] = {f32x16{}, f32x16{}};
@@ -203,13 +256,13 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
     for (int ks = 0; ks < NS; ++ks)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) s[kb] = mfma(frag_rows<D>(K(cur), 32 * kb, ks), qf[ks], s[kb]);
-    if (k0 + 64 > p.kv_seq || (p.causal && k0 + 64 > q0)) {
+    if (M || k0 + 64 > p.kv_seq || (p.causal && k0 + 64 > q0)) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
-          if (key >= p.kv_seq || (p.causal && key > query)) s[kb][i] = -INFINITY;
+          if (key >= nk || (M && key < first) || (p.causal && key > query)) s[kb][i] = -INFINITY;
         }
     }
     float mb = -INFINITY;
@@ -225,26 +278,32 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
 #pragma unroll
     for (int i = 0; i < NB; ++i) o[i] *= alpha;
     m = mn;
-    bf16x8 pf[4];
+    bf16x8 pf[4], pl[4];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int part = 0; part < 2; ++part) {
-        u32x4 w;
+        u32x4 w, r;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float w0 = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * part + 2 * e], c, -shift));
           const float w1 = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * part + 2 * e + 1], c, -shift));
           l += w0 + w1;
           w[e] = pack2(w0, w1);
+          if constexpr (M) r[e] = rest2(w0, w1, w[e]);
         }
         pf[2 * kb + part] = (bf16x8)w;
+        if constexpr (M) pl[2 * kb + part] = (bf16x8)r;
       }
-    // O' (D x 32 queries) += V' P', the weights rounded to bf16.
+    // O' (D x 32 queries) += V' P', the weights rounded to bf16 (M: in two parts).
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-      for (int db = 0; db < NB; ++db) o[db] = mfma(frag_tr<D>(V(cur), 32 * db, ks), pf[ks], o[db]);
+      for (int db = 0; db < NB; ++db) {
+        const bf16x8 vt = frag_tr<D>(V(cur), 32 * db, ks);
+        if constexpr (M) o[db] = mfma(vt, pl[ks], o[db]);
+        o[db] = mfma(vt, pf[ks], o[db]);
+      }
     if (j + 1 < nsteps) {
       // The other stage was last read in step j - 1, before the barrier that ended it.
       sk.store(K(cur ^ 1));
@@ -274,21 +333,25 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int d = 32 * db + 8 * g + 4 * lh;
-      *reinterpret_cast<u32x2*>(obase + d) =
+      *reinterpret_cast<u32x2_any*>(obase + d) =
           u32x2{pack2(o[db][4 * g] * inv, o[db][4 * g + 1] * inv), pack2(o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv)};
     }
   if (lh == 0 && p.lse) p.lse[((int64_t)b * p.seq + query) * p.heads + h] = (m + log2f(l)) * kLn2;
 }
 
-template <int D>
+template <int D, bool M>
 __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void mfma_attn_fwd(MArgs p) {
+  if constexpr (M) {
+    fwd_block<D, true>(p, gridDim.x - 1 - blockIdx.x, blockIdx.z, -1);
+    return;
+  }
   // Split: one part of one block; else a block and, causal, its mirror (one call site, inlined once).
   const bool split = p.nsplit > 1;
   const int nb = (p.seq + 127) / 128;
   const int npass = split ? 1 : passes(p.causal, blockIdx.x, nb);
   for (int pass = 0; pass < npass; ++pass) {
     if (pass > 0) __syncthreads();
-    fwd_block<D>(p, split ? blockIdx.x : block_of(pass, blockIdx.x, nb), split ? blockIdx.z / p.nsplit : blockIdx.z,
+    fwd_block<D, false>(p, split ? blockIdx.x : block_of(pass, blockIdx.x, nb), split ? blockIdx.z / p.nsplit : blockIdx.z,
                  split ? blockIdx.z % p.nsplit : -1);
   }
 }
@@ -362,8 +425,7 @@ struct DeltaArgs {
   int32_t d;
 };
 
-// D / 8 lanes per (batch, position, head) row, 16 bytes each (the builder
-// checks the strides and bases for it); each lane group takes kDeltaRowsM
+// D / 8 lanes per (batch, position, head) row, 16 bytes each; each lane group takes kDeltaRowsM
 // rows, 64 / (D / 8) apart, every load issued before the first product.
 // Rows are numbered with the head fastest, so a load instruction covers
 // consecutive rows; row numbers fit 32 bits (the builder checks).
@@ -387,8 +449,8 @@ __global__ __launch_bounds__(256) void mfma_attn_delta(DeltaArgs a) {
   for (int i = 0; i < kDeltaRowsM; ++i) {
     // Rows past the end re-read the last one; nothing is written for them.
     const int64_t at = at_of(min(row0 + R * i, total - 1));
-    ow[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.o + at));
-    gw[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.dout + at));
+    ow[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p.o + at));
+    gw[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p.dout + at));
   }
   // Every load out before any of their data is used.
   __builtin_amdgcn_sched_barrier(0);
@@ -412,32 +474,94 @@ __global__ __launch_bounds__(256) void mfma_attn_delta(DeltaArgs a) {
 // with queries on the registers and keys on the lanes, so that P and dS feed
 // the products over queries straight from the accumulators.
 
+// One step under device-held masks, its two halves of 32 queries in turn (P
+// and dS in two bf16 parts each take twice the registers of one).
+template <int D, int DO>
+__device__ __forceinline__ void dkdv_masked_step(const MArgs& p, const uint16_t* Qt, const uint16_t* Gt, const float* L,
+                                                 int qq0, int key, int nk, int dh, const bf16x8 (&kf)[D / 16],
+                                                 const bf16x8 (&vf)[D / 16], f32x16 (&dk)[DO / 32],
+                                                 f32x16 (&dv)[DO / 32]) {
+  const int lh = threadIdx.x % 64 / 32;
+  const float c = p.scale * kLog2e;
+#pragma unroll
+  for (int jj = 0; jj < 2; ++jj) {
+    f32x16 s = f32x16{}, dp = f32x16{};
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) {
+      s = mfma(frag_rows<D>(Qt, 32 * jj, ks), kf[ks], s);
+      dp = mfma(frag_rows<D>(Gt, 32 * jj, ks), vf[ks], dp);
+    }
+#pragma unroll
+    for (int part = 0; part < 2; ++part) {
+      u32x4 ph, pl, sh, sl;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float w[2], x[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int i = 8 * part + 2 * e + u;
+          const int qi = 32 * jj + 8 * (i / 4) + 4 * lh + i % 4, query = qq0 + qi;
+          const bool seen = query < p.seq && key < nk && key >= __float_as_int(L[128 + qi]) && (!p.causal || key <= query);
+          w[u] = seen ? __builtin_amdgcn_exp2f(fmaf(s[i], c, -L[qi])) : 0.0f;
+          x[u] = seen ? w[u] * (dp[i] - L[64 + qi]) : 0.0f;
+        }
+        ph[e] = pack2(w[0], w[1]), pl[e] = rest2(w[0], w[1], ph[e]);
+        sh[e] = pack2(x[0], x[1]), sl[e] = rest2(x[0], x[1], sh[e]);
+      }
+#pragma unroll
+      for (int db = 0; db < DO / 32; ++db) {
+        const bf16x8 g = frag_tr<D>(Gt, DO * dh + 32 * db, 2 * jj + part), q = frag_tr<D>(Qt, DO * dh + 32 * db, 2 * jj + part);
+        dv[db] = mfma(g, (bf16x8)pl, dv[db]);
+        dk[db] = mfma(q, (bf16x8)sl, dk[db]);
+        dv[db] = mfma(g, (bf16x8)ph, dv[db]);
+        dk[db] = mfma(q, (bf16x8)sh, dk[db]);
+      }
+    }
+  }
+}
+
 // Query tiles [qstart, qstop) for the keys of kblk: all of them (split <
 // 0), or part `split` of the sweep, which leaves its unscaled fp32 dK', dV'.
-template <int D, int DO>
+template <int D, int DO, bool M>
 __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const int dh, const int b,
                                            const int split) {
   constexpr int NS = D / 16, NBO = DO / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-  float* stats = reinterpret_cast<float*>(lds + 4 * kTile<D>);  // [stage][lse * log2e (64) | delta (64)]
+  constexpr int kStats = M ? 192 : 128;
+  // [stage][lse * log2e (64) | delta (64) | M: first keys, as ints (64)]
+  float* stats = reinterpret_cast<float*>(lds + 4 * kTile<D>);
   const int hk = blockIdx.y;
   const int group = p.heads / p.kv_heads;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
   const int kw0 = kblk * 128, key = kw0 + wave * 32 + lr;
   const int64_t koff = (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
   bf16x8 kf[NS], vf[NS];
-  row_operand<D>(p.k + koff + (int64_t)key * p.k_ss, key < p.kv_seq, kf);
-  row_operand<D>(p.v + koff + (int64_t)key * p.k_ss, key < p.kv_seq, vf);
+  const int nk = keys_of<M>(p, b);
+  row_operand<D>(p.k + koff + (int64_t)key * p.k_ss, key < nk, kf);
+  row_operand<D>(p.v + koff + (int64_t)key * p.k_ss, key < nk, vf);
   f32x16 dk[NBO], dv[NBO];
 #pragma unroll
   for (int i = 0; i < NBO; ++i) dk[i] = f32x16{}, dv[i] = f32x16{};
   const float c = p.scale * kLog2e;
   auto Q = [&](int s) { return lds + 2 * s * kTile<D>; };
   auto G = [&](int s) { return lds + (2 * s + 1) * kTile<D>; };
-  auto Ls = [&](int s) { return stats + 128 * s; };
+  auto Ls = [&](int s) { return stats + kStats * s; };
   const int qfirst = p.causal ? kw0 / 64 * 64 : 0;
-  const int qstart = split < 0 ? qfirst : qfirst + split * p.span;
-  const int qstop = split < 0 ? p.seq : min(p.seq, qstart + p.span);
+  int qstart = split < 0 ? qfirst : qfirst + split * p.span;
+  int qstop = split < 0 ? p.seq : min(p.seq, qstart + p.span);
+  if constexpr (M) {
+    if (kw0 >= nk) qstop = qstart;  // no key of the block: zeros
+    if (p.starts && kw0 < nk) {
+      // The span of queries that see any of the block's keys.
+      int lo = 0x7fffffff, hi = 0x7fffffff;  // hi: the least of -j
+      for (int j = qstart + threadIdx.x; j < qstop; j += 256)
+        if (first_of(p, j, b) < kw0 + 128) lo = min(lo, j), hi = min(hi, -j);
+      int* at = reinterpret_cast<int*>(stats + 2 * kStats);
+      lo = least(lo, at), hi = least(hi, at);
+      qstop = lo == 0x7fffffff ? qstart : 1 - hi;
+      qstart = lo == 0x7fffffff ? qstart : lo / 64 * 64;
+    }
+  }
   const int nsteps = qstart < qstop ? (qstop - qstart + 63) / 64 : 0;
   Stage<D> sq, sg;
   float st = 0.0f;  // threads 0..127: a query's lse * log2e or delta
@@ -448,12 +572,15 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
       const int j = q0 + threadIdx.x % 64;
       const int64_t row = ((int64_t)b * p.seq + j) * p.heads + h;
       st = j < p.seq ? (threadIdx.x < 64 ? p.lse[row] * kLog2e : p.delta[row]) : 0.0f;
+    } else if (M && threadIdx.x < 192) {
+      const int j = q0 + threadIdx.x % 64;
+      st = __int_as_float(j < p.seq ? first_of(p, j, b) : 0x7fffffff);
     }
   };
   auto store = [&](int s) {
     sq.store(Q(s));
     sg.store(G(s));
-    if (threadIdx.x < 128) Ls(s)[threadIdx.x] = st;
+    if (threadIdx.x < kStats) Ls(s)[threadIdx.x] = st;
   };
   for (int h = hk * group; h < (hk + 1) * group; ++h) {
     const uint16_t* qbase = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
@@ -469,6 +596,12 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
       const uint16_t *Qt = Q(cur), *Gt = G(cur);
       const float* L = Ls(cur);
       // S = Q K', dP = dO V' (64 queries x 32 keys): query 32 jj + 8 (i / 4) + 4 lh + i % 4 in register i.
+      if constexpr (M) {
+        dkdv_masked_step<D, DO>(p, Qt, Gt, L, qq0, key, nk, dh, kf, vf, dk, dv);
+        if (j + 1 < nsteps) store(cur ^ 1);
+        __syncthreads();
+        continue;
+      }
       f32x16 s[2] = {f32x16{}, f32x16{}}, dp[2] = {f32x16{}, f32x16{}};
 #pragma unroll
       for (int ks = 0; ks < NS; ++ks)
@@ -541,22 +674,26 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
     for (int g = 0; g < 4; ++g) {
       const int d = DO * dh + 32 * db + 8 * g + 4 * lh;
       const float sc = p.scale;
-      *reinterpret_cast<u32x2*>(p.dk + out + d) =
+      *reinterpret_cast<u32x2_any*>(p.dk + out + d) =
           u32x2{pack2(dk[db][4 * g] * sc, dk[db][4 * g + 1] * sc), pack2(dk[db][4 * g + 2] * sc, dk[db][4 * g + 3] * sc)};
-      *reinterpret_cast<u32x2*>(p.dv + out + d) =
+      *reinterpret_cast<u32x2_any*>(p.dv + out + d) =
           u32x2{pack2(dv[db][4 * g], dv[db][4 * g + 1]), pack2(dv[db][4 * g + 2], dv[db][4 * g + 3])};
     }
 }
 
-template <int D, int DO>
+template <int D, int DO, bool M>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void mfma_attn_dkdv(MArgs p) {
+  if constexpr (M) {
+    dkdv_block<D, DO, true>(p, blockIdx.x, 0, blockIdx.z, -1);
+    return;
+  }
   constexpr int halves = D / DO;
   const bool split = p.nsplit > 1;
   const int nb = (p.kv_seq + 127) / 128, x = blockIdx.x / halves;
   const int npass = split ? 1 : passes(p.causal, x, nb);
   for (int pass = 0; pass < npass; ++pass) {
     if (pass > 0) __syncthreads();
-    dkdv_block<D, DO>(p, split ? x : block_of(pass, x, nb), blockIdx.x % halves, split ? blockIdx.z / p.nsplit : blockIdx.z,
+    dkdv_block<D, DO, false>(p, split ? x : block_of(pass, x, nb), blockIdx.x % halves, split ? blockIdx.z / p.nsplit : blockIdx.z,
                       split ? blockIdx.z % p.nsplit : -1);
   }
 }
@@ -568,7 +705,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void mfma_attn_dkdv(MArgs p) 
 
 // Keys [k_lo, k_hi) for query block qb: all of them (split < 0), or part
 // `split` of the sweep, which leaves its unscaled fp32 dQ'.
-template <int D>
+template <int D, bool M>
 __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int b, const int split) {
   constexpr int NS = D / 16, NB = D / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
@@ -590,16 +727,24 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
   f32x16 dq[NB];
 #pragma unroll
   for (int i = 0; i < NB; ++i) dq[i] = f32x16{};
-  const int qlast = min(qb * 128 + 127, p.seq - 1);
-  const int kend = p.causal ? min(p.kv_seq, qlast + 1) : p.kv_seq;
-  const int k_lo = split < 0 ? 0 : split * p.span, k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
+  const int nk = keys_of<M>(p, b), qlast = min(qb * 128 + 127, p.seq - 1);
+  const int kend = p.causal ? min(nk, qlast + 1) : nk;
+  int k_lo = split < 0 ? 0 : split * p.span, first = 0;
+  if constexpr (M) {
+    // The sweep starts at the block's least first key, a wave's share of it at the wave's.
+    if (p.starts) {
+      first = query < p.seq ? first_of(p, query, b) : 0x7fffffff;
+      k_lo = max(0, min(least(first, reinterpret_cast<int*>(lds + 4 * kTile<D>)), nk)) / 64 * 64;
+    }
+  }
+  const int k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
   const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
   Stage<D> sk, sv;
   auto K = [&](int s) { return lds + 2 * s * kTile<D>; };
   auto V = [&](int s) { return lds + (2 * s + 1) * kTile<D>; };
   if (nsteps > 0) {
-    sk.load(kbase, p.k_ss, k_lo, p.kv_seq);
-    sv.load(vbase, p.k_ss, k_lo, p.kv_seq);
+    sk.load(kbase, p.k_ss, k_lo, nk);
+    sv.load(vbase, p.k_ss, k_lo, nk);
     sk.store(K(0));
     sv.store(V(0));
   }
@@ -607,8 +752,8 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
   for (int j = 0; j < nsteps; ++j) {
     const int cur = j & 1, k0 = k_lo + 64 * j;
     if (j + 1 < nsteps) {
-      sk.load(kbase, p.k_ss, k0 + 64, p.kv_seq);
-      sv.load(vbase, p.k_ss, k0 + 64, p.kv_seq);
+      sk.load(kbase, p.k_ss, k0 + 64, nk);
+      sv.load(vbase, p.k_ss, k0 + 64, nk);
     }
     f32x16 s[2] = {f32x16{}, f32x16{}}, dp[2] = {f32x16{}, f32x16{}};
 #pragma unroll
@@ -618,12 +763,12 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
         s[kb] = mfma(frag_rows<D>(K(cur), 32 * kb, ks), qf[ks], s[kb]);
         dp[kb] = mfma(frag_rows<D>(V(cur), 32 * kb, ks), gf[ks], dp[kb]);
       }
-    bf16x8 sf[4];
+    bf16x8 sf[4], sl[4];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int part = 0; part < 2; ++part) {
-        u32x4 w;
+        u32x4 w, r;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           float x[2];
@@ -631,18 +776,24 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
           for (int u = 0; u < 2; ++u) {
             const int i = 8 * part + 2 * e + u;
             const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
-            const bool seen = key < p.kv_seq && (!p.causal || key <= query);
+            const bool seen = key < nk && (!M || key >= first) && (!p.causal || key <= query);
             const float pw = seen ? __builtin_amdgcn_exp2f(fmaf(s[kb][i], c, -l2)) : 0.0f;
-            x[u] = pw * (dp[kb][i] - dl);
+            x[u] = M && !seen ? 0.0f : pw * (dp[kb][i] - dl);
           }
           w[e] = pack2(x[0], x[1]);
+          if constexpr (M) r[e] = rest2(x[0], x[1], w[e]);
         }
         sf[2 * kb + part] = (bf16x8)w;
+        if constexpr (M) sl[2 * kb + part] = (bf16x8)r;
       }
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-      for (int db = 0; db < NB; ++db) dq[db] = mfma(frag_tr<D>(K(cur), 32 * db, ks), sf[ks], dq[db]);
+      for (int db = 0; db < NB; ++db) {
+        const bf16x8 kt = frag_tr<D>(K(cur), 32 * db, ks);
+        if constexpr (M) dq[db] = mfma(kt, sl[ks], dq[db]);
+        dq[db] = mfma(kt, sf[ks], dq[db]);
+      }
     if (j + 1 < nsteps) {
       sk.store(K(cur ^ 1));
       sv.store(V(cur ^ 1));
@@ -668,19 +819,23 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
     for (int g = 0; g < 4; ++g) {
       const int d = 32 * db + 8 * g + 4 * lh;
       const float sc = p.scale;
-      *reinterpret_cast<u32x2*>(out + d) =
+      *reinterpret_cast<u32x2_any*>(out + d) =
           u32x2{pack2(dq[db][4 * g] * sc, dq[db][4 * g + 1] * sc), pack2(dq[db][4 * g + 2] * sc, dq[db][4 * g + 3] * sc)};
     }
 }
 
-template <int D>
+template <int D, bool M>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void mfma_attn_dq(MArgs p) {
+  if constexpr (M) {
+    dq_block<D, true>(p, gridDim.x - 1 - blockIdx.x, blockIdx.z, -1);
+    return;
+  }
   const bool split = p.nsplit > 1;
   const int nb = (p.seq + 127) / 128;
   const int npass = split ? 1 : passes(p.causal, blockIdx.x, nb);
   for (int pass = 0; pass < npass; ++pass) {
     if (pass > 0) __syncthreads();
-    dq_block<D>(p, split ? blockIdx.x : block_of(pass, blockIdx.x, nb), split ? blockIdx.z / p.nsplit : blockIdx.z,
+    dq_block<D, false>(p, split ? blockIdx.x : block_of(pass, blockIdx.x, nb), split ? blockIdx.z / p.nsplit : blockIdx.z,
                 split ? blockIdx.z % p.nsplit : -1);
   }
 }
@@ -711,6 +866,7 @@ MArgs margs_of(const th_attention_desc* d) {
   a.kv_seq = d->kv_seq > 0 ? d->kv_seq : d->seq;
   a.heads = d->heads, a.kv_heads = d->kv_heads, a.batch = d->batch, a.causal = d->causal;
   a.scale = d->scale > 0 ? d->scale : 1.0f / sqrtf((float)d->head_dim);
+  a.starts = d->starts, a.lengths = d->lengths;
   return a;
 }
 
@@ -726,7 +882,7 @@ double visible_pairs(const MArgs& a) {
 template <int D>
 int fwd_launch(const th_attention_desc* d, th_launch** out) {
   const size_t lds = 4 * (size_t)kTile<D> * sizeof(uint16_t);
-  TH_HIP(hipFuncSetAttribute((const void*)mfma_attn_fwd<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  TH_HIP(hipFuncSetAttribute((const void*)mfma_attn_fwd<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   MArgs a = margs_of(d);
   const int nqb = (d->seq + 127) / 128;
   const th::Split sp = th::split_of((int64_t)nqb * d->heads * d->batch, a.kv_seq);
@@ -734,7 +890,7 @@ int fwd_launch(const th_attention_desc* d, th_launch** out) {
   TH_REQUIRE((int64_t)d->batch * sp.n <= 65535, "attention: grid too large");
   th::Builder b("attention_fwd_mfma", 7);
   const dim3 grid = sp.n > 1 ? dim3(nqb, d->heads, d->batch * sp.n) : dim3(blocks_of(d->seq, d->causal), d->heads, d->batch);
-  int k = b.kernel((const void*)mfma_attn_fwd<D>, D == 64 ? "mfma_attn_fwd_d64" : D == 128 ? "mfma_attn_fwd_d128"
+  int k = b.kernel((const void*)mfma_attn_fwd<D, false>, D == 64 ? "mfma_attn_fwd_d64" : D == 128 ? "mfma_attn_fwd_d128"
                                                                                           : "mfma_attn_fwd_d256",
                    grid, dim3(256), (uint32_t)lds, a);
   b.ref(0, k, TH_OFFSET(MArgs, q));
@@ -768,9 +924,9 @@ int bwd_launch(const th_attention_desc* d, th_launch** out) {
   constexpr int DO = D == 256 ? 128 : D;
   const size_t lds_kv = 4 * (size_t)kTile<D> * sizeof(uint16_t);
   const size_t lds_dkdv = lds_kv + 2 * 128 * sizeof(float);
-  TH_HIP(hipFuncSetAttribute((const void*)mfma_attn_dkdv<D, DO>, hipFuncAttributeMaxDynamicSharedMemorySize,
+  TH_HIP(hipFuncSetAttribute((const void*)mfma_attn_dkdv<D, DO, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                              (int)lds_dkdv));
-  TH_HIP(hipFuncSetAttribute((const void*)mfma_attn_dq<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_kv));
+  TH_HIP(hipFuncSetAttribute((const void*)mfma_attn_dq<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_kv));
   MArgs a = margs_of(d);
   th::Builder b("attention_bwd_mfma", 11);
   const int64_t rows = (int64_t)d->batch * d->seq * d->heads;
@@ -791,7 +947,7 @@ int bwd_launch(const th_attention_desc* d, th_launch** out) {
   const dim3 gkv = skv.n > 1 ? dim3(nkb * (D / DO), d->kv_heads, d->batch * skv.n)
                              : dim3(blocks_of(a.kv_seq, d->causal) * (D / DO), d->kv_heads, d->batch);
   const dim3 gq = sq.n > 1 ? dim3(nqb, d->heads, d->batch * sq.n) : dim3(blocks_of(d->seq, d->causal), d->heads, d->batch);
-  int k1 = b.kernel((const void*)mfma_attn_dkdv<D, DO>, D == 64 ? "mfma_attn_dkdv_d64" : D == 128 ? "mfma_attn_dkdv_d128"
+  int k1 = b.kernel((const void*)mfma_attn_dkdv<D, DO, false>, D == 64 ? "mfma_attn_dkdv_d64" : D == 128 ? "mfma_attn_dkdv_d128"
                                                                                                : "mfma_attn_dkdv_d256",
                     gkv, dim3(256), (uint32_t)lds_dkdv, akv);
   if (skv.n > 1) {
@@ -810,7 +966,7 @@ int bwd_launch(const th_attention_desc* d, th_launch** out) {
     b.ref(7, ks, TH_OFFSET(SumArgs, out));
     b.ref(8, kv, TH_OFFSET(SumArgs, out));
   }
-  int k2 = b.kernel((const void*)mfma_attn_dq<D>, D == 64 ? "mfma_attn_dq_d64" : D == 128 ? "mfma_attn_dq_d128"
+  int k2 = b.kernel((const void*)mfma_attn_dq<D, false>, D == 64 ? "mfma_attn_dq_d64" : D == 128 ? "mfma_attn_dq_d128"
                                                                                        : "mfma_attn_dq_d256",
                     gq, dim3(256), (uint32_t)lds_kv, aq);
   if (sq.n > 1) {
@@ -831,6 +987,64 @@ int bwd_launch(const th_attention_desc* d, th_launch** out) {
     for (int kk : {k0, k1, k2}) b.ref(v, kk, offs[v]);
   for (int kk : {k0, k1, k2}) b.ws_ref(kk, TH_OFFSET(MArgs, delta), at_delta);
   for (int v : {0, 1, 2, 3, 5, 6, 7, 8}) b.align(v, 16);
+  const double BH = (double)d->batch * d->heads, BHk = (double)d->batch * d->kv_heads;
+  b.work(2.0 * BH * a.seq * D * 4 + 2.0 * BHk * a.kv_seq * D * 4 + 8.0 * BH * a.seq,
+         2.5 * 4.0 * BH * D * visible_pairs(a), (int64_t)gkv.x * gkv.y * gkv.z);
+  *out = b.release();
+  return TH_OK;
+}
+
+// Under device-held masks (or rows the kernels above do not take): whole
+// sweeps, a workgroup per block of 128.
+constexpr int kMaskLds = 2 * 192 * sizeof(float) + 16;  // the dK/dV stages' statistics and four ints
+
+template <int D>
+int masked_fwd_launch(const th_attention_desc* d, th_launch** out) {
+  const size_t lds = 4 * (size_t)kTile<D> * sizeof(uint16_t) + 16;
+  const void* fn = (const void*)mfma_attn_fwd<D, true>;
+  TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  MArgs a = margs_of(d);
+  th::Builder b("attention_fwd_mfma", 7);
+  const dim3 grid((d->seq + 127) / 128, d->heads, d->batch);
+  const int k = b.kernel(fn, D == 64 ? "mfma_attn_fwd_masked_d64" : "mfma_attn_fwd_masked_d128", grid, dim3(256),
+                         (uint32_t)lds, a);
+  const size_t offs[7] = {TH_OFFSET(MArgs, q),   TH_OFFSET(MArgs, k),      TH_OFFSET(MArgs, v),
+                          TH_OFFSET(MArgs, o),   TH_OFFSET(MArgs, lse),    TH_OFFSET(MArgs, starts),
+                          TH_OFFSET(MArgs, lengths)};
+  for (int v = 0; v < 7; ++v) b.ref(v, k, offs[v]);
+  const double BH = (double)d->batch * d->heads, BHk = (double)d->batch * d->kv_heads;
+  b.work(2.0 * BH * a.seq * D * 2 + 2.0 * BHk * a.kv_seq * D * 2 + 4.0 * BH * a.seq, 4.0 * BH * D * visible_pairs(a),
+         (int64_t)grid.x * grid.y * grid.z);
+  *out = b.release();
+  return TH_OK;
+}
+
+template <int D>
+int masked_bwd_launch(const th_attention_desc* d, th_launch** out) {
+  const size_t tiles = 4 * (size_t)kTile<D> * sizeof(uint16_t), lds_dkdv = tiles + kMaskLds, lds_dq = tiles + 16;
+  const void *f1 = (const void*)mfma_attn_dkdv<D, D, true>, *f2 = (const void*)mfma_attn_dq<D, true>;
+  TH_HIP(hipFuncSetAttribute(f1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dkdv));
+  TH_HIP(hipFuncSetAttribute(f2, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq));
+  MArgs a = margs_of(d);
+  th::Builder b("attention_bwd_mfma", 11);
+  const int64_t rows = (int64_t)d->batch * d->seq * d->heads;
+  const uint64_t at_delta = b.workspace((uint64_t)rows * sizeof(float));
+  constexpr int kDeltaBlockRows = 4 * (64 / (D / 8)) * kDeltaRowsM;
+  const int k0 = b.kernel((const void*)mfma_attn_delta<D>, "mfma_attn_delta",
+                          dim3((unsigned)((rows + kDeltaBlockRows - 1) / kDeltaBlockRows)), dim3(256), 0, DeltaArgs{a, D});
+  const dim3 gkv((a.kv_seq + 127) / 128, d->kv_heads, d->batch), gq((d->seq + 127) / 128, d->heads, d->batch);
+  const int k1 = b.kernel(f1, D == 64 ? "mfma_attn_dkdv_masked_d64" : "mfma_attn_dkdv_masked_d128", gkv, dim3(256),
+                          (uint32_t)lds_dkdv, a);
+  const int k2 = b.kernel(f2, D == 64 ? "mfma_attn_dq_masked_d64" : "mfma_attn_dq_masked_d128", gq, dim3(256),
+                          (uint32_t)lds_dq, a);
+  const size_t offs[11] = {TH_OFFSET(MArgs, q),      TH_OFFSET(MArgs, k),  TH_OFFSET(MArgs, v),  TH_OFFSET(MArgs, o),
+                           TH_OFFSET(MArgs, lse),    TH_OFFSET(MArgs, dout), TH_OFFSET(MArgs, dq), TH_OFFSET(MArgs, dk),
+                           TH_OFFSET(MArgs, dv),     TH_OFFSET(MArgs, starts), TH_OFFSET(MArgs, lengths)};
+  // The delta kernel's arguments are MArgs followed by d: the same offsets.
+  for (int kk : {k0, k1, k2}) {
+    for (int v = 0; v < 11; ++v) b.ref(v, kk, offs[v]);
+    b.ws_ref(kk, TH_OFFSET(MArgs, delta), at_delta);
+  }
   const double BH = (double)d->batch * d->heads, BHk = (double)d->batch * d->kv_heads;
   b.work(2.0 * BH * a.seq * D * 4 + 2.0 * BHk * a.kv_seq * D * 4 + 8.0 * BH * a.seq,
          2.5 * 4.0 * BH * D * visible_pairs(a), (int64_t)gkv.x * gkv.y * gkv.z);
@@ -885,6 +1099,21 @@ int build_attention_mfma_bwd(const th_attention_desc* d, th_launch** out) {
     case 128: return bwd_launch<128>(d, out);
     default: return bwd_launch<256>(d, out);
   }
+}
+
+// bf16 at head dims 64 and 128 under device-held masks, and rows of any
+// alignment and strides (descriptors the general kernels' checks passed).
+bool masked_attention_takes(const th_attention_desc* d) {
+  return !(d->flags & TH_ATTN_F32) && (d->head_dim == 64 || d->head_dim == 128) &&
+         (int64_t)d->batch * d->seq * d->heads < 2147483648LL;
+}
+
+int build_attention_masked_fwd(const th_attention_desc* d, th_launch** out) {
+  return d->head_dim == 64 ? masked_fwd_launch<64>(d, out) : masked_fwd_launch<128>(d, out);
+}
+
+int build_attention_masked_bwd(const th_attention_desc* d, th_launch** out) {
+  return d->head_dim == 64 ? masked_bwd_launch<64>(d, out) : masked_bwd_launch<128>(d, out);
 }
 
 }  // namespace th

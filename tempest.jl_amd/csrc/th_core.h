@@ -217,6 +217,11 @@ int build_attention_general_bwd(const th_attention_desc* d, th_launch** out);
 bool mfma_attention_takes(const th_attention_desc* d);
 int build_attention_mfma_fwd(const th_attention_desc* d, th_launch** out);
 int build_attention_mfma_bwd(const th_attention_desc* d, th_launch** out);
+// The same kernels under device-held masks, for descriptors the general
+// kernels' checks have passed.
+bool masked_attention_takes(const th_attention_desc* d);
+int build_attention_masked_fwd(const th_attention_desc* d, th_launch** out);
+int build_attention_masked_bwd(const th_attention_desc* d, th_launch** out);
 // A few queries over a long cache (attention_decode.hip), for descriptors the
 // two above have checked; `align`: what q, k, v, o keep when repointed;
 // `masks`: values 5 and 6 (starts, lengths) are the launch's.
