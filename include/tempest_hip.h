@@ -156,6 +156,15 @@ int th_launch_run(th_launch* launch);
  * src/Compiler/Implement/Implement.jl (repoint!), ext/CUDAExt.jl:1086-1090. */
 int th_launch_repoint(th_launch* launch, int value, void* ptr);
 
+/* th_launch_run for each of `n` launches, in order. */
+int th_launches_run(th_launch* const* host_launches, int n);
+
+/* th_launch_repoint for `n` values at once: value values[i] of launches[i] at
+ * base + offsets[i] (the places of one allocation that holds several values,
+ * as a compiled program's results). */
+int th_launches_place(th_launch* const* host_launches, const int32_t* host_values, const uint64_t* host_offsets,
+                      int n, void* base);
+
 /* The launch's algorithmic work.  Feeds Implement.estimate,
  * src/Compiler/Implement/Implement.jl:61-82. */
 int th_launch_work(th_launch* launch, th_work* host_out);

@@ -725,6 +725,18 @@ int th_launch_repoint(th_launch* l, int value, void* ptr) {
   return TH_OK;
 }
 
+int th_launches_run(th_launch* const* launches, int n) {
+  for (int i = 0; i < n; ++i)
+    if (int r = th_launch_run(launches[i])) return r;
+  return TH_OK;
+}
+
+int th_launches_place(th_launch* const* launches, const int32_t* values, const uint64_t* offsets, int n, void* base) {
+  for (int i = 0; i < n; ++i)
+    if (int r = th_launch_repoint(launches[i], values[i], static_cast<char*>(base) + offsets[i])) return r;
+  return TH_OK;
+}
+
 int th_launch_work(th_launch* l, th_work* out) {
   TH_REQUIRE(l != nullptr, "th_launch_work: null launch");
   *out = l->work;

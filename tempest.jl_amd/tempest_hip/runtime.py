@@ -21,6 +21,7 @@ stays there; ``programs.py`` states each plan it would form):
 from __future__ import annotations
 
 import ctypes
+import math
 from dataclasses import dataclass, field
 from typing import Callable, Sequence
 
@@ -234,19 +235,24 @@ class Executable:
                 self.result_at[name] = (at, nbytes)
                 at += (nbytes + 255) // 256 * 256
         self.results = target.allocate(torch.uint8, max(at, 256))
+        self._lent = False  # whether `results` is a call's, its caller's to keep
         for name, v in program.values.items():
             if v.role == "stored":
                 self.addresses[name] = self.arena.addresses[self.storage.slots[name]]
             elif v.role == "result":
-                off, nbytes = self.result_at[name]
-                t = self.results[off:off + nbytes].view(v.dtype)
-                self.own[name] = t
-                self.addresses[name] = t.data_ptr()
+                self.addresses[name] = self.results.data_ptr() + self.result_at[name][0]
         self._check(inputs)
         for name, x in zip(program.inputs, inputs):
             self._take(name, x, point)
         self.launches = [g.build(dict(self.addresses)) for g in program.groups]
         self._place_workspaces(pool)
+        # Every place a launch holds a result's address, as th_launches_place takes them.
+        refs = [(l.handle.value, i, self.result_at[v][0]) for g, l in zip(program.groups, self.launches)
+                for i, v in enumerate(g.values) if v in self.result_at]
+        n = max(1, len(refs))
+        self._result_refs = ((ctypes.c_void_p * n)(*(r[0] for r in refs)), (ctypes.c_int32 * n)(*(r[1] for r in refs)),
+                             (ctypes.c_uint64 * n)(*(r[2] for r in refs)), len(refs))
+        self._handles = (ctypes.c_void_p * max(1, len(self.launches)))(*(l.handle.value for l in self.launches))
         self.graph: Graph | Direct | None = None
         self._moved: set[int] = set()
 
@@ -326,10 +332,48 @@ class Executable:
 
     # -- running --------------------------------------------------------------
 
+    def _results_at(self, memory: torch.Tensor, lent: bool) -> None:
+        """Have the launches write their results to ``memory`` (laid out as ``result_at``)."""
+        base = memory.data_ptr()
+        self.results, self._lent = memory, lent
+        for name, (off, _) in self.result_at.items():
+            self.addresses[name] = base + off
+        self._alive()
+        call("th_launches_place", *self._result_refs, base)
+
+    def _alive(self) -> None:
+        for l in self.launches:
+            l.handle  # raises for a destroyed launch
+
+    def lend(self) -> bool:
+        """Give the next run a result allocation of its own, which its caller
+        keeps: nothing that runs later writes there.  False, and nothing
+        changed, where torch would not order the allocation with the launches
+        (another current stream than the library's) or the recording is a
+        graph, whose every node with a result would be retargeted."""
+        if isinstance(self.graph, Graph):
+            return False
+        stream = ctypes.c_void_p()
+        call("th_get_stream", ctypes.byref(stream))
+        if (stream.value or 0) != torch.cuda.current_stream(self.target.device).cuda_stream:
+            return False
+        self._results_at(torch.empty_like(self.results), lent=True)
+        return True
+
+    def _home(self) -> None:
+        """Results lent to a caller stay as they are: a run of the executable's
+        own writes to memory of its own."""
+        if self._lent:
+            self._results_at(torch.empty_like(self.results), lent=False)
+
     def execute(self) -> "Executable":
         """execute!(ex) (runtime.jl:1158): each launch in order."""
-        for l in self.launches:
-            l()
+        self._home()
+        return self._run()
+
+    def _run(self) -> "Executable":
+        self._alive()
+        call("th_launches_run", self._handles, len(self.launches))
         self._moved.clear()  # the launches themselves carry the new addresses
         return self
 
@@ -337,6 +381,7 @@ class Executable:
         """capture!(ex) (runtime.jl:1185): one graph of every launch, or the
         launches themselves where the target measures direct launches faster
         for this many kernels (HIPTarget.graph_pays); ``graph`` forces it."""
+        self._home()
         if self.graph is not None:
             self.graph = self.target.recapture(self.graph, self.launches, as_graph=graph)
         else:
@@ -353,6 +398,7 @@ class Executable:
         """replay!(ex) (runtime.jl:1208): retarget what moved, then one graph launch."""
         if self.graph is None:
             raise RuntimeError("replay before capture")
+        self._home()
         if isinstance(self.graph, Graph):
             for k in sorted(self._moved):
                 self.target.retarget(self.graph, k,
@@ -363,11 +409,13 @@ class Executable:
         return self
 
     def outputs(self) -> list[torch.Tensor]:
-        """outputs(ex): the result buffers themselves (the next run overwrites them)."""
+        """outputs(ex): the result buffers themselves (the next run overwrites
+        them; after a compiled call, what it returned)."""
         out = []
         for name in self.program.outputs:
             v = self.program.values[name]
-            t = self.own[name]
+            off, nbytes = self.result_at[name]
+            t = self.results[off:off + nbytes].view(v.dtype)
             out.append(t[0] if v.scalar else t.view(*reversed(v.dims)) if len(v.dims) > 1 else t)
         return out
 
@@ -412,9 +460,16 @@ class Compiled:
         for name in program.outputs:
             v = program.values[name]
             off, nbytes = ex.result_at[name]
-            self._layout.append((off, nbytes, v.dtype, v.scalar, tuple(reversed(v.dims)) if len(v.dims) > 1 else None))
-        spans = [(off, off + nbytes) for off, nbytes, _, scalar, _ in self._layout if scalar]
-        self._numbers = (min(a for a, _ in spans), max(b for _, b in spans)) if spans else None
+            shape = tuple(reversed(v.dims)) if len(v.dims) > 1 else (max(1, v.count),)
+            strides = tuple(math.prod(shape[i + 1:]) for i in range(len(shape)))
+            self._layout.append((v.dtype, v.scalar, shape, strides, off // _ELEMENT[v.dtype]))
+        spans = [ex.result_at[n] for n in program.outputs if program.values[n].scalar]
+        self._numbers = (min(a for a, _ in spans), max(a + n for a, n in spans)) if spans else None
+        if spans:
+            lo, hi = self._numbers
+            self._host = torch.empty((hi - lo + 255) // 256 * 256, dtype=torch.uint8, pin_memory=True)
+            self._host_numbers = [self._host.view(dt)[at - lo // _ELEMENT[dt]] if scalar else None
+                                  for dt, scalar, _, _, at in self._layout]
 
     def __call__(self, *args: torch.Tensor):
         sig = [(getattr(x, "dtype", None), tuple(getattr(x, "shape", ()))) for x in args]
@@ -422,6 +477,12 @@ class Compiled:
             raise ValueError(f"call does not match the compiled signature {self.signature}: {sig}")
         ex = self.executable
         ex.point(*args)
+        # The results go to an allocation that this call's caller keeps: a copy
+        # into one would read and write them once more (1 GiB: 418 us of a
+        # 1049 us call).
+        if ex.lend():
+            ex._run()
+            return self._returned(ex.results, lent=True)
         ex.replay() if ex.graph is not None else ex.execute()
         return self.returned()
 
@@ -429,18 +490,28 @@ class Compiled:
         """Arrays copied, numbers read to the host (compile.jl:334-349): one
         copy of the result allocation, whose views are the arrays returned,
         then one read of the span holding the numbers."""
-        fresh = self.executable.results.clone()
-        host = None
+        return self._returned(self.executable.results.clone(), lent=False)
+
+    def _returned(self, fresh: torch.Tensor, lent: bool):
+        # The arrays first: the device is still at work on the numbers.
+        typed = {}
+        out = []
+        for dtype, scalar, shape, strides, at in self._layout:
+            if scalar:
+                out.append(None)
+                continue
+            if dtype not in typed:
+                typed[dtype] = fresh.view(dtype)
+            out.append(typed[dtype].as_strided(shape, strides, at))
         if self._numbers is not None:
             lo, hi = self._numbers
-            host = fresh[lo:hi].cpu()
-        out = []
-        for off, nbytes, dtype, scalar, shape in self._layout:
-            if scalar:
-                out.append(host[off - self._numbers[0]:off - self._numbers[0] + nbytes].view(dtype)[0].item())
+            if lent:  # on the library's stream, which is torch's current one
+                call("th_download", self._host.data_ptr(), fresh.data_ptr() + lo, hi - lo)
             else:
-                t = fresh[off:off + nbytes].view(dtype)
-                out.append(t.view(*shape) if shape is not None else t)
+                self._host[:hi - lo].copy_(fresh[lo:hi])
+            for i, number in enumerate(self._host_numbers):
+                if number is not None:
+                    out[i] = number.item()
         return tuple(out)
 
 

@@ -462,3 +462,37 @@ def test_pool_destroyed_before_its_blocks(target):
     with pytest.raises(HIPError, match="destroyed"):
         _lib.call("th_pool_alloc", p, ctypes.c_uint64(256), ctypes.c_uint64(256), ctypes.byref(b))
     _lib.call("th_pool_free", p, a)
+
+
+def test_a_call_keeps_what_it_returned(target):
+    """Results are written to memory of the call's own: later
+    calls, and runs, recordings and retargets of the executable itself, leave
+    them as they were, and what the executable's outputs are follows."""
+    import tempest_hip as th
+    rows, n = 600, 1000
+    announce("lent results")
+    arrays = [(torch.randn(rows, n, device="cuda"), torch.randn(rows, n, device="cuda")) for _ in range(4)]
+    prog = th.programs.softmax_columns(rows, n)
+    wants = []
+    for x, g in arrays:
+        ex = th.prepare(prog, target, x, g).execute()
+        wants.append([t.clone() for t in ex.outputs()])
+    comp = th.compile(prog, target, *arrays[0])
+    first, second = comp(*arrays[0]), comp(*arrays[1])
+    ex = comp.executable
+    assert torch.equal(ex.outputs()[1], wants[1][1])
+    ex.point(*arrays[2]).replay()          # not into what `second` holds
+    assert torch.equal(ex.outputs()[1], wants[2][1])
+    third = comp(*arrays[2])
+    ex.point(*arrays[3]).execute()
+    ex.capture(graph=True)
+    fourth = comp(*arrays[3])              # a graph: the results copied
+    ex.replay()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        torch.cuda.synchronize()
+        fifth = comp(*arrays[3])           # another current stream
+        torch.cuda.synchronize()
+    torch.cuda.synchronize()
+    for got, want in zip((first, second, third, fourth), wants):
+        assert got[0] == want[0].item() and torch.equal(got[1], want[1])
+    assert torch.equal(fifth[1], wants[3][1])
