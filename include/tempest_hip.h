@@ -578,9 +578,9 @@ enum { TH_EPI_STORE = 0, TH_EPI_GELU = 1, TH_EPI_SQUARE_LOSS = 2, TH_EPI_GELU_BA
  *     128 x 128 tiles (16-byte loads along a unit stride, K split like the
  *     others), half factors or a half result on 64 x 64 tiles (unsplit).
  *     fp32 factors run only here unless TH_GEMM_BF16X3.
- * TH_TILE_AUTO chooses: the 256 x 256 kernel where it takes the product and
- * fills the device (split or not), else the largest middle tile that gives
- * 256 workgroups (the smallest if none does), else the general kernel.
+ * TH_TILE_AUTO chooses the least estimated time among the 256 x 256 kernel
+ * and the middle tiles (which it also gives fused epilogues, where the 256 x
+ * 256 kernel would take them), else the general kernel.
  * `splits` parts of K (256 and middle tiles, TH_EPI_STORE) are summed by a
  * second launch, with the bias and D; 0 chooses (parts when the tiles alone
  * would leave the device idle), 1 none.  th_gemm_tune measures the choices.

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <map>
 #include <mutex>
@@ -18,29 +19,25 @@
 namespace thg {
 namespace {
 
-struct RowSumArgs {
-  const float* partial;  // parts x m
-  uint16_t* out;         // m, bf16
-  int32_t m, parts;
-};
-
-// out[i] = sum over parts of partial[p, i], in part order.
-__global__ __launch_bounds__(256) void sum_parts(RowSumArgs a) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= a.m) return;
-  a.out[i] = bf16_bits(thd::sum_in_order(a.partial + i, a.m, a.parts));
-}
-
-struct LossArgs {
-  const float* partial;
+struct SumArgs {
+  const float* rows;       // parts x m
+  uint16_t* out;           // m, bf16
+  const float* loss_parts; // count, or null
   float* loss;
-  int32_t count;
+  int32_t m, parts, count;
 };
 
-__global__ __launch_bounds__(256) void sum_loss(LossArgs a) {
+// The folds an epilogue leaves: out[i] = sum over parts of rows[p, i], in
+// part order, 256 rows a workgroup; and, in the last workgroup, the loss.
+__global__ __launch_bounds__(256) void sum_epilogue(SumArgs a) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (blockIdx.x < (a.m + 255) / 256) {
+    if (i < a.m) a.out[i] = bf16_bits(thd::sum_in_order(a.rows + i, a.m, a.parts));
+    return;
+  }
   __shared__ double lds[4];
   double s = 0.0;
-  for (int i = threadIdx.x; i < a.count; i += 256) s += (double)a.partial[i];
+  for (int j = threadIdx.x; j < a.count; j += 256) s += (double)a.loss_parts[j];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
   if (threadIdx.x % 64 == 0) lds[threadIdx.x / 64] = s;
@@ -48,37 +45,42 @@ __global__ __launch_bounds__(256) void sum_loss(LossArgs a) {
   if (threadIdx.x == 0) a.loss[0] = (float)(lds[0] + lds[1] + lds[2] + lds[3]);
 }
 
-// The parts of K summed (in part order), plus the bias and what the product
-// is added to, rounded once to the result's type (fp32, bf16 or fp16):
-// C_z = D_z + sum_s W_zs + bias.
-struct ReduceArgs {
-  const float* ws;       // [batch][splits][m x n], column-major at ld m
-  void* c;               // result, column-major at c_ld, product z at c_batch
-  const uint16_t* bias;  // bf16, m, or null
-  const void* d;         // or null: laid out as C at d_ld, d_batch
-  int64_t c_ld, c_batch, d_ld, d_batch;
-  int32_t m, n, splits, c_dtype;
-};
-
-__global__ __launch_bounds__(256) void sum_splits(ReduceArgs a) {
-  const int64_t mn = (int64_t)a.m * a.n;
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (e >= mn) return;
-  const int64_t z = blockIdx.y;
-  const int64_t i = e % a.m, j = e / a.m;
-  float v = thd::sum_in_order(a.ws + z * a.splits * mn + e, mn, a.splits);
-  if (a.bias) v += bf16_float(a.bias[i]);
-  const int64_t at_d = z * a.d_batch + i + j * a.d_ld, at = z * a.c_batch + i + j * a.c_ld;
-  if (a.c_dtype == TH_F32) {
-    if (a.d) v += static_cast<const float*>(a.d)[at_d];
-    static_cast<float*>(a.c)[at] = v;
-  } else if (a.c_dtype == TH_F16) {
-    if (a.d) v += (float)__builtin_bit_cast(_Float16, static_cast<const uint16_t*>(a.d)[at_d]);
-    static_cast<uint16_t*>(a.c)[at] = __builtin_bit_cast(uint16_t, (_Float16)v);
-  } else {
-    if (a.d) v += bf16_float(static_cast<const uint16_t*>(a.d)[at_d]);
-    static_cast<uint16_t*>(a.c)[at] = bf16_bits(v);
+// The launch of sum_epilogue after an epilogue with row sums (`parts` x m at
+// at_rows of the workspace) and, for the square loss, `count` loss partials.
+void add_sums(th::Builder& b, const th_gemm_desc* d, uint64_t at_rows, int parts, uint64_t at_loss, int count) {
+  const bool loss = d->epilogue == TH_EPI_SQUARE_LOSS;
+  SumArgs s{nullptr, static_cast<uint16_t*>(d->row_sums), nullptr, d->loss, d->m, parts, count};
+  const int k = b.kernel((const void*)sum_epilogue, loss ? "sum_rows_and_loss" : "sum_rows",
+                         dim3((d->m + 255) / 256 + (loss ? 1 : 0)), dim3(256), 0, s);
+  b.ref(6, k, TH_OFFSET(SumArgs, out));
+  b.ws_ref(k, TH_OFFSET(SumArgs, rows), at_rows);
+  if (loss) {
+    b.ref(7, k, TH_OFFSET(SumArgs, loss));
+    b.ws_ref(k, TH_OFFSET(SumArgs, loss_parts), at_loss);
   }
+}
+
+// The launch that folds parts of K (mid_fold): `g` as the parts were written,
+// with what the result takes from `d` filled in here.
+int add_fold(th::Builder& b, const th_gemm_desc* d, MidArgs g, uint64_t at_parts) {
+  const bool accumulate = (d->flags & TH_GEMM_ACCUMULATE) != 0;
+  g.c = d->c, g.c_ld = d->c_ld, g.c_batch = d->c_batch, g.result = d->c_dtype;
+  g.d = accumulate ? d->d : nullptr;
+  g.d_ld = d->d_ld ? d->d_ld : d->c_ld;
+  g.d_batch = d->d_ld ? d->d_batch : d->c_batch;
+  g.bias = static_cast<const uint16_t*>(d->bias);
+  g.aux = static_cast<const uint16_t*>(d->aux), g.aux_ld = d->aux_ld;
+  g.aux_out = static_cast<uint16_t*>(d->aux_out);
+  g.m = d->m, g.n = d->n, g.epilogue = d->epilogue;
+  const unsigned blocks = (unsigned)(((d->m + 127) / 128) * (int64_t)((d->n + kFoldColumns - 1) / kFoldColumns));
+  const int k = b.kernel(mid_fold_kernel(), "sum_splits", dim3(blocks, 1, std::max(1, d->batch)), dim3(256), 0, g);
+  b.ws_ref(k, TH_OFFSET(MidArgs, parts), at_parts);
+  b.ref(2, k, TH_OFFSET(MidArgs, c));
+  b.ref(3, k, TH_OFFSET(MidArgs, bias));
+  b.ref(4, k, TH_OFFSET(MidArgs, aux));
+  b.ref(5, k, TH_OFFSET(MidArgs, aux_out));
+  b.ref(8, k, TH_OFFSET(MidArgs, d));
+  return k;
 }
 
 bool aligned(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) % bytes) == 0; }
@@ -151,6 +153,8 @@ static bool mid_takes(const th_gemm_desc* d) {
   return aligned(d->a, 16) && aligned(d->b, 16);
 }
 
+constexpr int kMidStep = 64;  // parts of K on the middle tiles are multiples of it
+
 static int mid_rows(int tile) { return tile == TH_TILE_64X128 || tile == TH_TILE_64X64 ? 64 : 128; }
 static int mid_cols(int tile) { return tile == TH_TILE_128X64 || tile == TH_TILE_64X64 ? 64 : 128; }
 
@@ -178,25 +182,90 @@ static int auto_splits(const th_gemm_desc* d, int tile) {
   return (int)std::max<int64_t>(1, std::min<int64_t>((256 + tiles - 1) / tiles, d->k / least));
 }
 
-// TH_TILE_AUTO: the 256 x 256 kernel where it takes the product and fills
-// the device (split or not) or nothing else takes it, else the largest middle
-// tile that gives 256 workgroups (the smallest if none does), else the
-// general kernel.
-static int choose_tile(const th_gemm_desc* d) {
-  const bool mid = mid_takes(d);
-  if (tile_kernel_takes(d) &&
-      (!mid || tiles_of(d, kTile, kTile) * auto_splits(d, TH_TILE_256) >= 128))
-    return TH_TILE_256;
-  if (mid) {
-    for (int t : {TH_TILE_128X128, TH_TILE_128X64, TH_TILE_64X128})
-      if (tiles_of(d, mid_rows(t), mid_cols(t)) >= 256) return t;
-    return TH_TILE_64X64;
+// Whether the 256 x 256 kernel runs its direct sweep: whole tiles of C, whole
+// steps of K, 32-bit byte offsets.
+static bool interior_256(const th_gemm_desc* d) {
+  const int64_t a_bytes = 2 * (d->a_k == 1 ? (int64_t)(d->m - 1) * d->a_m + d->k : (int64_t)(d->k - 1) * d->a_k + d->m);
+  const int64_t b_bytes = 2 * (d->b_k == 1 ? (int64_t)(d->n - 1) * d->b_n + d->k : (int64_t)(d->k - 1) * d->b_k + d->n);
+  return d->m % kTile == 0 && d->n % kTile == 0 && d->k % kDepth == 0 && a_bytes <= 0x7fffffff && b_bytes <= 0x7fffffff;
+}
+
+// Microseconds a product takes on a tile with K in `splits` parts, fitted to
+// what the kernels measure on this device (2.4 GHz, 256 CUs): a step of 64 of
+// K takes `alone` us with one workgroup on a CU and `pair` with two (the 256 x
+// 256 kernel has room for one), the end of a tile `end`; a launch 3; the fold
+// of parts 3 and their bytes at 8 TB/s.  Steps measured at 768 x 1024 x 3072,
+// 4096 x 512 x 4096, 2048^3, 4096^3, 4096 x 2048 x 16384: 64 x 64 0.27 / 0.43 to 0.55,
+// 128 x 64 0.44 / 0.75, 128 x 128 0.75 / 1.0 to 1.05, 256 x 256 1.55 to 1.8
+// (over twice that where its tiles are ragged: 2000 x 8000 x 520 58.6 us
+// against 33.8 on 128 x 128 tiles).  The estimate only has to order them.
+static double estimate(const th_gemm_desc* d, int tile, int splits) {
+  struct Cost { double alone, pair, end; };
+  const Cost c = tile == TH_TILE_256       ? (interior_256(d) ? Cost{1.7, 1.7, 5.0} : Cost{4.0, 4.0, 8.0})
+                 : tile == TH_TILE_128X128 ? Cost{0.75, 1.05, 2.0}
+                 : tile == TH_TILE_64X64   ? Cost{0.27, 0.5, 0.5}
+                                           : Cost{0.44, 0.75, 1.0};
+  const bool big = tile == TH_TILE_256;
+  const int64_t work = (big ? tiles_of(d, kTile, kTile) : tiles_of(d, mid_rows(tile), mid_cols(tile))) * splits;
+  const int64_t room = big ? 256 : 512;  // workgroups the device holds
+  const double steps = ((d->k + splits - 1) / splits + 63) / 64;
+  const int64_t rounds = work / room, rest = work % room;
+  double t = 3.0 + rounds * (steps * c.pair + c.end);
+  if (rest > 0) t += steps * (rest <= 256 ? c.alone : c.pair) + c.end;
+  if (splits > 1 || (big && (d->flags & TH_GEMM_ACCUMULATE)))
+    t += 3.0 + 8.0 * splits * std::max(1, d->batch) * (double)d->m * d->n / 8e6;
+  return t;
+}
+
+// Where the library chooses the tile: the kernel, and unless the caller
+// names them the parts of K (at least 256 deep), with the least estimate
+// among the 256 x 256 kernel (parts as it splits by itself) and the middle
+// tiles, where they take the product; else the general kernel.  The middle
+// tiles take what the 256 x 256 kernel takes, fused epilogues included, which
+// then run in the fold of the parts.
+static int choose_tile(const th_gemm_desc* d, int* splits) {
+  const bool big = tile_kernel_takes(d), mid = d->epilogue == TH_EPI_STORE ? mid_takes(d) : big;
+  *splits = d->splits > 0 ? d->splits : 1;
+  if (!big && !mid) return TH_TILE_GENERAL;
+  int best = TH_TILE_GENERAL;
+  double least = INFINITY;
+  auto consider = [&](int tile, int s) {
+    const double t = estimate(d, tile, s);
+    if (t < least) least = t, best = tile, *splits = s;
+  };
+  const int asked = d->splits;
+  if (big) {
+    const int s = asked > 0 ? asked : auto_splits(d, TH_TILE_256);
+    // An fp32 result with a bias stays refused where the 256 x 256 tiles fill the device.
+    if (d->c_dtype == TH_F32 && d->bias && tiles_of(d, kTile, kTile) * s >= 128) return *splits = s, TH_TILE_256;
+    consider(TH_TILE_256, s);
   }
-  return TH_TILE_GENERAL;
+  if (mid)
+    for (int t : {TH_TILE_128X128, TH_TILE_64X128, TH_TILE_128X64, TH_TILE_64X64})
+      for (int s = 1; s <= 16 && (s == 1 || (asked == 0 && d->k / s >= 256)); ++s) consider(t, asked > 0 ? asked : s);
+  return best;
 }
 
 static int build_tile256(const th_gemm_desc* d, th_launch** out);
-static int build_mid(const th_gemm_desc* d, int tile, th_launch** out);
+static int build_mid(const th_gemm_desc* d, int tile, int splits, th_launch** out);
+
+// What a fused epilogue needs, on whichever kernel.
+static int check_epilogue(const th_gemm_desc* d) {
+  const int epi = d->epilogue;
+  if (epi == TH_EPI_STORE) return TH_OK;
+  TH_REQUIRE(d->c_dtype == TH_BF16, "th_build_gemm: fused epilogues write bf16");
+  TH_REQUIRE(!d->bias || aligned(d->bias, 8), "th_build_gemm: bias must be 8-byte aligned");
+  TH_REQUIRE(d->splits <= 1, "th_build_gemm: only a plain product splits K");
+  if (epi == TH_EPI_GELU)
+    TH_REQUIRE(d->aux_out && d->bias && aligned(d->aux_out, 8), "th_build_gemm: GELU needs bias and aux_out");
+  if (epi == TH_EPI_SQUARE_LOSS)
+    TH_REQUIRE(d->bias && d->loss && d->row_sums, "th_build_gemm: the square loss needs bias, loss, row_sums");
+  if (epi == TH_EPI_GELU_BACKWARD)
+    TH_REQUIRE(d->aux && d->row_sums && d->aux_ld >= d->m && d->aux_ld % 4 == 0 && aligned(d->aux, 8),
+               "th_build_gemm: the GELU backward needs aux (8-byte aligned, ld >= m, ld % 4 == 0) and row_sums");
+  return TH_OK;
+}
+
 static int build_bf16x3(const th_gemm_desc* d, th_launch** out);
 
 extern "C" int th_build_gemm(const th_gemm_desc* d, th_launch** out) {
@@ -217,7 +286,8 @@ extern "C" int th_build_gemm(const th_gemm_desc* d, th_launch** out) {
   TH_REQUIRE(d->tile >= TH_TILE_AUTO && d->tile <= TH_TILE_GENERAL, "th_build_gemm: unknown tile");
   TH_REQUIRE(d->splits >= 0, "th_build_gemm: splits must be >= 0");
   if (d->flags & TH_GEMM_BF16X3) return build_bf16x3(d, out);
-  const int tile = d->tile == TH_TILE_AUTO ? choose_tile(d) : d->tile;
+  int splits = 0;
+  const int tile = d->tile == TH_TILE_AUTO ? choose_tile(d, &splits) : d->tile;
   if (tile == TH_TILE_GENERAL) return th::build_gemm_general(d, out);
   if (tile == TH_TILE_256) {
     TH_REQUIRE(tile_kernel_takes(d),
@@ -225,10 +295,14 @@ extern "C" int th_build_gemm(const th_gemm_desc* d, th_launch** out) {
                "and the other strides multiples of 8 and 16-byte aligned operands");
     return build_tile256(d, out);
   }
+  if (d->tile == TH_TILE_AUTO) {
+    if (int r = check_epilogue(d)) return r;
+    return build_mid(d, tile, splits, out);
+  }
   TH_REQUIRE(mid_takes(d),
              "th_build_gemm: the middle tiles take bf16 or fp16 factors with a unit stride on each operand, the other "
              "strides multiples of 8, 16-byte aligned operands, TH_EPI_STORE and a result of the factors' type or fp32");
-  return build_mid(d, tile, out);
+  return build_mid(d, tile, d->splits > 0 ? d->splits : auto_splits(d, tile), out);
 }
 
 static int build_tile256(const th_gemm_desc* d, th_launch** out) {
@@ -238,18 +312,9 @@ static int build_tile256(const th_gemm_desc* d, th_launch** out) {
   const int epi = d->epilogue;
   const int la = d->a_k == 1 ? kK : kMN;
   const int lb = d->b_k == 1 ? kK : kMN;
-  TH_REQUIRE(d->c_dtype == TH_BF16 || (d->c_dtype == TH_F32 && epi == TH_EPI_STORE),
-             "th_build_gemm: fused epilogues write bf16");
+  if (int r = check_epilogue(d)) return r;
   TH_REQUIRE(!d->bias || aligned(d->bias, 8), "th_build_gemm: bias must be 8-byte aligned");
   TH_REQUIRE(!(d->c_dtype == TH_F32 && d->bias), "th_build_gemm: an fp32 result takes no bias");
-  if (epi == TH_EPI_GELU)
-    TH_REQUIRE(d->aux_out && d->bias && aligned(d->aux_out, 8), "th_build_gemm: GELU needs bias and aux_out");
-  if (epi == TH_EPI_SQUARE_LOSS)
-    TH_REQUIRE(d->bias && d->loss && d->row_sums, "th_build_gemm: the square loss needs bias, loss, row_sums");
-  if (epi == TH_EPI_GELU_BACKWARD)
-    TH_REQUIRE(d->aux && d->row_sums && d->aux_ld >= M && d->aux_ld % 4 == 0 && aligned(d->aux, 8),
-               "th_build_gemm: the GELU backward needs aux (8-byte aligned, ld >= m, ld % 4 == 0) and row_sums");
-
   const int tiles_m = (M + kTile - 1) / kTile, tiles_n = (N + kTile - 1) / kTile;
   // K split over parts (each a multiple of 64 deep) where asked, or where the
   // tiles alone would leave most CUs idle.
@@ -263,12 +328,9 @@ static int build_tile256(const th_gemm_desc* d, th_launch** out) {
   TH_REQUIRE(splits <= 65535 && batch <= 65535, "th_build_gemm: grid too large");
   // Parts and what is added go through an fp32 workspace and a second launch.
   const bool staged = splits > 1 || accumulate;
-  // Interior tiles read through 32-bit buffer offsets: operands past 2 GiB
-  // take the bounds-checked kernel, which addresses with 64-bit pointers.
-  const int64_t a_bytes = 2 * (la == kK ? (int64_t)(M - 1) * d->a_m + K : (int64_t)(K - 1) * d->a_k + M);
-  const int64_t b_bytes = 2 * (lb == kK ? (int64_t)(N - 1) * d->b_n + K : (int64_t)(K - 1) * d->b_k + N);
-  const bool check = (M % kTile) || (N % kTile) || (K % kDepth) || (ksplit % kDepth) || a_bytes > 0x7fffffff ||
-                     b_bytes > 0x7fffffff;
+  // Ragged tiles and operands past 2 GiB take the bounds-checked kernel,
+  // which addresses with 64-bit pointers.
+  const bool check = !interior_256(d) || ksplit % kDepth;
   const void* fn = nullptr;
   const char* name = "";
   switch (epi) {
@@ -333,28 +395,11 @@ static int build_tile256(const th_gemm_desc* d, th_launch** out) {
   for (int v : {0, 1, 2}) b.align(v, 16);
   for (int v : {3, 4, 5}) b.align(v, 8);
   if (staged) {
-    ReduceArgs ra{nullptr, d->c, static_cast<const uint16_t*>(d->bias),
-                  accumulate ? d->d : nullptr, d->c_ld, d->c_batch, d->d_ld ? d->d_ld : d->c_ld,
-                  d->d_ld ? d->d_batch : d->c_batch, M, N, splits, d->c_dtype};
-    int kr = b.kernel((const void*)sum_splits, "sum_splits", dim3((unsigned)((mn + 255) / 256), batch), dim3(256), 0,
-                      ra);
-    b.ref(2, kr, TH_OFFSET(ReduceArgs, c));
-    b.ref(3, kr, TH_OFFSET(ReduceArgs, bias));
-    b.ref(8, kr, TH_OFFSET(ReduceArgs, d));
-    b.ws_ref(kr, TH_OFFSET(ReduceArgs, ws), at_parts);
+    MidArgs f{};
+    f.part_ld = M, f.part_split = mn, f.part_batch = (int64_t)splits * mn, f.splits = splits;
+    add_fold(b, d, f, at_parts);
   }
-  if (sums) {
-    RowSumArgs rs{nullptr, static_cast<uint16_t*>(d->row_sums), M, 2 * tiles_n};
-    int k2 = b.kernel((const void*)sum_parts, "sum_parts", dim3((M + 255) / 256), dim3(256), 0, rs);
-    b.ref(6, k2, TH_OFFSET(RowSumArgs, out));
-    b.ws_ref(k2, TH_OFFSET(RowSumArgs, partial), at_sums);
-  }
-  if (epi == TH_EPI_SQUARE_LOSS) {
-    LossArgs ls{nullptr, d->loss, 4 * blocks};
-    int k3 = b.kernel((const void*)sum_loss, "sum_loss", dim3(1), dim3(256), 0, ls);
-    b.ref(7, k3, TH_OFFSET(LossArgs, loss));
-    b.ws_ref(k3, TH_OFFSET(LossArgs, partial), at_sums + (uint64_t)2 * tiles_n * M * sizeof(float));
-  }
+  if (sums) add_sums(b, d, at_sums, 2 * tiles_n, at_sums + (uint64_t)2 * tiles_n * M * sizeof(float), 4 * blocks);
   const double mm = M, nn = N, kk = K, bb = batch;
   const double cbytes = d->c_dtype == TH_F32 ? 4 : 2;
   double bytes = bb * (2.0 * (mm * kk + kk * nn) + cbytes * mm * nn * (accumulate ? 2 : 1));
@@ -364,74 +409,98 @@ static int build_tile256(const th_gemm_desc* d, th_launch** out) {
   return TH_OK;
 }
 
-// The middle tiles: one launch of the tile kernel, and for parts of K a
-// second that sums them (with the bias and D) into the result.
-static int build_mid(const th_gemm_desc* d, int tile, th_launch** out) {
+// The middle tiles: one launch of the tile kernel, for parts of K a second
+// that folds them, and for an epilogue with folds a last one that ends them.
+static int build_mid(const th_gemm_desc* d, int tile, int splits, th_launch** out) {
   const int M = d->m, N = d->n, K = d->k;
   const int batch = d->batch > 0 ? d->batch : 1;
   const bool accumulate = (d->flags & TH_GEMM_ACCUMULATE) != 0;
   const bool f16 = (d->flags & TH_GEMM_F16_FACTORS) != 0;
   int bm = 0, bn = 0, lds = 0;
-  const void* fn = mid_kernel(tile, f16, d->a_k == 1, d->b_k == 1, &bm, &bn, &lds);
+  const bool a_kc = d->a_k == 1, b_kc = d->b_k == 1;
+  const void* fn = mid_kernel(tile, f16, a_kc, b_kc, &bm, &bn, &lds);
   TH_REQUIRE(fn != nullptr, "th_build_gemm: unknown tile");
+  TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
   const int64_t tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn;
   TH_REQUIRE(tiles_m * tiles_n <= 0x7fffffff, "th_build_gemm: grid too large");
-  int splits = d->splits > 0 ? d->splits : auto_splits(d, tile);
   int ksplit = K;
   if (splits > 1) {
-    ksplit = ((K + splits - 1) / splits + 31) / 32 * 32;
+    ksplit = ((K + splits - 1) / splits + kMidStep - 1) / kMidStep * kMidStep;
     splits = (K + ksplit - 1) / ksplit;
   }
   TH_REQUIRE(splits <= 65535 && batch <= 65535, "th_build_gemm: grid too large");
   const bool staged = splits > 1;
-  const int64_t mn = (int64_t)M * N;
+  const bool sums = d->epilogue >= TH_EPI_SQUARE_LOSS;
   th::Builder b("gemm_mid", 9);
   MidArgs g{};
   g.a = static_cast<const uint16_t*>(d->a);
   g.b = static_cast<const uint16_t*>(d->b);
   g.a_m = d->a_m, g.a_k = d->a_k, g.a_batch = d->a_batch;
   g.b_k = d->b_k, g.b_n = d->b_n, g.b_batch = d->b_batch;
-  g.m = M, g.n = N, g.k = K, g.ksplit = ksplit, g.tiles_m = (int32_t)tiles_m;
-  uint64_t at_parts = 0;
+  g.m = M, g.n = N, g.k = K, g.ksplit = ksplit, g.splits = splits;
+  g.tiles_m = (int32_t)tiles_m, g.tiles_n = (int32_t)tiles_n, g.epilogue = d->epilogue;
+  // Direct loads take 16-byte chunks that lie inside a row or outside all of
+  // them, at 32-bit byte offsets.
+  const int64_t a_bytes = 2 * (a_kc ? (int64_t)(M - 1) * d->a_m + K : (int64_t)(K - 1) * d->a_k + M);
+  const int64_t b_bytes = 2 * (b_kc ? (int64_t)(N - 1) * d->b_n + K : (int64_t)(K - 1) * d->b_k + N);
+  g.direct = (a_kc || M % 8 == 0) && (b_kc || N % 8 == 0) && a_bytes <= 0x7fffffff && b_bytes <= 0x7fffffff &&
+             d->a_m >= 0 && d->a_k >= 0 && d->b_n >= 0 && d->b_k >= 0;
+  uint64_t at_parts = 0, at_rows = 0, at_loss = 0;
   if (staged) {
-    // Each part's fp32 sums, [batch][part][m x n] column-major at ld m.
-    at_parts = b.workspace((uint64_t)batch * splits * mn * sizeof(float));
-    g.c = nullptr, g.c_ld = M, g.c_batch = (int64_t)splits * mn, g.c_split = mn, g.result = TH_F32;
+    // Each part's fp32 sums, [batch][part][n][m], m padded to 8.
+    g.part_ld = (M + 7) / 8 * 8, g.part_split = g.part_ld * N, g.part_batch = g.part_split * splits;
+    at_parts = b.workspace((uint64_t)batch * g.part_batch * sizeof(float));
   } else {
-    g.c = d->c, g.c_ld = d->c_ld, g.c_batch = d->c_batch, g.c_split = 0, g.result = d->c_dtype;
+    g.c = d->c, g.c_ld = d->c_ld, g.c_batch = d->c_batch, g.result = d->c_dtype;
     g.d = accumulate ? d->d : nullptr;
     g.d_ld = d->d_ld ? d->d_ld : d->c_ld;
     g.d_batch = d->d_ld ? d->d_batch : d->c_batch;
     g.bias = static_cast<const uint16_t*>(d->bias);
+    g.aux = static_cast<const uint16_t*>(d->aux), g.aux_ld = d->aux_ld;
+    g.aux_out = static_cast<uint16_t*>(d->aux_out);
   }
-  const char* name = staged ? "gemm_mid_parts_f32" : "gemm_mid";
-  int k = b.kernel(fn, name, dim3((unsigned)(tiles_m * tiles_n), splits, batch), dim3(256), (uint32_t)lds, g);
+  // Column blocks of row sums and workgroups of loss partials, as the kernel that finishes has them.
+  const int nb = staged ? (N + kFoldColumns - 1) / kFoldColumns : (int)tiles_n;
+  const int64_t blocks = staged ? (int64_t)((M + 127) / 128) * nb : tiles_m * tiles_n;
+  if (sums) {
+    at_rows = b.workspace((uint64_t)nb * M * sizeof(float));
+    at_loss = b.workspace((uint64_t)blocks * sizeof(float));
+  }
+  const char* name = staged ? "gemm_mid_parts_f32"
+                     : d->epilogue == TH_EPI_STORE       ? "gemm_mid"
+                     : d->epilogue == TH_EPI_GELU        ? "gemm_mid_gelu"
+                     : d->epilogue == TH_EPI_SQUARE_LOSS ? "gemm_mid_square_loss"
+                                                         : "gemm_mid_gelu_backward";
+  const int k = b.kernel(fn, name, dim3((unsigned)(tiles_m * tiles_n), splits, batch), dim3(256), (uint32_t)lds, g);
   b.ref(0, k, TH_OFFSET(MidArgs, a));
   b.ref(1, k, TH_OFFSET(MidArgs, b));
+  b.align(0, 16);
+  b.align(1, 16);
+  int last = k;
   if (staged) {
-    b.ws_ref(k, TH_OFFSET(MidArgs, c), at_parts);
+    b.ws_ref(k, TH_OFFSET(MidArgs, parts), at_parts);
+    last = add_fold(b, d, g, at_parts);
   } else {
     b.ref(2, k, TH_OFFSET(MidArgs, c));
     b.ref(3, k, TH_OFFSET(MidArgs, bias));
+    b.ref(4, k, TH_OFFSET(MidArgs, aux));
+    b.ref(5, k, TH_OFFSET(MidArgs, aux_out));
     b.ref(8, k, TH_OFFSET(MidArgs, d));
   }
-  b.align(0, 16);
-  b.align(1, 16);
-  if (staged) {
-    ReduceArgs ra{nullptr, d->c, static_cast<const uint16_t*>(d->bias),
-                  accumulate ? d->d : nullptr, d->c_ld, d->c_batch, d->d_ld ? d->d_ld : d->c_ld,
-                  d->d_ld ? d->d_batch : d->c_batch, M, N, splits, d->c_dtype};
-    int kr = b.kernel((const void*)sum_splits, "sum_splits", dim3((unsigned)((mn + 255) / 256), batch), dim3(256), 0,
-                      ra);
-    b.ref(2, kr, TH_OFFSET(ReduceArgs, c));
-    b.ref(3, kr, TH_OFFSET(ReduceArgs, bias));
-    b.ref(8, kr, TH_OFFSET(ReduceArgs, d));
-    b.ws_ref(kr, TH_OFFSET(ReduceArgs, ws), at_parts);
+  if (sums) {
+    b.ws_ref(last, TH_OFFSET(MidArgs, row_parts), at_rows);
+    b.ws_ref(last, TH_OFFSET(MidArgs, loss_parts), at_loss);
+    add_sums(b, d, at_rows, nb, at_loss, (int)blocks);
+  }
+  if (d->epilogue != TH_EPI_STORE) {  // as the 256 x 256 kernel asks of a fused product
+    b.align(2, 16);
+    for (int v : {3, 4, 5}) b.align(v, 8);
   }
   const double mm = M, nn = N, kk = K, bb = batch;
   const double cbytes = d->c_dtype == TH_F32 ? 4 : 2;
-  b.work(bb * (2.0 * (mm * kk + kk * nn) + cbytes * mm * nn * (accumulate ? 2 : 1)), 2.0 * bb * mm * nn * kk,
-         tiles_m * tiles_n * splits * batch);
+  double bytes = bb * (2.0 * (mm * kk + kk * nn) + cbytes * mm * nn * (accumulate ? 2 : 1));
+  if (d->epilogue == TH_EPI_GELU || d->epilogue == TH_EPI_GELU_BACKWARD) bytes += 2.0 * mm * nn;
+  b.work(bytes, 2.0 * bb * mm * nn * kk, tiles_m * tiles_n * splits * batch);
   *out = b.release();
   return TH_OK;
 }
@@ -545,7 +614,7 @@ int splits_used(const th_gemm_desc* d, int tile, int splits) {
   if (tile == TH_TILE_GENERAL) return 1;
   int s = splits > 0 ? splits : auto_splits(d, tile);
   if (s <= 1) return 1;
-  const int step = tile == TH_TILE_256 ? kDepth : 32;
+  const int step = tile == TH_TILE_256 ? kDepth : kMidStep;
   const int ks = ((d->k + s - 1) / s + step - 1) / step * step;
   return (d->k + ks - 1) / ks;
 }

@@ -133,6 +133,31 @@ def test_mlp_program_matches_oracle(target, batch, d_in, hidden, d_out):
         assert relative(g, r) < BF16_TOL, name
 
 
+@pytest.mark.parametrize("batch,d_in,hidden,d_out,kernels", [
+    (136, 4104, 72, 200, ["sum_splits", "square_loss"]),        # the GELU in the fold of parts of K = d_in
+    (128, 200, 4104, 136, ["gelu<", "sum_splits"]),             # the square loss and its sums there
+    (72, 136, 200, 4104, ["gelu<", "square_loss<", "sum_splits"]),  # the GELU backward, whose K is d_out, there
+    (8, 8, 8, 8, ["gelu<", "square_loss", "gelu_backward<"]), (1000, 264, 520, 392, ["gelu<"])])
+def test_mlp_epilogues_on_the_middle_tiles(target, batch, d_in, hidden, d_out, kernels):
+    """Fused products at sizes no tile divides: K past its whole steps of 64,
+    tiles cut by m and n, the epilogue and its row sums and loss in the tile's
+    own kernel or in the fold of the parts of K."""
+    import tempest_hip as th
+    announce("mlp middle tiles", batch, d_in, hidden, d_out)
+    W1, b1, W2, b2, x = _mlp_inputs(batch, d_in, hidden, d_out, 11)
+    args = [_col(a) for a in (W1, b1, W2, b2, x)]
+    comp = th.compile(th.programs.mlp(batch, d_in, hidden, d_out), target, *args)
+    said = " ".join(l.describe() for l in comp.executable.launches)
+    assert "gemm_bf16" not in said and all(k in said for k in kernels), said
+    loss, dW1, db1, dW2, db2, dx = comp(*args)
+    ref = interpret.mlp_grad(W1, b1, W2, b2, x)
+    assert abs(loss - ref[0]) <= BF16_TOL * abs(ref[0])
+    got = [_julia(dW1, (hidden, d_in)), _julia(db1, (hidden,)), _julia(dW2, (d_out, hidden)),
+           _julia(db2, (d_out,)), _julia(dx, (d_in, batch))]
+    for name, g, r in zip(("dW1", "db1", "dW2", "db2", "dx"), got, ref[1:]):
+        assert relative(g, r) < BF16_TOL, name
+
+
 def test_mlp_config3_full_size_against_fp32(target):
     """Config 3 at its size against torch in float32 on the same bf16 inputs
     (the floating-point reference of the same ops)."""
