@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "th_core.h"
 
@@ -180,14 +181,22 @@ __global__ __launch_bounds__(256) void gemm_general(GenGemmArgs p) {
 
 // ---- fp32 factors: 128 x 128 tiles, K split over parts ----------------------------
 // A workgroup of four waves takes a 128 x 128 tile of C, each wave 64 x 64 as
-// 2 x 2 blocks of v_mfma_f32_32x32x2_f32 (exact products, fp32 sums).  K
-// moves 16 at a time through LDS ([k][m] and [k][n] rows of 160 floats: the
-// two k rows a wave reads at once fall on different banks), the next slice
-// held in registers while the current one is multiplied.  Interior slices of
-// operands with a unit stride load 16 bytes a thread; edges and other
-// strides load element by element, bounds-checked.  K may be split over
-// parts (grid.y), each writing its fp32 sums to the launch's workspace, and a
-// second kernel adds the parts (in part order) and D.
+// 2 x 2 blocks.  The bf16 matrix cores multiply 16 times as fast as the fp32
+// ones, so each factor is split on its way into LDS into three bf16 parts (all
+// of fp32's 24 bits) and the six products of parts down to 2^-18 of a b, of
+// nine, are summed in fp32 (v_mfma_f32_32x32x16_bf16), the leading ones apart
+// from the others; what is left out is at most 2^-25 of each a b, under the
+// rounding of the sums.  Error against float64 (norm-wise, normal
+// factors), with fp32 products and so: 4096^3 1.1e-6 and 4.0e-7, 2000 x 1500 x
+// 1030 5.7e-7 and 1.9e-7, 256 x 256 x 8192 2.5e-7 and 1.6e-7; time 1289 and 800
+// to 860 us, 156 and 66, 32 and 21.  What bounds it now: of a step's 1.0 us (one
+// workgroup on a CU; 1.56 two) the products take 0.43, the rest is LDS traffic
+// and the wait at its barrier.  A tile whose sums are not finite, or with a row of values all
+// under 2^-90, is computed again on the fp32 matrix cores
+// (v_mfma_f32_32x32x2_f32), as every tile was before.
+// K moves 16 at a time through two LDS stages, the next two slices held in
+// registers (SplitOp).  K may be split over parts (grid.y), each writing its fp32 sums to the
+// launch's workspace, and a second kernel adds the parts (in part order) and D.
 
 constexpr int kFT = 128;        // C tile
 constexpr int kFK = 16;         // K per step
@@ -208,6 +217,17 @@ struct F32GemmArgs {
 };
 
 typedef float f32x16g __attribute__((ext_vector_type(16)));
+typedef float f32x2g __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2g __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8g __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4g __attribute__((ext_vector_type(4)));
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+typedef uint32_t u32x2g __attribute__((ext_vector_type(2)));
+typedef uint16_t u16x2g __attribute__((ext_vector_type(2)));
+// 16-byte pieces of a stage: operand, part, half of 16 k, row; the halves 128
+// bytes apart modulo the banks, so that quads of both halves write at once.
+constexpr int kSplitHalf = kFT + 8;
+constexpr int kSplitStage = 2 * 3 * 2 * kSplitHalf;
 
 // A's 128 x 16 slice at (m0, k0) into LDS As[k][m]: eight values a thread.
 __device__ __forceinline__ void f32_load_a(const F32GemmArgs& p, const float* a, int m0, int k0, int kend,
@@ -299,18 +319,15 @@ __device__ __forceinline__ void f32_store_b(const F32GemmArgs& p, float* Bs, con
   }
 }
 
-__global__ __launch_bounds__(256, 2) void gemm_f32(F32GemmArgs p) {
-  __shared__ __attribute__((aligned(16))) float As[2][kFK * kFRow];
-  __shared__ __attribute__((aligned(16))) float Bs[2][kFK * kFRow];
-  const int tiles_m = (p.m + kFT - 1) / kFT;
-  const int m0 = (blockIdx.x % tiles_m) * kFT, n0 = (blockIdx.x / tiles_m) * kFT;
-  const int part = blockIdx.y, z = blockIdx.z;
-  const int kbeg = part * p.ksplit, kend = min(p.k, kbeg + p.ksplit);
-  const float* a = p.a + z * p.a_batch;
-  const float* b = p.b + z * p.b_batch;
+// The sweep in full precision on the fp32 matrix cores: what gemm_f32 falls
+// back on.
+__device__ __forceinline__ void f32_sweep(const F32GemmArgs& p, const float* a, const float* b, int m0, int n0,
+                                          int kbeg, int kend, float* lds, f32x16g (&acc)[2][2]) {
+  float* As = lds;  // two stages each
+  float* Bs = lds + 2 * kFK * kFRow;
+  constexpr int kStage = kFK * kFRow;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int wm = (wave / 2) * 64, wn = (wave % 2) * 64;
-  f32x16g acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -318,8 +335,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32(F32GemmArgs p) {
   f32x4 ra[2], rb[2];
   f32_load_a(p, a, m0, kbeg, kend, ra);
   f32_load_b(p, b, n0, kbeg, kend, rb);
-  f32_store_a(p, As[0], ra);
-  f32_store_b(p, Bs[0], rb);
+  f32_store_a(p, As, ra);
+  f32_store_b(p, Bs, rb);
   __syncthreads();
   const int steps = (kend - kbeg + kFK - 1) / kFK;
   for (int st = 0; st < steps; ++st) {
@@ -331,8 +348,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32(F32GemmArgs p) {
     }
     // v_mfma_f32_32x32x2_f32: lane l gives A(row l % 32, k l / 32) and
     // B(k l / 32, column l % 32).
-    const float* A = As[cur];
-    const float* B = Bs[cur];
+    const float* A = As + cur * kStage;
+    const float* B = Bs + cur * kStage;
 #pragma unroll
     for (int kk = 0; kk < kFK; kk += 2) {
       const int kr = kk + lane / 32;
@@ -347,11 +364,205 @@ __global__ __launch_bounds__(256, 2) void gemm_f32(F32GemmArgs p) {
         for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
     }
     if (st + 1 < steps) {
-      f32_store_a(p, As[cur ^ 1], ra);
-      f32_store_b(p, Bs[cur ^ 1], rb);
+      f32_store_a(p, As + (cur ^ 1) * kStage, ra);
+      f32_store_b(p, Bs + (cur ^ 1) * kStage, rb);
     }
     __syncthreads();
   }
+}
+
+// One operand's 128 x 16 slice a step: eight values a thread, as two quads of
+// consecutive k.  KC (k the smaller stride): quad q is row t / 4 + 64 q, k 4 (t
+// % 4) + (0..3), 64 bytes of a row by four lanes; else row t % 128, k 8 (t /
+// 128) + 4 q + (0..3), a lane a row, so that a load covers 64 rows side by side.
+template <bool KC>
+struct SplitOp {
+  const float* at[2];
+  int64_t s_k;
+  int k[2];
+  bool unit;
+  uint32_t to[2];   // the quads' places in a stage, in 8-byte units
+  u16x2g most[2];   // the largest leading parts of each quad so far, as bf16 bits
+
+  __device__ __forceinline__ void init(const float* base, int64_t s_r, int64_t s_k_, int row0, int rows) {
+    const int t = threadIdx.x;
+    s_k = s_k_, unit = s_k_ == 1;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int lr = KC ? t / 4 + 64 * q : t % kFT;
+      k[q] = KC ? 4 * (t % 4) : 8 * (t / kFT) + 4 * q;
+      at[q] = base + (int64_t)min(row0 + lr, rows - 1) * s_r + (int64_t)k[q] * s_k;
+      to[q] = 2 * (k[q] / 8 * kSplitHalf + lr) + k[q] / 4 % 2;
+      most[q] = u16x2g{0, 0};
+    }
+  }
+  // The slice at k0, whole (nothing but loads, so that none waits for
+  // another) or cut at kend (zeros past it); rows past the last read it again.
+  __device__ __forceinline__ void load(int k0, f32x4 (&x)[2]) const {
+    const int64_t step = (int64_t)k0 * s_k;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const float* from = at[q] + step;
+      if (KC && unit) {
+        x[q] = *reinterpret_cast<const f32x4_any*>(from);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[q][i] = from[i * s_k];
+      }
+    }
+  }
+  __device__ __forceinline__ void load_cut(int k0, int kend, f32x4 (&x)[2]) const {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[q][i] = k0 + k[q] + i < kend ? at[q][(int64_t)(k0 + i) * s_k] : 0.0f;
+  }
+  // x = part 0 + part 1 + part 2 in bf16 (8 bits each, rounded to nearest:
+  // what is left is at most 2^-27 of x).
+  __device__ __forceinline__ void split(const f32x4 (&x)[2], u32x2g (&w)[2][3]) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float u = x[q][2 * i], v = x[q][2 * i + 1];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+          w[q][s][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2g{u, v}, bf16x2g));
+          if (s == 2) break;
+          u -= __uint_as_float(w[q][s][i] << 16), v -= __uint_as_float(w[q][s][i] & 0xffff0000u);
+        }
+        most[q] = __builtin_elementwise_max(most[q], __builtin_bit_cast(u16x2g, w[q][0][i] & 0x7fff7fffu));
+      }
+  }
+  __device__ __forceinline__ void store(u32x2g* stage, const u32x2g (&w)[2][3]) const {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int s = 0; s < 3; ++s) stage[to[q] + s * 4 * kSplitHalf] = w[q][s];
+  }
+  // Whether a quad's values were all under 2^-90, not all zero.
+  __device__ __forceinline__ bool tiny() const {
+    constexpr int limit = (127 - 90) << 7;
+    bool t = false;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int x = max((int)most[q][0], (int)most[q][1]);
+      t |= x > 0 && x < limit;
+    }
+    return t;
+  }
+};
+
+template <bool AKC, bool BKC>
+__global__ __launch_bounds__(256, 2) void gemm_f32(F32GemmArgs p) {
+  // [stage][operand][part][half of 16 k][row]: 16 bytes, eight k of a row; a
+  // fragment is 32 rows of each half, read whole lines.
+  __shared__ __attribute__((aligned(16))) u32x4g lds[2 * kSplitStage];
+  static_assert(sizeof(lds) >= 4 * kFK * kFRow * sizeof(float), "the fp32 sweep's stages fit");
+  const int tiles_m = (p.m + kFT - 1) / kFT;
+  const int m0 = (blockIdx.x % tiles_m) * kFT, n0 = (blockIdx.x / tiles_m) * kFT;
+  const int part = blockIdx.y, z = blockIdx.z;
+  const int kbeg = part * p.ksplit, kend = min(p.k, kbeg + p.ksplit);
+  const float* a = p.a + z * p.a_batch;
+  const float* b = p.b + z * p.b_batch;
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int wm = (wave / 2) * 64, wn = (wave % 2) * 64;
+  f32x16g acc[2][2], low[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16g{}, low[i][j] = f32x16g{};
+  SplitOp<AKC> A;
+  SplitOp<BKC> B;
+  A.init(a, p.a_m, p.a_k, m0, p.m);
+  B.init(b, p.b_n, p.b_k, n0, p.n);
+  // Two slices in flight in registers: a slice's loads lead its split by a
+  // whole step's products.
+  f32x4 a0[2], a1[2], b0[2], b1[2];
+  auto stage = [&](int st) { return lds + (st & 1) * kSplitStage; };
+  const int steps = (kend - kbeg + kFK - 1) / kFK, whole = (kend - kbeg) / kFK;
+  auto load = [&](int st, f32x4 (&x)[2], f32x4 (&y)[2]) {
+    const int k0 = kbeg + st * kFK;
+    if (st < whole) {
+      A.load(k0, x);
+      B.load(k0, y);
+    } else {
+      A.load_cut(k0, kend, x);
+      B.load_cut(k0, kend, y);
+    }
+  };
+  // Step st's products; slice st + 1 (in x, y) goes to the other stage, slice
+  // st + 2's loads are issued into xn, yn.  The split's vector work sits
+  // between the products: one wave's products leave the vector ALU idle.
+  auto step = [&](int st, const f32x4 (&x)[2], const f32x4 (&y)[2], f32x4 (&xn)[2], f32x4 (&yn)[2]) {
+    if (st + 2 < steps) load(st + 2, xn, yn);
+    const u32x4g* at = stage(st) + (lane / 32) * kSplitHalf + lane % 32;
+    bf16x8g fa[3][2], fb[3][2];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        fa[s][i] = __builtin_bit_cast(bf16x8g, at[s * 2 * kSplitHalf + wm + 32 * i]);
+        fb[s][i] = __builtin_bit_cast(bf16x8g, at[(3 + s) * 2 * kSplitHalf + wn + 32 * i]);
+      }
+    u32x2g wa[2][3], wb[2][3];
+    A.split(x, wa);
+    B.split(y, wb);
+    // The parts' products down to 2^-18 of a b, the leading one in sums of its own.
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      constexpr int pa[6] = {0, 1, 0, 2, 1, 0}, pb[6] = {0, 0, 1, 0, 1, 2};
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          f32x16g& to = q == 0 ? acc[i][j] : low[i][j];
+          to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[pa[q]][i], fb[pb[q]][j], to, 0, 0, 0);
+        }
+    }
+    u32x2g* next = reinterpret_cast<u32x2g*>(stage(st + 1));
+    A.store(next, wa);  // past the last step: a stage nothing reads again
+    B.store(next + 6 * 2 * kSplitHalf, wb);
+#pragma unroll
+    for (int q = 0; q < 24; ++q) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product
+      __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // five vector instructions
+    }
+    __syncthreads();
+  };
+  {
+    u32x2g w[2][3];
+    load(0, a0, b0);
+    if (steps > 1) {
+      load(1, a1, b1);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) a1[q] = b1[q] = f32x4{};
+    }
+    A.split(a0, w);
+    A.store(reinterpret_cast<u32x2g*>(stage(0)), w);
+    B.split(b0, w);
+    B.store(reinterpret_cast<u32x2g*>(stage(0)) + 6 * 2 * kSplitHalf, w);
+  }
+  __syncthreads();
+  for (int st = 0; st < steps; st += 2) {
+    step(st, a1, b1, a0, b0);
+    if (st + 1 < steps) step(st + 1, a0, b0, a1, b1);
+  }
+  // Sums that are not finite (an infinity or a NaN among the factors, whose
+  // parts are NaN; or an overflow), and rows whose every value is so small
+  // that its lower parts fall under bf16's normal range: the tile again in
+  // full precision.
+  bool again = A.tiny() || B.tiny();
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      acc[i][j] += low[i][j];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) again |= !(fabsf(acc[i][j][e]) < INFINITY);
+    }
+  if (__syncthreads_or(again)) f32_sweep(p, a, b, m0, n0, kbeg, kend, reinterpret_cast<float*>(lds), acc);
   // Lane l holds C(rows 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32) of each block.
   float* c = p.c + z * p.c_batch + part * p.c_part;
   const float* d = p.d ? p.d + z * p.d_batch : nullptr;
@@ -363,15 +574,16 @@ __global__ __launch_bounds__(256, 2) void gemm_f32(F32GemmArgs p) {
       if (n >= p.n) continue;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int mb = m0 + wm + 32 * i + 8 * q + 4 * (lane / 32);
+        const int m = m0 + wm + 32 * i + 8 * q + 4 * (lane / 32);
+        f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        const int64_t at = (int64_t)m + (int64_t)n * p.c_ld, at_d = (int64_t)m + (int64_t)n * p.d_ld;
+        if (m + 4 <= p.m) {
+          if (d) v += *reinterpret_cast<const f32x4_any*>(d + at_d);
+          *reinterpret_cast<f32x4_any*>(c + at) = v;
+        } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int m = mb + e;
-          if (m < p.m) {
-            float v = acc[i][j][4 * q + e];
-            if (d) v += d[(int64_t)m + (int64_t)n * p.d_ld];
-            c[(int64_t)m + (int64_t)n * p.c_ld] = v;
-          }
+          for (int e = 0; e < 4; ++e)
+            if (m + e < p.m) c[at + e] = d ? v[e] + d[at_d + e] : v[e];
         }
       }
     }
@@ -518,14 +730,17 @@ int build_gemm_general(const th_gemm_desc* d, th_launch** out) {
   return TH_OK;
 }
 
-// The parts of K an fp32 product takes when the caller leaves them: enough
-// for about 256 workgroups where the tiles alone give fewer than 128, each
-// part at least 32 deep (two steps: 256 x 256 x 8192 takes 64 parts, 256 x
-// 512 x 384 twelve).
+// The parts of K an fp32 product takes when the caller leaves them: as many as
+// keep its workgroups within the 512 the device holds, where the tiles alone
+// are fewer than 256, each part at least 256 deep (128 where the tiles are under
+// a quarter of the device).  In one part and as chosen: 2000 x 1500 x 1030 (192
+// tiles) 72 us and, in two, 66; 3500 x 640 x 2600 (140) 148 and 91 in three;
+// 1100 x 1000 x 3000 (72) 172 and 63 to 73 in six or seven; 1500 x 1300 x 400
+// (132) 26 in one, 30 in two.
 static int f32_splits(const th_gemm_desc* d) {
   const int64_t tiles = (int64_t)((d->m + kFT - 1) / kFT) * ((d->n + kFT - 1) / kFT) * std::max(1, d->batch);
-  if (tiles >= 128 || d->k < 64) return 1;
-  return (int)std::max<int64_t>(1, std::min<int64_t>((256 + tiles - 1) / tiles, d->k / 32));
+  if (tiles >= 256) return 1;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(512 / tiles, d->k / (tiles < 64 ? 128 : 256)));
 }
 
 static bool f32_vector(const void* base, int64_t unit_other, int64_t other, int64_t batch_stride, int n_batch) {
@@ -577,7 +792,10 @@ static int build_gemm_f32(const th_gemm_desc* d, th_launch** out) {
     a.d = acc ? static_cast<const float*>(d->d) : nullptr;
     a.d_ld = d->d_ld ? d->d_ld : d->c_ld, a.d_batch = d->d_ld ? d->d_batch : d->c_batch;
   }
-  int k = b.kernel((const void*)gemm_f32, "gemm_f32_128x128", dim3((unsigned)tiles, splits, batch), dim3(256), 0, a);
+  const bool akc = d->a_k <= d->a_m, bkc = d->b_k <= d->b_n;
+  const void* fn = akc ? (bkc ? (const void*)gemm_f32<true, true> : (const void*)gemm_f32<true, false>)
+                       : (bkc ? (const void*)gemm_f32<false, true> : (const void*)gemm_f32<false, false>);
+  int k = b.kernel(fn, "gemm_f32_128x128", dim3((unsigned)tiles, splits, batch), dim3(256), 0, a);
   b.ref(0, k, TH_OFFSET(F32GemmArgs, a));
   b.ref(1, k, TH_OFFSET(F32GemmArgs, b));
   if (staged) {

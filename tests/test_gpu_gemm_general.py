@@ -384,3 +384,60 @@ def test_bf16x3_tuned_and_refusals(target):
         L.gemm(*args, c_dtype=L.BF16, factors=L.F32, bf16x3=True)
     with pytest.raises(HIPError, match="bf16x3"):
         L.gemm(*args, c_dtype=L.F32, factors=L.F32, bf16x3=True, tile=L.TILE_GENERAL)
+
+
+@pytest.mark.parametrize("a_kfast,b_kfast", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("k", [1, 15, 16, 17, 33, 257])
+def test_f32_split_factors_at_the_edges(target, a_kfast, b_kfast, k):
+    """The 128 x 128 kernel's slices of 16: one cut, one whole, one of each,
+    rows cut by the tile.  Each factor is carried in three bf16 parts (2^-27 of
+    it left out, and products of parts under 2^-26 of a b), the sums in fp32:
+    the error stays under the fp32 sums' own bound."""
+    announce("fp32 split factors", k, a_kfast, b_kfast)
+    A, B, ta, tb, st = _f32_operands(130, 200, k, a_kfast, b_kfast, k)
+    got, l = _run_f32(130, 200, k, ta, tb, st, splits=1)
+    assert "gemm_f32_128x128" in l.describe()
+    bound = np.abs(A[0]) @ np.abs(B[0]) * (k + 8) * 2.0 ** -24
+    assert np.all(np.abs(got[0] - A[0] @ B[0]) <= bound)
+
+
+def test_f32_split_factors_of_any_value(target):
+    """Whole numbers are exact; infinities and NaN give what fp32 products
+    give; values near fp32's largest and rows of values under bf16's reach
+    (each computed again on the fp32 matrix cores) keep fp32's accuracy."""
+    announce("fp32 split factors values")
+    rng = np.random.default_rng(5)
+
+    def run(a, b):
+        ta, tb = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+        m, k, n = a.shape[0], a.shape[1], b.shape[1]
+        return _run_f32(m, n, k, ta, tb, {"a_m": k, "a_k": 1, "b_k": n, "b_n": 1, "a_batch": 0, "b_batch": 0},
+                        splits=1)[0][0]
+    f32 = np.float32
+    a = rng.integers(-2000, 2000, (130, 40)).astype(f32)
+    b = rng.integers(-100, 100, (40, 140)).astype(f32)
+    assert np.array_equal(run(a, b), a.astype(np.float64) @ b.astype(np.float64))
+    x, y = rng.standard_normal((130, 40)).astype(f32), rng.standard_normal((40, 140)).astype(f32)
+    for v in (np.inf, -np.inf, np.nan):
+        z = x.copy()
+        z[3, 7] = v
+        with np.errstate(invalid="ignore"):
+            want = z.astype(np.float64) @ y.astype(np.float64)
+        got = run(z, y)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+        keep = np.isfinite(want)
+        assert relative(got[keep], want[keep]) < TOL_F32
+    one = np.ones((40, 140), f32)  # infinity times a factor whose lower parts are zero is infinity
+    z = np.abs(x)
+    z[5, 0] = np.inf
+    assert np.all(np.isposinf(run(z, one)[5])) and np.all(np.isfinite(run(z, one)[6]))
+    big = x.copy()
+    big[:, 0] = 3.4e38  # rounds to infinity in bf16
+    small = y.copy()
+    small[0] *= 1e-3
+    assert relative(run(big, small), big.astype(np.float64) @ small.astype(np.float64)) < TOL_F32
+    for s in (1e-28, 1e-33, 1e-37):  # a whole row scaled down
+        z = x.copy()
+        z[9] *= f32(s)
+        want = z.astype(np.float64) @ y.astype(np.float64)
+        assert relative(run(z, y)[9], want[9]) < TOL_F32, s
