@@ -30,9 +30,7 @@
 // vector ALUs ran before): a first key per query and a key count per sequence.
 // A forward or dQ workgroup starts at its queries' least first key, a dK/dV
 // workgroup finds the span of queries that see any of its keys, so packed
-// documents cost their own pairs and not the sequence's; blocks are not
-// paired with their mirror (the work follows the documents), the last ones,
-// the longest without documents, go first.  The general kernels hold P and dS
+// documents cost their own pairs and not the sequence's.  The general kernels hold P and dS
 // in fp32, so here each is hi + lo in bf16 (2^-17 relative) and takes two
 // products, on operands that are bf16 already.  Rows may start at any element.
 // B2 H12 S2048 d64 in documents of about 256, forward + backward: 5981 us on
@@ -193,11 +191,11 @@ struct Stage {
 template <int D>
 constexpr int kTile = 64 * (D + 8);  // bf16 elements of a tile in LDS
 
-// Causal sweeps do less work for earlier query blocks (and later key
-// blocks): workgroup x takes blocks x and nb - 1 - x, so every workgroup
-// sweeps about the same number of tiles.
-__device__ __forceinline__ int passes(bool causal, int x, int nb) { return causal && 2 * x + 1 != nb ? 2 : 1; }
-__device__ __forceinline__ int block_of(int pass, int x, int nb) { return pass == 0 ? x : nb - 1 - x; }
+// The grid is (heads, batch, blocks): blocks slowest, so that under a causal
+// mask the longest sweeps start first and the short ones fill in behind them,
+// and, (heads x batch) a multiple of 8, a head's blocks share an XCD's L2.
+// (Before, a workgroup took a block and its mirror: even work, but half the
+// workgroups, and the chip half empty where they are few.)
 
 // ---- forward ---------------------------------------------------------------------
 
@@ -208,7 +206,7 @@ template <int D, bool M>
 __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const int b, const int split) {
   constexpr int NS = D / 16, NB = D / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-  const int h = blockIdx.y;
+  const int h = blockIdx.x;
   const int hk = h / (p.heads / p.kv_heads);
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
   const int q0 = qb * 128 + wave * 32, query = q0 + lr;
@@ -341,19 +339,9 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
 
 template <int D, bool M>
 __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void mfma_attn_fwd(MArgs p) {
-  if constexpr (M) {
-    fwd_block<D, true>(p, gridDim.x - 1 - blockIdx.x, blockIdx.z, -1);
-    return;
-  }
-  // Split: one part of one block; else a block and, causal, its mirror (one call site, inlined once).
   const bool split = p.nsplit > 1;
-  const int nb = (p.seq + 127) / 128;
-  const int npass = split ? 1 : passes(p.causal, blockIdx.x, nb);
-  for (int pass = 0; pass < npass; ++pass) {
-    if (pass > 0) __syncthreads();
-    fwd_block<D, false>(p, split ? blockIdx.x : block_of(pass, blockIdx.x, nb), split ? blockIdx.z / p.nsplit : blockIdx.z,
-                 split ? blockIdx.z % p.nsplit : -1);
-  }
+  const int z = gridDim.z - 1 - blockIdx.z;  // the last queries, the longest sweeps, first
+  fwd_block<D, M>(p, split ? z / p.nsplit : z, blockIdx.y, split ? z % p.nsplit : -1);
 }
 
 // The parts of a split forward combined: per (b, query, head) row, M = max
@@ -530,7 +518,7 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
   constexpr int kStats = M ? 192 : 128;
   // [stage][lse * log2e (64) | delta (64) | M: first keys, as ints (64)]
   float* stats = reinterpret_cast<float*>(lds + 4 * kTile<D>);
-  const int hk = blockIdx.y;
+  const int hk = blockIdx.x;
   const int group = p.heads / p.kv_heads;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
   const int kw0 = kblk * 128, key = kw0 + wave * 32 + lr;
@@ -683,19 +671,10 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
 
 template <int D, int DO, bool M>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void mfma_attn_dkdv(MArgs p) {
-  if constexpr (M) {
-    dkdv_block<D, DO, true>(p, blockIdx.x, 0, blockIdx.z, -1);
-    return;
-  }
   constexpr int halves = D / DO;
   const bool split = p.nsplit > 1;
-  const int nb = (p.kv_seq + 127) / 128, x = blockIdx.x / halves;
-  const int npass = split ? 1 : passes(p.causal, x, nb);
-  for (int pass = 0; pass < npass; ++pass) {
-    if (pass > 0) __syncthreads();
-    dkdv_block<D, DO, false>(p, split ? x : block_of(pass, x, nb), blockIdx.x % halves, split ? blockIdx.z / p.nsplit : blockIdx.z,
-                      split ? blockIdx.z % p.nsplit : -1);
-  }
+  const int z = blockIdx.z, x = split ? z / p.nsplit : z;  // the first keys, the longest sweeps, first
+  dkdv_block<D, DO, M>(p, x / halves, x % halves, blockIdx.y, split ? z % p.nsplit : -1);
 }
 
 // ---- backward: dQ ----------------------------------------------------------------------
@@ -709,7 +688,7 @@ template <int D, bool M>
 __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int b, const int split) {
   constexpr int NS = D / 16, NB = D / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-  const int h = blockIdx.y;
+  const int h = blockIdx.x;
   const int hk = h / (p.heads / p.kv_heads);
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
   const int q0 = qb * 128 + wave * 32, query = q0 + lr;
@@ -826,28 +805,12 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
 
 template <int D, bool M>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void mfma_attn_dq(MArgs p) {
-  if constexpr (M) {
-    dq_block<D, true>(p, gridDim.x - 1 - blockIdx.x, blockIdx.z, -1);
-    return;
-  }
   const bool split = p.nsplit > 1;
-  const int nb = (p.seq + 127) / 128;
-  const int npass = split ? 1 : passes(p.causal, blockIdx.x, nb);
-  for (int pass = 0; pass < npass; ++pass) {
-    if (pass > 0) __syncthreads();
-    dq_block<D, false>(p, split ? blockIdx.x : block_of(pass, blockIdx.x, nb), split ? blockIdx.z / p.nsplit : blockIdx.z,
-                split ? blockIdx.z % p.nsplit : -1);
-  }
+  const int z = gridDim.z - 1 - blockIdx.z;
+  dq_block<D, M>(p, split ? z / p.nsplit : z, blockIdx.y, split ? z % p.nsplit : -1);
 }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
-
-// Workgroups along a sequence of n positions in blocks of 128: causal ones
-// take a block and its mirror.
-unsigned blocks_of(int n, int causal) {
-  const unsigned nb = (unsigned)((n + 127) / 128);
-  return causal ? (nb + 1) / 2 : nb;
-}
 
 MArgs margs_of(const th_attention_desc* d) {
   MArgs a{};
@@ -887,9 +850,9 @@ int fwd_launch(const th_attention_desc* d, th_launch** out) {
   const int nqb = (d->seq + 127) / 128;
   const th::Split sp = th::split_of((int64_t)nqb * d->heads * d->batch, a.kv_seq);
   a.nsplit = sp.n, a.span = sp.span;
-  TH_REQUIRE((int64_t)d->batch * sp.n <= 65535, "attention: grid too large");
+  TH_REQUIRE((int64_t)nqb * sp.n <= 65535, "attention: grid too large");
   th::Builder b("attention_fwd_mfma", 7);
-  const dim3 grid = sp.n > 1 ? dim3(nqb, d->heads, d->batch * sp.n) : dim3(blocks_of(d->seq, d->causal), d->heads, d->batch);
+  const dim3 grid(d->heads, d->batch, nqb * sp.n);
   int k = b.kernel((const void*)mfma_attn_fwd<D, false>, D == 64 ? "mfma_attn_fwd_d64" : D == 128 ? "mfma_attn_fwd_d128"
                                                                                           : "mfma_attn_fwd_d256",
                    grid, dim3(256), (uint32_t)lds, a);
@@ -936,7 +899,7 @@ int bwd_launch(const th_attention_desc* d, th_launch** out) {
   const int nkb = (a.kv_seq + 127) / 128, nqb = (d->seq + 127) / 128;
   const th::Split skv = th::split_of((int64_t)nkb * (D / DO) * d->kv_heads * d->batch, d->seq);
   const th::Split sq = th::split_of((int64_t)nqb * d->heads * d->batch, a.kv_seq);
-  TH_REQUIRE((int64_t)d->batch * std::max(skv.n, sq.n) <= 65535, "attention: grid too large");
+  TH_REQUIRE((int64_t)nkb * (D / DO) * skv.n <= 65535 && (int64_t)nqb * sq.n <= 65535, "attention: grid too large");
   MArgs akv = a, aq = a;
   akv.nsplit = skv.n, akv.span = skv.span;
   aq.nsplit = sq.n, aq.span = sq.span;
@@ -944,9 +907,7 @@ int bwd_launch(const th_attention_desc* d, th_launch** out) {
   constexpr int kDeltaBlockRows = 4 * (64 / (D / 8)) * kDeltaRowsM;  // rows a workgroup
   int k0 = b.kernel((const void*)mfma_attn_delta<D>, "mfma_attn_delta",
                     dim3((unsigned)((rows + kDeltaBlockRows - 1) / kDeltaBlockRows)), dim3(256), 0, DeltaArgs{a, D});
-  const dim3 gkv = skv.n > 1 ? dim3(nkb * (D / DO), d->kv_heads, d->batch * skv.n)
-                             : dim3(blocks_of(a.kv_seq, d->causal) * (D / DO), d->kv_heads, d->batch);
-  const dim3 gq = sq.n > 1 ? dim3(nqb, d->heads, d->batch * sq.n) : dim3(blocks_of(d->seq, d->causal), d->heads, d->batch);
+  const dim3 gkv(d->kv_heads, d->batch, nkb * (D / DO) * skv.n), gq(d->heads, d->batch, nqb * sq.n);
   int k1 = b.kernel((const void*)mfma_attn_dkdv<D, DO, false>, D == 64 ? "mfma_attn_dkdv_d64" : D == 128 ? "mfma_attn_dkdv_d128"
                                                                                                : "mfma_attn_dkdv_d256",
                     gkv, dim3(256), (uint32_t)lds_dkdv, akv);
@@ -1005,7 +966,7 @@ int masked_fwd_launch(const th_attention_desc* d, th_launch** out) {
   TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   MArgs a = margs_of(d);
   th::Builder b("attention_fwd_mfma", 7);
-  const dim3 grid((d->seq + 127) / 128, d->heads, d->batch);
+  const dim3 grid(d->heads, d->batch, (d->seq + 127) / 128);
   const int k = b.kernel(fn, D == 64 ? "mfma_attn_fwd_masked_d64" : "mfma_attn_fwd_masked_d128", grid, dim3(256),
                          (uint32_t)lds, a);
   const size_t offs[7] = {TH_OFFSET(MArgs, q),   TH_OFFSET(MArgs, k),      TH_OFFSET(MArgs, v),
@@ -1032,7 +993,7 @@ int masked_bwd_launch(const th_attention_desc* d, th_launch** out) {
   constexpr int kDeltaBlockRows = 4 * (64 / (D / 8)) * kDeltaRowsM;
   const int k0 = b.kernel((const void*)mfma_attn_delta<D>, "mfma_attn_delta",
                           dim3((unsigned)((rows + kDeltaBlockRows - 1) / kDeltaBlockRows)), dim3(256), 0, DeltaArgs{a, D});
-  const dim3 gkv((a.kv_seq + 127) / 128, d->kv_heads, d->batch), gq((d->seq + 127) / 128, d->heads, d->batch);
+  const dim3 gkv(d->kv_heads, d->batch, (a.kv_seq + 127) / 128), gq(d->heads, d->batch, (d->seq + 127) / 128);
   const int k1 = b.kernel(f1, D == 64 ? "mfma_attn_dkdv_masked_d64" : "mfma_attn_dkdv_masked_d128", gkv, dim3(256),
                           (uint32_t)lds_dkdv, a);
   const int k2 = b.kernel(f2, D == 64 ? "mfma_attn_dq_masked_d64" : "mfma_attn_dq_masked_d128", gq, dim3(256),
@@ -1078,8 +1039,8 @@ bool mfma_attention_takes(const th_attention_desc* d) {
   for (int64_t s : {d->q_strides[0], d->q_strides[1], d->q_strides[2], d->k_strides[0], d->k_strides[1], d->k_strides[2]})
     if (s <= 0 || s % 8) return false;
   const int64_t kv = d->kv_seq > 0 ? d->kv_seq : d->seq;
-  return (d->seq + 127) / 128 <= 0x7fffffff && (kv + 127) / 128 * 2 <= 0x7fffffff && d->heads <= 65535 &&
-         d->batch <= 65535;
+  // (blocks of 128 positions along grid z, at most 8 parts or halves each)
+  return (d->seq + 127) / 128 <= 8191 && (kv + 127) / 128 <= 8191 && d->heads <= 65535 && d->batch <= 65535;
 }
 
 int build_attention_mfma_fwd(const th_attention_desc* d, th_launch** out) {
@@ -1104,8 +1065,9 @@ int build_attention_mfma_bwd(const th_attention_desc* d, th_launch** out) {
 // bf16 at head dims 64 and 128 under device-held masks, and rows of any
 // alignment and strides (descriptors the general kernels' checks passed).
 bool masked_attention_takes(const th_attention_desc* d) {
+  const int kv = d->kv_seq > 0 ? d->kv_seq : d->seq;
   return !(d->flags & TH_ATTN_F32) && (d->head_dim == 64 || d->head_dim == 128) &&
-         (int64_t)d->batch * d->seq * d->heads < 2147483648LL;
+         (int64_t)d->batch * d->seq * d->heads < 2147483648LL && (d->seq + 127) / 128 <= 65535 && (kv + 127) / 128 <= 65535;
 }
 
 int build_attention_masked_fwd(const th_attention_desc* d, th_launch** out) {
