@@ -100,6 +100,14 @@ __device__ __forceinline__ int first_of(const MArgs& p, int j, int b) {
   return p.starts ? p.starts[(int64_t)j + (int64_t)p.seq * b] - 1 : 0;
 }
 
+// The largest of x over the wave's lanes with a query (INT_MAX: none).
+__device__ __forceinline__ int most(int x) {
+  if (x == 0x7fffffff) x = 0;
+#pragma unroll
+  for (int i = 1; i < 64; i *= 2) x = max(x, __shfl_xor(x, i, 64));
+  return __builtin_amdgcn_readfirstlane(x);
+}
+
 // The least of x over the workgroup's 256 threads, through four ints of LDS;
 // a barrier on both sides.
 __device__ __forceinline__ int least(int x, int* at) {
@@ -209,7 +217,7 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
   const int h = blockIdx.x;
   const int hk = h / (p.heads / p.kv_heads);
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
-  const int q0 = qb * 128 + wave * 32, query = q0 + lr;
+  const int q0 = __builtin_amdgcn_readfirstlane(qb * 128 + wave * 32), query = q0 + lr;
   const uint16_t* qbase = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
   const uint16_t* kbase = p.k + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
   const uint16_t* vbase = p.v + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
@@ -230,6 +238,7 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
       k_lo = max(0, min(least(first, reinterpret_cast<int*>(lds + 4 * kTile<D>)), nk)) / 64 * 64;
     }
   }
+  const int last_first = M ? most(first) : 0;  // tiles from here on see no first key
   const int k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
   const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
   Stage<D> sk, sv;
@@ -254,7 +263,7 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
     for (int ks = 0; ks < NS; ++ks)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) s[kb] = mfma(frag_rows<D>(K(cur), 32 * kb, ks), qf[ks], s[kb]);
-    if (M || k0 + 64 > p.kv_seq || (p.causal && k0 + 64 > q0)) {
+    if (k0 + 64 > nk || k0 < last_first || (p.causal && k0 + 63 > q0)) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -462,48 +471,59 @@ __global__ __launch_bounds__(256) void mfma_attn_delta(DeltaArgs a) {
 // with queries on the registers and keys on the lanes, so that P and dS feed
 // the products over queries straight from the accumulators.
 
-// One step under device-held masks, its two halves of 32 queries in turn (P
-// and dS in two bf16 parts each take twice the registers of one).
-template <int D, int DO>
-__device__ __forceinline__ void dkdv_masked_step(const MArgs& p, const uint16_t* Qt, const uint16_t* Gt, const float* L,
-                                                 int qq0, int key, int nk, int dh, const bf16x8 (&kf)[D / 16],
-                                                 const bf16x8 (&vf)[D / 16], f32x16 (&dk)[DO / 32],
-                                                 f32x16 (&dv)[DO / 32]) {
+// Half a step: 32 queries (half jj of the tile) against the wave's 32 keys.
+// `edge`: some pair of them may be masked (compares and selects on every score
+// are a quarter of the step's vector work, so whole tiles go without).
+template <int D, int DO, bool M>
+__device__ __forceinline__ void dkdv_half(const MArgs& p, const uint16_t* Qt, const uint16_t* Gt, const float* L,
+                                          const int jj, const bool edge, int qq0, int key, int nk, int dh,
+                                          const bf16x8 (&kf)[D / 16], const bf16x8 (&vf)[D / 16],
+                                          f32x16 (&dk)[DO / 32], f32x16 (&dv)[DO / 32]) {
   const int lh = threadIdx.x % 64 / 32;
   const float c = p.scale * kLog2e;
+  // S = Q K', dP = dO V' (32 queries x 32 keys): query 32 jj + 8 (i / 4) + 4 lh + i % 4 in register i.
+  f32x16 s = f32x16{}, dp = f32x16{};
 #pragma unroll
-  for (int jj = 0; jj < 2; ++jj) {
-    f32x16 s = f32x16{}, dp = f32x16{};
+  for (int ks = 0; ks < D / 16; ++ks) {
+    s = mfma(frag_rows<D>(Qt, 32 * jj, ks), kf[ks], s);
+    dp = mfma(frag_rows<D>(Gt, 32 * jj, ks), vf[ks], dp);
+  }
+  // P into s, dS into dp.
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-      s = mfma(frag_rows<D>(Qt, 32 * jj, ks), kf[ks], s);
-      dp = mfma(frag_rows<D>(Gt, 32 * jj, ks), vf[ks], dp);
+  for (int i = 0; i < 16; ++i) {
+    const int qi = 32 * jj + 8 * (i / 4) + 4 * lh + i % 4;
+    s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c, -L[qi]));
+    dp[i] = s[i] * (dp[i] - L[64 + qi]);
+  }
+  if (edge) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int qi = 32 * jj + 8 * (i / 4) + 4 * lh + i % 4, query = qq0 + qi;
+      bool seen = query < p.seq && key < nk && (!p.causal || key <= query);
+      if constexpr (M) seen = seen && key >= __float_as_int(L[128 + qi]);
+      s[i] = seen ? s[i] : 0.0f;
+      dp[i] = seen ? dp[i] : 0.0f;
     }
+  }
 #pragma unroll
-    for (int part = 0; part < 2; ++part) {
-      u32x4 ph, pl, sh, sl;
+  for (int part = 0; part < 2; ++part) {
+    u32x4 ph, pl, sh, sl;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float w[2], x[2];
+    for (int e = 0; e < 4; ++e) {
+      const int i = 8 * part + 2 * e;
+      ph[e] = pack2(s[i], s[i + 1]), sh[e] = pack2(dp[i], dp[i + 1]);
+      if constexpr (M) pl[e] = rest2(s[i], s[i + 1], ph[e]), sl[e] = rest2(dp[i], dp[i + 1], sh[e]);
+    }
+    // dV' (DO features x 32 keys) += dO' P;  dK' += Q' dS.
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int i = 8 * part + 2 * e + u;
-          const int qi = 32 * jj + 8 * (i / 4) + 4 * lh + i % 4, query = qq0 + qi;
-          const bool seen = query < p.seq && key < nk && key >= __float_as_int(L[128 + qi]) && (!p.causal || key <= query);
-          w[u] = seen ? __builtin_amdgcn_exp2f(fmaf(s[i], c, -L[qi])) : 0.0f;
-          x[u] = seen ? w[u] * (dp[i] - L[64 + qi]) : 0.0f;
-        }
-        ph[e] = pack2(w[0], w[1]), pl[e] = rest2(w[0], w[1], ph[e]);
-        sh[e] = pack2(x[0], x[1]), sl[e] = rest2(x[0], x[1], sh[e]);
-      }
-#pragma unroll
-      for (int db = 0; db < DO / 32; ++db) {
-        const bf16x8 g = frag_tr<D>(Gt, DO * dh + 32 * db, 2 * jj + part), q = frag_tr<D>(Qt, DO * dh + 32 * db, 2 * jj + part);
+    for (int db = 0; db < DO / 32; ++db) {
+      const bf16x8 g = frag_tr<D>(Gt, DO * dh + 32 * db, 2 * jj + part), q = frag_tr<D>(Qt, DO * dh + 32 * db, 2 * jj + part);
+      if constexpr (M) {
         dv[db] = mfma(g, (bf16x8)pl, dv[db]);
         dk[db] = mfma(q, (bf16x8)sl, dk[db]);
-        dv[db] = mfma(g, (bf16x8)ph, dv[db]);
-        dk[db] = mfma(q, (bf16x8)sh, dk[db]);
       }
+      dv[db] = mfma(g, (bf16x8)ph, dv[db]);
+      dk[db] = mfma(q, (bf16x8)sh, dk[db]);
     }
   }
 }
@@ -515,8 +535,8 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
                                            const int split) {
   constexpr int NS = D / 16, NBO = DO / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-  constexpr int kStats = M ? 192 : 128;
-  // [stage][lse * log2e (64) | delta (64) | M: first keys, as ints (64)]
+  constexpr int kStats = M ? 196 : 128;
+  // [stage][lse * log2e (64) | delta (64) | M: first keys, as ints (64) | their largest (1) | -]
   float* stats = reinterpret_cast<float*>(lds + 4 * kTile<D>);
   const int hk = blockIdx.x;
   const int group = p.heads / p.kv_heads;
@@ -530,7 +550,6 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
   f32x16 dk[NBO], dv[NBO];
 #pragma unroll
   for (int i = 0; i < NBO; ++i) dk[i] = f32x16{}, dv[i] = f32x16{};
-  const float c = p.scale * kLog2e;
   auto Q = [&](int s) { return lds + 2 * s * kTile<D>; };
   auto G = [&](int s) { return lds + (2 * s + 1) * kTile<D>; };
   auto Ls = [&](int s) { return stats + kStats * s; };
@@ -552,6 +571,7 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
   }
   const int nsteps = qstart < qstop ? (qstop - qstart + 63) / 64 : 0;
   Stage<D> sq, sg;
+  int st_most = 0;
   float st = 0.0f;  // threads 0..127: a query's lse * log2e or delta
   auto load = [&](const uint16_t* qbase, const uint16_t* gbase, int h, int q0) {
     sq.load(qbase, p.q_ss, q0, p.seq);
@@ -562,13 +582,15 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
       st = j < p.seq ? (threadIdx.x < 64 ? p.lse[row] * kLog2e : p.delta[row]) : 0.0f;
     } else if (M && threadIdx.x < 192) {
       const int j = q0 + threadIdx.x % 64;
-      st = __int_as_float(j < p.seq ? first_of(p, j, b) : 0x7fffffff);
+      const int f = j < p.seq ? first_of(p, j, b) : 0x7fffffff;
+      st = __int_as_float(f), st_most = most(f);
     }
   };
   auto store = [&](int s) {
     sq.store(Q(s));
     sg.store(G(s));
-    if (threadIdx.x < kStats) Ls(s)[threadIdx.x] = st;
+    if (threadIdx.x < (M ? 192 : 128)) Ls(s)[threadIdx.x] = st;
+    if (M && threadIdx.x == 128) Ls(s)[192] = __int_as_float(st_most);
   };
   for (int h = hk * group; h < (hk + 1) * group; ++h) {
     const uint16_t* qbase = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
@@ -583,52 +605,11 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
       if (j + 1 < nsteps) load(qbase, gbase, h, qq0 + 64);
       const uint16_t *Qt = Q(cur), *Gt = G(cur);
       const float* L = Ls(cur);
-      // S = Q K', dP = dO V' (64 queries x 32 keys): query 32 jj + 8 (i / 4) + 4 lh + i % 4 in register i.
-      if constexpr (M) {
-        dkdv_masked_step<D, DO>(p, Qt, Gt, L, qq0, key, nk, dh, kf, vf, dk, dv);
-        if (j + 1 < nsteps) store(cur ^ 1);
-        __syncthreads();
-        continue;
-      }
-      f32x16 s[2] = {f32x16{}, f32x16{}}, dp[2] = {f32x16{}, f32x16{}};
+      const int kw = __builtin_amdgcn_readfirstlane(kw0 + wave * 32);
+      bool edge = qq0 + 64 > p.seq || kw + 32 > nk || (p.causal && kw + 31 > qq0);
+      if constexpr (M) edge = edge || kw < __builtin_amdgcn_readfirstlane(__float_as_int(L[192]));
 #pragma unroll
-      for (int ks = 0; ks < NS; ++ks)
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          s[jj] = mfma(frag_rows<D>(Qt, 32 * jj, ks), kf[ks], s[jj]);
-          dp[jj] = mfma(frag_rows<D>(Gt, 32 * jj, ks), vf[ks], dp[jj]);
-        }
-      bf16x8 pf[4], sf[4];
-#pragma unroll
-      for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-        for (int part = 0; part < 2; ++part) {
-          u32x4 wp, wd;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float w[2], x[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              const int i = 8 * part + 2 * e + u;
-              const int qi = 32 * jj + 8 * (i / 4) + 4 * lh + i % 4, query = qq0 + qi;
-              const bool seen = query < p.seq && key < p.kv_seq && (!p.causal || key <= query);
-              w[u] = seen ? __builtin_amdgcn_exp2f(fmaf(s[jj][i], c, -L[qi])) : 0.0f;
-              x[u] = w[u] * (dp[jj][i] - L[64 + qi]);
-            }
-            wp[e] = pack2(w[0], w[1]);
-            wd[e] = pack2(x[0], x[1]);
-          }
-          pf[2 * jj + part] = (bf16x8)wp;
-          sf[2 * jj + part] = (bf16x8)wd;
-        }
-      // dV' (DO features x 32 keys) += dO' P;  dK' += Q' dS.
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-        for (int db = 0; db < NBO; ++db) {
-          dv[db] = mfma(frag_tr<D>(Gt, DO * dh + 32 * db, ks), pf[ks], dv[db]);
-          dk[db] = mfma(frag_tr<D>(Qt, DO * dh + 32 * db, ks), sf[ks], dk[db]);
-        }
+      for (int jj = 0; jj < 2; ++jj) dkdv_half<D, DO, M>(p, Qt, Gt, L, jj, edge, qq0, key, nk, dh, kf, vf, dk, dv);
       if (j + 1 < nsteps) store(cur ^ 1);
       __syncthreads();
     }
@@ -691,7 +672,7 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
   const int h = blockIdx.x;
   const int hk = h / (p.heads / p.kv_heads);
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
-  const int q0 = qb * 128 + wave * 32, query = q0 + lr;
+  const int q0 = __builtin_amdgcn_readfirstlane(qb * 128 + wave * 32), query = q0 + lr;
   const int64_t qoff = (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)query * p.q_ss;
   const bool live = query < p.seq;
   bf16x8 qf[NS], gf[NS];
@@ -716,6 +697,7 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
       k_lo = max(0, min(least(first, reinterpret_cast<int*>(lds + 4 * kTile<D>)), nk)) / 64 * 64;
     }
   }
+  const int last_first = M ? most(first) : 0;  // tiles from here on see no first key
   const int k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
   const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
   Stage<D> sk, sv;
@@ -742,6 +724,21 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
         s[kb] = mfma(frag_rows<D>(K(cur), 32 * kb, ks), qf[ks], s[kb]);
         dp[kb] = mfma(frag_rows<D>(V(cur), 32 * kb, ks), gf[ks], dp[kb]);
       }
+    // dS' into dp, masked where the tile needs it.
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        dp[kb][i] = __builtin_amdgcn_exp2f(fmaf(s[kb][i], c, -l2)) * (dp[kb][i] - dl);
+    if (k0 + 64 > nk || k0 < last_first || (p.causal && k0 + 63 > q0)) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
+          dp[kb][i] = key < nk && (!M || key >= first) && (!p.causal || key <= query) ? dp[kb][i] : 0.0f;
+        }
+    }
     bf16x8 sf[4], sl[4];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
@@ -750,17 +747,9 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
         u32x4 w, r;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          float x[2];
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int i = 8 * part + 2 * e + u;
-            const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
-            const bool seen = key < nk && (!M || key >= first) && (!p.causal || key <= query);
-            const float pw = seen ? __builtin_amdgcn_exp2f(fmaf(s[kb][i], c, -l2)) : 0.0f;
-            x[u] = M && !seen ? 0.0f : pw * (dp[kb][i] - dl);
-          }
-          w[e] = pack2(x[0], x[1]);
-          if constexpr (M) r[e] = rest2(x[0], x[1], w[e]);
+          const int i = 8 * part + 2 * e;
+          w[e] = pack2(dp[kb][i], dp[kb][i + 1]);
+          if constexpr (M) r[e] = rest2(dp[kb][i], dp[kb][i + 1], w[e]);
         }
         sf[2 * kb + part] = (bf16x8)w;
         if constexpr (M) sl[2 * kb + part] = (bf16x8)r;
@@ -957,7 +946,7 @@ int bwd_launch(const th_attention_desc* d, th_launch** out) {
 
 // Under device-held masks (or rows the kernels above do not take): whole
 // sweeps, a workgroup per block of 128.
-constexpr int kMaskLds = 2 * 192 * sizeof(float) + 16;  // the dK/dV stages' statistics and four ints
+constexpr int kMaskLds = 2 * 196 * sizeof(float) + 16;  // the dK/dV stages' statistics and four ints
 
 template <int D>
 int masked_fwd_launch(const th_attention_desc* d, th_launch** out) {
