@@ -64,6 +64,9 @@ struct FArgs {
   int32_t nsplit, span;
   float* part;
   float* part_ml;
+  // The backward's dQ sweep, beside the dK/dV one above.
+  int32_t q_nsplit, q_span;
+  float* q_part;
 };
 
 __device__ __forceinline__ f32x16 mfma2(float a, float b, f32x16 c) {
@@ -188,11 +191,8 @@ struct StageF {
   }
 };
 
-// Causal sweeps do less work for earlier query blocks (and later key
-// blocks): workgroup x takes blocks x and nb - 1 - x (one pass each), so
-// every workgroup sweeps about the same number of tiles.
-__device__ __forceinline__ int passes(bool causal, int x, int nb) { return causal && 2 * x + 1 != nb ? 2 : 1; }
-__device__ __forceinline__ int block_of(int pass, int x, int nb) { return pass == 0 ? x : nb - 1 - x; }
+// The grid is (heads, batch, blocks): blocks slowest, the longest causal
+// sweeps first, the short ones filling in behind them.
 
 // ---- forward ---------------------------------------------------------------------
 
@@ -202,10 +202,10 @@ template <int D>
 __device__ __forceinline__ void fwd_block(const FArgs& p, const int qb, const int b, const int split) {
   constexpr int NB = D / 32;
   extern __shared__ __attribute__((aligned(16))) float flds[];
-  const int h = blockIdx.y;
+  const int h = blockIdx.x;
   const int hk = h / (p.heads / p.kv_heads);
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
-  const int q0 = qb * 128 + wave * 32, query = q0 + lr;
+  const int q0 = __builtin_amdgcn_readfirstlane(qb * 128 + wave * 32), query = q0 + lr;
   const float* qbase = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
   const float* kbase = p.k + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
   const float* vbase = p.v + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
@@ -240,7 +240,7 @@ __device__ __forceinline__ void fwd_block(const FArgs& p, const int qb, const in
     f32x16 s[2] = {f32x16{}, f32x16{}};
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) over_d<D>(K(cur), 32 * kb, qf, s[kb]);
-    if (k0 + 64 > p.kv_seq || (p.causal && k0 + 64 > q0)) {
+    if (k0 + 64 > p.kv_seq || (p.causal && k0 + 63 > q0)) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -295,15 +295,9 @@ __device__ __forceinline__ void fwd_block(const FArgs& p, const int qb, const in
 
 template <int D>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void f32_attn_fwd(FArgs p) {
-  // Split: one part of one block; else a block and, causal, its mirror (one call site).
   const bool split = p.nsplit > 1;
-  const int nb = (p.seq + 127) / 128;
-  const int npass = split ? 1 : passes(p.causal, blockIdx.x, nb);
-  for (int pass = 0; pass < npass; ++pass) {
-    if (pass > 0) __syncthreads();  // the first pass's last LDS reads are done
-    fwd_block<D>(p, split ? blockIdx.x : block_of(pass, blockIdx.x, nb), split ? blockIdx.z / p.nsplit : blockIdx.z,
-                 split ? blockIdx.z % p.nsplit : -1);
-  }
+  const int z = gridDim.z - 1 - blockIdx.z;  // the last queries first
+  fwd_block<D>(p, split ? z / p.nsplit : z, blockIdx.y, split ? z % p.nsplit : -1);
 }
 
 // The parts of a split forward combined: per (b, query, head) row, M = max
@@ -340,28 +334,38 @@ __global__ __launch_bounds__(256) void f32_attn_combine(FCombineArgs a) {
   if (c == 0 && p.lse) p.lse[row] = (mx + log2f(l)) * kLn2;
 }
 
-// dQ, dK or dV from a split sweep's parts: out = scale * sum_s part_s in
-// part order; rows [b][position][head] of `d` features.
-struct FSumArgs {
+// dK, dV and dQ from split sweeps' parts, one launch: out = scale * sum_s
+// part_s in part order; rows [b][position][head] of `d` features.
+struct FSumArgsOne {
   const float* part;
   float* out;
   int64_t sh, ss, sb;
-  int32_t positions, heads, batch, d, nsplit;
+  int32_t positions, heads, nsplit;
   float scale;
+  uint32_t blocks;  // workgroups, 256 quads of features each
+};
+struct FSumArgs {
+  FSumArgsOne of[3];
+  int32_t n, batch, d;
 };
 
-__global__ __launch_bounds__(256) void f32_attn_sum(FSumArgs a) {
-  const int quads = a.d / 4;
-  const int64_t rows = (int64_t)a.batch * a.positions * a.heads;
-  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(256) void f32_attn_sum(FSumArgs all) {
+  uint32_t block = blockIdx.x;
+  int which = 0;
+  while (which + 1 < all.n && block >= all.of[which].blocks) block -= all.of[which++].blocks;
+  const FSumArgsOne& a = all.of[which];
+  const int d = all.d, quads = d / 4;
+  const int64_t rows = (int64_t)all.batch * a.positions * a.heads;
+  const int64_t t = (int64_t)block * 256 + threadIdx.x;
   if (t >= rows * quads) return;
   const int64_t row = t / quads;
   const int c = 4 * (int)(t % quads);
   // Part s of this quad at a.part + (s rows + row) d + c: a stride of rows d / 4 quads.
-  f32x4 acc = thd::sum_in_order(reinterpret_cast<const f32x4*>(a.part + row * a.d + c), rows * a.d / 4, a.nsplit);
+  f32x4 acc = thd::sum_in_order(reinterpret_cast<const f32x4*>(a.part + row * d + c), rows * d / 4, a.nsplit);
+  acc *= a.scale;
   const int h = (int)(row % a.heads);
   const int64_t pos = (row / a.heads) % a.positions, b = row / ((int64_t)a.heads * a.positions);
-  *reinterpret_cast<f32x4*>(a.out + b * a.sb + h * a.sh + pos * a.ss + c) = acc * a.scale;
+  *reinterpret_cast<f32x4*>(a.out + b * a.sb + h * a.sh + pos * a.ss + c) = acc;
 }
 
 // ---- backward: delta = rowsum(dO .* O) ---------------------------------------------
@@ -422,11 +426,10 @@ __global__ __launch_bounds__(256) void f32_attn_delta(FDeltaArgs a) {
 // Query tiles [qstart, qstop) for the keys of kblk: all (split < 0) or part
 // `split`, which leaves its unscaled dK', dV'.
 template <int D>
-__device__ __forceinline__ void dkdv_block(const FArgs& p, const int kblk, const int b, const int split) {
+__device__ __forceinline__ void dkdv_block(const FArgs& p, const int kblk, const int hk, const int b, const int split) {
   constexpr int NB = D / 32;
   extern __shared__ __attribute__((aligned(16))) float flds[];
   float* stats = flds + 4 * kTileF<D>;  // [stage][lse * log2e (64) | delta (64)]
-  const int hk = blockIdx.y;
   const int group = p.heads / p.kv_heads;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lh = lane / 32;
   const int kw0 = kblk * 128, key = kw0 + wave * 32 + lane % 32;
@@ -474,6 +477,8 @@ __device__ __forceinline__ void dkdv_block(const FArgs& p, const int kblk, const
       if (j + 1 < nsteps) load(qbase, gbase, h, qq0 + 64);
       const float *Qt = Q(cur), *Gt = G(cur);
       const float* L = Ls(cur);
+      const int kw = __builtin_amdgcn_readfirstlane(kw0 + wave * 32);
+      const bool edge = qq0 + 64 > p.seq || kw + 32 > p.kv_seq || (p.causal && kw + 31 > qq0);
       // The tile's two halves of 32 queries in turn (half the score
       // accumulators live at once); the next tile goes to LDS after the first.
 #pragma unroll
@@ -485,11 +490,18 @@ __device__ __forceinline__ void dkdv_block(const FArgs& p, const int kblk, const
         // P into s, dS into dp.
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int qi = 32 * jj + 8 * (i / 4) + 4 * lh + i % 4, query = qq0 + qi;
-          const bool seen = query < p.seq && key < p.kv_seq && (!p.causal || key <= query);
-          const float w = seen ? __builtin_amdgcn_exp2f(fmaf(s[i], c, -L[qi])) : 0.0f;
-          s[i] = w;
-          dp[i] = w * (dp[i] - L[64 + qi]);
+          const int qi = 32 * jj + 8 * (i / 4) + 4 * lh + i % 4;
+          s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c, -L[qi]));
+          dp[i] = s[i] * (dp[i] - L[64 + qi]);
+        }
+        if (edge) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int query = qq0 + 32 * jj + 8 * (i / 4) + 4 * lh + i % 4;
+            const bool seen = query < p.seq && key < p.kv_seq && (!p.causal || key <= query);
+            s[i] = seen ? s[i] : 0.0f;
+            dp[i] = seen ? dp[i] : 0.0f;
+          }
         }
         // dV' (D x 32 keys) += dO' P;  dK' += Q' dS.
         over_positions<D>(Gt, 32 * jj, s, dv);
@@ -513,19 +525,6 @@ __device__ __forceinline__ void dkdv_block(const FArgs& p, const int kblk, const
   store_rows<D>(p.dv + out, dv, 1.0f);
 }
 
-template <int D>
-// One wave a SIMD: K and V of the wave's keys, dK' and dV' take D + D registers.
-__global__ __launch_bounds__(256, 1) void f32_attn_dkdv(FArgs p) {
-  const bool split = p.nsplit > 1;
-  const int nb = (p.kv_seq + 127) / 128;
-  const int npass = split ? 1 : passes(p.causal, blockIdx.x, nb);
-  for (int pass = 0; pass < npass; ++pass) {
-    if (pass > 0) __syncthreads();  // the first pass's last LDS reads are done
-    dkdv_block<D>(p, split ? blockIdx.x : block_of(pass, blockIdx.x, nb), split ? blockIdx.z / p.nsplit : blockIdx.z,
-                  split ? blockIdx.z % p.nsplit : -1);
-  }
-}
-
 // ---- backward: dQ ----------------------------------------------------------------------
 // A workgroup takes 128 queries (32 a wave) and sweeps key tiles of 64:
 // S' = K Q', dP' = V dO' (keys on the registers, queries on the lanes),
@@ -534,13 +533,12 @@ __global__ __launch_bounds__(256, 1) void f32_attn_dkdv(FArgs p) {
 // Keys [k_lo, k_hi) for query block qb: all (split < 0) or part `split`,
 // which leaves its unscaled dQ'.
 template <int D>
-__device__ __forceinline__ void dq_block(const FArgs& p, const int qb, const int b, const int split) {
+__device__ __forceinline__ void dq_block(const FArgs& p, const int qb, const int h, const int b, const int split) {
   constexpr int NB = D / 32;
   extern __shared__ __attribute__((aligned(16))) float flds[];
-  const int h = blockIdx.y;
   const int hk = h / (p.heads / p.kv_heads);
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lh = lane / 32;
-  const int q0 = qb * 128 + wave * 32, query = q0 + lane % 32;
+  const int q0 = __builtin_amdgcn_readfirstlane(qb * 128 + wave * 32), query = q0 + lane % 32;
   const int64_t qoff = (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)query * p.q_ss;
   const bool live = query < p.seq;
   float qf[D / 2], gf[D / 2];
@@ -557,7 +555,7 @@ __device__ __forceinline__ void dq_block(const FArgs& p, const int qb, const int
   for (int i = 0; i < NB; ++i) dq[i] = f32x16{};
   const int qlast = min(qb * 128 + 127, p.seq - 1);
   const int kend = p.causal ? min(p.kv_seq, qlast + 1) : p.kv_seq;
-  const int k_lo = split < 0 ? 0 : split * p.span, k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
+  const int k_lo = split < 0 ? 0 : split * p.q_span, k_hi = split < 0 ? kend : min(kend, k_lo + p.q_span);
   const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
   StageF<D> sk, sv;
   auto K = [&](int s) { return flds + 2 * s * kTileF<D>; };
@@ -584,10 +582,14 @@ __device__ __forceinline__ void dq_block(const FArgs& p, const int qb, const int
       // dS' into sc.
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
-        const bool seen = key < p.kv_seq && (!p.causal || key <= query);
-        const float pw = seen ? __builtin_amdgcn_exp2f(fmaf(sc[i], c, -l2)) : 0.0f;
-        sc[i] = pw * (dp[i] - dl);
+        sc[i] = __builtin_amdgcn_exp2f(fmaf(sc[i], c, -l2)) * (dp[i] - dl);
+      }
+      if (k0 + 64 > p.kv_seq || (p.causal && k0 + 63 > q0)) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
+          sc[i] = key < p.kv_seq && (!p.causal || key <= query) ? sc[i] : 0.0f;
+        }
       }
       over_positions<D>(K(cur), 32 * kb, sc, dq);
       if (kb == 0 && j + 1 < nsteps) {
@@ -599,30 +601,38 @@ __device__ __forceinline__ void dq_block(const FArgs& p, const int qb, const int
   }
   if (!live) return;
   if (split >= 0) {
-    store_rows<D>(p.part + ((((int64_t)split * p.batch + b) * p.seq + query) * p.heads + h) * D, dq, 1.0f);
+    store_rows<D>(p.q_part + ((((int64_t)split * p.batch + b) * p.seq + query) * p.heads + h) * D, dq, 1.0f);
     return;
   }
   store_rows<D>(p.dq + qoff, dq, p.scale);
 }
 
+// Both sweeps in one launch: neither needs the other, and alone each leaves
+// the device part empty at its end.  dK/dV workgroups, the first keys, the
+// longest causal sweeps, first; then the dQ ones, the last queries first.
+struct FBwdArgs {
+  FArgs p;  // first: its members sit at FArgs' offsets
+  uint32_t n_dkdv;
+};
+
+// One wave a SIMD: at d = 64 two would spill 10 registers (B2 H8 S2048, forward
+// and backward, 610 us against 468; S1024 179 against 181).
 template <int D>
-__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void f32_attn_dq(FArgs p) {
-  const bool split = p.nsplit > 1;
-  const int nb = (p.seq + 127) / 128;
-  const int npass = split ? 1 : passes(p.causal, blockIdx.x, nb);
-  for (int pass = 0; pass < npass; ++pass) {
-    if (pass > 0) __syncthreads();  // the first pass's last LDS reads are done
-    dq_block<D>(p, split ? blockIdx.x : block_of(pass, blockIdx.x, nb), split ? blockIdx.z / p.nsplit : blockIdx.z,
-                split ? blockIdx.z % p.nsplit : -1);
+__global__ __launch_bounds__(256, 1) void f32_attn_bwd(FBwdArgs a) {
+  const FArgs& p = a.p;
+  if (blockIdx.x < a.n_dkdv) {
+    const int hk = blockIdx.x % p.kv_heads, b = blockIdx.x / p.kv_heads % p.batch, z = blockIdx.x / p.kv_heads / p.batch;
+    const bool split = p.nsplit > 1;
+    dkdv_block<D>(p, split ? z / p.nsplit : z, hk, b, split ? z % p.nsplit : -1);
+    return;
   }
+  const uint32_t i = gridDim.x - 1 - blockIdx.x;  // (from the end: the last queries first)
+  const int h = i % p.heads, b = i / p.heads % p.batch, z = i / p.heads / p.batch;
+  const bool split = p.q_nsplit > 1;
+  dq_block<D>(p, split ? z / p.q_nsplit : z, h, b, split ? z % p.q_nsplit : -1);
 }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
-
-unsigned blocks_of(int n, int causal) {
-  const unsigned nb = (unsigned)((n + 127) / 128);
-  return causal ? (nb + 1) / 2 : nb;
-}
 
 FArgs fargs_of(const th_attention_desc* d) {
   FArgs a{};
@@ -659,9 +669,8 @@ int fwd_launch(const th_attention_desc* d, th_launch** out) {
   const int nqb = (d->seq + 127) / 128;
   const th::Split sp = th::split_of((int64_t)nqb * d->heads * d->batch, a.kv_seq);
   a.nsplit = sp.n, a.span = sp.span;
-  TH_REQUIRE((int64_t)d->batch * sp.n <= 65535, "attention: grid too large");
   th::Builder b("attention_fwd_f32mfma", 7);
-  const dim3 grid = sp.n > 1 ? dim3(nqb, d->heads, d->batch * sp.n) : dim3(blocks_of(d->seq, d->causal), d->heads, d->batch);
+  const dim3 grid(d->heads, d->batch, nqb * sp.n);
   int k = b.kernel((const void*)f32_attn_fwd<D>, D == 64 ? "f32_attn_fwd_d64" : "f32_attn_fwd_d128", grid, dim3(256),
                    (uint32_t)lds, a);
   b.ref(0, k, TH_OFFSET(FArgs, q));
@@ -690,73 +699,79 @@ int fwd_launch(const th_attention_desc* d, th_launch** out) {
   return TH_OK;
 }
 
+// The backward's launch: delta, both sweeps, and where small grids split
+// them (the dK/dV sweep over queries, the dQ sweep over keys) their sums.
 template <int D>
 int bwd_launch(const th_attention_desc* d, th_launch** out) {
-  const size_t lds_kv = 4 * (size_t)kTileF<D> * sizeof(float);
-  const size_t lds_dkdv = lds_kv + 2 * 128 * sizeof(float);
-  TH_HIP(hipFuncSetAttribute((const void*)f32_attn_dkdv<D>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)lds_dkdv));
-  TH_HIP(hipFuncSetAttribute((const void*)f32_attn_dq<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_kv));
+  const size_t lds = 4 * (size_t)kTileF<D> * sizeof(float) + 2 * 128 * sizeof(float);
+  const void* fn = (const void*)f32_attn_bwd<D>;
+  TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   FArgs a = fargs_of(d);
   th::Builder b("attention_bwd_f32mfma", 11);
   const int64_t rows = (int64_t)d->batch * d->seq * d->heads;
   const int64_t rows_k = (int64_t)d->batch * a.kv_seq * d->kv_heads;
-  const uint64_t at_delta = b.workspace((uint64_t)rows * sizeof(float));
-  // Small grids split the dK/dV sweep over queries and the dQ sweep over keys.
-  const int nkb = (a.kv_seq + 127) / 128, nqb = (d->seq + 127) / 128;
-  const th::Split skv = th::split_of((int64_t)nkb * d->kv_heads * d->batch, d->seq);
-  const th::Split sq = th::split_of((int64_t)nqb * d->heads * d->batch, a.kv_seq);
-  TH_REQUIRE((int64_t)d->batch * std::max(skv.n, sq.n) <= 65535, "attention: grid too large");
-  FArgs akv = a, aq = a;
-  akv.nsplit = skv.n, akv.span = skv.span;
-  aq.nsplit = sq.n, aq.span = sq.span;
   TH_REQUIRE(rows < 2147483648LL, "attention: batch x seq x heads must be under 2^31");
+  const uint64_t at_delta = b.workspace((uint64_t)rows * sizeof(float));
+  const int nkb = (a.kv_seq + 127) / 128, nqb = (d->seq + 127) / 128;
+  const int64_t gkv = (int64_t)nkb * d->kv_heads * d->batch, gq = (int64_t)nqb * d->heads * d->batch;
+  const th::Split skv = th::split_of(gkv, d->seq, 384), sq = th::split_of(gq, a.kv_seq, 384);
+  a.nsplit = skv.n, a.span = skv.span;
+  a.q_nsplit = sq.n, a.q_span = sq.span;
+  const int64_t n_dkdv = gkv * skv.n, blocks = n_dkdv + gq * sq.n;
+  TH_REQUIRE(blocks <= 0x7fffffff, "attention: grid too large");
   constexpr int kDeltaBlockRows = 4 * (64 / (D / 4)) * kDeltaRowsF;  // rows a workgroup
-  int k0 = b.kernel((const void*)f32_attn_delta<D>, "f32_attn_delta",
-                    dim3((unsigned)((rows + kDeltaBlockRows - 1) / kDeltaBlockRows)), dim3(256), 0, FDeltaArgs{a, D});
-  const dim3 gkv = skv.n > 1 ? dim3(nkb, d->kv_heads, d->batch * skv.n) : dim3(blocks_of(a.kv_seq, d->causal), d->kv_heads, d->batch);
-  const dim3 gq = sq.n > 1 ? dim3(nqb, d->heads, d->batch * sq.n) : dim3(blocks_of(d->seq, d->causal), d->heads, d->batch);
-  int k1 = b.kernel((const void*)f32_attn_dkdv<D>, D == 64 ? "f32_attn_dkdv_d64" : "f32_attn_dkdv_d128", gkv,
-                    dim3(256), (uint32_t)lds_dkdv, akv);
-  if (skv.n > 1) {
-    const uint64_t at_kv = b.workspace((uint64_t)2 * skv.n * rows_k * D * sizeof(float));
-    b.ws_ref(k1, TH_OFFSET(FArgs, part), at_kv);
-    const unsigned g = (unsigned)((rows_k * (D / 4) + 255) / 256);
-    // The outputs' pointers start as the descriptor's (repointing rewrites them with the others).
-    FSumArgs sk{nullptr, static_cast<float*>(d->dk), d->k_strides[0], d->k_strides[1], d->k_strides[2], a.kv_seq,
-                d->kv_heads, d->batch, D, skv.n, a.scale};
-    FSumArgs sv = sk;
-    sv.out = static_cast<float*>(d->dv), sv.scale = 1.0f;
-    const int ks = b.kernel((const void*)f32_attn_sum, "f32_attn_sum_dk", dim3(g), dim3(256), 0, sk);
-    const int kv = b.kernel((const void*)f32_attn_sum, "f32_attn_sum_dv", dim3(g), dim3(256), 0, sv);
-    b.ws_ref(ks, TH_OFFSET(FSumArgs, part), at_kv);
-    b.ws_ref(kv, TH_OFFSET(FSumArgs, part), at_kv + (uint64_t)skv.n * rows_k * D * sizeof(float));
-    b.ref(7, ks, TH_OFFSET(FSumArgs, out));
-    b.ref(8, kv, TH_OFFSET(FSumArgs, out));
-  }
-  int k2 = b.kernel((const void*)f32_attn_dq<D>, D == 64 ? "f32_attn_dq_d64" : "f32_attn_dq_d128", gq, dim3(256),
-                    (uint32_t)lds_kv, aq);
-  if (sq.n > 1) {
-    const uint64_t at_q = b.workspace((uint64_t)sq.n * rows * D * sizeof(float));
-    b.ws_ref(k2, TH_OFFSET(FArgs, part), at_q);
-    FSumArgs s1{nullptr, static_cast<float*>(d->dq), d->q_strides[0], d->q_strides[1], d->q_strides[2], d->seq,
-                d->heads, d->batch, D, sq.n, a.scale};
-    const int kq = b.kernel((const void*)f32_attn_sum, "f32_attn_sum_dq", dim3((unsigned)((rows * (D / 4) + 255) / 256)),
-                            dim3(256), 0, s1);
-    b.ws_ref(kq, TH_OFFSET(FSumArgs, part), at_q);
-    b.ref(6, kq, TH_OFFSET(FSumArgs, out));
-  }
+  const int k0 = b.kernel((const void*)f32_attn_delta<D>, "f32_attn_delta",
+                          dim3((unsigned)((rows + kDeltaBlockRows - 1) / kDeltaBlockRows)), dim3(256), 0, FDeltaArgs{a, D});
+  const int k1 = b.kernel(fn, D == 64 ? "f32_attn_dkdv_d64_f32_attn_dq_d64" : "f32_attn_dkdv_d128_f32_attn_dq_d128",
+                          dim3((unsigned)blocks), dim3(256), (uint32_t)lds, FBwdArgs{a, (uint32_t)n_dkdv});
   const size_t offs[9] = {TH_OFFSET(FArgs, q),  TH_OFFSET(FArgs, k),  TH_OFFSET(FArgs, v),
                           TH_OFFSET(FArgs, o),  TH_OFFSET(FArgs, lse), TH_OFFSET(FArgs, dout),
                           TH_OFFSET(FArgs, dq), TH_OFFSET(FArgs, dk),  TH_OFFSET(FArgs, dv)};
-  // The delta kernel's arguments are FArgs followed by d: the same offsets.
-  for (int v = 0; v < 9; ++v)
-    for (int kk : {k0, k1, k2}) b.ref(v, kk, offs[v]);
-  for (int kk : {k0, k1, k2}) b.ws_ref(kk, TH_OFFSET(FArgs, delta), at_delta);
+  // Both kernels' arguments begin with FArgs: the same offsets.
+  for (int kk : {k0, k1}) {
+    for (int v = 0; v < 9; ++v) b.ref(v, kk, offs[v]);
+    b.ws_ref(kk, TH_OFFSET(FArgs, delta), at_delta);
+  }
   for (int v : {0, 1, 2, 3, 5, 6, 7, 8}) b.align(v, 16);
+  if (skv.n > 1 || sq.n > 1) {
+    FSumArgs s{};
+    s.batch = d->batch, s.d = D;
+    // The outputs' pointers start as the descriptor's (repointing rewrites them with the others).
+    int values[3];
+    uint64_t ats[3];
+    unsigned total = 0;
+    auto add = [&](int value, float* to, const int64_t* strides, int positions, int heads, int parts, float scale,
+                   uint64_t at) {
+      const unsigned g = (unsigned)(((int64_t)d->batch * positions * heads * (D / 4) + 255) / 256);
+      values[s.n] = value, ats[s.n] = at;
+      s.of[s.n++] = FSumArgsOne{nullptr, to, strides[0], strides[1], strides[2], positions, heads, parts, scale, g};
+      total += g;
+    };
+    if (skv.n > 1) {
+      const uint64_t at = b.workspace((uint64_t)2 * skv.n * rows_k * D * sizeof(float));
+      b.ws_ref(k1, TH_OFFSET(FArgs, part), at);
+      add(7, a.dk, d->k_strides, a.kv_seq, d->kv_heads, skv.n, a.scale, at);
+      add(8, a.dv, d->k_strides, a.kv_seq, d->kv_heads, skv.n, 1.0f, at + (uint64_t)skv.n * rows_k * D * sizeof(float));
+    }
+    if (sq.n > 1) {
+      const uint64_t at = b.workspace((uint64_t)sq.n * rows * D * sizeof(float));
+      b.ws_ref(k1, TH_OFFSET(FArgs, q_part), at);
+      add(6, a.dq, d->q_strides, d->seq, d->heads, sq.n, a.scale, at);
+    }
+    const int k2 = b.kernel((const void*)f32_attn_sum,
+                            sq.n == 1   ? "f32_attn_sum_dk_dv"
+                                                              : skv.n == 1 ? "f32_attn_sum_dq"
+                                                                           : "f32_attn_sum_dk_dv_f32_attn_sum_dq",
+                            dim3(total), dim3(256), 0, s);
+    for (int i = 0; i < s.n; ++i) {
+      const size_t one = TH_OFFSET(FSumArgs, of) + i * sizeof(FSumArgsOne);
+      b.ref(values[i], k2, one + TH_OFFSET(FSumArgsOne, out));
+      b.ws_ref(k2, one + TH_OFFSET(FSumArgsOne, part), ats[i]);
+    }
+  }
   const double BH = (double)d->batch * d->heads, BHk = (double)d->batch * d->kv_heads;
   b.work(2.0 * BH * a.seq * D * 8 + 2.0 * BHk * a.kv_seq * D * 8 + 8.0 * BH * a.seq,
-         2.5 * 4.0 * BH * D * visible_pairs(a), (int64_t)gkv.x * gkv.y * gkv.z);
+         2.5 * 4.0 * BH * D * visible_pairs(a), n_dkdv);
   *out = b.release();
   return TH_OK;
 }
@@ -778,8 +793,8 @@ bool f32_attention_takes(const th_attention_desc* d) {
                           (const void*)d->dout, (const void*)d->dq, (const void*)d->dk, (const void*)d->dv})
     if (!aligned16(ptr)) return false;
   const int64_t kv = d->kv_seq > 0 ? d->kv_seq : d->seq;
-  return (d->seq + 127) / 128 <= 0x7fffffff && (kv + 127) / 128 <= 0x7fffffff && d->heads <= 65535 &&
-         d->batch <= 65535;
+  // (blocks of 128 positions along grid z, at most 8 parts each)
+  return (d->seq + 127) / 128 <= 8191 && (kv + 127) / 128 <= 8191 && d->heads <= 65535 && d->batch <= 65535;
 }
 
 int build_attention_f32_fwd(const th_attention_desc* d, th_launch** out) {

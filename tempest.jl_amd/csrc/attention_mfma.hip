@@ -79,6 +79,9 @@ struct MArgs {
   int32_t nsplit, span;
   float* part;
   float* part_ml;
+  // The backward's dQ sweep, beside the dK/dV one above.
+  int32_t q_nsplit, q_span;
+  float* q_part;
   const int32_t* starts;   // M only: (positions, batch), 1-based, or null
   const int32_t* lengths;  // M only: (batch), or null
 };
@@ -389,25 +392,34 @@ __global__ __launch_bounds__(256) void mfma_attn_combine(CombineArgs a) {
   if (c == 0 && p.lse) p.lse[row] = (mx + log2f(l)) * kLn2;
 }
 
-// dQ, dK or dV from a split sweep's parts: out = scale * sum_s part_s in
-// part order, rounded to bf16; rows [b][position][head] of `d` features.
-struct SumArgs {
+// dK, dV and dQ from split sweeps' parts, one launch: out = scale * sum_s
+// part_s in part order, rounded to bf16; rows [b][position][head] of `d` features.
+struct SumArgsOne {
   const float* part;
   uint16_t* out;
   int64_t sh, ss, sb;
-  int32_t positions, heads, batch, d, nsplit;
+  int32_t positions, heads, nsplit;
   float scale;
+  uint32_t blocks;  // workgroups, 256 quads of features each
+};
+struct SumArgs {
+  SumArgsOne of[3];
+  int32_t n, batch, d;
 };
 
-__global__ __launch_bounds__(256) void mfma_attn_sum(SumArgs a) {
-  const int quads = a.d / 4;
-  const int64_t rows = (int64_t)a.batch * a.positions * a.heads;
-  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(256) void mfma_attn_sum(SumArgs all) {
+  uint32_t block = blockIdx.x;
+  int which = 0;
+  while (which + 1 < all.n && block >= all.of[which].blocks) block -= all.of[which++].blocks;
+  const SumArgsOne& a = all.of[which];
+  const int d = all.d, quads = d / 4;
+  const int64_t rows = (int64_t)all.batch * a.positions * a.heads;
+  const int64_t t = (int64_t)block * 256 + threadIdx.x;
   if (t >= rows * quads) return;
   const int64_t row = t / quads;
   const int c = 4 * (int)(t % quads);
   // Part s of this quad at a.part + (s rows + row) d + c: a stride of rows d / 4 quads.
-  f32x4 acc = thd::sum_in_order(reinterpret_cast<const f32x4*>(a.part + row * a.d + c), rows * a.d / 4, a.nsplit);
+  f32x4 acc = thd::sum_in_order(reinterpret_cast<const f32x4*>(a.part + row * d + c), rows * d / 4, a.nsplit);
   acc *= a.scale;
   const int h = (int)(row % a.heads);
   const int64_t pos = (row / a.heads) % a.positions, b = row / ((int64_t)a.heads * a.positions);
@@ -531,14 +543,13 @@ __device__ __forceinline__ void dkdv_half(const MArgs& p, const uint16_t* Qt, co
 // Query tiles [qstart, qstop) for the keys of kblk: all of them (split <
 // 0), or part `split` of the sweep, which leaves its unscaled fp32 dK', dV'.
 template <int D, int DO, bool M>
-__device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const int dh, const int b,
+__device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const int dh, const int hk, const int b,
                                            const int split) {
   constexpr int NS = D / 16, NBO = DO / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   constexpr int kStats = M ? 196 : 128;
   // [stage][lse * log2e (64) | delta (64) | M: first keys, as ints (64) | their largest (1) | -]
   float* stats = reinterpret_cast<float*>(lds + 4 * kTile<D>);
-  const int hk = blockIdx.x;
   const int group = p.heads / p.kv_heads;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
   const int kw0 = kblk * 128, key = kw0 + wave * 32 + lr;
@@ -650,14 +661,6 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
     }
 }
 
-template <int D, int DO, bool M>
-__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void mfma_attn_dkdv(MArgs p) {
-  constexpr int halves = D / DO;
-  const bool split = p.nsplit > 1;
-  const int z = blockIdx.z, x = split ? z / p.nsplit : z;  // the first keys, the longest sweeps, first
-  dkdv_block<D, DO, M>(p, x / halves, x % halves, blockIdx.y, split ? z % p.nsplit : -1);
-}
-
 // ---- backward: dQ ----------------------------------------------------------------------
 // A workgroup takes 128 queries (32 a wave) and sweeps key tiles of 64:
 // S' = K Q', dP' = V dO' (keys on the registers, queries on the lanes),
@@ -666,10 +669,9 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void mfma_attn_dkdv(MArgs p) 
 // Keys [k_lo, k_hi) for query block qb: all of them (split < 0), or part
 // `split` of the sweep, which leaves its unscaled fp32 dQ'.
 template <int D, bool M>
-__device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int b, const int split) {
+__device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int h, const int b, const int split) {
   constexpr int NS = D / 16, NB = D / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-  const int h = blockIdx.x;
   const int hk = h / (p.heads / p.kv_heads);
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
   const int q0 = __builtin_amdgcn_readfirstlane(qb * 128 + wave * 32), query = q0 + lr;
@@ -689,7 +691,7 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
   for (int i = 0; i < NB; ++i) dq[i] = f32x16{};
   const int nk = keys_of<M>(p, b), qlast = min(qb * 128 + 127, p.seq - 1);
   const int kend = p.causal ? min(nk, qlast + 1) : nk;
-  int k_lo = split < 0 ? 0 : split * p.span, first = 0;
+  int k_lo = split < 0 ? 0 : split * p.q_span, first = 0;
   if constexpr (M) {
     // The sweep starts at the block's least first key, a wave's share of it at the wave's.
     if (p.starts) {
@@ -698,7 +700,7 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
     }
   }
   const int last_first = M ? most(first) : 0;  // tiles from here on see no first key
-  const int k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
+  const int k_hi = split < 0 ? kend : min(kend, k_lo + p.q_span);
   const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
   Stage<D> sk, sv;
   auto K = [&](int s) { return lds + 2 * s * kTile<D>; };
@@ -771,7 +773,7 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
   if (!live) return;
   if (split >= 0) {
     const int64_t row = (((int64_t)split * p.batch + b) * p.seq + query) * p.heads + h;
-    float* pq = p.part + row * D;
+    float* pq = p.q_part + row * D;
 #pragma unroll
     for (int db = 0; db < NB; ++db)
 #pragma unroll
@@ -792,11 +794,30 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
     }
 }
 
-template <int D, bool M>
-__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void mfma_attn_dq(MArgs p) {
-  const bool split = p.nsplit > 1;
-  const int z = gridDim.z - 1 - blockIdx.z;
-  dq_block<D, M>(p, split ? z / p.nsplit : z, blockIdx.y, split ? z % p.nsplit : -1);
+// Both sweeps in one launch: neither needs the other, and alone each leaves
+// the device part empty at its end (and, on small grids, all along).  The
+// first p's dK/dV workgroups, the first keys, the longest causal sweeps, first;
+// then the dQ ones, the last queries first.
+struct BwdArgs {
+  MArgs p;  // first: its members sit at MArgs' offsets
+  uint32_t n_dkdv;
+};
+
+template <int D, int DO, bool M>
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void mfma_attn_bwd(BwdArgs a) {
+  const MArgs& p = a.p;
+  if (blockIdx.x < a.n_dkdv) {
+    constexpr int halves = D / DO;
+    const int hk = blockIdx.x % p.kv_heads, b = blockIdx.x / p.kv_heads % p.batch, z = blockIdx.x / p.kv_heads / p.batch;
+    const bool split = p.nsplit > 1;
+    const int x = split ? z / p.nsplit : z;
+    dkdv_block<D, DO, M>(p, x / halves, x % halves, hk, b, split ? z % p.nsplit : -1);
+    return;
+  }
+  const uint32_t i = gridDim.x - 1 - blockIdx.x;  // (from the end: the last queries first)
+  const int h = i % p.heads, b = i / p.heads % p.batch, z = i / p.heads / p.batch;
+  const bool split = p.q_nsplit > 1;
+  dq_block<D, M>(p, split ? z / p.q_nsplit : z, h, b, split ? z % p.q_nsplit : -1);
 }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -839,7 +860,6 @@ int fwd_launch(const th_attention_desc* d, th_launch** out) {
   const int nqb = (d->seq + 127) / 128;
   const th::Split sp = th::split_of((int64_t)nqb * d->heads * d->batch, a.kv_seq);
   a.nsplit = sp.n, a.span = sp.span;
-  TH_REQUIRE((int64_t)nqb * sp.n <= 65535, "attention: grid too large");
   th::Builder b("attention_fwd_mfma", 7);
   const dim3 grid(d->heads, d->batch, nqb * sp.n);
   int k = b.kernel((const void*)mfma_attn_fwd<D, false>, D == 64 ? "mfma_attn_fwd_d64" : D == 128 ? "mfma_attn_fwd_d128"
@@ -871,82 +891,92 @@ int fwd_launch(const th_attention_desc* d, th_launch** out) {
   return TH_OK;
 }
 
-template <int D>
+constexpr int kMaskLds = 2 * 196 * sizeof(float) + 16;  // under masks: the dK/dV stages' statistics and four ints
+
+// The backward's launch: delta, both sweeps, and where small grids split
+// them (the dK/dV sweep over queries, the dQ sweep over keys) their sums.
+template <int D, bool M>
 int bwd_launch(const th_attention_desc* d, th_launch** out) {
   constexpr int DO = D == 256 ? 128 : D;
-  const size_t lds_kv = 4 * (size_t)kTile<D> * sizeof(uint16_t);
-  const size_t lds_dkdv = lds_kv + 2 * 128 * sizeof(float);
-  TH_HIP(hipFuncSetAttribute((const void*)mfma_attn_dkdv<D, DO, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)lds_dkdv));
-  TH_HIP(hipFuncSetAttribute((const void*)mfma_attn_dq<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_kv));
+  const size_t lds = 4 * (size_t)kTile<D> * sizeof(uint16_t) + (M ? kMaskLds : 2 * 128 * sizeof(float));
+  const void* fn = (const void*)mfma_attn_bwd<D, DO, M>;
+  TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   MArgs a = margs_of(d);
   th::Builder b("attention_bwd_mfma", 11);
   const int64_t rows = (int64_t)d->batch * d->seq * d->heads;
   const int64_t rows_k = (int64_t)d->batch * a.kv_seq * d->kv_heads;
-  const uint64_t at_delta = b.workspace((uint64_t)rows * sizeof(float));
-  // Small grids split the dK/dV sweep over queries and the dQ sweep over keys.
-  const int nkb = (a.kv_seq + 127) / 128, nqb = (d->seq + 127) / 128;
-  const th::Split skv = th::split_of((int64_t)nkb * (D / DO) * d->kv_heads * d->batch, d->seq);
-  const th::Split sq = th::split_of((int64_t)nqb * d->heads * d->batch, a.kv_seq);
-  TH_REQUIRE((int64_t)nkb * (D / DO) * skv.n <= 65535 && (int64_t)nqb * sq.n <= 65535, "attention: grid too large");
-  MArgs akv = a, aq = a;
-  akv.nsplit = skv.n, akv.span = skv.span;
-  aq.nsplit = sq.n, aq.span = sq.span;
   TH_REQUIRE(rows < 2147483648LL, "attention: batch x seq x heads must be under 2^31");
+  const uint64_t at_delta = b.workspace((uint64_t)rows * sizeof(float));
+  const int nkb = (a.kv_seq + 127) / 128, nqb = (d->seq + 127) / 128;
+  const int64_t gkv = (int64_t)nkb * (D / DO) * d->kv_heads * d->batch, gq = (int64_t)nqb * d->heads * d->batch;
+  const th::Split skv = M ? th::Split{1, 0} : th::split_of(gkv, d->seq, 384), sq = M ? th::Split{1, 0} : th::split_of(gq, a.kv_seq, 384);
+  a.nsplit = skv.n, a.span = skv.span;
+  a.q_nsplit = sq.n, a.q_span = sq.span;
+  const int64_t n_dkdv = gkv * skv.n, blocks = n_dkdv + gq * sq.n;
+  TH_REQUIRE(blocks <= 0x7fffffff, "attention: grid too large");
   constexpr int kDeltaBlockRows = 4 * (64 / (D / 8)) * kDeltaRowsM;  // rows a workgroup
-  int k0 = b.kernel((const void*)mfma_attn_delta<D>, "mfma_attn_delta",
-                    dim3((unsigned)((rows + kDeltaBlockRows - 1) / kDeltaBlockRows)), dim3(256), 0, DeltaArgs{a, D});
-  const dim3 gkv(d->kv_heads, d->batch, nkb * (D / DO) * skv.n), gq(d->heads, d->batch, nqb * sq.n);
-  int k1 = b.kernel((const void*)mfma_attn_dkdv<D, DO, false>, D == 64 ? "mfma_attn_dkdv_d64" : D == 128 ? "mfma_attn_dkdv_d128"
-                                                                                               : "mfma_attn_dkdv_d256",
-                    gkv, dim3(256), (uint32_t)lds_dkdv, akv);
-  if (skv.n > 1) {
-    const uint64_t at_kv = b.workspace((uint64_t)2 * skv.n * rows_k * D * sizeof(float));
-    b.ws_ref(k1, TH_OFFSET(MArgs, part), at_kv);
-    const unsigned g = (unsigned)((rows_k * (D / 4) + 255) / 256);
+  const int k0 = b.kernel((const void*)mfma_attn_delta<D>, "mfma_attn_delta",
+                          dim3((unsigned)((rows + kDeltaBlockRows - 1) / kDeltaBlockRows)), dim3(256), 0, DeltaArgs{a, D});
+  const char* name = M ? (D == 64 ? "mfma_attn_dkdv_masked_d64_mfma_attn_dq_masked_d64" : "mfma_attn_dkdv_masked_d128_mfma_attn_dq_masked_d128")
+                       : D == 64    ? "mfma_attn_dkdv_d64_mfma_attn_dq_d64"
+                       : D == 128   ? "mfma_attn_dkdv_d128_mfma_attn_dq_d128"
+                                    : "mfma_attn_dkdv_d256_mfma_attn_dq_d256";
+  const int k1 = b.kernel(fn, name, dim3((unsigned)blocks), dim3(256), (uint32_t)lds, BwdArgs{a, (uint32_t)n_dkdv});
+  const size_t offs[11] = {TH_OFFSET(MArgs, q),      TH_OFFSET(MArgs, k),  TH_OFFSET(MArgs, v),  TH_OFFSET(MArgs, o),
+                           TH_OFFSET(MArgs, lse),    TH_OFFSET(MArgs, dout), TH_OFFSET(MArgs, dq), TH_OFFSET(MArgs, dk),
+                           TH_OFFSET(MArgs, dv),     TH_OFFSET(MArgs, starts), TH_OFFSET(MArgs, lengths)};
+  // Both kernels' arguments begin with MArgs: the same offsets.
+  for (int kk : {k0, k1}) {
+    for (int v = 0; v < (M ? 11 : 9); ++v) b.ref(v, kk, offs[v]);
+    b.ws_ref(kk, TH_OFFSET(MArgs, delta), at_delta);
+  }
+  if (!M)
+    for (int v : {0, 1, 2, 3, 5, 6, 7, 8}) b.align(v, 16);
+  if (skv.n > 1 || sq.n > 1) {
+    SumArgs s{};
+    s.batch = d->batch, s.d = D;
     // The outputs' pointers start as the descriptor's (repointing rewrites them with the others).
-    SumArgs sk{nullptr, static_cast<uint16_t*>(d->dk), d->k_strides[0], d->k_strides[1], d->k_strides[2], a.kv_seq,
-               d->kv_heads, d->batch, D, skv.n, a.scale};
-    SumArgs sv = sk;
-    sv.out = static_cast<uint16_t*>(d->dv), sv.scale = 1.0f;
-    const int ks = b.kernel((const void*)mfma_attn_sum, "mfma_attn_sum_dk", dim3(g), dim3(256), 0, sk);
-    const int kv = b.kernel((const void*)mfma_attn_sum, "mfma_attn_sum_dv", dim3(g), dim3(256), 0, sv);
-    b.ws_ref(ks, TH_OFFSET(SumArgs, part), at_kv);
-    b.ws_ref(kv, TH_OFFSET(SumArgs, part), at_kv + (uint64_t)skv.n * rows_k * D * sizeof(float));
-    b.ref(7, ks, TH_OFFSET(SumArgs, out));
-    b.ref(8, kv, TH_OFFSET(SumArgs, out));
+    int values[3];
+    uint64_t ats[3];
+    unsigned total = 0;
+    auto add = [&](int value, uint16_t* to, const int64_t* strides, int positions, int heads, int parts, float scale,
+                   uint64_t at) {
+      const unsigned g = (unsigned)(((int64_t)d->batch * positions * heads * (D / 4) + 255) / 256);
+      values[s.n] = value, ats[s.n] = at;
+      s.of[s.n++] = SumArgsOne{nullptr, to, strides[0], strides[1], strides[2], positions, heads, parts, scale, g};
+      total += g;
+    };
+    if (skv.n > 1) {
+      const uint64_t at = b.workspace((uint64_t)2 * skv.n * rows_k * D * sizeof(float));
+      b.ws_ref(k1, TH_OFFSET(MArgs, part), at);
+      add(7, a.dk, d->k_strides, a.kv_seq, d->kv_heads, skv.n, a.scale, at);
+      add(8, a.dv, d->k_strides, a.kv_seq, d->kv_heads, skv.n, 1.0f, at + (uint64_t)skv.n * rows_k * D * sizeof(float));
+    }
+    if (sq.n > 1) {
+      const uint64_t at = b.workspace((uint64_t)sq.n * rows * D * sizeof(float));
+      b.ws_ref(k1, TH_OFFSET(MArgs, q_part), at);
+      add(6, a.dq, d->q_strides, d->seq, d->heads, sq.n, a.scale, at);
+    }
+    const int k2 = b.kernel((const void*)mfma_attn_sum,
+                            sq.n == 1   ? "mfma_attn_sum_dk_dv"
+                                                              : skv.n == 1 ? "mfma_attn_sum_dq"
+                                                                           : "mfma_attn_sum_dk_dv_mfma_attn_sum_dq",
+                            dim3(total), dim3(256), 0, s);
+    for (int i = 0; i < s.n; ++i) {
+      const size_t one = TH_OFFSET(SumArgs, of) + i * sizeof(SumArgsOne);
+      b.ref(values[i], k2, one + TH_OFFSET(SumArgsOne, out));
+      b.ws_ref(k2, one + TH_OFFSET(SumArgsOne, part), ats[i]);
+    }
   }
-  int k2 = b.kernel((const void*)mfma_attn_dq<D, false>, D == 64 ? "mfma_attn_dq_d64" : D == 128 ? "mfma_attn_dq_d128"
-                                                                                       : "mfma_attn_dq_d256",
-                    gq, dim3(256), (uint32_t)lds_kv, aq);
-  if (sq.n > 1) {
-    const uint64_t at_q = b.workspace((uint64_t)sq.n * rows * D * sizeof(float));
-    b.ws_ref(k2, TH_OFFSET(MArgs, part), at_q);
-    SumArgs s1{nullptr, static_cast<uint16_t*>(d->dq), d->q_strides[0], d->q_strides[1], d->q_strides[2], d->seq,
-               d->heads, d->batch, D, sq.n, a.scale};
-    const int kq = b.kernel((const void*)mfma_attn_sum, "mfma_attn_sum_dq", dim3((unsigned)((rows * (D / 4) + 255) / 256)),
-                            dim3(256), 0, s1);
-    b.ws_ref(kq, TH_OFFSET(SumArgs, part), at_q);
-    b.ref(6, kq, TH_OFFSET(SumArgs, out));
-  }
-  const size_t offs[9] = {TH_OFFSET(MArgs, q),  TH_OFFSET(MArgs, k),  TH_OFFSET(MArgs, v),
-                          TH_OFFSET(MArgs, o),  TH_OFFSET(MArgs, lse), TH_OFFSET(MArgs, dout),
-                          TH_OFFSET(MArgs, dq), TH_OFFSET(MArgs, dk),  TH_OFFSET(MArgs, dv)};
-  // The delta kernel's arguments are MArgs followed by d: the same offsets.
-  for (int v = 0; v < 9; ++v)
-    for (int kk : {k0, k1, k2}) b.ref(v, kk, offs[v]);
-  for (int kk : {k0, k1, k2}) b.ws_ref(kk, TH_OFFSET(MArgs, delta), at_delta);
-  for (int v : {0, 1, 2, 3, 5, 6, 7, 8}) b.align(v, 16);
   const double BH = (double)d->batch * d->heads, BHk = (double)d->batch * d->kv_heads;
   b.work(2.0 * BH * a.seq * D * 4 + 2.0 * BHk * a.kv_seq * D * 4 + 8.0 * BH * a.seq,
-         2.5 * 4.0 * BH * D * visible_pairs(a), (int64_t)gkv.x * gkv.y * gkv.z);
+         2.5 * 4.0 * BH * D * visible_pairs(a), n_dkdv);
   *out = b.release();
   return TH_OK;
 }
 
 // Under device-held masks (or rows the kernels above do not take): whole
 // sweeps, a workgroup per block of 128.
-constexpr int kMaskLds = 2 * 196 * sizeof(float) + 16;  // the dK/dV stages' statistics and four ints
 
 template <int D>
 int masked_fwd_launch(const th_attention_desc* d, th_launch** out) {
@@ -965,39 +995,6 @@ int masked_fwd_launch(const th_attention_desc* d, th_launch** out) {
   const double BH = (double)d->batch * d->heads, BHk = (double)d->batch * d->kv_heads;
   b.work(2.0 * BH * a.seq * D * 2 + 2.0 * BHk * a.kv_seq * D * 2 + 4.0 * BH * a.seq, 4.0 * BH * D * visible_pairs(a),
          (int64_t)grid.x * grid.y * grid.z);
-  *out = b.release();
-  return TH_OK;
-}
-
-template <int D>
-int masked_bwd_launch(const th_attention_desc* d, th_launch** out) {
-  const size_t tiles = 4 * (size_t)kTile<D> * sizeof(uint16_t), lds_dkdv = tiles + kMaskLds, lds_dq = tiles + 16;
-  const void *f1 = (const void*)mfma_attn_dkdv<D, D, true>, *f2 = (const void*)mfma_attn_dq<D, true>;
-  TH_HIP(hipFuncSetAttribute(f1, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dkdv));
-  TH_HIP(hipFuncSetAttribute(f2, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq));
-  MArgs a = margs_of(d);
-  th::Builder b("attention_bwd_mfma", 11);
-  const int64_t rows = (int64_t)d->batch * d->seq * d->heads;
-  const uint64_t at_delta = b.workspace((uint64_t)rows * sizeof(float));
-  constexpr int kDeltaBlockRows = 4 * (64 / (D / 8)) * kDeltaRowsM;
-  const int k0 = b.kernel((const void*)mfma_attn_delta<D>, "mfma_attn_delta",
-                          dim3((unsigned)((rows + kDeltaBlockRows - 1) / kDeltaBlockRows)), dim3(256), 0, DeltaArgs{a, D});
-  const dim3 gkv(d->kv_heads, d->batch, (a.kv_seq + 127) / 128), gq(d->heads, d->batch, (d->seq + 127) / 128);
-  const int k1 = b.kernel(f1, D == 64 ? "mfma_attn_dkdv_masked_d64" : "mfma_attn_dkdv_masked_d128", gkv, dim3(256),
-                          (uint32_t)lds_dkdv, a);
-  const int k2 = b.kernel(f2, D == 64 ? "mfma_attn_dq_masked_d64" : "mfma_attn_dq_masked_d128", gq, dim3(256),
-                          (uint32_t)lds_dq, a);
-  const size_t offs[11] = {TH_OFFSET(MArgs, q),      TH_OFFSET(MArgs, k),  TH_OFFSET(MArgs, v),  TH_OFFSET(MArgs, o),
-                           TH_OFFSET(MArgs, lse),    TH_OFFSET(MArgs, dout), TH_OFFSET(MArgs, dq), TH_OFFSET(MArgs, dk),
-                           TH_OFFSET(MArgs, dv),     TH_OFFSET(MArgs, starts), TH_OFFSET(MArgs, lengths)};
-  // The delta kernel's arguments are MArgs followed by d: the same offsets.
-  for (int kk : {k0, k1, k2}) {
-    for (int v = 0; v < 11; ++v) b.ref(v, kk, offs[v]);
-    b.ws_ref(kk, TH_OFFSET(MArgs, delta), at_delta);
-  }
-  const double BH = (double)d->batch * d->heads, BHk = (double)d->batch * d->kv_heads;
-  b.work(2.0 * BH * a.seq * D * 4 + 2.0 * BHk * a.kv_seq * D * 4 + 8.0 * BH * a.seq,
-         2.5 * 4.0 * BH * D * visible_pairs(a), (int64_t)gkv.x * gkv.y * gkv.z);
   *out = b.release();
   return TH_OK;
 }
@@ -1045,9 +1042,9 @@ int build_attention_mfma_fwd(const th_attention_desc* d, th_launch** out) {
 int build_attention_mfma_bwd(const th_attention_desc* d, th_launch** out) {
   if (int r = check_mfma(d, true)) return r;
   switch (d->head_dim) {
-    case 64: return bwd_launch<64>(d, out);
-    case 128: return bwd_launch<128>(d, out);
-    default: return bwd_launch<256>(d, out);
+    case 64: return bwd_launch<64, false>(d, out);
+    case 128: return bwd_launch<128, false>(d, out);
+    default: return bwd_launch<256, false>(d, out);
   }
 }
 
@@ -1064,7 +1061,7 @@ int build_attention_masked_fwd(const th_attention_desc* d, th_launch** out) {
 }
 
 int build_attention_masked_bwd(const th_attention_desc* d, th_launch** out) {
-  return d->head_dim == 64 ? masked_bwd_launch<64>(d, out) : masked_bwd_launch<128>(d, out);
+  return d->head_dim == 64 ? bwd_launch<64, true>(d, out) : bwd_launch<128, true>(d, out);
 }
 
 }  // namespace th

@@ -192,17 +192,20 @@ int rows_scratch_setup(int device);
 int device_alloc(size_t bytes, void** out);
 
 // The parts an attention sweep of `length` positions takes when `groups`
-// workgroups (unsplit, unpaired) would leave the device idle: enough for
-// about 512 workgroups where they are fewer than 256 (one a CU), at most 8,
+// workgroups (unsplit) would leave the device idle: enough for about `target`
+// workgroups where they are fewer than 256 (one a CU), at most 8,
 // each at least 128 positions (span, a multiple of 64).  Each wave's sweep
 // bounds a small grid; parts share it among more waves, at the cost of
-// fp32 partial results and a launch that adds them.
+// fp32 partial results and a launch that adds them.  Target 512 for a forward
+// (B2 H8 S1024 d64 18.8 us; 384: 20.6), 384 for each of a backward's sweeps, which
+// share their launch (B2 H8 S1024 d64 with the forward 55 us against 60 at 512,
+// 54 at 256; B1 H16 KV4 S1853 118, 127, 123).
 struct Split {
   int n, span;
 };
-inline Split split_of(int64_t groups, int length) {
+inline Split split_of(int64_t groups, int length, int target = 512) {
   if (groups >= 256 || length <= 128) return {1, 0};
-  int n = (int)std::min<int64_t>(8, (512 + groups - 1) / groups);
+  int n = (int)std::min<int64_t>(8, (target + groups - 1) / groups);
   n = std::min(n, (length + 127) / 128);
   if (n <= 1) return {1, 0};
   const int span = ((length + n - 1) / n + 63) / 64 * 64;
