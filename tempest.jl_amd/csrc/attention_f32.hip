@@ -1,13 +1,25 @@
-// Op class (c) for fp32 arrays on the matrix cores: v_mfma_f32_32x32x2_f32
-// (exact fp32 products, fp32 sums) at head dims 64 and 128, any lengths,
-// grouped heads, causal or not.  fp32 attention with device-held masks, and
-// other head dims, stay on attention_generic.hip.  The reference's cuTile
+// Op class (c) for fp32 arrays on the matrix cores at head dims 64 and 128, any
+// lengths, grouped heads, causal or not.  fp32 attention with device-held masks,
+// and other head dims, stay on attention_generic.hip.  The reference's cuTile
 // sweep takes fp32 arrays (its TF32 mode rounds the factors to 10 bits,
-// ext/cuTileExt/build.jl:326-532; TRIALS.md:2187); here the products are
-// exact, as its default precision asks (src/Compiler/runtime/target.jl:42-44).
+// ext/cuTileExt/build.jl:326-532; TRIALS.md:2187); here all of fp32's 24 bits
+// take part, as its default precision asks (src/Compiler/runtime/target.jl:42-44).
 //
-// The forms of the bf16 kernels of attention_mfma.hip, for one product of
-// depth 2 instead of 16:
+// The sweeps (*_parts) are the bf16 kernels' of attention_mfma.hip on operands
+// split into three bf16 parts, tiles on their way into LDS, P and dS in
+// registers: six products of parts (v_mfma_f32_32x32x16_bf16) for each product,
+// what they leave out at most 2^-25 of each a b.  The fp32 matrix cores take
+// 2.7 times as long for the same product.  Error against float64 over thirty
+// drawn shapes: 0.89 of the fp32 products' on average, at most 6.7e-7 where
+// theirs was 8.1e-7.  B2 H8 S1024 d64 causal, forward + backward: 168 us with
+// fp32 products, 124 so; S2048 469 and 309; B6 H16 KV8 S640 d128 568 and 471.  One
+// stage of LDS (the parts take 1.5 times fp32's bytes), the next tile in
+// registers, two barriers a step; bound by the vector work of the splits and
+// the wait at the barriers, the products being under half of the time.
+//
+// A block whose results are not finite, or all of whose staged values are under
+// 2^-90 (their lower parts fall under bf16's range), is computed again with fp32
+// products (v_mfma_f32_32x32x2_f32; *_block), forms of depth 2 instead of 16:
 //   - products over d (S' = K Q', S = Q K', dP = dO V'): lane half h takes d
 //     in [h D/2, (h + 1) D/2), step s the d h D/2 + s, so a lane's operand
 //     of four steps is one 16-byte read of a tile row (rows of D + 4 floats:
@@ -21,27 +33,20 @@
 //     lane's A operands of the NB blocks are NB adjacent floats of one tile
 //     row, one 8- or 16-byte read.
 // Everything else as there: tiles of 64 positions staged through registers a
-// step ahead (zeros past the sequence), one barrier a step, the online
-// softmax in exp2 units (folds.jl:186-222), P in fp32, lse = m + log(l);
-// the backward FA2's, deterministic: delta = rowsum(dO .* O); dK, dV per 128
-// keys sweeping the query tiles of each query head of the group; dQ per 128
-// queries sweeping the key tiles.  Keys past the keys' length and, causal,
-// keys after the query weigh 0; queries past the sequence are computed on
-// zeros and not stored.
+// step ahead (zeros past the sequence), the online softmax in exp2 units
+// (folds.jl:186-222), P in fp32, lse = m + log(l); the backward FA2's,
+// deterministic: delta = rowsum(dO .* O); dK, dV per 128 keys sweeping the query
+// tiles of each query head of the group; dQ per 128 queries sweeping the key
+// tiles.  Keys past the keys' length and, causal, keys after the query weigh 0;
+// queries past the sequence are computed on zeros and not stored.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 
+#include "attention_tiles.h"
 #include "th_core.h"
 
 namespace {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLn2 = 0.6931471805599453f;
 
 struct FArgs {
   const float* q;
@@ -71,12 +76,6 @@ struct FArgs {
 
 __device__ __forceinline__ f32x16 mfma2(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// The value lane l ^ 32 holds.
-__device__ __forceinline__ float other_half(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(threadIdx.x % 64 < 32 ? r[1] : r[0]);
 }
 
 template <int D>
@@ -291,13 +290,6 @@ __device__ __forceinline__ void fwd_block(const FArgs& p, const int qb, const in
   }
   store_rows<D>(p.o + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)query * p.q_ss, o, 1.0f / l);
   if (lh == 0 && p.lse) p.lse[((int64_t)b * p.seq + query) * p.heads + h] = (m + log2f(l)) * kLn2;
-}
-
-template <int D>
-__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void f32_attn_fwd(FArgs p) {
-  const bool split = p.nsplit > 1;
-  const int z = gridDim.z - 1 - blockIdx.z;  // the last queries first
-  fwd_block<D>(p, split ? z / p.nsplit : z, blockIdx.y, split ? z % p.nsplit : -1);
 }
 
 // The parts of a split forward combined: per (b, query, head) row, M = max
@@ -607,6 +599,426 @@ __device__ __forceinline__ void dq_block(const FArgs& p, const int qb, const int
   store_rows<D>(p.dq + qoff, dq, p.scale);
 }
 
+// ---- the sweeps in bf16 parts -------------------------------------------------------
+
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+// x = part 0 + part 1 + part 2 in bf16, two values a word (8 bits each, rounded
+// to nearest: what is left is at most 2^-27 of x).
+__device__ __forceinline__ void split2(float u, float v, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
+  w0 = pack2(u, v);
+  u -= __uint_as_float(w0 << 16), v -= __uint_as_float(w0 & 0xffff0000u);
+  w1 = pack2(u, v);
+  u -= __uint_as_float(w1 << 16), v -= __uint_as_float(w1 & 0xffff0000u);
+  w2 = pack2(u, v);
+}
+
+// An operand of eight values a lane, in its three parts.
+struct Parts {
+  bf16x8 of[3];
+};
+// Eight registers of an accumulator from register `at`.
+__device__ __forceinline__ Parts parts_of(const f32x16& x, const int at) {
+  u32x4 w[3];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    uint32_t w0, w1, w2;
+    split2(x[at + 2 * e], x[at + 2 * e + 1], w0, w1, w2);
+    w[0][e] = w0, w[1][e] = w1, w[2][e] = w2;
+  }
+  return Parts{{(bf16x8)w[0], (bf16x8)w[1], (bf16x8)w[2]}};
+}
+
+// c += a b: the products of parts down to 2^-18 of a b, the least first.
+__device__ __forceinline__ f32x16 mfma6(const Parts& a, const Parts& b, f32x16 c) {
+  c = mfma(a.of[2], b.of[0], c);
+  c = mfma(a.of[1], b.of[1], c);
+  c = mfma(a.of[0], b.of[2], c);
+  c = mfma(a.of[1], b.of[0], c);
+  c = mfma(a.of[0], b.of[1], c);
+  return mfma(a.of[0], b.of[0], c);
+}
+
+template <int D>
+constexpr int kPart = 64 * (D + 8);  // bf16 elements of one part of a tile
+template <int D>
+constexpr int kTileP = 3 * kPart<D>;
+
+template <int D>
+__device__ __forceinline__ Parts rows3(const uint16_t* t, int r0, int ks) {
+  return Parts{{frag_rows<D>(t, r0, ks), frag_rows<D>(t + kPart<D>, r0, ks), frag_rows<D>(t + 2 * kPart<D>, r0, ks)}};
+}
+template <int D>
+__device__ __forceinline__ Parts tr3(const uint16_t* t, int d0, int ks) {
+  return Parts{{frag_tr<D>(t, d0, ks), frag_tr<D>(t + kPart<D>, d0, ks), frag_tr<D>(t + 2 * kPart<D>, d0, ks)}};
+}
+
+// A position's row as the B operand of a product over d: d = 16 ks + 8 (lane /
+// 32) + (0..7); zeros for a position past the end.
+template <int D>
+__device__ __forceinline__ void row_parts(const float* row, bool live, Parts (&f)[D / 16]) {
+  const int lh = threadIdx.x % 64 / 32;
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) {
+    const float* at = row + 16 * ks + 8 * lh;
+    const f32x4 lo = live ? *reinterpret_cast<const f32x4*>(at) : f32x4{}, hi = live ? *reinterpret_cast<const f32x4*>(at + 4) : f32x4{};
+    u32x4 w[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const f32x4& x = e < 2 ? lo : hi;
+      uint32_t w0, w1, w2;
+      split2(x[2 * (e % 2)], x[2 * (e % 2) + 1], w0, w1, w2);
+      w[0][e] = w0, w[1][e] = w1, w[2][e] = w2;
+    }
+    f[ks] = Parts{{(bf16x8)w[0], (bf16x8)w[1], (bf16x8)w[2]}};
+  }
+}
+
+// A tile loaded into registers (StageF) and stored in its parts; `most`: the
+// largest leading parts this thread has stored.
+template <int D>
+struct StageP : StageF<D> {
+  u16x2 most = {0, 0};
+  __device__ void store(uint16_t* t) {
+#pragma unroll
+    for (int i = 0; i < StageF<D>::kPer; ++i) {
+      const int c = threadIdx.x + 256 * i, row = c / StageF<D>::kChunks, col = c % StageF<D>::kChunks;
+      const f32x4& x = this->r[i];
+      u32x2 w[3];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        uint32_t w0, w1, w2;
+        split2(x[2 * e], x[2 * e + 1], w0, w1, w2);
+        w[0][e] = w0, w[1][e] = w1, w[2][e] = w2;
+        most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, w0 & 0x7fff7fffu));
+      }
+#pragma unroll
+      for (int s = 0; s < 3; ++s) *reinterpret_cast<u32x2*>(t + s * kPart<D> + row * (D + 8) + 4 * col) = w[s];
+    }
+  }
+  // Whether all it stored was under 2^-90, and not all zero: the lower parts
+  // then fall under bf16's normal range.
+  __device__ bool tiny() const {
+    const int x = max((int)most[0], (int)most[1]);
+    return x > 0 && x < (127 - 90) << 7;
+  }
+};
+
+// d = 32 db + 8 g + 4 lh + (0..3) of a lane's position: out = x sc.
+template <int D>
+__device__ __forceinline__ void store_quads(float* row, const f32x16 (&x)[D / 32], float sc) {
+  const int lh = threadIdx.x % 64 / 32;
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(row + 32 * db + 8 * g + 4 * lh) =
+          f32x4{x[db][4 * g], x[db][4 * g + 1], x[db][4 * g + 2], x[db][4 * g + 3]} * sc;
+}
+template <int N>
+__device__ __forceinline__ bool finite(const f32x16 (&x)[N]) {
+  bool f = true;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) f = f && fabsf(x[i][e]) < INFINITY;
+  return f;
+}
+
+// fwd_block in bf16 parts; false, and nothing stored, where it has to be
+// computed in fp32 products.
+template <int D>
+__device__ __forceinline__ bool fwd_parts(const FArgs& p, const int qb, const int b, const int split) {
+  constexpr int NS = D / 16, NB = D / 32;
+  extern __shared__ __attribute__((aligned(16))) float flds[];
+  uint16_t* K = reinterpret_cast<uint16_t*>(flds);
+  uint16_t* V = K + kTileP<D>;
+  const int h = blockIdx.x;
+  const int hk = h / (p.heads / p.kv_heads);
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
+  const int q0 = __builtin_amdgcn_readfirstlane(qb * 128 + wave * 32), query = q0 + lr;
+  const float* kbase = p.k + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
+  const float* vbase = p.v + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
+  Parts qf[NS];
+  row_parts<D>(p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)query * p.q_ss, query < p.seq, qf);
+  f32x16 o[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) o[i] = f32x16{};
+  float m = -INFINITY, l = 0.0f;
+  const float c = p.scale * kLog2e;
+  const int qlast = min(qb * 128 + 127, p.seq - 1);
+  const int kend = p.causal ? min(p.kv_seq, qlast + 1) : p.kv_seq;
+  const int k_lo = split < 0 ? 0 : split * p.span, k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
+  const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
+  StageP<D> sk, sv;
+  if (nsteps > 0) {
+    sk.load(kbase, p.k_ss, k_lo, p.kv_seq);
+    sv.load(vbase, p.k_ss, k_lo, p.kv_seq);
+  }
+  for (int j = 0; j < nsteps; ++j) {
+    const int k0 = k_lo + 64 * j;
+    __syncthreads();  // the previous step's tile is read
+    sk.store(K);
+    sv.store(V);
+    if (j + 1 < nsteps) {
+      sk.load(kbase, p.k_ss, k0 + 64, p.kv_seq);
+      sv.load(vbase, p.k_ss, k0 + 64, p.kv_seq);
+    }
+    __syncthreads();
+    // S' (64 keys x 32 queries): key 32 kb + 8 (i / 4) + 4 lh + i % 4 in register i.
+    f32x16 s[2] = {f32x16{}, f32x16{}};
+#pragma unroll
+    for (int ks = 0; ks < NS; ++ks)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) s[kb] = mfma6(rows3<D>(K, 32 * kb, ks), qf[ks], s[kb]);
+    if (k0 + 64 > p.kv_seq || (p.causal && k0 + 63 > q0)) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
+          if (key >= p.kv_seq || (p.causal && key > query)) s[kb][i] = -INFINITY;
+        }
+    }
+    float mb = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mb = fmaxf(mb, s[kb][i]);
+    mb = fmaxf(mb, other_half(mb)) * c;
+    const float mn = fmaxf(m, mb);
+    const float shift = isfinite(mn) ? mn : 0.0f;  // lse_shift (folds.jl:194)
+    const float alpha = __builtin_amdgcn_exp2f(m - shift);
+    l *= alpha;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) o[i] *= alpha;
+    m = mn;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        s[kb][i] = __builtin_amdgcn_exp2f(fmaf(s[kb][i], c, -shift));
+        l += s[kb][i];
+      }
+      // O' (D x 32 queries) += V' P'.
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const Parts pw = parts_of(s[kb], 8 * half);
+#pragma unroll
+        for (int db = 0; db < NB; ++db) o[db] = mfma6(tr3<D>(V, 32 * db, 2 * kb + half), pw, o[db]);
+      }
+    }
+  }
+  l += other_half(l);
+  const bool good = query >= p.seq || (finite(o) && fabsf(l) < INFINITY);
+  if (__syncthreads_or(!good || sk.tiny() || sv.tiny())) return false;
+  if (query >= p.seq) return true;
+  if (split >= 0) {
+    const int64_t row = (((int64_t)split * p.batch + b) * p.seq + query) * p.heads + h;
+    store_quads<D>(p.part + row * D, o, 1.0f);
+    if (lh == 0) reinterpret_cast<f32x2*>(p.part_ml)[row] = f32x2{m, l};
+    return true;
+  }
+  store_quads<D>(p.o + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)query * p.q_ss, o, 1.0f / l);
+  if (lh == 0 && p.lse) p.lse[((int64_t)b * p.seq + query) * p.heads + h] = (m + log2f(l)) * kLn2;
+  return true;
+}
+
+// dkdv_block in bf16 parts; false, and nothing stored, as fwd_parts.
+template <int D>
+__device__ __forceinline__ bool dkdv_parts(const FArgs& p, const int kblk, const int hk, const int b, const int split) {
+  constexpr int NS = D / 16, NB = D / 32;
+  extern __shared__ __attribute__((aligned(16))) float flds[];
+  uint16_t* Q = reinterpret_cast<uint16_t*>(flds);
+  uint16_t* G = Q + kTileP<D>;
+  float* L = reinterpret_cast<float*>(G + kTileP<D>);  // lse * log2e (64) | delta (64)
+  const int group = p.heads / p.kv_heads;
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lh = lane / 32;
+  const int kw = __builtin_amdgcn_readfirstlane(kblk * 128 + wave * 32), key = kw + lane % 32;
+  const int64_t koff = (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
+  Parts kf[NS], vf[NS];
+  row_parts<D>(p.k + koff + (int64_t)key * p.k_ss, key < p.kv_seq, kf);
+  row_parts<D>(p.v + koff + (int64_t)key * p.k_ss, key < p.kv_seq, vf);
+  f32x16 dk[NB], dv[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) dk[i] = f32x16{}, dv[i] = f32x16{};
+  const float c = p.scale * kLog2e;
+  const int qfirst = p.causal ? kblk * 128 : 0;
+  const int qstart = split < 0 ? qfirst : qfirst + split * p.span;
+  const int qstop = split < 0 ? p.seq : min(p.seq, qstart + p.span);
+  const int nsteps = qstart < qstop ? (qstop - qstart + 63) / 64 : 0;
+  StageP<D> sq, sg;
+  float st = 0.0f;  // threads 0..127: a query's lse * log2e or delta
+  auto load = [&](int h, int q0) {
+    const int64_t qoff = (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
+    sq.load(p.q + qoff, p.q_ss, q0, p.seq);
+    sg.load(p.dout + qoff, p.q_ss, q0, p.seq);
+    if (threadIdx.x < 128) {
+      const int j = q0 + threadIdx.x % 64;
+      const int64_t row = ((int64_t)b * p.seq + j) * p.heads + h;
+      st = j < p.seq ? (threadIdx.x < 64 ? p.lse[row] * kLog2e : p.delta[row]) : 0.0f;
+    }
+  };
+  const int total = nsteps * group;  // steps over the group's query heads
+  if (total > 0) load(hk * group, qstart);
+  for (int j = 0, q = 0, h = hk * group; j < total; ++j) {
+    const int qq0 = qstart + 64 * q;
+    if (++q == nsteps) q = 0, ++h;
+    __syncthreads();  // the previous step's tile is read
+    sq.store(Q);
+    sg.store(G);
+    if (threadIdx.x < 128) L[threadIdx.x] = st;
+    if (j + 1 < total) load(h, qstart + 64 * q);
+    __syncthreads();
+    const bool edge = qq0 + 64 > p.seq || kw + 32 > p.kv_seq || (p.causal && kw + 31 > qq0);
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      // S = Q K', dP = dO V' (32 queries x 32 keys): query 32 jj + 8 (i / 4) + 4 lh + i % 4 in register i.
+      f32x16 s = {}, dp = {};
+#pragma unroll
+      for (int ks = 0; ks < NS; ++ks) {
+        s = mfma6(rows3<D>(Q, 32 * jj, ks), kf[ks], s);
+        dp = mfma6(rows3<D>(G, 32 * jj, ks), vf[ks], dp);
+      }
+      // P into s, dS into dp.
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int qi = 32 * jj + 8 * (i / 4) + 4 * lh + i % 4;
+        s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c, -L[qi]));
+        dp[i] = s[i] * (dp[i] - L[64 + qi]);
+      }
+      if (edge) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int query = qq0 + 32 * jj + 8 * (i / 4) + 4 * lh + i % 4;
+          const bool seen = query < p.seq && key < p.kv_seq && (!p.causal || key <= query);
+          s[i] = seen ? s[i] : 0.0f;
+          dp[i] = seen ? dp[i] : 0.0f;
+        }
+      }
+      // dV' (D x 32 keys) += dO' P;  dK' += Q' dS.
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const Parts pw = parts_of(s, 8 * half), sw = parts_of(dp, 8 * half);
+#pragma unroll
+        for (int db = 0; db < NB; ++db) {
+          dv[db] = mfma6(tr3<D>(G, 32 * db, 2 * jj + half), pw, dv[db]);
+          dk[db] = mfma6(tr3<D>(Q, 32 * db, 2 * jj + half), sw, dk[db]);
+        }
+      }
+    }
+  }
+  const bool good = key >= p.kv_seq || (finite(dk) && finite(dv));
+  if (__syncthreads_or(!good || sq.tiny() || sg.tiny())) return false;
+  if (key >= p.kv_seq) return true;
+  if (split >= 0) {
+    const int64_t rows = (int64_t)p.batch * p.kv_seq * p.kv_heads;
+    const int64_t row = (((int64_t)split * p.batch + b) * p.kv_seq + key) * p.kv_heads + hk;
+    store_quads<D>(p.part + row * D, dk, 1.0f);
+    store_quads<D>(p.part + ((int64_t)p.nsplit * rows + row) * D, dv, 1.0f);
+    return true;
+  }
+  const int64_t out = koff + (int64_t)key * p.k_ss;
+  store_quads<D>(p.dk + out, dk, p.scale);
+  store_quads<D>(p.dv + out, dv, 1.0f);
+  return true;
+}
+
+// dq_block in bf16 parts; false, and nothing stored, as fwd_parts.
+template <int D>
+__device__ __forceinline__ bool dq_parts(const FArgs& p, const int qb, const int h, const int b, const int split) {
+  constexpr int NS = D / 16, NB = D / 32;
+  extern __shared__ __attribute__((aligned(16))) float flds[];
+  uint16_t* K = reinterpret_cast<uint16_t*>(flds);
+  uint16_t* V = K + kTileP<D>;
+  const int hk = h / (p.heads / p.kv_heads);
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lh = lane / 32;
+  const int q0 = __builtin_amdgcn_readfirstlane(qb * 128 + wave * 32), query = q0 + lane % 32;
+  const int64_t qoff = (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)query * p.q_ss;
+  const bool live = query < p.seq;
+  Parts qf[NS], gf[NS];
+  row_parts<D>(p.q + qoff, live, qf);
+  row_parts<D>(p.dout + qoff, live, gf);
+  const int64_t srow = ((int64_t)b * p.seq + query) * p.heads + h;
+  const float l2 = live ? p.lse[srow] * kLog2e : 0.0f;
+  const float dl = live ? p.delta[srow] : 0.0f;
+  const float c = p.scale * kLog2e;
+  const float* kbase = p.k + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
+  const float* vbase = p.v + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
+  f32x16 dq[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) dq[i] = f32x16{};
+  const int qlast = min(qb * 128 + 127, p.seq - 1);
+  const int kend = p.causal ? min(p.kv_seq, qlast + 1) : p.kv_seq;
+  const int k_lo = split < 0 ? 0 : split * p.q_span, k_hi = split < 0 ? kend : min(kend, k_lo + p.q_span);
+  const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
+  StageP<D> sk, sv;
+  if (nsteps > 0) {
+    sk.load(kbase, p.k_ss, k_lo, p.kv_seq);
+    sv.load(vbase, p.k_ss, k_lo, p.kv_seq);
+  }
+  for (int j = 0; j < nsteps; ++j) {
+    const int k0 = k_lo + 64 * j;
+    __syncthreads();  // the previous step's tile is read
+    sk.store(K);
+    sv.store(V);
+    if (j + 1 < nsteps) {
+      sk.load(kbase, p.k_ss, k0 + 64, p.kv_seq);
+      sv.load(vbase, p.k_ss, k0 + 64, p.kv_seq);
+    }
+    __syncthreads();
+    const bool edge = k0 + 64 > p.kv_seq || (p.causal && k0 + 63 > q0);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      f32x16 s = {}, dp = {};
+#pragma unroll
+      for (int ks = 0; ks < NS; ++ks) {
+        s = mfma6(rows3<D>(K, 32 * kb, ks), qf[ks], s);
+        dp = mfma6(rows3<D>(V, 32 * kb, ks), gf[ks], dp);
+      }
+      // dS' into s.
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c, -l2)) * (dp[i] - dl);
+      if (edge) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
+          s[i] = key < p.kv_seq && (!p.causal || key <= query) ? s[i] : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const Parts sw = parts_of(s, 8 * half);
+#pragma unroll
+        for (int db = 0; db < NB; ++db) dq[db] = mfma6(tr3<D>(K, 32 * db, 2 * kb + half), sw, dq[db]);
+      }
+    }
+  }
+  if (__syncthreads_or((live && !finite(dq)) || sk.tiny() || sv.tiny())) return false;
+  if (!live) return true;
+  if (split >= 0)
+    store_quads<D>(p.q_part + ((((int64_t)split * p.batch + b) * p.seq + query) * p.heads + h) * D, dq, 1.0f);
+  else
+    store_quads<D>(p.dq + qoff, dq, p.scale);
+  return true;
+}
+
+// ---- the kernels ----------------------------------------------------------------------
+
+// LDS of either form: two tiles in parts, or two stages of two fp32 tiles.
+template <int D>
+constexpr size_t kLdsF = (2 * kTileP<D> * sizeof(uint16_t) > 4 * kTileF<D> * sizeof(float) ? 2 * kTileP<D> * sizeof(uint16_t)
+                                                                                           : 4 * kTileF<D> * sizeof(float)) +
+                         2 * 128 * sizeof(float);
+
+template <int D>
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void f32_attn_fwd(FArgs p) {
+  const bool split = p.nsplit > 1;
+  const int z = gridDim.z - 1 - blockIdx.z;  // the last queries first
+  const int qb = split ? z / p.nsplit : z, part = split ? z % p.nsplit : -1;
+  if (!fwd_parts<D>(p, qb, blockIdx.y, part)) fwd_block<D>(p, qb, blockIdx.y, part);
+}
+
 // Both sweeps in one launch: neither needs the other, and alone each leaves
 // the device part empty at its end.  dK/dV workgroups, the first keys, the
 // longest causal sweeps, first; then the dQ ones, the last queries first.
@@ -615,21 +1027,22 @@ struct FBwdArgs {
   uint32_t n_dkdv;
 };
 
-// One wave a SIMD: at d = 64 two would spill 10 registers (B2 H8 S2048, forward
-// and backward, 610 us against 468; S1024 179 against 181).
+// One wave a SIMD: with two, d = 64 spills around its sweeps.
 template <int D>
 __global__ __launch_bounds__(256, 1) void f32_attn_bwd(FBwdArgs a) {
   const FArgs& p = a.p;
   if (blockIdx.x < a.n_dkdv) {
     const int hk = blockIdx.x % p.kv_heads, b = blockIdx.x / p.kv_heads % p.batch, z = blockIdx.x / p.kv_heads / p.batch;
     const bool split = p.nsplit > 1;
-    dkdv_block<D>(p, split ? z / p.nsplit : z, hk, b, split ? z % p.nsplit : -1);
+    const int kblk = split ? z / p.nsplit : z, part = split ? z % p.nsplit : -1;
+    if (!dkdv_parts<D>(p, kblk, hk, b, part)) dkdv_block<D>(p, kblk, hk, b, part);
     return;
   }
   const uint32_t i = gridDim.x - 1 - blockIdx.x;  // (from the end: the last queries first)
   const int h = i % p.heads, b = i / p.heads % p.batch, z = i / p.heads / p.batch;
   const bool split = p.q_nsplit > 1;
-  dq_block<D>(p, split ? z / p.q_nsplit : z, h, b, split ? z % p.q_nsplit : -1);
+  const int qb = split ? z / p.q_nsplit : z, part = split ? z % p.q_nsplit : -1;
+  if (!dq_parts<D>(p, qb, h, b, part)) dq_block<D>(p, qb, h, b, part);
 }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -663,7 +1076,7 @@ double visible_pairs(const FArgs& a) {
 
 template <int D>
 int fwd_launch(const th_attention_desc* d, th_launch** out) {
-  const size_t lds = 4 * (size_t)kTileF<D> * sizeof(float);
+  const size_t lds = kLdsF<D>;
   TH_HIP(hipFuncSetAttribute((const void*)f32_attn_fwd<D>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   FArgs a = fargs_of(d);
   const int nqb = (d->seq + 127) / 128;
@@ -703,7 +1116,7 @@ int fwd_launch(const th_attention_desc* d, th_launch** out) {
 // them (the dK/dV sweep over queries, the dQ sweep over keys) their sums.
 template <int D>
 int bwd_launch(const th_attention_desc* d, th_launch** out) {
-  const size_t lds = 4 * (size_t)kTileF<D> * sizeof(float) + 2 * 128 * sizeof(float);
+  const size_t lds = kLdsF<D>;
   const void* fn = (const void*)f32_attn_bwd<D>;
   TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   FArgs a = fargs_of(d);

@@ -1,5 +1,5 @@
-"""fp32 attention on the matrix cores (v_mfma_f32_32x32x2_f32, exact fp32
-products and sums) at head dims 64 and 128: causal or not, grouped heads,
+"""fp32 attention on the matrix cores (each factor in three bf16 parts, fp32
+products where those do not reach) at head dims 64 and 128: causal or not, grouped heads,
 lengths that are not multiples of the 64-position tiles, more or fewer keys
 than queries.  Forward (o, lse) and backward (dq, dk, dv) against the float64
 oracle on the same inputs, to the fp32 tolerance; and the kernels that ran
@@ -8,7 +8,9 @@ import pytest
 import torch
 
 from conftest import announce
-from test_gpu_attention_general import TOL_F32, _check, _run
+from oracle import interpret
+from oracle.data import relative
+from test_gpu_attention_general import TOL_F32, _check, _np, _run
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +63,33 @@ def test_fp32_split_and_whole_sweeps(target, D, B, H, KV, S, causal, split):
     assert ("f32_attn_combine" in fwd.describe()) == split, fwd.describe()
     assert ("f32_attn_sum_dk" in bwd.describe() and "f32_attn_sum_dq" in bwd.describe()) == split, bwd.describe()
     _check(outs, q, k, v, g, causal, TOL_F32)
+
+
+@pytest.mark.parametrize("D,S,causal", [(64, 65, True), (64, 128, False), (64, 63, True), (128, 129, True),
+                                        (128, 64, False), (64, 1, True)])
+def test_fp32_values_out_of_the_parts_reach(target, D, S, causal):
+    """Tiles computed again with fp32 products: an infinity in V gives infinity
+    where it is seen and leaves the other features alone; gradients scaled far
+    under 2^-90 keep their relative accuracy, at the edges of tiles."""
+    announce("attn fp32 parts", D, S, causal)
+    gen = torch.Generator(device="cuda").manual_seed(D + S)
+    r = lambda: torch.randn(2, S, 2, D, device="cuda", generator=gen) * 0.5  # noqa: E731
+    q, k, v, g = r(), r(), r(), r()
+    outs, _ = _run(q, k, v, g, causal, True)
+    _check(outs, q, k, v, g, causal, TOL_F32)
+    small = g * 1e-30
+    outs, _ = _run(q, k, v, small, causal, True)
+    want = interpret.attention_bwd(*(_np(t) for t in (q, k, v, g)), causal)
+    for got, ref in zip(outs[2:], want):
+        assert relative(_np(got) * 1e30, ref) < TOL_F32, relative(_np(got) * 1e30, ref)
+    v[0, 0, 1, 3] = float("inf")
+    v[1, 0, 0, 5] = float("-inf")
+    outs, _ = _run(q, k, v, g, False, True)
+    o = outs[0]
+    assert torch.isposinf(o[0, :, 1, 3]).all() and torch.isneginf(o[1, :, 0, 5]).all()
+    rest = torch.ones_like(o, dtype=torch.bool)
+    rest[0, :, 1, 3] = rest[1, :, 0, 5] = False
+    clean = torch.where(torch.isfinite(v), v, torch.zeros_like(v))
+    ro, _ = interpret.attention_fwd(_np(q), _np(k), _np(clean), False)
+    keep = rest.cpu().numpy()
+    assert relative(_np(o)[keep], ro[keep]) < TOL_F32
