@@ -98,15 +98,53 @@ __device__ __forceinline__ int most(int x) {
   return __builtin_amdgcn_readfirstlane(x);
 }
 
-// The least of x over the workgroup's 256 threads, through four ints of LDS;
-// a barrier on both sides.
+// The least of x over the workgroup's 256 P threads, through 4 P ints of LDS; a
+// barrier on both sides.
+template <int P>
 __device__ __forceinline__ int least(int x, int* at) {
 #pragma unroll
   for (int i = 1; i < 64; i *= 2) x = min(x, __shfl_xor(x, i, 64));
   __syncthreads();
   if (threadIdx.x % 64 == 0) at[threadIdx.x / 64] = x;
   __syncthreads();
-  return min(min(at[0], at[1]), min(at[2], at[3]));
+  x = at[0];
+#pragma unroll
+  for (int i = 1; i < 4 * P; ++i) x = min(x, at[i]);
+  return x;
+}
+
+// P = 2: a workgroup of eight waves whose two halves take the tiles of one
+// sweep in turn, each with stages of its own, the second handing its fp32 sums
+// to the first through LDS at the end (a lane to the lane of the same place).
+// A sweep is a chain of steps, each waiting for the one before (about 1.5 us a
+// step of the forward, whatever the occupancy); where the sweeps are of uneven
+// length and few, the longest one is the launch's time, and this halves it.
+// The host takes it up to these workgroups, us before and after:
+//   causal forward whose keys are not split over workgroups, <= 512 (two a CU):
+//     B2 H16 S1853 d64 (480) 40.5 -> 35.0, B1 H16 S4000 d128 (512) 118 -> 103;
+//     1024: 54.6 -> 74.3, and sweeps of one length (not causal, 480) 45 -> 55.6,
+//     already split ones 53.5 -> 58 (with the backward);
+//   masked forward, <= 512: packed documents B2 H12 S2048 d64 (384), with the
+//     backward 114 -> 106; 768 workgroups 110 -> 118;
+//   masked backward at d64, <= 1024: the same documents (768) 106 -> 96,
+//     1 x 1500 x 8 heads 132 -> 90 in all; 1152 workgroups 133 -> 145.
+//   The unmasked backward gains nothing (600 workgroups 181 -> 192), and at d128
+//   one wave a SIMD holds a sweep.
+constexpr int64_t kFwdHalves = 512, kBwdHalves = 1024;
+
+template <int N>
+__device__ __forceinline__ void hand_over(const f32x16 (&x)[N], float* to) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) to[256 * (16 * i + e) + threadIdx.x % 256] = x[i][e];
+}
+template <int N>
+__device__ __forceinline__ void take_over(f32x16 (&x)[N], const float* from) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) x[i][e] += from[256 * (16 * i + e) + threadIdx.x % 256];
 }
 
 __device__ __forceinline__ float bf16_float(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
@@ -130,7 +168,7 @@ struct Stage {
   __device__ void load(const uint16_t* base, int64_t ss, int row0, int limit) {
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int c = threadIdx.x + 256 * i, row = c / kChunks, col = c % kChunks;
+      const int c = threadIdx.x % 256 + 256 * i, row = c / kChunks, col = c % kChunks;
       r[i] = row0 + row < limit ? (u32x4) * reinterpret_cast<const u32x4_any*>(base + (int64_t)(row0 + row) * ss + 8 * col)
                                 : u32x4{0, 0, 0, 0};
     }
@@ -138,7 +176,7 @@ struct Stage {
   __device__ void store(uint16_t* t) const {
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int c = threadIdx.x + 256 * i, row = c / kChunks, col = c % kChunks;
+      const int c = threadIdx.x % 256 + 256 * i, row = c / kChunks, col = c % kChunks;
       *reinterpret_cast<u32x4*>(t + row * (D + 8) + 8 * col) = r[i];
     }
   }
@@ -158,13 +196,13 @@ constexpr int kTile = 64 * (D + 8);  // bf16 elements of a tile in LDS
 // Keys [k_lo, k_hi) of query block qb: all of them (split < 0), or part
 // `split` of the sweep, which leaves its unnormalised O' and (m, l) for the
 // combining kernel.
-template <int D, bool M>
+template <int D, bool M, int P>
 __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const int b, const int split) {
   constexpr int NS = D / 16, NB = D / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   const int h = blockIdx.x;
   const int hk = h / (p.heads / p.kv_heads);
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
+  const int grp = P == 1 ? 0 : threadIdx.x / 256, wave = threadIdx.x / 64 % 4, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
   const int q0 = __builtin_amdgcn_readfirstlane(qb * 128 + wave * 32), query = q0 + lr;
   const uint16_t* qbase = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
   const uint16_t* kbase = p.k + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
@@ -183,27 +221,28 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
     // The sweep starts at the block's least first key, a wave's share of it at the wave's.
     if (p.starts) {
       first = query < p.seq ? first_of(p, query, b) : 0x7fffffff;
-      k_lo = max(0, min(least(first, reinterpret_cast<int*>(lds + 4 * kTile<D>)), nk)) / 64 * 64;
+      k_lo = max(0, min(least<P>(first, reinterpret_cast<int*>(lds + 4 * P * kTile<D>)), nk)) / 64 * 64;
     }
   }
   const int last_first = M ? most(first) : 0;  // tiles from here on see no first key
   const int k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
   const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
   Stage<D> sk, sv;
-  auto K = [&](int s) { return lds + 2 * s * kTile<D>; };
-  auto V = [&](int s) { return lds + (2 * s + 1) * kTile<D>; };
-  if (nsteps > 0) {
-    sk.load(kbase, p.k_ss, k_lo, nk);
-    sv.load(vbase, p.k_ss, k_lo, nk);
+  auto K = [&](int s) { return lds + (4 * grp + 2 * s) * kTile<D>; };
+  auto V = [&](int s) { return lds + (4 * grp + 2 * s + 1) * kTile<D>; };
+  const int mine = P == 1 ? nsteps : (nsteps + 1 - grp) / 2;  // tiles grp, grp + P, ...
+  if (mine > 0) {
+    sk.load(kbase, p.k_ss, k_lo + 64 * grp, nk);
+    sv.load(vbase, p.k_ss, k_lo + 64 * grp, nk);
     sk.store(K(0));
     sv.store(V(0));
   }
   __syncthreads();
-  for (int j = 0; j < nsteps; ++j) {
-    const int cur = j & 1, k0 = k_lo + 64 * j;
-    if (j + 1 < nsteps) {
-      sk.load(kbase, p.k_ss, k0 + 64, nk);
-      sv.load(vbase, p.k_ss, k0 + 64, nk);
+  auto step = [&](int j) {
+    const int cur = j & 1, k0 = k_lo + 64 * (P * j + grp);
+    if (j + 1 < mine) {
+      sk.load(kbase, p.k_ss, k0 + 64 * P, nk);
+      sv.load(vbase, p.k_ss, k0 + 64 * P, nk);
     }
     // S' (64 keys x 32 queries): keys 32 kb + 8 (i / 4) + 4 lh + i % 4 in register i.
     f32x16 s[2] = {f32x16{}, f32x16{}};
@@ -259,12 +298,33 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
         if constexpr (M) o[db] = mfma(vt, pl[ks], o[db]);
         o[db] = mfma(vt, pf[ks], o[db]);
       }
-    if (j + 1 < nsteps) {
+    if (j + 1 < mine) {
       // The other stage was last read in step j - 1, before the barrier that ended it.
       sk.store(K(cur ^ 1));
       sv.store(V(cur ^ 1));
     }
+  };
+  for (int j = 0; P * j < nsteps; ++j) {
+    if (P == 1 || j < mine) step(j);
     __syncthreads();
+  }
+  if constexpr (P == 2) {
+    float* x = reinterpret_cast<float*>(lds);
+    float* ml = x + 256 * 16 * NB;
+    if (grp == 1) {
+      hand_over(o, x);
+      ml[threadIdx.x % 256] = m, ml[256 + threadIdx.x % 256] = l;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    const float m1 = ml[threadIdx.x], mn = fmaxf(m, m1), shift = thd::lse_shift(mn);
+    const float a0 = __builtin_amdgcn_exp2f(m - shift), a1 = __builtin_amdgcn_exp2f(m1 - shift);
+    l = l * a0 + ml[256 + threadIdx.x] * a1;
+    m = mn;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[i][e] = o[i][e] * a0 + x[256 * (16 * i + e) + threadIdx.x] * a1;
   }
   l += other_half(l);
   if (query >= p.seq) return;
@@ -294,11 +354,11 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
   if (lh == 0 && p.lse) p.lse[((int64_t)b * p.seq + query) * p.heads + h] = (m + log2f(l)) * kLn2;
 }
 
-template <int D, bool M>
-__global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void mfma_attn_fwd(MArgs p) {
+template <int D, bool M, int P>
+__global__ __launch_bounds__(256 * P, D <= 128 ? 2 : 1) void mfma_attn_fwd(MArgs p) {
   const bool split = p.nsplit > 1;
   const int z = gridDim.z - 1 - blockIdx.z;  // the last queries, the longest sweeps, first
-  fwd_block<D, M>(p, split ? z / p.nsplit : z, blockIdx.y, split ? z % p.nsplit : -1);
+  fwd_block<D, M, P>(p, split ? z / p.nsplit : z, blockIdx.y, split ? z % p.nsplit : -1);
 }
 
 // The parts of a split forward combined: per (b, query, head) row, M = max
@@ -487,16 +547,16 @@ __device__ __forceinline__ void dkdv_half(const MArgs& p, const uint16_t* Qt, co
 
 // Query tiles [qstart, qstop) for the keys of kblk: all of them (split <
 // 0), or part `split` of the sweep, which leaves its unscaled fp32 dK', dV'.
-template <int D, int DO, bool M>
+template <int D, int DO, bool M, int P>
 __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const int dh, const int hk, const int b,
                                            const int split) {
   constexpr int NS = D / 16, NBO = DO / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   constexpr int kStats = M ? 196 : 128;
   // [stage][lse * log2e (64) | delta (64) | M: first keys, as ints (64) | their largest (1) | -]
-  float* stats = reinterpret_cast<float*>(lds + 4 * kTile<D>);
+  float* stats = reinterpret_cast<float*>(lds + 4 * P * kTile<D>);
   const int group = p.heads / p.kv_heads;
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
+  const int grp = P == 1 ? 0 : threadIdx.x / 256, tid = P == 1 ? threadIdx.x : threadIdx.x % 256, wave = tid / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
   const int kw0 = kblk * 128, key = kw0 + wave * 32 + lr;
   const int64_t koff = (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
   bf16x8 kf[NS], vf[NS];
@@ -506,9 +566,9 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
   f32x16 dk[NBO], dv[NBO];
 #pragma unroll
   for (int i = 0; i < NBO; ++i) dk[i] = f32x16{}, dv[i] = f32x16{};
-  auto Q = [&](int s) { return lds + 2 * s * kTile<D>; };
-  auto G = [&](int s) { return lds + (2 * s + 1) * kTile<D>; };
-  auto Ls = [&](int s) { return stats + kStats * s; };
+  auto Q = [&](int s) { return lds + (4 * grp + 2 * s) * kTile<D>; };
+  auto G = [&](int s) { return lds + (4 * grp + 2 * s + 1) * kTile<D>; };
+  auto Ls = [&](int s) { return stats + kStats * (2 * grp + s); };
   const int qfirst = p.causal ? kw0 / 64 * 64 : 0;
   int qstart = split < 0 ? qfirst : qfirst + split * p.span;
   int qstop = split < 0 ? p.seq : min(p.seq, qstart + p.span);
@@ -517,27 +577,28 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
     if (p.starts && kw0 < nk) {
       // The span of queries that see any of the block's keys.
       int lo = 0x7fffffff, hi = 0x7fffffff;  // hi: the least of -j
-      for (int j = qstart + threadIdx.x; j < qstop; j += 256)
+      for (int j = qstart + threadIdx.x; j < qstop; j += 256 * P)
         if (first_of(p, j, b) < kw0 + 128) lo = min(lo, j), hi = min(hi, -j);
-      int* at = reinterpret_cast<int*>(stats + 2 * kStats);
-      lo = least(lo, at), hi = least(hi, at);
+      int* at = reinterpret_cast<int*>(stats + 2 * P * kStats);
+      lo = least<P>(lo, at), hi = least<P>(hi, at);
       qstop = lo == 0x7fffffff ? qstart : 1 - hi;
       qstart = lo == 0x7fffffff ? qstart : lo / 64 * 64;
     }
   }
   const int nsteps = qstart < qstop ? (qstop - qstart + 63) / 64 : 0;
+  const int mine = P == 1 ? nsteps : (nsteps + 1 - grp) / 2;  // tiles grp, grp + P, ...
   Stage<D> sq, sg;
   int st_most = 0;
   float st = 0.0f;  // threads 0..127: a query's lse * log2e or delta
   auto load = [&](const uint16_t* qbase, const uint16_t* gbase, int h, int q0) {
     sq.load(qbase, p.q_ss, q0, p.seq);
     sg.load(gbase, p.q_ss, q0, p.seq);
-    if (threadIdx.x < 128) {
-      const int j = q0 + threadIdx.x % 64;
+    if (tid < 128) {
+      const int j = q0 + tid % 64;
       const int64_t row = ((int64_t)b * p.seq + j) * p.heads + h;
-      st = j < p.seq ? (threadIdx.x < 64 ? p.lse[row] * kLog2e : p.delta[row]) : 0.0f;
-    } else if (M && threadIdx.x < 192) {
-      const int j = q0 + threadIdx.x % 64;
+      st = j < p.seq ? (tid < 64 ? p.lse[row] * kLog2e : p.delta[row]) : 0.0f;
+    } else if (M && tid < 192) {
+      const int j = q0 + tid % 64;
       const int f = j < p.seq ? first_of(p, j, b) : 0x7fffffff;
       st = __int_as_float(f), st_most = most(f);
     }
@@ -545,20 +606,20 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
   auto store = [&](int s) {
     sq.store(Q(s));
     sg.store(G(s));
-    if (threadIdx.x < (M ? 192 : 128)) Ls(s)[threadIdx.x] = st;
-    if (M && threadIdx.x == 128) Ls(s)[192] = __int_as_float(st_most);
+    if (tid < (M ? 192 : 128)) Ls(s)[tid] = st;
+    if (M && tid == 128) Ls(s)[192] = __int_as_float(st_most);
   };
   for (int h = hk * group; h < (hk + 1) * group; ++h) {
     const uint16_t* qbase = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
     const uint16_t* gbase = p.dout + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
-    if (nsteps > 0) {
-      load(qbase, gbase, h, qstart);
+    if (mine > 0) {
+      load(qbase, gbase, h, qstart + 64 * grp);
       store(0);
     }
     __syncthreads();
-    for (int j = 0; j < nsteps; ++j) {
-      const int cur = j & 1, qq0 = qstart + 64 * j;
-      if (j + 1 < nsteps) load(qbase, gbase, h, qq0 + 64);
+    auto step = [&](int j) {
+      const int cur = j & 1, qq0 = qstart + 64 * (P * j + grp);
+      if (j + 1 < mine) load(qbase, gbase, h, qq0 + 64 * P);
       const uint16_t *Qt = Q(cur), *Gt = G(cur);
       const float* L = Ls(cur);
       const int kw = __builtin_amdgcn_readfirstlane(kw0 + wave * 32);
@@ -566,9 +627,23 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
       if constexpr (M) edge = edge || kw < __builtin_amdgcn_readfirstlane(__float_as_int(L[192]));
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) dkdv_half<D, DO, M>(p, Qt, Gt, L, jj, edge, qq0, key, nk, dh, kf, vf, dk, dv);
-      if (j + 1 < nsteps) store(cur ^ 1);
+      if (j + 1 < mine) store(cur ^ 1);
+    };
+    for (int j = 0; P * j < nsteps; ++j) {
+      if (P == 1 || j < mine) step(j);
       __syncthreads();
     }
+  }
+  if constexpr (P == 2) {
+    float* x = reinterpret_cast<float*>(lds);
+    if (grp == 1) {
+      hand_over(dk, x);
+      hand_over(dv, x + 256 * 16 * NBO);
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    take_over(dk, x);
+    take_over(dv, x + 256 * 16 * NBO);
   }
   // At D = 128 the key as an opaque copy, so that the output addresses below
   // are computed here rather than kept from the sweep's start: measured 4 %
@@ -613,12 +688,12 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
 
 // Keys [k_lo, k_hi) for query block qb: all of them (split < 0), or part
 // `split` of the sweep, which leaves its unscaled fp32 dQ'.
-template <int D, bool M>
+template <int D, bool M, int P>
 __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int h, const int b, const int split) {
   constexpr int NS = D / 16, NB = D / 32;
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   const int hk = h / (p.heads / p.kv_heads);
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
+  const int grp = P == 1 ? 0 : threadIdx.x / 256, wave = threadIdx.x / 64 % 4, lane = threadIdx.x % 64, lr = lane % 32, lh = lane / 32;
   const int q0 = __builtin_amdgcn_readfirstlane(qb * 128 + wave * 32), query = q0 + lr;
   const int64_t qoff = (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)query * p.q_ss;
   const bool live = query < p.seq;
@@ -641,27 +716,28 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
     // The sweep starts at the block's least first key, a wave's share of it at the wave's.
     if (p.starts) {
       first = query < p.seq ? first_of(p, query, b) : 0x7fffffff;
-      k_lo = max(0, min(least(first, reinterpret_cast<int*>(lds + 4 * kTile<D>)), nk)) / 64 * 64;
+      k_lo = max(0, min(least<P>(first, reinterpret_cast<int*>(lds + 4 * P * kTile<D>)), nk)) / 64 * 64;
     }
   }
   const int last_first = M ? most(first) : 0;  // tiles from here on see no first key
   const int k_hi = split < 0 ? kend : min(kend, k_lo + p.q_span);
   const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
   Stage<D> sk, sv;
-  auto K = [&](int s) { return lds + 2 * s * kTile<D>; };
-  auto V = [&](int s) { return lds + (2 * s + 1) * kTile<D>; };
-  if (nsteps > 0) {
-    sk.load(kbase, p.k_ss, k_lo, nk);
-    sv.load(vbase, p.k_ss, k_lo, nk);
+  auto K = [&](int s) { return lds + (4 * grp + 2 * s) * kTile<D>; };
+  auto V = [&](int s) { return lds + (4 * grp + 2 * s + 1) * kTile<D>; };
+  const int mine = P == 1 ? nsteps : (nsteps + 1 - grp) / 2;  // tiles grp, grp + P, ...
+  if (mine > 0) {
+    sk.load(kbase, p.k_ss, k_lo + 64 * grp, nk);
+    sv.load(vbase, p.k_ss, k_lo + 64 * grp, nk);
     sk.store(K(0));
     sv.store(V(0));
   }
   __syncthreads();
-  for (int j = 0; j < nsteps; ++j) {
-    const int cur = j & 1, k0 = k_lo + 64 * j;
-    if (j + 1 < nsteps) {
-      sk.load(kbase, p.k_ss, k0 + 64, nk);
-      sv.load(vbase, p.k_ss, k0 + 64, nk);
+  auto step = [&](int j) {
+    const int cur = j & 1, k0 = k_lo + 64 * (P * j + grp);
+    if (j + 1 < mine) {
+      sk.load(kbase, p.k_ss, k0 + 64 * P, nk);
+      sv.load(vbase, p.k_ss, k0 + 64 * P, nk);
     }
     f32x16 s[2] = {f32x16{}, f32x16{}}, dp[2] = {f32x16{}, f32x16{}};
 #pragma unroll
@@ -709,11 +785,21 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
         if constexpr (M) dq[db] = mfma(kt, sl[ks], dq[db]);
         dq[db] = mfma(kt, sf[ks], dq[db]);
       }
-    if (j + 1 < nsteps) {
+    if (j + 1 < mine) {
       sk.store(K(cur ^ 1));
       sv.store(V(cur ^ 1));
     }
+  };
+  for (int j = 0; P * j < nsteps; ++j) {
+    if (P == 1 || j < mine) step(j);
     __syncthreads();
+  }
+  if constexpr (P == 2) {
+    float* x = reinterpret_cast<float*>(lds);
+    if (grp == 1) hand_over(dq, x);
+    __syncthreads();
+    if (grp == 1) return;
+    take_over(dq, x);
   }
   if (!live) return;
   if (split >= 0) {
@@ -748,21 +834,21 @@ struct BwdArgs {
   uint32_t n_dkdv;
 };
 
-template <int D, int DO, bool M>
-__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void mfma_attn_bwd(BwdArgs a) {
+template <int D, int DO, bool M, int P>
+__global__ __launch_bounds__(256 * P, D <= 64 ? 2 : 1) void mfma_attn_bwd(BwdArgs a) {
   const MArgs& p = a.p;
   if (blockIdx.x < a.n_dkdv) {
     constexpr int halves = D / DO;
     const int hk = blockIdx.x % p.kv_heads, b = blockIdx.x / p.kv_heads % p.batch, z = blockIdx.x / p.kv_heads / p.batch;
     const bool split = p.nsplit > 1;
     const int x = split ? z / p.nsplit : z;
-    dkdv_block<D, DO, M>(p, x / halves, x % halves, hk, b, split ? z % p.nsplit : -1);
+    dkdv_block<D, DO, M, P>(p, x / halves, x % halves, hk, b, split ? z % p.nsplit : -1);
     return;
   }
   const uint32_t i = gridDim.x - 1 - blockIdx.x;  // (from the end: the last queries first)
   const int h = i % p.heads, b = i / p.heads % p.batch, z = i / p.heads / p.batch;
   const bool split = p.q_nsplit > 1;
-  dq_block<D, M>(p, split ? z / p.q_nsplit : z, h, b, split ? z % p.q_nsplit : -1);
+  dq_block<D, M, P>(p, split ? z / p.q_nsplit : z, h, b, split ? z % p.q_nsplit : -1);
 }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -799,17 +885,19 @@ double visible_pairs(const MArgs& a) {
 
 template <int D>
 int fwd_launch(const th_attention_desc* d, th_launch** out) {
-  const size_t lds = 4 * (size_t)kTile<D> * sizeof(uint16_t);
-  TH_HIP(hipFuncSetAttribute((const void*)mfma_attn_fwd<D, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   MArgs a = margs_of(d);
   const int nqb = (d->seq + 127) / 128;
   const th::Split sp = th::split_of((int64_t)nqb * d->heads * d->batch, a.kv_seq);
   a.nsplit = sp.n, a.span = sp.span;
   th::Builder b("attention_fwd_mfma", 7);
   const dim3 grid(d->heads, d->batch, nqb * sp.n);
-  int k = b.kernel((const void*)mfma_attn_fwd<D, false>, D == 64 ? "mfma_attn_fwd_d64" : D == 128 ? "mfma_attn_fwd_d128"
+  const int P = D <= 128 && d->causal && sp.n == 1 && (int64_t)grid.x * grid.y * grid.z <= kFwdHalves ? 2 : 1;
+  const size_t lds = 4 * P * (size_t)kTile<D> * sizeof(uint16_t);
+  const void* fn = P == 2 ? (const void*)mfma_attn_fwd<D, false, D <= 128 ? 2 : 1> : (const void*)mfma_attn_fwd<D, false, 1>;
+  TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  int k = b.kernel(fn, D == 64 ? "mfma_attn_fwd_d64" : D == 128 ? "mfma_attn_fwd_d128"
                                                                                           : "mfma_attn_fwd_d256",
-                   grid, dim3(256), (uint32_t)lds, a);
+                   grid, dim3(256 * P), (uint32_t)lds, a);
   b.ref(0, k, TH_OFFSET(MArgs, q));
   b.ref(1, k, TH_OFFSET(MArgs, k));
   b.ref(2, k, TH_OFFSET(MArgs, v));
@@ -843,9 +931,6 @@ constexpr int kMaskLds = 2 * 196 * sizeof(float) + 16;  // under masks: the dK/d
 template <int D, bool M>
 int bwd_launch(const th_attention_desc* d, th_launch** out) {
   constexpr int DO = D == 256 ? 128 : D;
-  const size_t lds = 4 * (size_t)kTile<D> * sizeof(uint16_t) + (M ? kMaskLds : 2 * 128 * sizeof(float));
-  const void* fn = (const void*)mfma_attn_bwd<D, DO, M>;
-  TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   MArgs a = margs_of(d);
   th::Builder b("attention_bwd_mfma", 11);
   const int64_t rows = (int64_t)d->batch * d->seq * d->heads;
@@ -859,6 +944,10 @@ int bwd_launch(const th_attention_desc* d, th_launch** out) {
   a.q_nsplit = sq.n, a.q_span = sq.span;
   const int64_t n_dkdv = gkv * skv.n, blocks = n_dkdv + gq * sq.n;
   TH_REQUIRE(blocks <= 0x7fffffff, "attention: grid too large");
+  const int P = D == 64 && M && blocks <= kBwdHalves ? 2 : 1;
+  const size_t lds = P * (4 * (size_t)kTile<D> * sizeof(uint16_t) + (M ? kMaskLds : 2 * 128 * sizeof(float)));
+  const void* fn = P == 2 ? (const void*)mfma_attn_bwd<D, DO, M, D == 64 && M ? 2 : 1> : (const void*)mfma_attn_bwd<D, DO, M, 1>;
+  TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   constexpr int kDeltaBlockRows = 4 * (64 / (D / 8)) * kDeltaRowsM;  // rows a workgroup
   const int k0 = b.kernel((const void*)mfma_attn_delta<D>, "mfma_attn_delta",
                           dim3((unsigned)((rows + kDeltaBlockRows - 1) / kDeltaBlockRows)), dim3(256), 0, DeltaArgs{a, D});
@@ -866,7 +955,7 @@ int bwd_launch(const th_attention_desc* d, th_launch** out) {
                        : D == 64    ? "mfma_attn_dkdv_d64_mfma_attn_dq_d64"
                        : D == 128   ? "mfma_attn_dkdv_d128_mfma_attn_dq_d128"
                                     : "mfma_attn_dkdv_d256_mfma_attn_dq_d256";
-  const int k1 = b.kernel(fn, name, dim3((unsigned)blocks), dim3(256), (uint32_t)lds, BwdArgs{a, (uint32_t)n_dkdv});
+  const int k1 = b.kernel(fn, name, dim3((unsigned)blocks), dim3(256 * P), (uint32_t)lds, BwdArgs{a, (uint32_t)n_dkdv});
   const size_t offs[11] = {TH_OFFSET(MArgs, q),      TH_OFFSET(MArgs, k),  TH_OFFSET(MArgs, v),  TH_OFFSET(MArgs, o),
                            TH_OFFSET(MArgs, lse),    TH_OFFSET(MArgs, dout), TH_OFFSET(MArgs, dq), TH_OFFSET(MArgs, dk),
                            TH_OFFSET(MArgs, dv),     TH_OFFSET(MArgs, starts), TH_OFFSET(MArgs, lengths)};
@@ -925,13 +1014,14 @@ int bwd_launch(const th_attention_desc* d, th_launch** out) {
 
 template <int D>
 int masked_fwd_launch(const th_attention_desc* d, th_launch** out) {
-  const size_t lds = 4 * (size_t)kTile<D> * sizeof(uint16_t) + 16;
-  const void* fn = (const void*)mfma_attn_fwd<D, true>;
-  TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   MArgs a = margs_of(d);
   th::Builder b("attention_fwd_mfma", 7);
   const dim3 grid(d->heads, d->batch, (d->seq + 127) / 128);
-  const int k = b.kernel(fn, D == 64 ? "mfma_attn_fwd_masked_d64" : "mfma_attn_fwd_masked_d128", grid, dim3(256),
+  const int P = (int64_t)grid.x * grid.y * grid.z <= kFwdHalves ? 2 : 1;
+  const size_t lds = 4 * P * (size_t)kTile<D> * sizeof(uint16_t) + 4 * P * sizeof(int);
+  const void* fn = P == 2 ? (const void*)mfma_attn_fwd<D, true, 2> : (const void*)mfma_attn_fwd<D, true, 1>;
+  TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  const int k = b.kernel(fn, D == 64 ? "mfma_attn_fwd_masked_d64" : "mfma_attn_fwd_masked_d128", grid, dim3(256 * P),
                          (uint32_t)lds, a);
   const size_t offs[7] = {TH_OFFSET(MArgs, q),   TH_OFFSET(MArgs, k),      TH_OFFSET(MArgs, v),
                           TH_OFFSET(MArgs, o),   TH_OFFSET(MArgs, lse),    TH_OFFSET(MArgs, starts),
