@@ -22,7 +22,7 @@
 //   dn_output       one workgroup per chunk: P, O.
 //   dn_state_grad   one eight-wave workgroup per (sequence, 32 columns): the state
 //                   gradient swept back over chunks; stores dU and dS_{n+1}.
-//   dn_grad_a/b     one workgroup per chunk: the chunk's products' gradients,
+//   dn_grad         one workgroup per chunk: the chunk's products' gradients,
 //                   the inverse's (dA = -T' dT T'), the decays', a's.
 #include <hip/hip_runtime.h>
 
@@ -59,10 +59,6 @@ struct DnArgs {
   float* P;     // [c][64][64]
   float* dU;    // [c][64][128]
   float* dSn;   // [c][128][128] gradient w.r.t. the chunk's end state
-  float* dQg;   // [c][64][128]
-  float* dW;    // [c][64][128]
-  float* dKd;   // [c][64][128]
-  float* dP;    // [c][64][64]
   float* dg;    // [c][kDgParts]: <S, dSn> by (column slice, wave) of the state gradient
   int64_t s_h, s_t, s_b;  // strides (elements) of q, k, v, o, dout, dq, dk, dv along head, position, batch
   int64_t g_h, g_t, g_b;  // strides of a, beta, da, dbeta
@@ -131,6 +127,14 @@ constexpr int kLdS = 36;   // LDS row of 32 fp32
 
 __device__ __forceinline__ f32x4v quad(const float* row) { return *reinterpret_cast<const f32x4v*>(row); }
 
+// x, hidden from the compiler's known bits: of a lane number below 16 it would
+// make (16 b + x) an `or`, whose rows it then addresses one by one from a
+// register each, not from one register and the instruction's offset.
+__device__ __forceinline__ int plain(int x) {
+  asm("" : "+v"(x));
+  return x;
+}
+
 // The four k of lane g's quad along a column: X(k, c) at x[k * ld + c].
 __device__ __forceinline__ f32x4v column_quad(const float* x, int ld, int k0, int c) {
   return f32x4v{x[k0 * ld + c], x[(k0 + 1) * ld + c], x[(k0 + 2) * ld + c], x[(k0 + 3) * ld + c]};
@@ -175,31 +179,6 @@ __device__ __forceinline__ f32x4v mma_split(const Split8& a, const Split8& b, f3
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, b.hi, c, 0, 0, 0);
 }
 
-// acc[bi][bj] += X(i0 + 16 bi .., k) Y(j0 + 16 bj .., k) over k in [0, K):
-// both operands with k along their rows (row-major in LDS, stride kLd);
-// kExactX: X's fp32 values are bf16 values (no lo part).
-template <int BI, int BJ, bool kExactX = false>
-__device__ __forceinline__ void mm_nt(f32x4v (&acc)[BI][BJ], const float* X, int i0, const float* Y, int j0, int K) {
-  const int r = threadIdx.x % 16, g = (threadIdx.x % 64) / 16;
-  for (int kb = 0; kb < K; kb += 32) {
-    Split8 a[BI], b[BJ];
-#pragma unroll
-    for (int bi = 0; bi < BI; ++bi) {
-      const float* row = X + (i0 + 16 * bi + r) * kLd + kb + 8 * g;
-      a[bi] = split8<kExactX>(quad(row), quad(row + 4));
-    }
-#pragma unroll
-    for (int bj = 0; bj < BJ; ++bj) {
-      const float* row = Y + (j0 + 16 * bj + r) * kLd + kb + 8 * g;
-      b[bj] = split8<false>(quad(row), quad(row + 4));
-    }
-#pragma unroll
-    for (int bi = 0; bi < BI; ++bi)
-#pragma unroll
-      for (int bj = 0; bj < BJ; ++bj) acc[bi][bj] = mma_split<kExactX, false>(a[bi], b[bj], acc[bi][bj]);
-  }
-}
-
 // acc[bi][bj] += X(i0 + 16 bi .., k) Y(k, j0 + 16 bj ..) over k in [0, K), each
 // operand read along its rows (X(i, k) = X[i * ldx + k], Y(k, j) = Y[j * ldy + k])
 // or, when XT / YT, along its columns (X(i, k) = X[k * ldx + i], Y(k, j) =
@@ -207,7 +186,7 @@ __device__ __forceinline__ void mm_nt(f32x4v (&acc)[BI][BJ], const float* X, int
 template <bool XT, bool YT, int BI, int BJ>
 __device__ __forceinline__ void mm_gen(f32x4v (&acc)[BI][BJ], const float* X, int ldx, int i0, const float* Y, int ldy,
                                        int j0, int K) {
-  const int r = threadIdx.x % 16, g = (threadIdx.x % 64) / 16;
+  const int r = plain(threadIdx.x % 16), g = plain((threadIdx.x % 64) / 16);
   auto xq = [&](int k0, int i) { return XT ? column_quad(X, ldx, k0, i) : quad(X + i * ldx + k0); };
   auto yq = [&](int k0, int j) { return YT ? column_quad(Y, ldy, k0, j) : quad(Y + j * ldy + k0); };
   for (int kb = 0; kb < K; kb += 32) {
@@ -232,51 +211,13 @@ __device__ __forceinline__ void clear(f32x4v (&acc)[BI][BJ]) {
     for (int bj = 0; bj < BJ; ++bj) acc[bi][bj] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
 }
 
-// rows x 128 fp32 from global (row stride 128) into LDS rows of kLd, 16-byte pieces.
 // Each staging helper issues all of a thread's loads before its first LDS
 // store, so their latencies overlap instead of adding up.
-__device__ __forceinline__ void stage_f32(float* dst, const float* src) {
-  constexpr int n = kC * 32 / 256;
-  float4 x[n];
-#pragma unroll
-  for (int u = 0; u < n; ++u) {
-    const int e = threadIdx.x + 256 * u;
-    x[u] = *reinterpret_cast<const float4*>(src + (e / 32) * kD + 4 * (e % 32));
-  }
-#pragma unroll
-  for (int u = 0; u < n; ++u) {
-    const int e = threadIdx.x + 256 * u;
-    *reinterpret_cast<float4*>(dst + (e / 32) * kLd + 4 * (e % 32)) = x[u];
-  }
-}
-
-// 64 x 128 bf16 of a (d, heads, positions, batch) array into LDS as fp32 rows of kLd.
-__device__ __forceinline__ void stage_bf16(float* dst, const uint16_t* src, int64_t s_t) {
-  constexpr int n = kC * 16 / 256;
-  uint4 x[n];
-#pragma unroll
-  for (int q = 0; q < n; ++q) {
-    const int e = threadIdx.x + 256 * q;
-    x[q] = *reinterpret_cast<const uint4*>(src + (e / 16) * s_t + 8 * (e % 16));
-  }
-#pragma unroll
-  for (int q = 0; q < n; ++q) {
-    const int e = threadIdx.x + 256 * q;
-    const int r = e / 16, c8 = 8 * (e % 16);
-    const uint4 w = x[q];
-    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-    float f[8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) f[2 * j] = bf((uint16_t)u[j]), f[2 * j + 1] = bf((uint16_t)(u[j] >> 16));
-    *reinterpret_cast<float4*>(dst + r * kLd + c8) = make_float4(f[0], f[1], f[2], f[3]);
-    *reinterpret_cast<float4*>(dst + r * kLd + c8 + 4) = make_float4(f[4], f[5], f[6], f[7]);
-  }
-}
 
 // Block (bi, bj) of acc to out (row stride ld), rows i0 + 16 bi + 4 g + v, columns j0 + 16 bj + r, times s.
 template <int BI, int BJ>
 __device__ __forceinline__ void store_blocks(float* out, int ld, const f32x4v (&acc)[BI][BJ], int i0, int j0, float s) {
-  const int r = threadIdx.x % 16, g = (threadIdx.x % 64) / 16;
+  const int r = plain(threadIdx.x % 16), g = plain((threadIdx.x % 64) / 16);
 #pragma unroll
   for (int bi = 0; bi < BI; ++bi)
 #pragma unroll
@@ -331,7 +272,7 @@ struct ColBf16 {  // (x, k) at bf16 p[k * ld + x]
 // acc[bi][bj] += X(i0 + 16 bi .., k) Y(k, j0 + 16 bj ..) over k in [0, K).
 template <int BI, int BJ, class XR, class YR>
 __device__ __forceinline__ void mm_by(f32x4v (&acc)[BI][BJ], const XR& X, int i0, const YR& Y, int j0, int K) {
-  const int r = threadIdx.x % 16, g = (threadIdx.x % 64) / 16;
+  const int r = plain(threadIdx.x % 16), g = plain((threadIdx.x % 64) / 16);
   for (int kb = 0; kb < K; kb += 32) {
     const int k0 = kb + 8 * g;
     Split8 b[BJ];
@@ -878,115 +819,102 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_state_grad(DnArgs p) {
   }
 }
 
-// ---- backward: the chunk's products (part a) ---------------------------------------
-// dQg = dO S', dW = -dU S', dKd = U dSn', dP = lower(dO U'),
-// every product on the matrix cores (split bf16).  Two phases through LDS: dO, dU
-// and S, then U and dSn (dO stays).  Wave w computes columns 32 w .. 32 w + 31
-// of the 64 x 128 results and row block w of dP.
-
-// S and dSn are read by rows straight from memory (each wave's 32 rows, for
-// both products that use them at once), so only dO and one 64-row operand
-// live in LDS and two workgroups share a CU.
-constexpr size_t kGaLds = 2 * kC * kLd * sizeof(float);
-
-// acc1 += X1 Y', acc2 += X2 Y' over k in [0, K): X1, X2 rows i0 .. of LDS
-// (stride kLd), Y rows j0 + 16 bj .. of memory (stride kD), each Y quad read once;
-// kExact1: X1's fp32 values are bf16 values.
-template <int BI, int BJ, bool kExact1 = false>
-__device__ __forceinline__ void mm_nt2(f32x4v (&acc1)[BI][BJ], const float* X1, f32x4v (&acc2)[BI][BJ], const float* X2,
-                                       int i0, const float* Y, int j0, int K) {
-  const int r = threadIdx.x % 16, g = (threadIdx.x % 64) / 16;
-  for (int kb = 0; kb < K; kb += 32) {
-    Split8 a1[BI], a2[BI], b[BJ];
-#pragma unroll
-    for (int bj = 0; bj < BJ; ++bj) {
-      const float* row = Y + (j0 + 16 * bj + r) * kD + kb + 8 * g;
-      b[bj] = split8<false>(quad(row), quad(row + 4));
-    }
-#pragma unroll
-    for (int bi = 0; bi < BI; ++bi) {
-      const float* r1 = X1 + (i0 + 16 * bi + r) * kLd + kb + 8 * g;
-      const float* r2 = X2 + (i0 + 16 * bi + r) * kLd + kb + 8 * g;
-      a1[bi] = split8<kExact1>(quad(r1), quad(r1 + 4));
-      a2[bi] = split8<false>(quad(r2), quad(r2 + 4));
-    }
-#pragma unroll
-    for (int bi = 0; bi < BI; ++bi)
-#pragma unroll
-      for (int bj = 0; bj < BJ; ++bj) {
-        acc1[bi][bj] = mma_split<kExact1, false>(a1[bi], b[bj], acc1[bi][bj]);
-        acc2[bi][bj] = mma_split<false, false>(a2[bi], b[bj], acc2[bi][bj]);
-      }
-  }
-}
-
-__global__ __launch_bounds__(256, 2) void dn_grad_a(DnArgs p) {
-  extern __shared__ float lds[];
-  float* dO = lds;              // [64][kLd]
-  float* X = dO + kC * kLd;     // [64][kLd]: dU, then U
-  const Chunk ck = chunk_of(p, blockIdx.x);
-  const int t = threadIdx.x, w = t / 64;
-  const float* Sc = p.S + ck.c * kD * kD;
-  const float* dSc = p.dSn + ck.c * kD * kD;
-  stage_bf16(dO, p.dout + ck.row0, p.s_t);
-  stage_f32(X, p.dU + ck.c * kC * kD);
-  __syncthreads();
-  {
-    f32x4v q[4][2], wq[4][2];
-    clear(q);
-    clear(wq);
-    mm_nt2<4, 2, true>(q, dO, wq, X, 0, Sc, 32 * w, kD);  // dO: bf16 values
-    store_blocks(p.dQg + ck.c * kC * kD, kD, q, 0, 32 * w, 1.0f);
-    store_blocks(p.dW + ck.c * kC * kD, kD, wq, 0, 32 * w, -1.0f);
-  }
-  __syncthreads();
-  stage_f32(X, p.U + ck.c * kC * kD);
-  __syncthreads();
-  {
-    f32x4v kd[4][2];
-    clear(kd);
-    mm_by(kd, RowF32{X, kLd}, 0, RowF32{dSc, kD}, 32 * w, kD);
-    store_blocks(p.dKd + ck.c * kC * kD, kD, kd, 0, 32 * w, 1.0f);
-  }
-  {
-    // Row block w of dP: blocks (w, jb) for jb <= w, the diagonal masked, zeros above.
-    const int r = t % 16, g = (t % 64) / 16;
-    float* dPc = p.dP + ck.c * kC * kC;
-    for (int jb = 0; jb < 4; ++jb) {
-      f32x4v acc[1][1];
-      clear(acc);
-      if (jb <= w) mm_nt<1, 1, true>(acc, dO, 16 * w, X, 16 * jb, kD);  // dO: bf16 values
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = 16 * w + 4 * g + v, j = 16 * jb + r;
-        dPc[i * kC + j] = i >= j ? acc[0][0][v] : 0.0f;
-      }
-    }
-  }
-}
-
-// ---- backward: the chunk's WY form, decays and gates (part b) -----------------------
-// Every product on the matrix cores, split bf16 (mm_by below); Q and K sit in LDS
-// as bf16 (their exact values) and are widened as they are read, V is read
-// from global where it is needed, and dW, dU~ take turns in one fp32 buffer.
-// The row sums of the gate gradients are complete within a wave (each wave
-// owns 16 rows of the 64 x 64 work, and 32 of the 128 columns of the
-// 64 x 128 work, whose partials go to LDS by wave) and are folded in a fixed
+// ---- backward: the chunk's products, WY form, decays and gates ---------------------
+// dQg = dO S', dW = -dU S', dKd = U dSn', dP = lower(dO U'), then everything
+// that follows from them: dT, dA = -T' dT T', the gate gradients and dQ, dK, dV.
+// Bound by memory: a chunk reads 336 KB of states, U, dU, T and arrays and
+// writes 48.  The products stay in the registers that the outputs sum in (dQg
+// in dQ's, dKd and T' dW in dK's, dP in the lanes that form dQK), so none of
+// them goes through memory; as two kernels that passed dQg, dW, dKd and dP on
+// (224 KB a chunk, out and back) the same took 1293 us at B4 H16 T8192, now 1022.
+//
+// Every product on the matrix cores, split bf16; dO, Q and K sit in LDS as
+// bf16 (their exact values) and are widened as they are read; U, dU and dW take
+// turns in one fp32 buffer, which M and N then share; V, T, S and dSn are
+// read from memory by the products that use them (S and dSn by rows, each
+// wave's 32).  Under 80 KB, so two workgroups share a CU.
+// Wave w: columns 32 w .. 32 w + 31 of the 64 x 128 work, rows 16 w .. of the
+// 64 x 64 work.  The row sums of the gate gradients are complete within a wave,
+// the column work's partials go to LDS by wave and are folded in a fixed
 // order, so the result does not depend on timing.
 
-// dW, dU~ and T are read straight from memory by the products that use them,
-// so LDS holds Q, K, M and N only and two workgroups share a CU; dQK = dP o
-// Gamma (lower) takes N once N's own last use is past.
-constexpr size_t kGbLds = 2 * kC * kLdH * sizeof(uint16_t) + 2 * kC * kLdC * sizeof(float) +
-                          (2 * kC + 5 * 4 * kC + 2 * kC) * sizeof(float);
+// acc1 += X1 Y', acc2 += X2 Y' over k in [0, K): rows i0 .. of X1 and X2, each
+// quad of Y read once.
+template <int BI, int BJ, class X1, class X2, class YR>
+__device__ __forceinline__ void mm_by2(f32x4v (&acc1)[BI][BJ], const X1& x1, f32x4v (&acc2)[BI][BJ], const X2& x2,
+                                       int i0, const YR& Y, int j0, int K) {
+  const int r = plain(threadIdx.x % 16), g = plain((threadIdx.x % 64) / 16);
+  for (int kb = 0; kb < K; kb += 32) {
+    const int k0 = kb + 8 * g;
+    Split8 b[BJ];
+#pragma unroll
+    for (int bj = 0; bj < BJ; ++bj)
+      b[bj] = split8<YR::kExact>(Y.quad(j0 + 16 * bj + r, k0), Y.quad(j0 + 16 * bj + r, k0 + 4));
+#pragma unroll
+    for (int bi = 0; bi < BI; ++bi) {
+      const int i = i0 + 16 * bi + r;
+      const Split8 a1 = split8<X1::kExact>(x1.quad(i, k0), x1.quad(i, k0 + 4));
+      const Split8 a2 = split8<X2::kExact>(x2.quad(i, k0), x2.quad(i, k0 + 4));
+#pragma unroll
+      for (int bj = 0; bj < BJ; ++bj) {
+        acc1[bi][bj] = mma_split<X1::kExact, YR::kExact>(a1, b[bj], acc1[bi][bj]);
+        acc2[bi][bj] = mma_split<X2::kExact, YR::kExact>(a2, b[bj], acc2[bi][bj]);
+      }
+    }
+  }
+}
 
-__global__ __launch_bounds__(256, 2) void dn_grad_b(DnArgs p) {
+// 64 x 128 fp32 rows of memory (stride kD) or bf16 rows (stride s_t), requested
+// under the products before the LDS they go to is free.
+struct HeldF32 {
+  static constexpr int n = kC * 32 / 256;
+  f32x4v x[n];
+  __device__ void load(const float* src) {
+#pragma unroll
+    for (int u = 0; u < n; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      x[u] = quad(src + (e / 32) * kD + 4 * (e % 32));
+    }
+  }
+  __device__ void store(float* dst) const {
+#pragma unroll
+    for (int u = 0; u < n; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      *reinterpret_cast<f32x4v*>(dst + (e / 32) * kLd + 4 * (e % 32)) = x[u];
+    }
+  }
+};
+struct HeldBf16 {
+  static constexpr int n = kC * (kD / 8) / 256;
+  u32x4v x[n];
+  __device__ void load(const uint16_t* src, int64_t s_t) {
+#pragma unroll
+    for (int u = 0; u < n; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      x[u] = *reinterpret_cast<const u32x4v*>(src + (e / (kD / 8)) * s_t + 8 * (e % (kD / 8)));
+    }
+  }
+  __device__ void store(uint16_t* dst) const {
+#pragma unroll
+    for (int u = 0; u < n; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      *reinterpret_cast<u32x4v*>(dst + (e / (kD / 8)) * kLdH + 8 * (e % (kD / 8))) = x[u];
+    }
+  }
+};
+
+constexpr int kGradX = 2 * kC * kLdC > kC * kLd ? 2 * kC * kLdC : kC * kLd;
+constexpr size_t kGradLds = 2 * kC * kLdH * sizeof(uint16_t) + kGradX * sizeof(float) +
+                            (2 * kC + 5 * 4 * kC + 2 * kC) * sizeof(float);
+
+__global__ __launch_bounds__(256, 2) void dn_grad(DnArgs p) {
   extern __shared__ float lds[];
-  uint16_t* Qh = reinterpret_cast<uint16_t*>(lds);       // [64][kLdH]
+  uint16_t* Qh = reinterpret_cast<uint16_t*>(lds);       // [64][kLdH]: dO, then Q
   uint16_t* Kh = Qh + kC * kLdH;                          // [64][kLdH]
-  float* M = reinterpret_cast<float*>(Kh + kC * kLdH);   // [64][kLdC]: dT, then dA, then dG + dG'
+  float* X = reinterpret_cast<float*>(Kh + kC * kLdH);   // [64][kLd]: U, then dU, then dW
+  float* M = X;                    // [64][kLdC]: dT, then dA, then dG + dG'
   float* N = M + kC * kLdC;        // [64][kLdC]: T' dT, then dG, then dQK
-  float* wrow = N + kC * kLdC;     // [64]: sum_j w_ij
+  float* wrow = X + kGradX;        // [64]: sum_j w_ij
   float* brow = wrow + kC;         // [64]: sum_j dA Gamma G
   float* wcol = brow + kC;         // [4][64]: sum_i w_ij by wave
   float* kx = wcol + 4 * kC;       // [4][64]: k . dX by wave (columns)
@@ -997,37 +925,20 @@ __global__ __launch_bounds__(256, 2) void dn_grad_b(DnArgs p) {
   float* be = ca + kC;             // [64]
   const Chunk ck = chunk_of(p, blockIdx.x);
   const int t = threadIdx.x, w = t / 64;
-  const int r = t % 16, g = (t % 64) / 16;
-  const uint16_t* qg = p.q + ck.row0;
-  const uint16_t* kg = p.k + ck.row0;
+  const int r = plain(t % 16), g4 = plain((t % 64) / 16 * 4);  // 4 x the row group
   const uint16_t* vg = p.v + ck.row0;
   const float* Tc = p.T + ck.c * kC * kC;  // [64][64]
-  const float* dW = p.dW + ck.c * kC * kD;
-  const float* dUt = p.dU + ck.c * kC * kD;
   const int i0 = 16 * w;  // this wave's rows of the 64 x 64 work
-  // The first products' operands from memory (this wave's rows of dW and
-  // dU~, its lanes' V), requested before the staging so that their latency
-  // overlaps it: lane (r, g) takes k = 32 kb + 8 g + (0..7).
-  f32x4v dwq[8], duq[8];
-  uint2 vq[4][8];
-  {
-    const float* dWr = dW + (i0 + r) * kD + 8 * g;
-    const float* dUr = dUt + (i0 + r) * kD + 8 * g;
-#pragma unroll
-    for (int h = 0; h < 8; ++h) {
-      dwq[h] = quad(dWr + 32 * (h / 2) + 4 * (h % 2));
-      duq[h] = quad(dUr + 32 * (h / 2) + 4 * (h % 2));
-    }
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-      for (int h = 0; h < 8; ++h)
-        vq[bj][h] = *reinterpret_cast<const uint2*>(vg + (int64_t)(16 * bj + r) * p.s_t + 32 * (h / 2) + 8 * g + 4 * (h % 2));
-  }
-  stage_rows_bf16(Qh, qg, Kh, kg, p.s_t);
-  const float* dQg = p.dQg + ck.c * kC * kD;
-  const float* dKd = p.dKd + ck.c * kC * kD;
-  const float* dP = p.dP + ck.c * kC * kC;
+  const int d0 = 32 * w;  // and its columns of the 64 x 128 work
+  // This lane's place in block (0, 0) of its wave's columns of an array; the
+  // rows of the other blocks are uniform offsets from it.
+  const int64_t lane_at = ck.row0 + g4 * p.s_t + d0 + r;
+  const uint16_t* vl = p.v + lane_at;
+  uint16_t *dql = p.dq + lane_at, *dkl = p.dk + lane_at, *dvl = p.dv + lane_at;
+  HeldF32 held;
+  held.load(p.U + ck.c * kC * kD);
+  stage_rows_bf16(Qh, p.dout + ck.row0, Kh, p.k + ck.row0, p.s_t);
+  held.store(X);
   const float dg_part = t < kDgParts ? p.dg[ck.c * kDgParts + t] : 0.0f;
   if (t < 64) {
     ca[t] = p.ca[ck.c * kC + t];
@@ -1037,31 +948,129 @@ __global__ __launch_bounds__(256, 2) void dn_grad_b(DnArgs p) {
   const RowBf16 Kr{Kh, kLdH}, Qr{Qh, kLdH};
   const ColBf16 Kc{Kh, kLdH}, Qc{Qh, kLdH};
   const float last = ca[kC - 1];
-  // dT = dW X' + dU~ Y',  X = diag(beta e^ca) K, Y = diag(beta) V.
-  {
-    f32x4v xk[1][4], yv[1][4];
-    clear(xk);
-    clear(yv);
+  const RowF32 Xr{X, kLd};
+  const ColF32 Xc{X, kLd};
+  const RowBf16 Or{Qh, kLdH};
+  // U: dKd = U dSn' (kd; sk = k . dKd a row) and dP = lower(dO U') (this wave's rows).
+  f32x4v kd[4][2], dp[1][4];
+  clear(kd);
+  clear(dp);
+  mm_by(kd, Xr, 0, RowF32{p.dSn + ck.c * kD * kD, kD}, d0, kD);
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      const Split8 aw = split8<false>(dwq[2 * kb], dwq[2 * kb + 1]);
-      const Split8 au = split8<false>(duq[2 * kb], duq[2 * kb + 1]);
+  for (int bj = 0; bj < 4; ++bj)
+    if (bj <= w) {
+      f32x4v a1[1][1];
+      clear(a1);
+      mm_by(a1, Or, i0, Xr, 16 * bj, kD);
 #pragma unroll
-      for (int bj = 0; bj < 4; ++bj) {
-        const int x = 16 * bj + r, k0 = 32 * kb + 8 * g;
-        const Split8 bk = split8<true>(Kr.quad(x, k0), Kr.quad(x, k0 + 4));
-        xk[0][bj] = mma_split<false, true>(aw, bk, xk[0][bj]);
-        const uint2 v0 = vq[bj][2 * kb], v1 = vq[bj][2 * kb + 1];
-        const Split8 bv{__builtin_bit_cast(bf16x8v, u32x4v{v0.x, v0.y, v1.x, v1.y}),
-                        __builtin_bit_cast(bf16x8v, u32x4v{0u, 0u, 0u, 0u})};
-        yv[0][bj] = mma_split<false, true>(au, bv, yv[0][bj]);
-      }
+      for (int v = 0; v < 4; ++v) dp[0][bj][v] = i0 + g4 + v >= 16 * bj + r ? a1[0][0][v] : 0.0f;
     }
+#pragma unroll
+  for (int bi = 0; bi < 4; ++bi)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = 16 * bi + g4 + v;
+      const float ed = expf(last - ca[i]);
+      float sk = 0.0f;
+#pragma unroll
+      for (int bj = 0; bj < 2; ++bj) {
+        sk = fmaf(bf(Kh[i * kLdH + d0 + 16 * bj + r]), kd[bi][bj][v], sk);
+        float x = kd[bi][bj][v] * ed;
+        asm("" : "+v"(x));  // formed here: put off to its use, it would hold ed and dKd till then
+        kd[bi][bj][v] = x;
+      }
+      sk = row_group_sum(sk);
+      if (r == 0) kk[w * kC + i] = sk;
+    }
+  __syncthreads();
+  held.load(p.dU + ck.c * kC * kD);
+  held.store(X);
+  __syncthreads();
+  // dU: dV = beta T' dU~, dU~ V' (this wave's rows), dQg = dO S', dW = -dU S'.
+  f32x4v yv[1][4];
+  {
+    f32x4v dy[4][2];
+    clear(dy);
+    mm_by(dy, ColF32{Tc, kC}, 0, Xc, d0, kC);
+    // In two halves of row blocks: the V values of a half are all read
+    // before its first dV store (same element type: loaded in the loop,
+    // each read would wait for the previous store).
+#pragma unroll
+    for (int hb = 0; hb < 2; ++hb) {
+      uint32_t vh[2][4];  // the two bf16 of columns d0 + r, d0 + 16 + r
+#pragma unroll
+      for (int b2 = 0; b2 < 2; ++b2)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const uint16_t* vr = vl + (16 * (2 * hb + b2) + v) * p.s_t;
+          vh[b2][v] = (uint32_t)vr[0] | ((uint32_t)vr[16] << 16);
+        }
+#pragma unroll
+      for (int b2 = 0; b2 < 2; ++b2)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int bi = 2 * hb + b2, i = 16 * bi + g4 + v;
+          float sv = 0.0f;
+#pragma unroll
+          for (int bj = 0; bj < 2; ++bj) {
+            const float vv = bf((uint16_t)(vh[b2][v] >> (16 * bj))), yv1 = dy[bi][bj][v];
+            sv = fmaf(vv, yv1, sv);
+            dvl[(16 * bi + v) * p.s_t + 16 * bj] = to_bf(be[i] * yv1);
+          }
+          sv = row_group_sum(sv);
+          if (r == 0) vy[w * kC + i] = sv;
+        }
+    }
+    clear(yv);
+    mm_by(yv, Xr, i0, RowBf16{vg, p.s_t}, 0, kD);
+  }
+  f32x4v dq[4][2];
+  {
+    HeldBf16 q;
+    f32x4v wq[4][2];
+    clear(dq);
+    clear(wq);
+    mm_by2(dq, Or, wq, Xr, 0, RowF32{p.S + ck.c * kD * kD, kD}, d0, kD);
+    __syncthreads();
+    store_blocks(X, kLd, wq, 0, d0, -1.0f);
+    q.load(p.q + ck.row0, p.s_t);
+    q.store(Qh);
+  }
+  __syncthreads();
+  // dW: dX = T' dW into dK's sum (beta e^ca dX + e^(last - ca) dKd), and
+  // dT = dW X' + dU~ Y',  X = diag(beta e^ca) K, Y = diag(beta) V; the row sums q . dQg and k . dX.
+  {
+    f32x4v dx[4][2];
+    clear(dx);
+    mm_by(dx, ColF32{Tc, kC}, 0, Xc, d0, kC);
+#pragma unroll
+    for (int bi = 0; bi < 4; ++bi)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = 16 * bi + g4 + v;
+        const float e = expf(ca[i]);
+        float sq = 0.0f, sx = 0.0f;
+#pragma unroll
+        for (int bj = 0; bj < 2; ++bj) {
+          const int d = d0 + 16 * bj + r;
+          sq = fmaf(bf(Qh[i * kLdH + d]), dq[bi][bj][v], sq);
+          sx = fmaf(bf(Kh[i * kLdH + d]), dx[bi][bj][v], sx);
+          dq[bi][bj][v] *= e;
+          kd[bi][bj][v] = fmaf(be[i] * e, dx[bi][bj][v], kd[bi][bj][v]);
+        }
+        sq = row_group_sum(sq);
+        sx = row_group_sum(sx);
+        if (r == 0) qq[w * kC + i] = sq, kx[w * kC + i] = sx;
+      }
+    f32x4v xk[1][4];
+    clear(xk);
+    mm_by(xk, Xr, i0, Kr, 0, kD);
+    __syncthreads();
 #pragma unroll
     for (int bj = 0; bj < 4; ++bj)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int i = i0 + 4 * g + v, l = 16 * bj + r;
+        const int i = i0 + g4 + v, l = 16 * bj + r;
         M[i * kLdC + l] = be[l] * (expf(ca[l]) * xk[0][bj][v] + yv[0][bj][v]);
       }
   }
@@ -1083,7 +1092,7 @@ __global__ __launch_bounds__(256, 2) void dn_grad_b(DnArgs p) {
     for (int bj = 0; bj < 4; ++bj)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int i = i0 + 4 * g + v, j = 16 * bj + r;
+        const int i = i0 + g4 + v, j = 16 * bj + r;
         M[i * kLdC + j] = i > j ? -acc[0][bj][v] : 0.0f;
       }
   }
@@ -1093,12 +1102,6 @@ __global__ __launch_bounds__(256, 2) void dn_grad_b(DnArgs p) {
   // dbeta_i gets sum_j dA Gamma G; w = (dA beta_i G + dP QK) o Gamma gives
   // dca_i += sum_j w_ij - sum_j w_ji.
   {
-    // This lane's dP values, loaded under the products below.
-    float dpv[4][4];
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) dpv[bj][v] = dP[(i0 + 4 * g + v) * kC + 16 * bj + r];
     f32x4v gk[1][4], qk[1][4];
     clear(gk);
     clear(qk);
@@ -1120,15 +1123,16 @@ __global__ __launch_bounds__(256, 2) void dn_grad_b(DnArgs p) {
     for (int bj = 0; bj < 4; ++bj)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int i = i0 + 4 * g + v, j = 16 * bj + r;
+        const int i = i0 + g4 + v, j = 16 * bj + r;
         const float gam = expf(ca[i] - ca[j]);
         const float dA = M[i * kLdC + j];
         const float gg = bj <= w ? gk[0][bj][v] : 0.0f, q = bj <= w ? qk[0][bj][v] : 0.0f;
         N[i * kLdC + j] = dA * be[i] * gam;
         rowb[v] += dA * gam * gg;
-        const float wv = i >= j ? (dA * be[i] * gg + dpv[bj][v] * q) * gam : 0.0f;
+        const float wv = i >= j ? (dA * be[i] * gg + dp[0][bj][v] * q) * gam : 0.0f;
         roww[v] += wv;
         colw[bj] += wv;
+        dp[0][bj][v] = i >= j ? dp[0][bj][v] * gam : 0.0f;  // dQK
       }
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -1137,14 +1141,14 @@ __global__ __launch_bounds__(256, 2) void dn_grad_b(DnArgs p) {
     }
     if (r == 0)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) wrow[i0 + 4 * g + v] = roww[v], brow[i0 + 4 * g + v] = rowb[v];
+      for (int v = 0; v < 4; ++v) wrow[i0 + g4 + v] = roww[v], brow[i0 + g4 + v] = rowb[v];
     // Column sums over this wave's 16 rows: the four row groups g, in order.
 #pragma unroll
     for (int bj = 0; bj < 4; ++bj) {
       float x = colw[bj];
       x += __shfl_xor(x, 16, 64);
       x += __shfl_xor(x, 32, 64);
-      if (g == 0) wcol[w * kC + 16 * bj + r] = x;
+      if (g4 == 0) wcol[w * kC + 16 * bj + r] = x;
     }
   }
   __syncthreads();
@@ -1155,139 +1159,23 @@ __global__ __launch_bounds__(256, 2) void dn_grad_b(DnArgs p) {
   }
   __syncthreads();
   // dQK = dP o Gamma (lower), read by two of the products below along its rows
-  // and its columns: formed once into N (free now), not at every read.
-  {
-    float x[kC * kC / 256];
-#pragma unroll
-    for (int u = 0; u < kC * kC / 256; ++u) x[u] = dP[t + 256 * u];
-#pragma unroll
-    for (int u = 0; u < kC * kC / 256; ++u) {
-      const int e = t + 256 * u, i = e / kC, j = e % kC;
-      N[i * kLdC + j] = i >= j ? x[u] * expf(ca[i] - ca[j]) : 0.0f;
-    }
-  }
+  // and its columns, into N (free now).
+  store_blocks(N, kLdC, dp, i0, 0, 1.0f);
   __syncthreads();
-  // dQ = e^ca dQg + dQK K;  dV = beta T' dU~;  dK = dQK' Q + (dG + dG') K +
-  // beta e^ca dX + e^(last - ca) dKd with dX = T' dW.  Wave w: columns
-  // 32 w .. 32 w + 31, one output at a time (two accumulator sets live).
-  {
-    const int d0 = 32 * w;
-    const RowF32 Rr{N, kLdC};  // dQK along its rows
-    const ColF32 Rc{N, kLdC};  // and along its columns
-    {
-      float gqv[4][4][2];  // this lane's dQg, loaded under the product
+  // dQ = e^ca dQg + dQK K;  dK = dQK' Q + (dG + dG') K + beta e^ca dX + e^(last - ca) dKd.
+  mm_by(dq, RowF32{N, kLdC}, 0, Kc, d0, kC);
+  mm_by(kd, ColF32{N, kLdC}, 0, Qc, d0, kC);
+  mm_by(kd, RowF32{M, kLdC}, 0, Kc, d0, kC);
 #pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
+  for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+    for (int v = 0; v < 4; ++v)
 #pragma unroll
-          for (int bj = 0; bj < 2; ++bj) gqv[bi][v][bj] = dQg[(16 * bi + 4 * g + v) * kD + d0 + 16 * bj + r];
-      f32x4v dq[4][2];
-      clear(dq);
-      mm_by(dq, Rr, 0, Kc, d0, kC);
-#pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = 16 * bi + 4 * g + v;
-          const float e = expf(ca[i]);
-          float sq = 0.0f;
-#pragma unroll
-          for (int bj = 0; bj < 2; ++bj) {
-            const int d = d0 + 16 * bj + r;
-            const float gq = gqv[bi][v][bj], qv = bf(Qh[i * kLdH + d]);
-            sq = fmaf(qv, gq, sq);
-            p.dq[ck.row0 + (int64_t)i * p.s_t + d] = to_bf(e * gq + dq[bi][bj][v]);
-          }
-          sq = row_group_sum(sq);
-          if (r == 0) qq[w * kC + i] = sq;
-        }
-    }
-    {
-      // This lane's V values, all read before the first dV store (same
-      // element type: loaded in the loop, each read would wait for the
-      // previous store).
-      f32x4v dy[4][2];
-      clear(dy);
-      mm_by(dy, ColF32{Tc, kC}, 0, ColF32{dUt, kD}, d0, kC);
-      // In two halves of row blocks: the V values of a half are all read
-      // before its first dV store (same element type: loaded in the loop,
-      // each read would wait for the previous store).
-#pragma unroll
-      for (int hb = 0; hb < 2; ++hb) {
-        uint32_t vh[2][4];  // the two bf16 of columns d0 + r, d0 + 16 + r
-#pragma unroll
-        for (int b2 = 0; b2 < 2; ++b2)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const uint16_t* vr = vg + (int64_t)(16 * (2 * hb + b2) + 4 * g + v) * p.s_t + d0 + r;
-            vh[b2][v] = (uint32_t)vr[0] | ((uint32_t)vr[16] << 16);
-          }
-#pragma unroll
-        for (int b2 = 0; b2 < 2; ++b2)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int bi = 2 * hb + b2, i = 16 * bi + 4 * g + v;
-            float sv = 0.0f;
-#pragma unroll
-            for (int bj = 0; bj < 2; ++bj) {
-              const int d = d0 + 16 * bj + r;
-              const float vv = bf((uint16_t)(vh[b2][v] >> (16 * bj))), yv = dy[bi][bj][v];
-              sv = fmaf(vv, yv, sv);
-              p.dv[ck.row0 + (int64_t)i * p.s_t + d] = to_bf(be[i] * yv);
-            }
-            sv = row_group_sum(sv);
-            if (r == 0) vy[w * kC + i] = sv;
-          }
+      for (int bj = 0; bj < 2; ++bj) {
+        const int64_t at = (16 * bi + v) * p.s_t + 16 * bj;
+        dql[at] = to_bf(dq[bi][bj][v]);
+        dkl[at] = to_bf(kd[bi][bj][v]);
       }
-    }
-    {
-      // dX first; its terms of dK (beta e^ca dX + e^(last - ca) dKd) then
-      // seed dK's accumulator, so one accumulator set is live at a time.
-      float gkv[4][4][2];  // this lane's dKd, loaded under the product
-#pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-#pragma unroll
-          for (int bj = 0; bj < 2; ++bj) gkv[bi][v][bj] = dKd[(16 * bi + 4 * g + v) * kD + d0 + 16 * bj + r];
-      f32x4v acc[4][2];
-      clear(acc);
-      mm_by(acc, ColF32{Tc, kC}, 0, ColF32{dW, kD}, d0, kC);
-#pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = 16 * bi + 4 * g + v;
-          const float e = expf(ca[i]), ed = expf(last - ca[i]);
-          float sx = 0.0f, sk = 0.0f;
-#pragma unroll
-          for (int bj = 0; bj < 2; ++bj) {
-            const int d = d0 + 16 * bj + r;
-            const float gk = gkv[bi][v][bj], kv = bf(Kh[i * kLdH + d]);
-            const float xv = acc[bi][bj][v];
-            sx = fmaf(kv, xv, sx);
-            sk = fmaf(kv, gk, sk);
-            acc[bi][bj][v] = be[i] * e * xv + ed * gk;
-          }
-          sx = row_group_sum(sx);
-          sk = row_group_sum(sk);
-          if (r == 0) kx[w * kC + i] = sx, kk[w * kC + i] = sk;
-        }
-      mm_by(acc, Rc, 0, Qc, d0, kC);
-      mm_by(acc, RowF32{M, kLdC}, 0, Kc, d0, kC);
-#pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-#pragma unroll
-          for (int bj = 0; bj < 2; ++bj) {
-            const int i = 16 * bi + 4 * g + v, d = d0 + 16 * bj + r;
-            p.dk[ck.row0 + (int64_t)i * p.s_t + d] = to_bf(acc[bi][bj][v]);
-          }
-    }
-  }
-  __syncthreads();
   // Fold the partials in a fixed order (lane i: row i), then da = the
   // reverse cumulative sum of dca, dca_63 also taking sum kd + dg g.
   if (t < 64) {
@@ -1325,18 +1213,19 @@ __global__ __launch_bounds__(256, 2) void dn_grad_b(DnArgs p) {
 
 bool aligned(const void* q, int bytes) { return (reinterpret_cast<uintptr_t>(q) % bytes) == 0; }
 
+// ca, T, W, Ut, S, U, P; for the backward dU, dSn, dg
+constexpr int kSlots = 10;
 struct Workspace {
-  size_t offs[14];
+  size_t offs[kSlots];
   size_t bytes;
 };
 
 Workspace workspace(int64_t chunks, bool backward) {
-  const size_t sizes[14] = {(size_t)kC, (size_t)kC * kC, (size_t)kC * kD, (size_t)kC * kD, (size_t)kD * kD,
-                            (size_t)kC * kD, (size_t)kC * kC, (size_t)kC * kD, (size_t)kD * kD, (size_t)kC * kD,
-                            (size_t)kC * kD, (size_t)kC * kD, (size_t)kC * kC, (size_t)kDgParts};
+  const size_t sizes[kSlots] = {(size_t)kC,      (size_t)kC * kC, (size_t)kC * kD, (size_t)kC * kD, (size_t)kD * kD,
+                                (size_t)kC * kD, (size_t)kC * kC, (size_t)kC * kD, (size_t)kD * kD, (size_t)kDgParts};
   Workspace w{};
   size_t at = 0;
-  for (int i = 0; i < 14; ++i) {
+  for (int i = 0; i < kSlots; ++i) {
     w.offs[i] = at;
     if (i < 7 || backward) at += ((sizes[i] * chunks * sizeof(float)) + 255) & ~(size_t)255;
   }
@@ -1384,12 +1273,11 @@ int build(const th_deltanet_desc* d, bool backward, th_launch** out) {
   a.da = d->da;
   a.dbeta = d->dbeta;
   // The per-chunk intermediates (ca, T, W, Ut, S, U, P; for the backward dU,
-  // dSn, dQg, dW, dKd, dP, dg) lie in the launch's workspace at w.offs.
-  const size_t slot_args[14] = {TH_OFFSET(DnArgs, ca),  TH_OFFSET(DnArgs, T),   TH_OFFSET(DnArgs, W),
-                                TH_OFFSET(DnArgs, Ut),  TH_OFFSET(DnArgs, S),   TH_OFFSET(DnArgs, U),
-                                TH_OFFSET(DnArgs, P),   TH_OFFSET(DnArgs, dU),  TH_OFFSET(DnArgs, dSn),
-                                TH_OFFSET(DnArgs, dQg), TH_OFFSET(DnArgs, dW),  TH_OFFSET(DnArgs, dKd),
-                                TH_OFFSET(DnArgs, dP),  TH_OFFSET(DnArgs, dg)};
+  // dSn, dg) lie in the launch's workspace at w.offs.
+  const size_t slot_args[kSlots] = {TH_OFFSET(DnArgs, ca), TH_OFFSET(DnArgs, T),  TH_OFFSET(DnArgs, W),
+                                    TH_OFFSET(DnArgs, Ut), TH_OFFSET(DnArgs, S),  TH_OFFSET(DnArgs, U),
+                                    TH_OFFSET(DnArgs, P),  TH_OFFSET(DnArgs, dU), TH_OFFSET(DnArgs, dSn),
+                                    TH_OFFSET(DnArgs, dg)};
   a.s_h = d->strides[0];
   a.s_t = d->strides[1];
   a.s_b = d->strides[2];
@@ -1400,10 +1288,10 @@ int build(const th_deltanet_desc* d, bool backward, th_launch** out) {
   a.heads = d->heads;
   a.seq = d->seq;
   a.chunks = d->seq / kC;
-  const void* fns[7] = {(const void*)dn_chunk_prep, (const void*)dn_state_scan, (const void*)dn_output,
-                        (const void*)dn_state_grad, (const void*)dn_grad_a, (const void*)dn_grad_b, nullptr};
-  const size_t ldss[6] = {kPrepLds, kScanLds, kOutLds, kSgLds, kGaLds, kGbLds};
-  for (int i = 0; i < 6; ++i) TH_HIP(hipFuncSetAttribute(fns[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldss[i]));
+  const void* fns[5] = {(const void*)dn_chunk_prep, (const void*)dn_state_scan, (const void*)dn_output,
+                        (const void*)dn_state_grad, (const void*)dn_grad};
+  const size_t ldss[5] = {kPrepLds, kScanLds, kOutLds, kSgLds, kGradLds};
+  for (int i = 0; i < 5; ++i) TH_HIP(hipFuncSetAttribute(fns[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldss[i]));
   th::Builder b(backward ? "deltanet_fwd_bwd" : "deltanet_fwd", 12);
   const uint64_t at_ws = b.workspace(w.bytes);
   // A gradient with no o given keeps it in the workspace, at q's strides.
@@ -1413,15 +1301,14 @@ int build(const th_deltanet_desc* d, bool backward, th_launch** out) {
   const uint64_t at_o = own_o ? b.workspace(o_bytes) : 0;
   const unsigned nchunks = (unsigned)chunks;
   const unsigned scans = (unsigned)((int64_t)d->batch * d->heads * (kD / kCols));
-  int ks[6];
+  int ks[5];
   int nk = 0;
   ks[nk++] = b.kernel(fns[0], "dn_chunk_prep", dim3(nchunks), dim3(256), (uint32_t)kPrepLds, a);
   ks[nk++] = b.kernel(fns[1], "dn_state_scan", dim3(scans), dim3(kScanThreads), (uint32_t)kScanLds, a);
   ks[nk++] = b.kernel(fns[2], "dn_output", dim3(nchunks), dim3(256), (uint32_t)kOutLds, a);
   if (backward) {
     ks[nk++] = b.kernel(fns[3], "dn_state_grad", dim3(scans), dim3(kScanThreads), (uint32_t)kSgLds, a);
-    ks[nk++] = b.kernel(fns[4], "dn_grad_a", dim3(nchunks), dim3(256), (uint32_t)kGaLds, a);
-    ks[nk++] = b.kernel(fns[5], "dn_grad_b", dim3(nchunks), dim3(256), (uint32_t)kGbLds, a);
+    ks[nk++] = b.kernel(fns[4], "dn_grad", dim3(nchunks), dim3(256), (uint32_t)kGradLds, a);
   }
   const size_t offs[12] = {TH_OFFSET(DnArgs, q),  TH_OFFSET(DnArgs, k),  TH_OFFSET(DnArgs, v),     TH_OFFSET(DnArgs, a),
                            TH_OFFSET(DnArgs, beta), TH_OFFSET(DnArgs, o), TH_OFFSET(DnArgs, dout), TH_OFFSET(DnArgs, dq),
@@ -1431,7 +1318,7 @@ int build(const th_deltanet_desc* d, bool backward, th_launch** out) {
       for (int i = 0; i < nk; ++i) b.ref(v, ks[i], offs[v]);
   if (own_o)
     for (int i = 0; i < nk; ++i) b.ws_ref(ks[i], offs[5], at_o);
-  for (int j = 0; j < 14; ++j)
+  for (int j = 0; j < kSlots; ++j)
     if (j < 7 || backward)
       for (int i = 0; i < nk; ++i) b.ws_ref(ks[i], slot_args[j], at_ws + w.offs[j]);
   for (int v : {0, 1, 2, 5, 6, 7, 8, 9}) b.align(v, 16);

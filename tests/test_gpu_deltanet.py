@@ -80,3 +80,22 @@ def test_config5_full_size_sampled_sequences(target):
         for name, g, r in zip(("dq", "dk", "dv", "da", "dbeta"),
                               (pick(dq), pick(dk), pick(dv), pickg(da), pickg(dbeta)), grads):
             assert relative(g, r) < TOL, (b, h, name)
+
+
+@pytest.mark.parametrize("B,T,H,decay", [(1, 64, 1, 1.0), (1, 192, 2, 0.0), (2, 128, 3, 0.3), (1, 320, 1, 1.0)])
+def test_gate_gradients_to_the_products_precision(target, B, T, H, decay):
+    """da and dbeta are fp32 and depend on every product of a chunk's gradient,
+    each exact to about 2^-16: through the at most six products in a row of
+    the longest path, 6 x 2^-16 < 1e-4 of the float64 oracle, norm-wise; from
+    no decay at all to about e^-51 over a chunk (the kernels form the decay
+    between every two positions, either way round: fp32 holds up to e^88)."""
+    import tempest_hip as th
+    announce("deltanet gates", B, T, H, decay)
+    q, k, v, a, beta, do = _inputs(B, T, H, 3 * T + H)
+    a = (a * decay).contiguous()
+    comp = th.compile(th.programs.deltanet(B, H, T), target, q, k, v, a, beta, do)
+    out = comp(q, k, v, a, beta, do)
+    grads = interpret.deltanet_grad(*[_np(x).astype(np.float64) for x in (q, k, v, a, beta, do)])
+    for name, got, ref in (("da", out[4], grads[3]), ("dbeta", out[5], grads[4])):
+        err = relative(_np(got).reshape(B, T, H), ref)
+        assert err < 1e-4, (name, err)
