@@ -121,6 +121,9 @@ __device__ __forceinline__ void cumulative_gates(float* ca, const DnArgs& p, con
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+typedef short s16x4v __attribute__((ext_vector_type(4)));
+typedef short s16x8v __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) s16x4v lds_s16x4v;
 constexpr int kLd = 132;   // LDS row of 128 fp32
 constexpr int kLdC = 68;   // LDS row of 64 fp32
 constexpr int kLdS = 36;   // LDS row of 32 fp32
@@ -226,73 +229,142 @@ __device__ __forceinline__ void store_blocks(float* out, int ld, const f32x4v (&
       for (int v = 0; v < 4; ++v) out[(int64_t)(i0 + 16 * bi + 4 * g + v) * ld + j0 + 16 * bj + r] = s * acc[bi][bj][v];
 }
 
-// Operand readers for mm_by: quad(x, k) is this lane's (x, k .. k + 3).
-struct RowF32 {  // (x, k) at p[x * ld + k]
-  static constexpr bool kExact = false;
+// Operand readers for mm_by: block(x0, k0) is the block (x0 .. x0 + 15, k0 .. k0 + 31)
+// as this lane l = 16 g + r holds it: (x0 + r, k0 + 8 g .. k0 + 8 g + 7).
+// Those over fp32 split it at each read; Planes hold an operand split once
+// where it was written (hi and lo as bf16, what split8 gives), read as they are:
+// the splits were most of the instructions of a kernel whose waves read each
+// operand several times over.
+__device__ __forceinline__ int lane_r() { return plain(threadIdx.x % 16); }
+__device__ __forceinline__ int lane_g8() { return plain((threadIdx.x % 64) / 16 * 8); }
+template <bool kExactValues>
+struct RowFloats {  // (x, k) at p[x * ld + k]
+  static constexpr bool kExact = kExactValues;
   const float* p;
   int ld;
-  __device__ f32x4v quad(int x, int k) const { return *reinterpret_cast<const f32x4v*>(p + x * ld + k); }
-};
-struct ColF32 {  // (x, k) at p[k * ld + x]
-  static constexpr bool kExact = false;
-  const float* p;
-  int ld;
-  __device__ f32x4v quad(int x, int k) const { return column_quad(p, ld, k, x); }
-};
-struct RowF32Bf {  // (x, k) at p[x * ld + k], fp32 holding bf16 values
-  static constexpr bool kExact = true;
-  const float* p;
-  int ld;
-  __device__ f32x4v quad(int x, int k) const { return *reinterpret_cast<const f32x4v*>(p + x * ld + k); }
-};
-struct ColF32Bf {  // (x, k) at p[k * ld + x], fp32 holding bf16 values
-  static constexpr bool kExact = true;
-  const float* p;
-  int ld;
-  __device__ f32x4v quad(int x, int k) const { return column_quad(p, ld, k, x); }
-};
-struct RowBf16 {  // (x, k) at bf16 p[x * ld + k]
-  static constexpr bool kExact = true;
-  const uint16_t* p;
-  int64_t ld;
-  __device__ f32x4v quad(int x, int k) const {
-    const uint2 w = *reinterpret_cast<const uint2*>(p + x * ld + k);
-    return f32x4v{bf((uint16_t)w.x), bf((uint16_t)(w.x >> 16)), bf((uint16_t)w.y), bf((uint16_t)(w.y >> 16))};
+  __device__ Split8 block(int x0, int k0, int r, int g8) const {
+    const float* at = p + (x0 + r) * ld + k0 + g8;
+    return split8<kExact>(quad(at), quad(at + 4));
   }
 };
-struct ColBf16 {  // (x, k) at bf16 p[k * ld + x]
+template <bool kExactValues>
+struct ColFloats {  // (x, k) at p[k * ld + x]
+  static constexpr bool kExact = kExactValues;
+  const float* p;
+  int ld;
+  __device__ Split8 block(int x0, int k0, int r, int g8) const {
+    return split8<kExact>(column_quad(p, ld, k0 + g8, x0 + r), column_quad(p, ld, k0 + g8 + 4, x0 + r));
+  }
+};
+typedef RowFloats<false> RowF32;
+typedef ColFloats<false> ColF32;
+typedef RowFloats<true> RowF32Bf;  // fp32 holding bf16 values
+typedef ColFloats<true> ColF32Bf;
+
+// Eight bf16 along a row of memory or LDS, 16-byte aligned.
+__device__ __forceinline__ bf16x8v row8(const uint16_t* p) {
+  return __builtin_bit_cast(bf16x8v, *reinterpret_cast<const u32x4v*>(p));
+}
+// Eight rows k0 + g8 .. of column x0 + r of LDS rows of ld bf16:
+// ds_read_b64_tr_b16 hands lane i of each 16 element i % 4 of the 8-byte pieces
+// that lanes 4 k + i / 4 address; lane j addresses row j / 4, columns
+// 4 (j % 4) .., so lane i gets rows 0..3 of column i, and a second read rows 4..7.
+__device__ __forceinline__ bf16x8v column8(const uint16_t* p, int ld, int x0, int k0, int r, int g8) {
+  const uint16_t* at = p + (k0 + g8 + r / 4) * ld + x0 + 4 * (r % 4);
+  const s16x4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4v*)at);
+  const s16x4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4v*)(at + 4 * ld));
+  return __builtin_bit_cast(bf16x8v, s16x8v{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+}
+__device__ __forceinline__ bf16x8v none8() { return __builtin_bit_cast(bf16x8v, u32x4v{0u, 0u, 0u, 0u}); }
+template <class Ld>
+struct RowBf16At {  // (x, k) at bf16 p[x * ld + k]
+  static constexpr bool kExact = true;
+  const uint16_t* p;
+  Ld ld;
+  __device__ Split8 block(int x0, int k0, int r, int g8) const { return Split8{row8(p + (x0 + r) * ld + k0 + g8), none8()}; }
+};
+typedef RowBf16At<int> RowBf16;       // in LDS
+typedef RowBf16At<int64_t> RowBf16G;  // in memory
+struct ColBf16 {  // (x, k) at bf16 p[k * ld + x], in LDS
   static constexpr bool kExact = true;
   const uint16_t* p;
   int ld;
-  __device__ f32x4v quad(int x, int k) const {
-    return f32x4v{bf(p[k * ld + x]), bf(p[(k + 1) * ld + x]), bf(p[(k + 2) * ld + x]), bf(p[(k + 3) * ld + x])};
+  __device__ Split8 block(int x0, int k0, int r, int g8) const { return Split8{column8(p, ld, x0, k0, r, g8), none8()}; }
+};
+struct Planes {  // rows of ld bf16 in LDS, twice
+  uint16_t *hi, *lo;
+  int ld;
+  // Two values, at (i, j) and (i + 1, j).
+  __device__ void put_rows(int i, int j, float a, float b) const {
+    const uint32_t h = pk2(a, b), l = pk2(a - __uint_as_float(h << 16), b - __uint_as_float(h & 0xffff0000u));
+    const int at = i * ld + j;
+    hi[at] = (uint16_t)h, hi[at + ld] = (uint16_t)(h >> 16);
+    lo[at] = (uint16_t)l, lo[at + ld] = (uint16_t)(l >> 16);
+  }
+  // The same at (i, j) and (i, j + 1), j even.
+  __device__ void put(int i, int j, float a, float b) const {
+    const uint32_t h = pk2(a, b), l = pk2(a - __uint_as_float(h << 16), b - __uint_as_float(h & 0xffff0000u));
+    *reinterpret_cast<uint32_t*>(hi + i * ld + j) = h;
+    *reinterpret_cast<uint32_t*>(lo + i * ld + j) = l;
   }
 };
+struct RowPlanes {  // (x, k) at (x, k)
+  static constexpr bool kExact = false;
+  Planes p;
+  __device__ Split8 block(int x0, int k0, int r, int g8) const {
+    const int at = (x0 + r) * p.ld + k0 + g8;
+    return Split8{row8(p.hi + at), row8(p.lo + at)};
+  }
+};
+struct ColPlanes {  // (x, k) at (k, x)
+  static constexpr bool kExact = false;
+  Planes p;
+  __device__ Split8 block(int x0, int k0, int r, int g8) const {
+    return Split8{column8(p.hi, p.ld, x0, k0, r, g8), column8(p.lo, p.ld, x0, k0, r, g8)};
+  }
+};
+// The blocks of acc, rows i0 .. and columns j0 .., times s, to planes.
+template <int BI, int BJ>
+__device__ __forceinline__ void store_planes(const Planes& to, const f32x4v (&acc)[BI][BJ], int i0, int j0, float s) {
+  const int r = lane_r(), g4 = plain((threadIdx.x % 64) / 16 * 4);
+#pragma unroll
+  for (int bi = 0; bi < BI; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < BJ; ++bj)
+#pragma unroll
+      for (int v = 0; v < 4; v += 2)
+        to.put_rows(i0 + 16 * bi + g4 + v, j0 + 16 * bj + r, s * acc[bi][bj][v], s * acc[bi][bj][v + 1]);
+}
 
 // acc[bi][bj] += X(i0 + 16 bi .., k) Y(k, j0 + 16 bj ..) over k in [0, K).
 template <int BI, int BJ, class XR, class YR>
 __device__ __forceinline__ void mm_by(f32x4v (&acc)[BI][BJ], const XR& X, int i0, const YR& Y, int j0, int K) {
-  const int r = plain(threadIdx.x % 16), g = plain((threadIdx.x % 64) / 16);
+  const int r = lane_r(), g8 = lane_g8();
   for (int kb = 0; kb < K; kb += 32) {
-    const int k0 = kb + 8 * g;
     Split8 b[BJ];
 #pragma unroll
-    for (int bj = 0; bj < BJ; ++bj)
-      b[bj] = split8<YR::kExact>(Y.quad(j0 + 16 * bj + r, k0), Y.quad(j0 + 16 * bj + r, k0 + 4));
+    for (int bj = 0; bj < BJ; ++bj) b[bj] = Y.block(j0 + 16 * bj, kb, r, g8);
     // The rows of X one block at a time: only one of its split blocks live.
 #pragma unroll
     for (int bi = 0; bi < BI; ++bi) {
-      const Split8 a = split8<XR::kExact>(X.quad(i0 + 16 * bi + r, k0), X.quad(i0 + 16 * bi + r, k0 + 4));
+      const Split8 a = X.block(i0 + 16 * bi, kb, r, g8);
 #pragma unroll
       for (int bj = 0; bj < BJ; ++bj) acc[bi][bj] = mma_split<XR::kExact, YR::kExact>(a, b[bj], acc[bi][bj]);
     }
   }
 }
 
-// Sum over the 16 lanes of a row group (lanes 16 g .. 16 g + 15), a fixed tree.
+// Sum over the 16 lanes of a row group (lanes 16 g .. 16 g + 15), a fixed tree
+// (1, 2, 4, 8 apart; by then alike within the group of lanes that a mirror swaps).
+template <int kDpp>
+__device__ __forceinline__ float moved(float x) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), kDpp, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float row_group_sum(float x) {
-#pragma unroll
-  for (int o = 1; o < 16; o <<= 1) x += __shfl_xor(x, o, 64);
+  x += moved<0xB1>(x);   // quad_perm 1, 0, 3, 2
+  x += moved<0x4E>(x);   // quad_perm 2, 3, 0, 1
+  x += moved<0x141>(x);  // row_half_mirror
+  x += moved<0x140>(x);  // row_mirror
   return x;
 }
 
@@ -826,7 +898,7 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_state_grad(DnArgs p) {
 // writes 48.  The products stay in the registers that the outputs sum in (dQg
 // in dQ's, dKd and T' dW in dK's, dP in the lanes that form dQK), so none of
 // them goes through memory; as two kernels that passed dQg, dW, dKd and dP on
-// (224 KB a chunk, out and back) the same took 1293 us at B4 H16 T8192, now 1022.
+// (224 KB a chunk, out and back) the same took 1293 us at B4 H16 T8192, now 889.
 //
 // Every product on the matrix cores, split bf16; dO, Q and K sit in LDS as
 // bf16 (their exact values) and are widened as they are read; U, dU and dW take
@@ -838,23 +910,19 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_state_grad(DnArgs p) {
 // the column work's partials go to LDS by wave and are folded in a fixed
 // order, so the result does not depend on timing.
 
-// acc1 += X1 Y', acc2 += X2 Y' over k in [0, K): rows i0 .. of X1 and X2, each
-// quad of Y read once.
+// acc1 += X1 Y, acc2 += X2 Y over k in [0, K): rows i0 .. of X1 and X2, each
+// block of Y read once.
 template <int BI, int BJ, class X1, class X2, class YR>
 __device__ __forceinline__ void mm_by2(f32x4v (&acc1)[BI][BJ], const X1& x1, f32x4v (&acc2)[BI][BJ], const X2& x2,
                                        int i0, const YR& Y, int j0, int K) {
-  const int r = plain(threadIdx.x % 16), g = plain((threadIdx.x % 64) / 16);
+  const int r = lane_r(), g8 = lane_g8();
   for (int kb = 0; kb < K; kb += 32) {
-    const int k0 = kb + 8 * g;
     Split8 b[BJ];
 #pragma unroll
-    for (int bj = 0; bj < BJ; ++bj)
-      b[bj] = split8<YR::kExact>(Y.quad(j0 + 16 * bj + r, k0), Y.quad(j0 + 16 * bj + r, k0 + 4));
+    for (int bj = 0; bj < BJ; ++bj) b[bj] = Y.block(j0 + 16 * bj, kb, r, g8);
 #pragma unroll
     for (int bi = 0; bi < BI; ++bi) {
-      const int i = i0 + 16 * bi + r;
-      const Split8 a1 = split8<X1::kExact>(x1.quad(i, k0), x1.quad(i, k0 + 4));
-      const Split8 a2 = split8<X2::kExact>(x2.quad(i, k0), x2.quad(i, k0 + 4));
+      const Split8 a1 = x1.block(i0 + 16 * bi, kb, r, g8), a2 = x2.block(i0 + 16 * bi, kb, r, g8);
 #pragma unroll
       for (int bj = 0; bj < BJ; ++bj) {
         acc1[bi][bj] = mma_split<X1::kExact, YR::kExact>(a1, b[bj], acc1[bi][bj]);
@@ -876,11 +944,15 @@ struct HeldF32 {
       x[u] = quad(src + (e / 32) * kD + 4 * (e % 32));
     }
   }
-  __device__ void store(float* dst) const {
+  __device__ void store(const Planes& to) const {
 #pragma unroll
     for (int u = 0; u < n; ++u) {
-      const int e = threadIdx.x + 256 * u;
-      *reinterpret_cast<f32x4v*>(dst + (e / 32) * kLd + 4 * (e % 32)) = x[u];
+      const int e = threadIdx.x + 256 * u, at = (e / 32) * to.ld + 4 * (e % 32);
+      const u32x2v h = {pk2(x[u][0], x[u][1]), pk2(x[u][2], x[u][3])};
+      const u32x2v l = {pk2(x[u][0] - __uint_as_float(h[0] << 16), x[u][1] - __uint_as_float(h[0] & 0xffff0000u)),
+                        pk2(x[u][2] - __uint_as_float(h[1] << 16), x[u][3] - __uint_as_float(h[1] & 0xffff0000u))};
+      *reinterpret_cast<u32x2v*>(to.hi + at) = h;
+      *reinterpret_cast<u32x2v*>(to.lo + at) = l;
     }
   }
 };
@@ -903,7 +975,9 @@ struct HeldBf16 {
   }
 };
 
-constexpr int kGradX = 2 * kC * kLdC > kC * kLd ? 2 * kC * kLdC : kC * kLd;
+constexpr int kLdP = 72;                // LDS row of 64 bf16
+constexpr int kGradX = 2 * kC * kLdP;   // floats: M and N as planes; U, dU and dW take 2 kC kLdH / 2
+static_assert(kGradX >= kC * kLdH && kC * kLdP >= kC * kLdC, "");
 constexpr size_t kGradLds = 2 * kC * kLdH * sizeof(uint16_t) + kGradX * sizeof(float) +
                             (2 * kC + 5 * 4 * kC + 2 * kC) * sizeof(float);
 
@@ -911,10 +985,13 @@ __global__ __launch_bounds__(256, 2) void dn_grad(DnArgs p) {
   extern __shared__ float lds[];
   uint16_t* Qh = reinterpret_cast<uint16_t*>(lds);       // [64][kLdH]: dO, then Q
   uint16_t* Kh = Qh + kC * kLdH;                          // [64][kLdH]
-  float* X = reinterpret_cast<float*>(Kh + kC * kLdH);   // [64][kLd]: U, then dU, then dW
-  float* M = X;                    // [64][kLdC]: dT, then dA, then dG + dG'
-  float* N = M + kC * kLdC;        // [64][kLdC]: T' dT, then dG, then dQK
-  float* wrow = X + kGradX;        // [64]: sum_j w_ij
+  uint16_t* x0 = Kh + kC * kLdH;
+  const Planes X{x0, x0 + kC * kLdH, kLdH};               // [64][kLdH]: U, then dU, then dW
+  const Planes M{x0, x0 + kC * kLdP, kLdP};               // [64][kLdP]: dT, then dG + dG'
+  uint16_t* n0 = x0 + 2 * kC * kLdP;
+  const Planes Np{n0, n0 + kC * kLdP, kLdP};              // [64][kLdP]: dQK
+  float* N = reinterpret_cast<float*>(n0);                // [64][kLdC] before: T' dT, then dG
+  float* wrow = reinterpret_cast<float*>(x0) + kGradX;    // [64]: sum_j w_ij
   float* brow = wrow + kC;         // [64]: sum_j dA Gamma G
   float* wcol = brow + kC;         // [4][64]: sum_i w_ij by wave
   float* kx = wcol + 4 * kC;       // [4][64]: k . dX by wave (columns)
@@ -948,8 +1025,8 @@ __global__ __launch_bounds__(256, 2) void dn_grad(DnArgs p) {
   const RowBf16 Kr{Kh, kLdH}, Qr{Qh, kLdH};
   const ColBf16 Kc{Kh, kLdH}, Qc{Qh, kLdH};
   const float last = ca[kC - 1];
-  const RowF32 Xr{X, kLd};
-  const ColF32 Xc{X, kLd};
+  const RowPlanes Xr{X};
+  const ColPlanes Xc{X};
   const RowBf16 Or{Qh, kLdH};
   // U: dKd = U dSn' (kd; sk = k . dKd a row) and dP = lower(dO U') (this wave's rows).
   f32x4v kd[4][2], dp[1][4];
@@ -1022,7 +1099,7 @@ __global__ __launch_bounds__(256, 2) void dn_grad(DnArgs p) {
         }
     }
     clear(yv);
-    mm_by(yv, Xr, i0, RowBf16{vg, p.s_t}, 0, kD);
+    mm_by(yv, Xr, i0, RowBf16G{vg, p.s_t}, 0, kD);
   }
   f32x4v dq[4][2];
   {
@@ -1032,7 +1109,7 @@ __global__ __launch_bounds__(256, 2) void dn_grad(DnArgs p) {
     clear(wq);
     mm_by2(dq, Or, wq, Xr, 0, RowF32{p.S + ck.c * kD * kD, kD}, d0, kD);
     __syncthreads();
-    store_blocks(X, kLd, wq, 0, d0, -1.0f);
+    store_planes(X, wq, 0, d0, -1.0f);
     q.load(p.q + ck.row0, p.s_t);
     q.store(Qh);
   }
@@ -1067,37 +1144,26 @@ __global__ __launch_bounds__(256, 2) void dn_grad(DnArgs p) {
     mm_by(xk, Xr, i0, Kr, 0, kD);
     __syncthreads();
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
+    for (int bj = 0; bj < 4; ++bj) {
+      const float bl = be[16 * bj + r], el = expf(ca[16 * bj + r]);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = i0 + g4 + v, l = 16 * bj + r;
-        M[i * kLdC + l] = be[l] * (expf(ca[l]) * xk[0][bj][v] + yv[0][bj][v]);
-      }
+      for (int v = 0; v < 4; ++v) xk[0][bj][v] = bl * (el * xk[0][bj][v] + yv[0][bj][v]);
+    }
+    store_planes(M, xk, i0, 0, 1.0f);
   }
   __syncthreads();
   // N = T' dT.
   {
     f32x4v acc[1][4];
     clear(acc);
-    mm_by(acc, ColF32{Tc, kC}, i0, ColF32{M, kLdC}, 0, kC);
+    mm_by(acc, ColF32{Tc, kC}, i0, ColPlanes{M}, 0, kC);
     store_blocks(N, kLdC, acc, i0, 0, 1.0f);
   }
   __syncthreads();
-  // dA = -(N T') o strict lower (into M).
-  {
-    f32x4v acc[1][4];
-    clear(acc);
-    mm_by(acc, RowF32{N, kLdC}, i0, RowF32{Tc, kC}, 0, kC);
-#pragma unroll
-    for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = i0 + g4 + v, j = 16 * bj + r;
-        M[i * kLdC + j] = i > j ? -acc[0][bj][v] : 0.0f;
-      }
-  }
-  // Every row of this wave's M was written by this wave; the other waves'
-  // rows are not read before the next barrier.
+  // dA = -(N T') o strict lower (this wave's rows of N are its own).
+  f32x4v dA[1][4];
+  clear(dA);
+  mm_by(dA, RowF32{N, kLdC}, i0, RowF32{Tc, kC}, 0, kC);
   // With G = K K', QK = Q K', Gamma: dG = dA o beta_i o Gamma (into N);
   // dbeta_i gets sum_j dA Gamma G; w = (dA beta_i G + dP QK) o Gamma gives
   // dca_i += sum_j w_ij - sum_j w_ji.
@@ -1125,11 +1191,11 @@ __global__ __launch_bounds__(256, 2) void dn_grad(DnArgs p) {
       for (int v = 0; v < 4; ++v) {
         const int i = i0 + g4 + v, j = 16 * bj + r;
         const float gam = expf(ca[i] - ca[j]);
-        const float dA = M[i * kLdC + j];
+        const float da = i > j ? -dA[0][bj][v] : 0.0f;
         const float gg = bj <= w ? gk[0][bj][v] : 0.0f, q = bj <= w ? qk[0][bj][v] : 0.0f;
-        N[i * kLdC + j] = dA * be[i] * gam;
-        rowb[v] += dA * gam * gg;
-        const float wv = i >= j ? (dA * be[i] * gg + dp[0][bj][v] * q) * gam : 0.0f;
+        N[i * kLdC + j] = da * be[i] * gam;
+        rowb[v] += da * gam * gg;
+        const float wv = i >= j ? (da * be[i] * gg + dp[0][bj][v] * q) * gam : 0.0f;
         roww[v] += wv;
         colw[bj] += wv;
         dp[0][bj][v] = i >= j ? dp[0][bj][v] * gam : 0.0f;  // dQK
@@ -1153,19 +1219,19 @@ __global__ __launch_bounds__(256, 2) void dn_grad(DnArgs p) {
   }
   __syncthreads();
   // M <- dG + dG'.
-  for (int e = t; e < kC * kC; e += 256) {
-    const int i = e / kC, j = e % kC;
-    M[i * kLdC + j] = N[i * kLdC + j] + N[j * kLdC + i];
+  for (int e = t; e < kC * kC / 2; e += 256) {
+    const int i = e / (kC / 2), j = 2 * (e % (kC / 2));
+    M.put(i, j, N[i * kLdC + j] + N[j * kLdC + i], N[i * kLdC + j + 1] + N[(j + 1) * kLdC + i]);
   }
   __syncthreads();
   // dQK = dP o Gamma (lower), read by two of the products below along its rows
   // and its columns, into N (free now).
-  store_blocks(N, kLdC, dp, i0, 0, 1.0f);
+  store_planes(Np, dp, i0, 0, 1.0f);
   __syncthreads();
   // dQ = e^ca dQg + dQK K;  dK = dQK' Q + (dG + dG') K + beta e^ca dX + e^(last - ca) dKd.
-  mm_by(dq, RowF32{N, kLdC}, 0, Kc, d0, kC);
-  mm_by(kd, ColF32{N, kLdC}, 0, Qc, d0, kC);
-  mm_by(kd, RowF32{M, kLdC}, 0, Kc, d0, kC);
+  mm_by(dq, RowPlanes{Np}, 0, Kc, d0, kC);
+  mm_by(kd, ColPlanes{Np}, 0, Qc, d0, kC);
+  mm_by(kd, RowPlanes{M}, 0, Kc, d0, kC);
 #pragma unroll
   for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
