@@ -87,6 +87,16 @@ __device__ __forceinline__ Chunk chunk_of(const DnArgs& p, int64_t c) {
   return k;
 }
 
+// Chunk n of the sequence whose first chunk is `first` (its divisions done once).
+__device__ __forceinline__ Chunk chunk_at(const DnArgs& p, const Chunk& first, int n) {
+  Chunk k = first;
+  k.n = n;
+  k.c += n;
+  k.row0 += (int64_t)n * kC * p.s_t;
+  k.grow0 += (int64_t)n * kC * p.g_t;
+  return k;
+}
+
 // ca = inclusive cumulative sum of a over the chunk (wave 0), into LDS.
 __device__ __forceinline__ void cumulative_gates(float* ca, const DnArgs& p, const Chunk& ck) {
   if (threadIdx.x < 64) {
@@ -107,14 +117,11 @@ __device__ __forceinline__ void cumulative_gates(float* ca, const DnArgs& p, con
 // that are bf16 values, Q K V, have no lo).  The three bf16 products of 32 k
 // take 48 matrix-core cycles, the eight fp32 ones (v_mfma_f32_16x16x4_f32)
 // for the same k would take 256.
-// Operands sit in LDS as fp32 rows of kLd floats: a row's 16-byte quads land
-// on distinct bank quads for 16 consecutive rows (kLd / 4 odd), and a column
-// read by 16 consecutive rows x 4 row groups hits 64 distinct banks
-// (kLd = 4 mod 16).
+// Operands sit in LDS as rows padded by 16 bytes: the 16-byte pieces of 16
+// consecutive rows land on distinct banks.
 //
 // Lane l = 16 g + r of a 16 x 16 block over 32 consecutive k takes the eight
-// k = kb + 8 g + (0..7): two quads per operand when k runs along its rows,
-// split to bf16, each pairing A(i0 + r, k) with B(k, j0 + r); the products'
+// k = kb + 8 g + (0..7), each pairing A(i0 + r, k) with B(k, j0 + r); the products'
 // k slot g then holds the same k in both operands.  The block
 // C(i0 + 4 g + v, j0 + r) sits in register v of lane l.
 
@@ -124,9 +131,9 @@ typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
 typedef short s16x4v __attribute__((ext_vector_type(4)));
 typedef short s16x8v __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) s16x4v lds_s16x4v;
-constexpr int kLd = 132;   // LDS row of 128 fp32
 constexpr int kLdC = 68;   // LDS row of 64 fp32
 constexpr int kLdS = 36;   // LDS row of 32 fp32
+constexpr int kLdT = 40;   // LDS row of 32 bf16
 
 __device__ __forceinline__ f32x4v quad(const float* row) { return *reinterpret_cast<const f32x4v*>(row); }
 
@@ -182,30 +189,6 @@ __device__ __forceinline__ f32x4v mma_split(const Split8& a, const Split8& b, f3
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.hi, b.hi, c, 0, 0, 0);
 }
 
-// acc[bi][bj] += X(i0 + 16 bi .., k) Y(k, j0 + 16 bj ..) over k in [0, K), each
-// operand read along its rows (X(i, k) = X[i * ldx + k], Y(k, j) = Y[j * ldy + k])
-// or, when XT / YT, along its columns (X(i, k) = X[k * ldx + i], Y(k, j) =
-// Y[k * ldy + j]).  Strides satisfy ld / 4 odd and ld = 4 mod 16.
-template <bool XT, bool YT, int BI, int BJ>
-__device__ __forceinline__ void mm_gen(f32x4v (&acc)[BI][BJ], const float* X, int ldx, int i0, const float* Y, int ldy,
-                                       int j0, int K) {
-  const int r = plain(threadIdx.x % 16), g = plain((threadIdx.x % 64) / 16);
-  auto xq = [&](int k0, int i) { return XT ? column_quad(X, ldx, k0, i) : quad(X + i * ldx + k0); };
-  auto yq = [&](int k0, int j) { return YT ? column_quad(Y, ldy, k0, j) : quad(Y + j * ldy + k0); };
-  for (int kb = 0; kb < K; kb += 32) {
-    const int k0 = kb + 8 * g;
-    Split8 a[BI], b[BJ];
-#pragma unroll
-    for (int bi = 0; bi < BI; ++bi) a[bi] = split8<false>(xq(k0, i0 + 16 * bi + r), xq(k0 + 4, i0 + 16 * bi + r));
-#pragma unroll
-    for (int bj = 0; bj < BJ; ++bj) b[bj] = split8<false>(yq(k0, j0 + 16 * bj + r), yq(k0 + 4, j0 + 16 * bj + r));
-#pragma unroll
-    for (int bi = 0; bi < BI; ++bi)
-#pragma unroll
-      for (int bj = 0; bj < BJ; ++bj) acc[bi][bj] = mma_split<false, false>(a[bi], b[bj], acc[bi][bj]);
-  }
-}
-
 template <int BI, int BJ>
 __device__ __forceinline__ void clear(f32x4v (&acc)[BI][BJ]) {
 #pragma unroll
@@ -237,9 +220,8 @@ __device__ __forceinline__ void store_blocks(float* out, int ld, const f32x4v (&
 // operand several times over.
 __device__ __forceinline__ int lane_r() { return plain(threadIdx.x % 16); }
 __device__ __forceinline__ int lane_g8() { return plain((threadIdx.x % 64) / 16 * 8); }
-template <bool kExactValues>
-struct RowFloats {  // (x, k) at p[x * ld + k]
-  static constexpr bool kExact = kExactValues;
+struct RowF32 {  // (x, k) at p[x * ld + k]
+  static constexpr bool kExact = false;
   const float* p;
   int ld;
   __device__ Split8 block(int x0, int k0, int r, int g8) const {
@@ -247,19 +229,14 @@ struct RowFloats {  // (x, k) at p[x * ld + k]
     return split8<kExact>(quad(at), quad(at + 4));
   }
 };
-template <bool kExactValues>
-struct ColFloats {  // (x, k) at p[k * ld + x]
-  static constexpr bool kExact = kExactValues;
+struct ColF32 {  // (x, k) at p[k * ld + x]
+  static constexpr bool kExact = false;
   const float* p;
   int ld;
   __device__ Split8 block(int x0, int k0, int r, int g8) const {
     return split8<kExact>(column_quad(p, ld, k0 + g8, x0 + r), column_quad(p, ld, k0 + g8 + 4, x0 + r));
   }
 };
-typedef RowFloats<false> RowF32;
-typedef ColFloats<false> ColF32;
-typedef RowFloats<true> RowF32Bf;  // fp32 holding bf16 values
-typedef ColFloats<true> ColF32Bf;
 
 // Eight bf16 along a row of memory or LDS, 16-byte aligned.
 __device__ __forceinline__ bf16x8v row8(const uint16_t* p) {
@@ -300,6 +277,14 @@ struct Planes {  // rows of ld bf16 in LDS, twice
     const int at = i * ld + j;
     hi[at] = (uint16_t)h, hi[at + ld] = (uint16_t)(h >> 16);
     lo[at] = (uint16_t)l, lo[at + ld] = (uint16_t)(l >> 16);
+  }
+  // Four at (i, j) .. (i, j + 3), j a multiple of 4.
+  __device__ void put(int i, int j, f32x4v x) const {
+    const u32x2v h = {pk2(x[0], x[1]), pk2(x[2], x[3])};
+    const u32x2v l = {pk2(x[0] - __uint_as_float(h[0] << 16), x[1] - __uint_as_float(h[0] & 0xffff0000u)),
+                      pk2(x[2] - __uint_as_float(h[1] << 16), x[3] - __uint_as_float(h[1] & 0xffff0000u))};
+    *reinterpret_cast<u32x2v*>(hi + i * ld + j) = h;
+    *reinterpret_cast<u32x2v*>(lo + i * ld + j) = l;
   }
   // The same at (i, j) and (i, j + 1), j even.
   __device__ void put(int i, int j, float a, float b) const {
@@ -487,6 +472,12 @@ __global__ __launch_bounds__(256, 2) void dn_chunk_prep(DnArgs p) {
 // the products on the matrix cores (split bf16).  While a chunk's products run,
 // the next chunk's W, U~ columns, K and ca are loaded into registers.
 
+// The two sweeps (this and the state gradient's) are serial chains bound by the
+// instructions of a chunk, so each operand is split to bf16 once, as it goes to
+// LDS, the state stays in registers (LDS holds its halves for the products, and
+// an fp32 copy for 16-byte stores), and a sequence's place is found once, not
+// by divisions a chunk: B4 H16 T8192, 128 chunks a sweep, 515 -> 468 us and,
+// backward, 810 -> 679 against fp32 operands split at each wave's read.
 // Eight waves, two on each SIMD: one workgroup per CU (its LDS), and a
 // chunk's serial chain (stage, product, product, update) split eight ways.
 constexpr int kScanThreads = 512;
@@ -520,12 +511,13 @@ __device__ __forceinline__ void scan_load(ScanInputs& in, const DnArgs& p, const
 }
 
 // The inputs to LDS; K as Kd = diag(e^(ca_63 - ca)) K (ca of the same chunk, already in LDS).
-__device__ __forceinline__ void scan_store(const ScanInputs& in, float* W, float* Ut, float* Kd, const float* ca) {
+__device__ __forceinline__ void scan_store(const ScanInputs& in, const Planes& W, float* Ut, const Planes& Kd,
+                                           const float* ca) {
   const int t = threadIdx.x;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int x = t + kScanThreads * e, r = x / 32, c = 4 * (x % 32);
-    *reinterpret_cast<f32x4v*>(W + r * kLd + c) = in.w[e];
+    W.put(r, c, in.w[e]);
   }
   *reinterpret_cast<f32x4v*>(Ut + (t / 8) * kLdS + 4 * (t % 8)) = in.u;
   const float last = ca[kC - 1];
@@ -536,9 +528,8 @@ __device__ __forceinline__ void scan_store(const ScanInputs& in, float* W, float
     const u32x4v uk = in.k[e];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-      *reinterpret_cast<f32x4v*>(Kd + r * kLd + c + 4 * h) =
-          f32x4v{ed * bf((uint16_t)uk[2 * h]), ed * bf((uint16_t)(uk[2 * h] >> 16)), ed * bf((uint16_t)uk[2 * h + 1]),
-                 ed * bf((uint16_t)(uk[2 * h + 1] >> 16))};
+      Kd.put(r, c + 4 * h, f32x4v{ed * bf((uint16_t)uk[2 * h]), ed * bf((uint16_t)(uk[2 * h] >> 16)), ed * bf((uint16_t)uk[2 * h + 1]),
+                 ed * bf((uint16_t)(uk[2 * h + 1] >> 16))});
   }
 }
 
@@ -563,31 +554,43 @@ __device__ __forceinline__ ScanSlot scan_slot() {
   return ScanSlot{(int64_t)whole + x / kSlices, (x % kSlices) * kCols};
 }
 
-constexpr size_t kScanLds = (2 * kC * kLd + kC * kLdS + kD * kLdS + kC * kLdS + kC) * sizeof(float);
+constexpr size_t kScanLds = (2 * kC * kLdH + kC * kLdS + kD * kLdS + kD * kLdT + kC * kLdS + kC * kLdT + kC) * sizeof(float);
 
 __global__ __launch_bounds__(kScanThreads, 1) void dn_state_scan(DnArgs p) {
   extern __shared__ float lds[];
-  float* W = lds;                 // [64][kLd]
-  float* Kd = W + kC * kLd;       // [64][kLd]: diag(e^(ca_63 - ca)) K
-  float* Ut = Kd + kC * kLd;      // [64][kLdS]: U~ columns col0 .. col0 + 31
-  float* S = Ut + kC * kLdS;      // [128][kLdS]: the state's 32 columns
+  uint16_t* at = reinterpret_cast<uint16_t*>(lds);
+  auto planes = [&](int rows, int ld) {
+    const Planes x{at, at + rows * ld, ld};
+    at += 2 * rows * ld;
+    return x;
+  };
+  const Planes W = planes(kC, kLdH);   // [64][kLdH]
+  const Planes Kd = planes(kC, kLdH);  // [64][kLdH]: diag(e^(ca_63 - ca)) K
+  const Planes Sp = planes(kD, kLdT);  // [128][kLdT]: the state's 32 columns
+  const Planes Up = planes(kC, kLdT);  // [64][kLdT]: U
+  float* Ut = reinterpret_cast<float*>(at);  // [64][kLdS]: U~ columns col0 .. col0 + 31
+  float* S = Ut + kC * kLdS;      // [128][kLdS]: the state, as memory takes it
   float* U = S + kD * kLdS;       // [64][kLdS]
   float* ca = U + kC * kLdS;      // [64]
   const int t = threadIdx.x, w = t / 64;
-  const int r = t % 16, g = (t % 64) / 16;
+  const int r = plain(t % 16), g4 = plain((t % 64) / 16 * 4);
   const ScanSlot slot = scan_slot();
   const int64_t seq = slot.seq;
   const int col0 = slot.col0;
   for (int e = t; e < kD * kLdS; e += kScanThreads) S[e] = 0.0f;
+  for (int e = t; e < kD * kLdT; e += kScanThreads) Sp.hi[e] = 0, Sp.lo[e] = 0;
+  f32x4v st[1][2];  // the state: rows 16 w + 4 g + v, columns 16 bj + r
+  clear(st);
+  const Chunk first = chunk_of(p, seq * p.chunks);
   ScanInputs in;
-  scan_load(in, p, chunk_of(p, seq * p.chunks), col0);
+  scan_load(in, p, first, col0);
   if (t < kC) ca[t] = in.ca;
   __syncthreads();
   scan_store(in, W, Ut, Kd, ca);
   for (int n = 0; n < p.chunks; ++n) {
-    const Chunk ck = chunk_of(p, seq * p.chunks + n);
+    const Chunk ck = chunk_at(p, first, n);
     __syncthreads();
-    if (n + 1 < p.chunks) scan_load(in, p, chunk_of(p, seq * p.chunks + n + 1), col0);
+    if (n + 1 < p.chunks) scan_load(in, p, chunk_at(p, first, n + 1), col0);
     const float gl = expf(ca[kC - 1]);
     // The chunk's starting state, stored for the output and the backward: read
     // now, written to memory at the chunk's end (and U with it), after the
@@ -606,12 +609,14 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_state_scan(DnArgs p) {
       f32x4v ws[1][1];
       clear(ws);
       const int i0 = 16 * (w % 4), j0 = 16 * (w / 4);
-      mm_gen<false, true>(ws, W, kLd, i0, S, kLdS, j0, kD);
+      mm_by(ws, RowPlanes{W}, i0, ColPlanes{Sp}, j0, kD);
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int i = i0 + 4 * g + v, j = j0 + r;
-        U[i * kLdS + j] = Ut[i * kLdS + j] - ws[0][0][v];
+        const int i = i0 + g4 + v, j = j0 + r;
+        ws[0][0][v] = Ut[i * kLdS + j] - ws[0][0][v];
+        U[i * kLdS + j] = ws[0][0][v];
       }
+      store_planes(Up, ws, i0, j0, 1.0f);
     }
     __syncthreads();
     // U for memory, 16 bytes a thread.
@@ -620,20 +625,14 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_state_scan(DnArgs p) {
     {
       f32x4v ku[1][2];
       clear(ku);
-      mm_gen<true, true>(ku, Kd, kLd, 16 * w, U, kLdS, 0, kC);
-      float nw[2][4];
+      mm_by(ku, ColPlanes{Kd}, 16 * w, ColPlanes{Up}, 0, kC);
 #pragma unroll
       for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = 16 * w + 4 * g + v, j = 16 * bj + r;
-          nw[bj][v] = gl * S[i * kLdS + j] + ku[0][bj][v];
-        }
+        for (int v = 0; v < 4; ++v) st[0][bj][v] = gl * st[0][bj][v] + ku[0][bj][v];
       __syncthreads();  // every wave has read S, U and this chunk's inputs
-#pragma unroll
-      for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) S[(16 * w + 4 * g + v) * kLdS + 16 * bj + r] = nw[bj][v];
+      store_blocks(S, kLdS, st, 16 * w, 0, 1.0f);
+      store_planes(Sp, st, 16 * w, 0, 1.0f);
     }
     if (n + 1 < p.chunks) {
       if (t < kC) ca[t] = in.ca;
@@ -716,8 +715,8 @@ __global__ __launch_bounds__(256, 2) void dn_output(DnArgs p) {
 // the previous chunk's inputs (P, the dO columns, Q, K, W, ca) are loaded
 // into registers; they go to LDS once the chunk is done with its own.
 
-constexpr size_t kSgLds =
-    (kC * kLdC + kC * kLdS + 3 * kC * kLd + kD * kLdS + kC * kLdS + kC) * sizeof(float);
+constexpr int kLdP = 72;   // LDS row of 64 bf16
+constexpr size_t kSgLds = (kC * kLdP + kC * kLdT / 2 + 2 * kC * kLdH + kC * kLdH / 2 + kD * kLdS + kD * kLdT + kC * kLdT + kC) * sizeof(float);
 
 // One chunk's inputs as this thread loads them (plain vector types, so the
 // whole set stays in registers).
@@ -748,64 +747,70 @@ __device__ __forceinline__ void sg_load(SgInputs& in, const DnArgs& p, const Chu
 }
 
 // The inputs to LDS; Q as Qg = diag(e^ca) Q (ca of the same chunk, already in LDS).
-__device__ __forceinline__ void sg_store(const SgInputs& in, float* P, float* dO, float* Qg, float* K, float* W,
-                                         const float* ca) {
+__device__ __forceinline__ void sg_store(const SgInputs& in, const Planes& P, uint16_t* dO, const Planes& Qg, uint16_t* K,
+                                         const Planes& W, const float* ca) {
   const int t = threadIdx.x;
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
-    const int x = t + kScanThreads * e, r = x / 16, c = 4 * (x % 16);
-    *reinterpret_cast<f32x4v*>(P + r * kLdC + c) = in.p[e];
+    const int x = t + kScanThreads * e;
+    P.put(x / 16, 4 * (x % 16), in.p[e]);
   }
-  *reinterpret_cast<f32x4v*>(dO + (t / 8) * kLdS + 4 * (t % 8)) =
-      f32x4v{bf((uint16_t)in.d[0]), bf((uint16_t)(in.d[0] >> 16)), bf((uint16_t)in.d[1]), bf((uint16_t)(in.d[1] >> 16))};
+  *reinterpret_cast<u32x2v*>(dO + (t / 8) * kLdT + 4 * (t % 8)) = in.d;
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int x = t + kScanThreads * e, r = x / 16, c = 8 * (x % 16);
     const float eq = expf(ca[r]);
-    const u32x4v uq = in.q[e], uk = in.k[e];
+    const u32x4v uq = in.q[e];
+    *reinterpret_cast<u32x4v*>(K + r * kLdH + c) = in.k[e];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      *reinterpret_cast<f32x4v*>(Qg + r * kLd + c + 4 * h) =
-          f32x4v{eq * bf((uint16_t)uq[2 * h]), eq * bf((uint16_t)(uq[2 * h] >> 16)), eq * bf((uint16_t)uq[2 * h + 1]),
-                 eq * bf((uint16_t)(uq[2 * h + 1] >> 16))};
-      *reinterpret_cast<f32x4v*>(K + r * kLd + c + 4 * h) =
-          f32x4v{bf((uint16_t)uk[2 * h]), bf((uint16_t)(uk[2 * h] >> 16)), bf((uint16_t)uk[2 * h + 1]),
-                 bf((uint16_t)(uk[2 * h + 1] >> 16))};
-    }
+    for (int h = 0; h < 2; ++h)
+      Qg.put(r, c + 4 * h, f32x4v{eq * bf((uint16_t)uq[2 * h]), eq * bf((uint16_t)(uq[2 * h] >> 16)),
+                                  eq * bf((uint16_t)uq[2 * h + 1]), eq * bf((uint16_t)(uq[2 * h + 1] >> 16))});
   }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int x = t + kScanThreads * e, r = x / 32, c = 4 * (x % 32);
-    *reinterpret_cast<f32x4v*>(W + r * kLd + c) = in.w[e];
+    const int x = t + kScanThreads * e;
+    W.put(x / 32, 4 * (x % 32), in.w[e]);
   }
 }
 
 __global__ __launch_bounds__(kScanThreads, 1) void dn_state_grad(DnArgs p) {
   extern __shared__ float lds[];
-  float* P = lds;                  // [64][kLdC]
-  float* dO = P + kC * kLdC;       // [64][kLdS]: columns col0 .. col0 + 31 of dO
-  float* Qg = dO + kC * kLdS;      // [64][kLd]: diag(e^ca) Q
-  float* K = Qg + kC * kLd;        // [64][kLd]
-  float* W = K + kC * kLd;         // [64][kLd]
-  float* dS = W + kC * kLd;        // [128][kLdS]: the state gradient's 32 columns
-  float* dU = dS + kD * kLdS;      // [64][kLdS]
-  float* ca = dU + kC * kLdS;      // [64]
+  uint16_t* at = reinterpret_cast<uint16_t*>(lds);
+  auto planes = [&](int rows, int ld) {
+    const Planes x{at, at + rows * ld, ld};
+    at += 2 * rows * ld;
+    return x;
+  };
+  const Planes P = planes(kC, kLdP);    // [64][kLdP]
+  const Planes Qg = planes(kC, kLdH);   // [64][kLdH]: diag(e^ca) Q
+  const Planes W = planes(kC, kLdH);    // [64][kLdH]
+  const Planes dSp = planes(kD, kLdT);  // [128][kLdT]: the state gradient's 32 columns
+  const Planes dUp = planes(kC, kLdT);  // [64][kLdT]: dU
+  uint16_t* dO = at;                    // [64][kLdT]: columns col0 .. col0 + 31 of dO
+  uint16_t* K = dO + kC * kLdT;         // [64][kLdH]
+  float* dS = reinterpret_cast<float*>(K + kC * kLdH);  // [128][kLdS]: the state gradient, as memory takes it
+  float* ca = dS + kD * kLdS;           // [64]
   const int t = threadIdx.x, w = t / 64;
-  const int r = t % 16, g = (t % 64) / 16;
+  const int g4 = plain((t % 64) / 16 * 4);
   const ScanSlot slot = scan_slot();
   const int64_t seq = slot.seq;
   const int col0 = slot.col0;
   for (int e = t; e < kD * kLdS; e += kScanThreads) dS[e] = 0.0f;
+  for (int e = t; e < kD * kLdT; e += kScanThreads) dSp.hi[e] = 0, dSp.lo[e] = 0;
+  f32x4v st[1][2];  // the state gradient: rows 16 w + 4 g + v, columns 16 bj + r
+  clear(st);
+  const Chunk first = chunk_of(p, seq * p.chunks);
   SgInputs in;
   {
-    const Chunk ck = chunk_of(p, seq * p.chunks + p.chunks - 1);
+    const Chunk ck = chunk_at(p, first, p.chunks - 1);
     sg_load(in, p, ck, col0);
     if (t < kC) ca[t] = in.ca;
     __syncthreads();
     sg_store(in, P, dO, Qg, K, W, ca);
   }
   for (int n = p.chunks - 1; n >= 0; --n) {
-    const Chunk ck = chunk_of(p, seq * p.chunks + n);
+    const Chunk ck = chunk_at(p, first, n);
     __syncthreads();
     // This chunk's starting state, where this thread's dS values below sit:
     // dg's partial sums take it at the chunk's end.
@@ -815,7 +820,7 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_state_grad(DnArgs p) {
       const int e = t + kScanThreads * u, row = e / 8, c = 4 * (e % 8);
       s_in[u] = *reinterpret_cast<const f32x4v*>(p.S + ck.c * kD * kD + row * kD + col0 + c);
     }
-    if (n > 0) sg_load(in, p, chunk_of(p, seq * p.chunks + n - 1), col0);
+    if (n > 0) sg_load(in, p, chunk_at(p, first, n - 1), col0);
     const float last = ca[kC - 1];
     // The gradient at the chunk's end state: read now, written to memory at
     // the chunk's end (and dU with it), after the previous chunk's inputs are
@@ -830,43 +835,34 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_state_grad(DnArgs p) {
     }
     // dU (64 x 32): wave w takes the 16 x 16 block at rows 16 (w mod 4),
     // columns 16 (w / 4).
+    const int i0 = 16 * (w % 4), j0 = 16 * (w / 4);
+    f32x4v du[1][1];
     {
-      f32x4v pd[1][1], kd[1][1];
-      clear(pd);
+      f32x4v kd[1][1];
+      clear(du);
       clear(kd);
-      const int i0 = 16 * (w % 4), j0 = 16 * (w / 4);
-      mm_by(pd, ColF32{P, kLdC}, i0, ColF32Bf{dO, kLdS}, j0, kC);  // dO: bf16 values
-      mm_by(kd, RowF32Bf{K, kLd}, i0, ColF32{dS, kLdS}, j0, kD);  // K: bf16 values
+      mm_by(du, ColPlanes{P}, i0, ColBf16{dO, kLdT}, j0, kC);
+      mm_by(kd, RowBf16{K, kLdH}, i0, ColPlanes{dSp}, j0, kD);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = i0 + 4 * g + v;
-        dU[i * kLdS + j0 + r] = pd[0][0][v] + expf(last - ca[i]) * kd[0][0][v];
-      }
+      for (int v = 0; v < 4; ++v) du[0][0][v] += expf(last - ca[i0 + g4 + v]) * kd[0][0][v];
+      store_planes(dUp, du, i0, j0, 1.0f);
     }
     __syncthreads();
-    // dU for memory, 16 bytes a thread.
-    const f32x4v du_out = *reinterpret_cast<const f32x4v*>(dU + (t / 8) * kLdS + 4 * (t % 8));
     // dS <- Qg' dO + g dS - W' dU (128 x 32): wave w takes rows 16 w .. 16 w + 15.
     {
       f32x4v qd[1][2], wu[1][2];
       clear(qd);
       clear(wu);
-      mm_by(qd, ColF32{Qg, kLd}, 16 * w, ColF32Bf{dO, kLdS}, 0, kC);
-      mm_gen<true, true>(wu, W, kLd, 16 * w, dU, kLdS, 0, kC);
+      mm_by(qd, ColPlanes{Qg}, 16 * w, ColBf16{dO, kLdT}, 0, kC);
+      mm_by(wu, ColPlanes{W}, 16 * w, ColPlanes{dUp}, 0, kC);
       const float gl = expf(last);
-      float nw[2][4];
 #pragma unroll
       for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = 16 * w + 4 * g + v, j = 16 * bj + r;
-          nw[bj][v] = qd[0][bj][v] + gl * dS[i * kLdS + j] - wu[0][bj][v];
-        }
+        for (int v = 0; v < 4; ++v) st[0][bj][v] = qd[0][bj][v] + gl * st[0][bj][v] - wu[0][bj][v];
       __syncthreads();  // every wave has read dS, dU and this chunk's inputs
-#pragma unroll
-      for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) dS[(16 * w + 4 * g + v) * kLdS + 16 * bj + r] = nw[bj][v];
+      store_blocks(dS, kLdS, st, 16 * w, 0, 1.0f);
+      store_planes(dSp, st, 16 * w, 0, 1.0f);
     }
     if (n > 0) {
       if (t < kC) ca[t] = in.ca;
@@ -879,7 +875,7 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_state_grad(DnArgs p) {
       const int e = t + kScanThreads * u, row = e / 8, c = 4 * (e % 8);
       *reinterpret_cast<f32x4v*>(dSc + row * kD + col0 + c) = ds_out[u];
     }
-    *reinterpret_cast<f32x4v*>(p.dU + ck.c * kC * kD + (t / 8) * kD + col0 + 4 * (t % 8)) = du_out;
+    store_blocks(p.dU + ck.c * kC * kD + col0, kD, du, i0, j0, 1.0f);
     // This wave's part of dg = <S, dSn>.
     float dot = 0.0f;
 #pragma unroll
@@ -947,12 +943,8 @@ struct HeldF32 {
   __device__ void store(const Planes& to) const {
 #pragma unroll
     for (int u = 0; u < n; ++u) {
-      const int e = threadIdx.x + 256 * u, at = (e / 32) * to.ld + 4 * (e % 32);
-      const u32x2v h = {pk2(x[u][0], x[u][1]), pk2(x[u][2], x[u][3])};
-      const u32x2v l = {pk2(x[u][0] - __uint_as_float(h[0] << 16), x[u][1] - __uint_as_float(h[0] & 0xffff0000u)),
-                        pk2(x[u][2] - __uint_as_float(h[1] << 16), x[u][3] - __uint_as_float(h[1] & 0xffff0000u))};
-      *reinterpret_cast<u32x2v*>(to.hi + at) = h;
-      *reinterpret_cast<u32x2v*>(to.lo + at) = l;
+      const int e = threadIdx.x + 256 * u;
+      to.put(e / 32, 4 * (e % 32), x[u]);
     }
   }
 };
@@ -975,7 +967,6 @@ struct HeldBf16 {
   }
 };
 
-constexpr int kLdP = 72;                // LDS row of 64 bf16
 constexpr int kGradX = 2 * kC * kLdP;   // floats: M and N as planes; U, dU and dW take 2 kC kLdH / 2
 static_assert(kGradX >= kC * kLdH && kC * kLdP >= kC * kLdC, "");
 constexpr size_t kGradLds = 2 * kC * kLdH * sizeof(uint16_t) + kGradX * sizeof(float) +
