@@ -1201,7 +1201,7 @@ extern "C" int th_build_attention_fwd(const th_attention_desc* d, th_launch** ou
              "attention: a sequence of K or V must span under 2 GiB (seq x position stride x 2 bytes)");
   TH_HIP(hipFuncSetAttribute((const void*)attn_fwd, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFwdLds));
   AttnArgs a = args_of(d);
-  th::Builder b("attention_fwd", 7);  // values 5, 6 (the masks) are read only by the general kernels
+  th::Builder b("attention_fwd", 7);  // values 5, 6 (the masks): no mask reaches these kernels
   int k = b.kernel((const void*)attn_fwd, "attn_fwd", dim3(blocks_x(d->seq / kFwdQ, d->causal), d->heads, d->batch),
                    dim3(256), (uint32_t)kFwdLds, a);
   b.ref(0, k, TH_OFFSET(AttnArgs, q));
@@ -1227,7 +1227,7 @@ extern "C" int th_build_attention_bwd(const th_attention_desc* d, th_launch** ou
                                         : th::build_attention_general_bwd(d, out);
   if (int r = check_desc(d, true)) return r;
   AttnArgs a = args_of(d);
-  th::Builder b("attention_bwd", 11);  // values 9, 10 (the masks) are read only by the general kernels
+  th::Builder b("attention_bwd", 11);  // values 9, 10 (the masks): no mask reaches these kernels
   // The dK/dV sweep loads Q and dO tiles directly into LDS with 32-bit byte
   // offsets from a (batch, head) base.
   TH_REQUIRE((double)d->seq * d->q_strides[1] * 2 < 2147483648.0,

@@ -1,8 +1,10 @@
 // Op class (c), general shapes: attention forward and backward for any head
 // dimension up to 256, any sequence lengths (keys may be fewer or more than
 // queries), fp32 or bf16 arrays, grouped heads, and the masks the device
-// holds (a first key per query, a key count per sequence).  What the
-// matrix-core kernels of attention.hip do not take runs here: the reference's
+// holds (a first key per query, a key count per sequence).  What none of the
+// matrix-core kernels takes runs here (attention.hip, attention_mfma.hip with
+// and without masks, attention_decode.hip, attention_f32.hip: the builders here ask the masked
+// and decode ones first): the reference's
 // cuDNN claim covers d <= 256 (ext/cuDNNExt.jl:95-100) and its tests use
 // D = 4, 8, 16, 32 at odd lengths, packed documents and decode over a cache
 // (test/fixtures/programs.jl:110-113, test/cuda/attention.jl:10-16,218-271).

@@ -1,7 +1,6 @@
 // Op class (c) on the matrix cores at head dims 64, 128 and 256 and any
 // lengths: what the tuned kernels of attention.hip (head dim 128, lengths in
-// 128s) do not take, short of fp32 arrays and device-held masks, which stay
-// on attention_generic.hip.  The reference's cuDNN claim takes half
+// 128s) do not take, short of fp32 arrays (attention_f32.hip).  The reference's cuDNN claim takes half
 // precision d <= 256 on tensor cores (ext/cuDNNExt.jl:90-100) and its cuTile
 // sweep any tile (ext/cuTileExt/build.jl:326-493); d = 64 and d = 256 are
 // the head dims models use beside 128.
@@ -34,7 +33,7 @@
 // in fp32, so here each is hi + lo in bf16 (2^-17 relative) and takes two
 // products, on operands that are bf16 already.  Rows may start at any element.
 // B2 H12 S2048 d64 in documents of about 256, forward + backward: 5981 us on
-// the general kernels, 190 here.
+// the general kernels, 96 here.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -123,7 +122,8 @@ __device__ __forceinline__ int least(int x, int* at) {
 //   causal forward whose keys are not split over workgroups, <= 512 (two a CU):
 //     B2 H16 S1853 d64 (480) 40.5 -> 35.0, B1 H16 S4000 d128 (512) 118 -> 103;
 //     1024: 54.6 -> 74.3, and sweeps of one length (not causal, 480) 45 -> 55.6,
-//     already split ones 53.5 -> 58 (with the backward);
+//     already split ones 53.5 -> 58 (with the backward); short
+//     sweeps in place of a split: beside the rule;
 //   masked forward, <= 512: packed documents B2 H12 S2048 d64 (384), with the
 //     backward 114 -> 106; 768 workgroups 110 -> 118;
 //   masked backward at d64, <= 1024: the same documents (768) 106 -> 96,
@@ -887,11 +887,25 @@ template <int D>
 int fwd_launch(const th_attention_desc* d, th_launch** out) {
   MArgs a = margs_of(d);
   const int nqb = (d->seq + 127) / 128;
-  const th::Split sp = th::split_of((int64_t)nqb * d->heads * d->batch, a.kv_seq);
+  const int64_t groups = (int64_t)nqb * d->heads * d->batch;
+  th::Split sp = th::split_of(groups, a.kv_seq);
+  bool halves = sp.n == 1 && d->causal && groups <= kFwdHalves;
+  // Short sweeps that would be split: halves in place of a twofold split, without its
+  // partial results and (whole) its second launch.  us, split alone and so, forward:
+  // whole, B2 H8 S512 d64 causal (64 workgroups) 14.4, 11.3; B1 H16 S700 d128 (96)
+  // 26.3, 19.7 and not causal 28.8, 21.3; half the parts, B1 H4 S1000 d64 (32) 16.0,
+  // 14.5, S2000 19.4, 18.4, B2 H8 S1024 18.4, 18.1.  Longer ones fill the device
+  // better split: B1 H2 S8000 d64 46.5, halved 63.7; whole S1024 d128 (24) 18.0, 27.4.
+  if (D <= 128 && sp.n > 1 && a.kv_seq <= 768 && groups >= 64) {
+    sp = {1, 0}, halves = true;
+  } else if (D == 64 && sp.n >= 4 && a.kv_seq <= 2048) {
+    const int n = sp.n / 2, span = ((a.kv_seq + n - 1) / n + 63) / 64 * 64;
+    sp = {(a.kv_seq + span - 1) / span, span}, halves = true;
+  }
   a.nsplit = sp.n, a.span = sp.span;
   th::Builder b("attention_fwd_mfma", 7);
   const dim3 grid(d->heads, d->batch, nqb * sp.n);
-  const int P = D <= 128 && d->causal && sp.n == 1 && (int64_t)grid.x * grid.y * grid.z <= kFwdHalves ? 2 : 1;
+  const int P = D <= 128 && halves ? 2 : 1;
   const size_t lds = 4 * P * (size_t)kTile<D> * sizeof(uint16_t);
   const void* fn = P == 2 ? (const void*)mfma_attn_fwd<D, false, D <= 128 ? 2 : 1> : (const void*)mfma_attn_fwd<D, false, 1>;
   TH_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));

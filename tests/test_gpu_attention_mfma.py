@@ -109,13 +109,16 @@ def test_split_and_whole_sweeps(target, D, B, H, KV, S, causal, split):
 
 
 @pytest.mark.parametrize("D,B,H,KV,S,Sk", [
+    (64, 1, 32, 8, 129, 768), (128, 1, 32, 8, 140, 700),  # 64 workgroups, whole sweeps in halves
+    (64, 1, 4, 2, 1000, 1000), (64, 1, 4, 4, 1025, 2048),  # parts in halves, a last part that is short
     (64, 4, 32, 8, 129, 129),   # 256 workgroups: three tiles, then one, to the halves of a sweep
     (64, 4, 32, 32, 255, 64),   # one tile: the second half has none
     (64, 8, 32, 8, 200, 330),   # 512 workgroups, the last that are halved
     (64, 9, 32, 8, 130, 130),   # 576: not halved
     (128, 4, 32, 8, 129, 193), (128, 2, 2, 1, 5, 5), (128, 4, 33, 33, 260, 260)])
-def test_forward_sweeps_in_halves(target, D, B, H, KV, S, Sk):
-    """Causal forwards whose sweeps two halves of a workgroup share, at the
+@pytest.mark.parametrize("causal", [True, False])
+def test_forward_sweeps_in_halves(target, D, B, H, KV, S, Sk, causal):
+    """Forwards whose sweeps two halves of a workgroup share, at the
     edges of tiles and on both sides of the workgroups up to which they do:
     o and lse against the float64 oracle."""
     announce("attn mfma halves", D, B, H, KV, S, Sk)
@@ -123,9 +126,9 @@ def test_forward_sweeps_in_halves(target, D, B, H, KV, S, Sk):
     q, k, v, _ = _inputs(B, S, Sk, H, KV, D, D + 5 * S + Sk)
     o = torch.empty_like(q)
     lse = torch.empty(B, S, H, device="cuda")
-    L.attention_fwd(B, H, KV, S, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), causal=True,
+    L.attention_fwd(B, H, KV, S, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), causal=causal,
                     head_dim=D, kv_seq=Sk)()
     torch.cuda.synchronize()
-    ro, rl = interpret.attention_fwd(_np(q), _np(k), _np(v), True)
+    ro, rl = interpret.attention_fwd(_np(q), _np(k), _np(v), causal)
     assert relative(_np(o), ro) < TOL_BF16, relative(_np(o), ro)
     assert np.max(np.abs(_np(lse) - rl)) < 1e-3 * max(1.0, np.abs(rl).max())
