@@ -573,10 +573,12 @@ enum { TH_EPI_STORE = 0, TH_EPI_GELU = 1, TH_EPI_SQUARE_LOSS = 2, TH_EPI_GELU_BA
  *     (bias allowed), a result of the factors' type or fp32: the output tiles
  *     the reference's product sketch searches for half factors
  *     (ext/cuTileExt/contract.jl:36-39);
- *   TH_TILE_GENERAL: anything with TH_EPI_STORE and no bias, on the fp32
- *     matrix cores, any shape and strides: fp32 factors with an fp32 result on
- *     128 x 128 tiles (16-byte loads along a unit stride, K split like the
- *     others), half factors or a half result on 64 x 64 tiles (unsplit).
+ *   TH_TILE_GENERAL: anything with TH_EPI_STORE and no bias, any shape and
+ *     strides: fp32 factors with an fp32 result on 128 x 128 tiles (each factor
+ *     as three bf16 parts on the bf16 matrix cores, in fp32's precision; the fp32
+ *     matrix cores where a part would leave bf16's range; K split like the
+ *     others) or, few and short, 32 x 32 ones, half factors or a half
+ *     result on 64 x 64 tiles of the fp32 matrix cores (unsplit).
  *     fp32 factors run only here unless TH_GEMM_BF16X3.
  * TH_TILE_AUTO chooses the least estimated time among the 256 x 256 kernel
  * and the middle tiles (which it also gives fused epilogues, where the 256 x
@@ -666,10 +668,13 @@ int th_build_gemm_grouped(const th_gemm_desc* descs, int count, th_launch** host
  * key/value head h / (heads / kv_heads).  lse is fp32, (1, heads, positions,
  * batch): element (h, s, b) at h + heads*(s + seq*b), the natural log-sum-exp
  * of each query's scaled scores.  scale <= 0 means 1/sqrt(head_dim).
- * Two implementations: bf16 with head_dim 128, seq a multiple of 128, keys
- * as many as queries and no device-held masks runs the matrix-core kernels;
- * anything else with head_dim 1..256 (fp32 or bf16 arrays, any lengths,
- * starts and lengths masks) runs the general kernels, which compute in fp32
+ * On the matrix cores: bf16 with head_dim 128, seq a multiple of 128, keys
+ * as many as queries and no device-held masks (the tuned kernels); bf16 with
+ * head_dim 64, 128 or 256 at any lengths; bf16 with head_dim 64 or 128 under
+ * starts and lengths masks; a few bf16 queries over a long cache (head_dim 64 or 128,
+ * seq times heads / kv_heads at most 16, the forward); fp32 with head_dim
+ * 64 or 128 and no masks (three bf16 parts a factor, fp32's precision).
+ * Anything else with head_dim 1..256 runs the general kernels, in fp32
  * on the vector ALUs (the cuDNN claim's d <= 256, ext/cuDNNExt.jl:95-100, and
  * the reference's attention tests, test/cuda/attention.jl:10-16,218-271). */
 typedef struct th_attention_desc {
