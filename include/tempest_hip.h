@@ -159,11 +159,12 @@ int th_launch_repoint(th_launch* launch, int value, void* ptr);
 /* th_launch_run for each of `n` launches, in order. */
 int th_launches_run(th_launch* const* host_launches, int n);
 
-/* th_launch_repoint for `n` values at once: value values[i] of launches[i] at
- * base + offsets[i] (the places of one allocation that holds several values,
- * as a compiled program's results). */
-int th_launches_place(th_launch* const* host_launches, const int32_t* host_values, const uint64_t* host_offsets,
-                      int n, void* base);
+/* th_launches_run with value values[i] of holders[i] at lent + offsets[i] (i <
+ * refs: the places of one allocation that holds several values, as a compiled
+ * program's results), for these launches only: on return, also with an error,
+ * every one of them is at home + offsets[i]. */
+int th_launches_lend(th_launch* const* host_launches, int n, th_launch* const* host_holders,
+                     const int32_t* host_values, const uint64_t* host_offsets, int refs, void* lent, void* home);
 
 /* The launch's algorithmic work.  Feeds Implement.estimate,
  * src/Compiler/Implement/Implement.jl:61-82. */

@@ -731,10 +731,19 @@ int th_launches_run(th_launch* const* launches, int n) {
   return TH_OK;
 }
 
-int th_launches_place(th_launch* const* launches, const int32_t* values, const uint64_t* offsets, int n, void* base) {
-  for (int i = 0; i < n; ++i)
-    if (int r = th_launch_repoint(launches[i], values[i], static_cast<char*>(base) + offsets[i])) return r;
-  return TH_OK;
+int th_launches_lend(th_launch* const* launches, int n, th_launch* const* holders, const int32_t* values,
+                     const uint64_t* offsets, int refs, void* lent, void* home) {
+  auto place = [&](void* base) {
+    for (int i = 0; i < refs; ++i)
+      if (int r = th_launch_repoint(holders[i], values[i], static_cast<char*>(base) + offsets[i])) return r;
+    return (int)TH_OK;
+  };
+  int r = place(lent);
+  if (r == TH_OK) r = th_launches_run(launches, n);
+  // A launch's arguments are copied as it is issued: the launches are back at
+  // `home` whatever became of the run.
+  const int back = place(home);
+  return r != TH_OK ? r : back;
 }
 
 int th_launch_work(th_launch* l, th_work* out) {

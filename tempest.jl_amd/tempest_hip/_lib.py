@@ -147,7 +147,7 @@ SIGNATURES: dict[str, list] = {
     "th_launch_run": [c_void_p],
     "th_launch_repoint": [c_void_p, c_int, c_void_p],
     "th_launches_run": [P(c_void_p), c_int],
-    "th_launches_place": [P(c_void_p), P(c_i32), P(c_u64), c_int, c_void_p],
+    "th_launches_lend": [P(c_void_p), c_int, P(c_void_p), P(c_i32), P(c_u64), c_int, c_void_p, c_void_p],
     "th_launch_work": [c_void_p, P(Work)],
     "th_launch_describe": [c_void_p, c_char_p, c_size],
     "th_launch_destroy": [c_void_p],

@@ -211,10 +211,25 @@ class PoolSlots:
             pass
 
 
+def _shown(name: str, doc: str) -> property:
+    """An attribute that tells its reader where the executable's results lie, or
+    that runs into them: reading it ends what only a program that sees nothing
+    but its calls' results may have (Executable.lend)."""
+    def read(self):
+        self._settle()
+        return getattr(self, name)
+    return property(read, doc=doc)
+
+
 class Executable:
     """A prepared program: its storage, launches and (once captured) graph.
     Its slots lie in one arena slab, or, given a Pool, are taken from the
     pool's reserved range one by one."""
+
+    results = _shown("_results", "The results' one allocation, for as long as the executable.")
+    addresses = _shown("_addresses", "Where each value lies.")
+    launches = _shown("_launches", "A launch a group, in order.")
+    graph = _shown("_graph", "What capture recorded, or None.")
 
     def __init__(self, program: Program, target: HIPTarget, inputs: Sequence[torch.Tensor], point: bool = True,
                  pool: Pool | None = None):
@@ -224,7 +239,7 @@ class Executable:
         self.arena = Arena(self.storage.sizes) if pool is None else PoolSlots(pool, self.storage.sizes)
         self.own: dict[str, torch.Tensor] = {}
         self.bound: dict[str, torch.Tensor] = {}
-        self.addresses: dict[str, int] = {}
+        self._addresses: dict[str, int] = {}
         # The results share one allocation, each at a 256-byte boundary, so a
         # call returns them with one copy and reads its numbers at once.
         self.result_at: dict[str, tuple[int, int]] = {}
@@ -234,26 +249,28 @@ class Executable:
                 nbytes = max(1, v.count) * _ELEMENT[v.dtype]
                 self.result_at[name] = (at, nbytes)
                 at += (nbytes + 255) // 256 * 256
-        self.results = target.allocate(torch.uint8, max(at, 256))
-        self._lent = False  # whether `results` is a call's, its caller's to keep
+        self._results = target.allocate(torch.uint8, max(at, 256))
+        self._seen = False  # whether anyone has been told where the results lie
+        # What the last run wrote instead, the stream it ran on, the memory's version then.
+        self._last: tuple[torch.Tensor, torch.cuda.Stream, int] | None = None
         for name, v in program.values.items():
             if v.role == "stored":
-                self.addresses[name] = self.arena.addresses[self.storage.slots[name]]
+                self._addresses[name] = self.arena.addresses[self.storage.slots[name]]
             elif v.role == "result":
-                self.addresses[name] = self.results.data_ptr() + self.result_at[name][0]
+                self._addresses[name] = self._results.data_ptr() + self.result_at[name][0]
         self._check(inputs)
         for name, x in zip(program.inputs, inputs):
             self._take(name, x, point)
-        self.launches = [g.build(dict(self.addresses)) for g in program.groups]
+        self._launches = [g.build(dict(self._addresses)) for g in program.groups]
         self._place_workspaces(pool)
-        # Every place a launch holds a result's address, as th_launches_place takes them.
-        refs = [(l.handle.value, i, self.result_at[v][0]) for g, l in zip(program.groups, self.launches)
+        # Every place a launch holds a result's address, as th_launches_lend takes them.
+        refs = [(l.handle.value, i, self.result_at[v][0]) for g, l in zip(program.groups, self._launches)
                 for i, v in enumerate(g.values) if v in self.result_at]
         n = max(1, len(refs))
         self._result_refs = ((ctypes.c_void_p * n)(*(r[0] for r in refs)), (ctypes.c_int32 * n)(*(r[1] for r in refs)),
                              (ctypes.c_uint64 * n)(*(r[2] for r in refs)), len(refs))
-        self._handles = (ctypes.c_void_p * max(1, len(self.launches)))(*(l.handle.value for l in self.launches))
-        self.graph: Graph | Direct | None = None
+        self._handles = (ctypes.c_void_p * max(1, len(self._launches)))(*(l.handle.value for l in self._launches))
+        self._graph: Graph | Direct | None = None
         self._moved: set[int] = set()
 
     def _place_workspaces(self, pool: Pool | None) -> None:
@@ -262,20 +279,20 @@ class Executable:
         again in one arena (or taken from the pool), the launches repointed
         to it.  The first arena, built before the workspaces were known,
         goes."""
-        self.workspaces = [l.workspace() for l in self.launches]
+        self.workspaces = [l.workspace() for l in self._launches]
         if not any(self.workspaces):
             return
         sizes = list(self.storage.sizes) + [w for w in self.workspaces if w]
         arena = Arena(sizes) if pool is None else PoolSlots(pool, sizes)
         for name, v in self.program.values.items():
             if v.role == "stored":
-                self.addresses[name] = arena.addresses[self.storage.slots[name]]
-        for g, l in zip(self.program.groups, self.launches):
+                self._addresses[name] = arena.addresses[self.storage.slots[name]]
+        for g, l in zip(self.program.groups, self._launches):
             for i, v in enumerate(g.values):
                 if v in self.program.values and self.program.values[v].role == "stored":
-                    l.repoint(i, self.addresses[v])
+                    l.repoint(i, self._addresses[v])
         j = len(self.storage.sizes)
-        for l, w in zip(self.launches, self.workspaces):
+        for l, w in zip(self._launches, self.workspaces):
             if w:
                 l.set_workspace(arena.addresses[j])
                 j += 1
@@ -297,7 +314,7 @@ class Executable:
         v = self.program.values[name]
         if point and self.target.pointable(x, x.data_ptr()):
             self.bound[name] = x
-            self.addresses[name] = x.data_ptr()
+            self._addresses[name] = x.data_ptr()
             self.own.pop(name, None)
         else:
             buf = self.own.get(name)
@@ -306,7 +323,7 @@ class Executable:
                 self.own[name] = buf
             self.target.upload_into(buf, x.reshape(-1))
             self.bound.pop(name, None)
-            self.addresses[name] = buf.data_ptr()
+            self._addresses[name] = buf.data_ptr()
 
     def bind(self, *inputs: torch.Tensor) -> "Executable":
         """bind!(ex, inputs...) (runtime.jl:719): copy into own buffers."""
@@ -319,11 +336,11 @@ class Executable:
     def _rebind(self, inputs, point: bool) -> "Executable":
         self._check(inputs)
         for name, x in zip(self.program.inputs, inputs):
-            before = self.addresses[name]
+            before = self._addresses[name]
             self._take(name, x, point)
-            after = self.addresses[name]
+            after = self._addresses[name]
             if after != before:
-                for k, (g, l) in enumerate(zip(self.program.groups, self.launches)):
+                for k, (g, l) in enumerate(zip(self.program.groups, self._launches)):
                     for i, v in enumerate(g.values):
                         if v == name:
                             l.repoint(i, after)
@@ -332,48 +349,54 @@ class Executable:
 
     # -- running --------------------------------------------------------------
 
-    def _results_at(self, memory: torch.Tensor, lent: bool) -> None:
-        """Have the launches write their results to ``memory`` (laid out as ``result_at``)."""
-        base = memory.data_ptr()
-        self.results, self._lent = memory, lent
-        for name, (off, _) in self.result_at.items():
-            self.addresses[name] = base + off
-        self._alive()
-        call("th_launches_place", *self._result_refs, base)
-
     def _alive(self) -> None:
-        for l in self.launches:
+        for l in self._launches:
             l.handle  # raises for a destroyed launch
 
-    def lend(self) -> bool:
-        """Give the next run a result allocation of its own, which its caller
-        keeps: nothing that runs later writes there.  False, and nothing
-        changed, where torch would not order the allocation with the launches
-        (another current stream than the library's) or the recording is a
-        graph, whose every node with a result would be retargeted."""
-        if isinstance(self.graph, Graph):
-            return False
-        stream = ctypes.c_void_p()
-        call("th_get_stream", ctypes.byref(stream))
-        if (stream.value or 0) != torch.cuda.current_stream(self.target.device).cuda_stream:
-            return False
-        self._results_at(torch.empty_like(self.results), lent=True)
-        return True
+    def lend(self) -> torch.Tensor | None:
+        """One run whose results go to memory of its own, laid out as
+        ``result_at``, which its caller keeps; every launch, and so every
+        recording, timing or run of it, stays at the executable's results.
+        None, and nothing run, where those are what the caller has to have
+        (someone knows where they lie), where torch would not order the memory
+        with the launches (another current stream than the library's), or
+        where the recording is a graph, whose every node with a result would
+        be retargeted."""
+        if self._seen or isinstance(self._graph, Graph):
+            return None
+        handle = ctypes.c_void_p()
+        call("th_get_stream", ctypes.byref(handle))
+        stream = torch.cuda.current_stream(self.target.device)
+        if (handle.value or 0) != stream.cuda_stream:
+            return None
+        self._alive()
+        self._last = None
+        memory = torch.empty_like(self._results)
+        call("th_launches_lend", self._handles, len(self._launches), *self._result_refs, memory.data_ptr(),
+             self._results.data_ptr())
+        self._moved.clear()
+        self._last = memory, stream, 0 if memory.is_inference() else memory._version
+        return memory
 
-    def _home(self) -> None:
-        """Results lent to a caller stay as they are: a run of the executable's
-        own writes to memory of its own."""
-        if self._lent:
-            self._results_at(torch.empty_like(self.results), lent=False)
+    def _settle(self) -> None:
+        """From here on every run's results are where the executable says, the
+        last one's too: copied there on the stream that it ran on, or, where
+        their holder has written over them, computed again."""
+        self._seen = True
+        if self._last is None:
+            return
+        (memory, stream, version), self._last = self._last, None
+        with torch.cuda.stream(stream):
+            if memory.is_inference() or memory._version == version:
+                self._results.copy_(memory)
+            else:
+                self.execute()
 
     def execute(self) -> "Executable":
         """execute!(ex) (runtime.jl:1158): each launch in order."""
-        self._home()
-        return self._run()
-
-    def _run(self) -> "Executable":
+        self._last = None
         self._alive()
-        call("th_launches_run", self._handles, len(self.launches))
+        call("th_launches_run", self._handles, len(self._launches))
         self._moved.clear()  # the launches themselves carry the new addresses
         return self
 
@@ -381,48 +404,47 @@ class Executable:
         """capture!(ex) (runtime.jl:1185): one graph of every launch, or the
         launches themselves where the target measures direct launches faster
         for this many kernels (HIPTarget.graph_pays); ``graph`` forces it."""
-        self._home()
-        if self.graph is not None:
-            self.graph = self.target.recapture(self.graph, self.launches, as_graph=graph)
+        if self._graph is not None:
+            self._graph = self.target.recapture(self._graph, self._launches, as_graph=graph)
         else:
-            self.graph = self.target.capture(self.launches, graph=graph)
+            self._graph = self.target.capture(self._launches, graph=graph)
         self._moved.clear()
         return self
 
     @property
     def graphed(self) -> bool:
         """Whether what capture recorded replays as a graph."""
-        return isinstance(self.graph, Graph)
+        return isinstance(self._graph, Graph)
 
     def replay(self) -> "Executable":
         """replay!(ex) (runtime.jl:1208): retarget what moved, then one graph launch."""
-        if self.graph is None:
+        if self._graph is None:
             raise RuntimeError("replay before capture")
-        self._home()
-        if isinstance(self.graph, Graph):
+        self._last = None
+        if isinstance(self._graph, Graph):
             for k in sorted(self._moved):
-                self.target.retarget(self.graph, k,
-                                     [Move(n, 0, self.addresses[n], 0) for n in self.program.groups[k].values],
+                self.target.retarget(self._graph, k,
+                                     [Move(n, 0, self._addresses[n], 0) for n in self.program.groups[k].values],
                                      lambda: None)
         self._moved.clear()
-        self.target.replay(self.graph)
+        self.target.replay(self._graph)
         return self
 
     def outputs(self) -> list[torch.Tensor]:
-        """outputs(ex): the result buffers themselves (the next run overwrites
-        them; after a compiled call, what it returned)."""
+        """outputs(ex): the result buffers themselves (the next run overwrites them)."""
         out = []
+        results = self.results
         for name in self.program.outputs:
             v = self.program.values[name]
             off, nbytes = self.result_at[name]
-            t = self.results[off:off + nbytes].view(v.dtype)
+            t = results[off:off + nbytes].view(v.dtype)
             out.append(t[0] if v.scalar else t.view(*reversed(v.dims)) if len(v.dims) > 1 else t)
         return out
 
     def work(self) -> tuple[float, float]:
         """Algorithmic bytes and flops of one run, summed over launches."""
         b = f = 0.0
-        for l in self.launches:
+        for l in self._launches:
             w = l.work()
             b += w.bytes
             f += w.flops
@@ -431,11 +453,11 @@ class Executable:
     def explain(self) -> str:
         """explain (runtime.jl:1216-1238): each kernel and what runs it."""
         ws = sum(1 for w in self.workspaces if w)
-        lines = [f"{self.program.name}: {len(self.launches)} launches, arena {self.arena.bytes} bytes "
+        lines = [f"{self.program.name}: {len(self._launches)} launches, arena {self.arena.bytes} bytes "
                  f"in {len(self.storage.sizes)} slots" + (f" and {ws} workspaces" if ws else "")]
-        for g, l in zip(self.program.groups, self.launches):
+        for g, l in zip(self.program.groups, self._launches):
             lines.append(f"  {g.name}: reads {', '.join(g.reads)}; writes {', '.join(g.writes)}; {l.describe()}")
-        if self.graph is not None:
+        if self._graph is not None:
             lines.append("  replays as " + ("one graph" if self.graphed else "its launches, one by one (cheaper "
                                             "than a graph for this many kernels on this device)"))
         return "\n".join(lines)
@@ -480,17 +502,20 @@ class Compiled:
         # The results go to an allocation that this call's caller keeps: a copy
         # into one would read and write them once more (1 GiB: 418 us of a
         # 1049 us call).
-        if ex.lend():
-            ex._run()
-            return self._returned(ex.results, lent=True)
-        ex.replay() if ex.graph is not None else ex.execute()
+        lent = ex.lend()
+        if lent is not None:
+            return self._returned(lent, lent=True)
+        ex.replay() if ex._graph is not None else ex.execute()
         return self.returned()
 
     def returned(self):
         """Arrays copied, numbers read to the host (compile.jl:334-349): one
         copy of the result allocation, whose views are the arrays returned,
         then one read of the span holding the numbers."""
-        return self._returned(self.executable.results.clone(), lent=False)
+        ex = self.executable
+        if ex._last is not None:
+            ex._settle()
+        return self._returned(ex._results.clone(), lent=False)
 
     def _returned(self, fresh: torch.Tensor, lent: bool):
         # The arrays first: the device is still at work on the numbers.

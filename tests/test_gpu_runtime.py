@@ -496,3 +496,49 @@ def test_a_call_keeps_what_it_returned(target):
     for got, want in zip((first, second, third, fourth), wants):
         assert got[0] == want[0].item() and torch.equal(got[1], want[1])
     assert torch.equal(fifth[1], wants[3][1])
+
+
+def test_recordings_and_runs_beside_calls(target):
+    """A graph recorded from an executable's launches, a launch run by hand
+    and a run under another current stream write to the executable's own
+    results, which its calls leave in place; what calls returned stays."""
+    import tempest_hip as th
+    rows, n = 500, 1000
+    announce("recordings beside calls")
+    arrays = [(torch.randn(rows, n, device="cuda"), torch.randn(rows, n, device="cuda")) for _ in range(4)]
+    prog = th.programs.softmax_columns(rows, n)
+    wants = [[t.clone() for t in th.prepare(prog, target, x, g).execute().outputs()] for x, g in arrays]
+    same = lambda got, want: got[0] == want[0].item() and torch.equal(got[1], want[1])  # noqa: E731
+    plain = th.compile(prog, target, *arrays[0])
+    kept = [plain(*a) for a in arrays]           # never looked into: results lent every time
+    torch.cuda.synchronize()
+    assert all(same(k, w) for k, w in zip(kept, wants))
+    comp = th.compile(prog, target, *arrays[0])
+    first = comp(*arrays[0])
+    ex = comp.executable
+    graph = target.capture(ex.launches, graph=True)  # of arrays[0]
+    home = ex.results.data_ptr()
+    second = comp(*arrays[1])
+    for _ in range(3):
+        ex.results.zero_()
+        target.replay(graph)
+        torch.cuda.synchronize()
+        assert ex.results.data_ptr() == home and torch.equal(ex.outputs()[1], wants[0][1])
+    graph.release()
+    ex.point(*arrays[2])
+    for l in ex.launches:
+        l()
+    assert torch.equal(ex.outputs()[1], wants[2][1]) and torch.equal(ex.outputs()[0], wants[2][0])
+    third = comp(*arrays[2])
+    other = th.compile(prog, target, *arrays[0])
+    before = other(*arrays[0])
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        bytes_before = torch.cuda.memory_allocated()
+        held = torch.cuda.memory_allocated()
+        other.executable.point(*arrays[3]).execute()
+        assert torch.cuda.memory_allocated() <= held
+        torch.cuda.synchronize()
+        fourth = other(*arrays[3])
+        torch.cuda.synchronize()
+    assert all(same(k, w) for k, w in zip((first, second, third, fourth, before), (*wants, wants[0])))
