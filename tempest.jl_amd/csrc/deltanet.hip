@@ -1181,7 +1181,9 @@ __global__ __launch_bounds__(256, 2) void dn_grad(DnArgs p) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int i = i0 + g4 + v, j = 16 * bj + r;
-        const float gam = expf(ca[i] - ca[j]);
+        // (Above the diagonal the exponent is positive: past e^88 it would be
+        // an infinity times that 0.)
+        const float gam = i >= j ? expf(ca[i] - ca[j]) : 0.0f;
         const float da = i > j ? -dA[0][bj][v] : 0.0f;
         const float gg = bj <= w ? gk[0][bj][v] : 0.0f, q = bj <= w ? qk[0][bj][v] : 0.0f;
         N[i * kLdC + j] = da * be[i] * gam;

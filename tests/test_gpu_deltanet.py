@@ -87,8 +87,7 @@ def test_gate_gradients_to_the_products_precision(target, B, T, H, decay):
     """da and dbeta are fp32 and depend on every product of a chunk's gradient,
     each exact to about 2^-16: through the at most six products in a row of
     the longest path, 6 x 2^-16 < 1e-4 of the float64 oracle, norm-wise; from
-    no decay at all to about e^-51 over a chunk (the kernels form the decay
-    between every two positions, either way round: fp32 holds up to e^88)."""
+    no decay at all to about e^-51 over a chunk."""
     import tempest_hip as th
     announce("deltanet gates", B, T, H, decay)
     q, k, v, a, beta, do = _inputs(B, T, H, 3 * T + H)
@@ -99,3 +98,24 @@ def test_gate_gradients_to_the_products_precision(target, B, T, H, decay):
     for name, got, ref in (("da", out[4], grads[3]), ("dbeta", out[5], grads[4])):
         err = relative(_np(got).reshape(B, T, H), ref)
         assert err < 1e-4, (name, err)
+
+
+@pytest.mark.parametrize("B,T,H,decay", [(1, 128, 2, 3.0), (1, 192, 1, 10.0)])
+def test_gates_that_decay_past_fp32_within_a_chunk(target, B, T, H, decay):
+    """A chunk's decay of e^-150 and e^-500, whose inverse fp32 does not
+    hold: every gradient finite and, where the last state is gone, the
+    oracle's."""
+    import tempest_hip as th
+    announce("deltanet strong gates", B, T, H, decay)
+    q, k, v, a, beta, do = _inputs(B, T, H, 7 * T + H)
+    a = (a * decay).contiguous()
+    comp = th.compile(th.programs.deltanet(B, H, T), target, q, k, v, a, beta, do)
+    out = [_np(x) for x in comp(q, k, v, a, beta, do)]
+    args = [_np(x).astype(np.float64) for x in (q, k, v, a, beta)]
+    assert np.abs(args[3].reshape(B, T // 64, 64, H).sum(axis=2)).max() > 88 * decay / 3
+    refs = [interpret.deltanet_chunked(*args), *interpret.deltanet_grad(*args, _np(do).astype(np.float64))]
+    for name, got, ref in zip(("o", "dq", "dk", "dv", "da", "dbeta"), out, refs):
+        assert np.isfinite(got).all() and np.isfinite(ref).all(), name
+        # bf16 results: TOL; the fp32 ones as in the test above.
+        err = relative(got.reshape(ref.shape), ref)
+        assert err < (1e-4 if name in ("da", "dbeta") else TOL), (name, err)
