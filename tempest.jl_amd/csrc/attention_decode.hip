@@ -19,12 +19,11 @@
 //     of O' += V' P' as they stand, the keys of slot 8 g + j being 4 g + j and
 //     16 + 4 g + j - 4; V' comes from whole rows of V (16 lanes of one row a
 //     load) by an 8 x 8 transpose of halves inside each lane (v_perm_b32);
-//   - the weights stay at fp32's level as in the general kernels: P = hi + lo
-//     in bf16 (16 bits of each weight), two products on V, whose values are
-//     bf16 already.
+//   - the weights are fp32's as in the general kernels: P in three bf16 parts
+//     (weights2), three products on V, whose values are bf16 already.
 // Rows of q, k, v, o may start at any even address.  B16 H32 KV8, 4096 keys of
 // 128 features, lengths of 1/8 to all of it (151 MB on average): 3593 us on the
-// general kernels, 45 here, 40 of them this sweep (3.8 TB/s; the copy rate is
+// general kernels, 45 here (44 with weights of 16 bits), 40 of them this sweep (3.8 TB/s; the copy rate is
 // 5.2) and 5 the fold.  Measured and not kept: parts for 1024, 4096 or 8192
 // workgroups (50, 52, 52 us), non-temporal loads (46), a lane's four K pieces
 // adjacent (46).
@@ -32,23 +31,16 @@
 
 #include <cmath>
 
+#include "attention_tiles.h"
 #include "th_core.h"
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // Rows start where the caller's strides put them: loads and stores of 16 and 8
 // bytes that assume the elements' own alignment.
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
 typedef u32x2 u32x2_any __attribute__((aligned(2)));
 
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLn2 = 0.6931471805599453f;
 constexpr int kRows = 16;    // query rows a workgroup holds
 constexpr int kBlock = 32;   // keys a wave takes at a time
 constexpr int kStep = 128;   // keys the four waves take at a time
@@ -76,10 +68,6 @@ __device__ __forceinline__ int keys_of(const DecodeArgs& p, int b) {
   int n = p.kv_seq;
   if (p.lengths) n = min(max(p.lengths[b], 0), n);
   return p.causal ? min(n, p.seq) : n;
-}
-
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
 
 // One block's operands in flight: K as A operands (key l % 16 of each half,
@@ -167,7 +155,7 @@ __global__ __launch_bounds__(256, 2) void mfma_attn_fwd_decode(DecodeArgs p) {
     const float shift = thd::lse_shift(mn);
     const float alpha = __builtin_amdgcn_exp2f(m - shift);
     m = mn;
-    u32x4 hi, lo;
+    u32x4 w0, w1, w2;
     float w[8], sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -177,8 +165,9 @@ __global__ __launch_bounds__(256, 2) void mfma_attn_fwd_decode(DecodeArgs p) {
     l = l * alpha + sum;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      hi[i] = pack2(w[2 * i], w[2 * i + 1]);
-      lo[i] = pack2(w[2 * i] - __uint_as_float(hi[i] << 16), w[2 * i + 1] - __uint_as_float(hi[i] & 0xffff0000u));
+      uint32_t x0, x1, x2;
+      weights2(w[2 * i], w[2 * i + 1], x0, x1, x2);
+      w0[i] = x0, w1[i] = x1, w2[i] = x2;
     }
     const bool tail = key0 + kBlock > nk;  // keys past the length: V may hold anything there
 #pragma unroll
@@ -199,8 +188,9 @@ __global__ __launch_bounds__(256, 2) void mfma_attn_fwd_decode(DecodeArgs p) {
       for (int u = 0; u < 2; ++u) {
         const bf16x8 a = __builtin_bit_cast(bf16x8, u ? odd : even);
         f32x4 t = o[2 * d2 + u] * alpha;
-        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, lo), t, 0, 0, 0);
-        o[2 * d2 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, hi), t, 0, 0, 0);
+        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, w2), t, 0, 0, 0);
+        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, w1), t, 0, 0, 0);
+        o[2 * d2 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, w0), t, 0, 0, 0);
       }
     }
   };

@@ -30,6 +30,22 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
 __device__ __forceinline__ uint32_t rest2(float a, float b, uint32_t packed) {
   return pack2(a - __uint_as_float(packed << 16), b - __uint_as_float(packed & 0xffff0000u));
 }
+// Two weights (>= 0) in three bf16 parts each, exactly for those from 2^-94 on,
+// every part of a positive weight positive: each is the top 8 bits of the number just below
+// what is left, and the last all of it.  An infinity among the values that the
+// weights multiply then stays one, as with the weight itself; nearest parts, which
+// are 0 or of both signs, would make it NaN.
+__device__ __forceinline__ void weights2(float u, float v, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
+  auto below = [](float x) { return __builtin_elementwise_sub_sat(__float_as_uint(x), 1u); };
+  auto high = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); };
+  uint32_t a = below(u), b = below(v);
+  w0 = high(a, b);
+  u -= __uint_as_float(a & 0xffff0000u), v -= __uint_as_float(b & 0xffff0000u);
+  a = below(u), b = below(v);
+  w1 = high(a, b);
+  u -= __uint_as_float(a & 0xffff0000u), v -= __uint_as_float(b & 0xffff0000u);
+  w2 = high(__float_as_uint(u), __float_as_uint(v));
+}
 // The value lane l ^ 32 holds.
 __device__ __forceinline__ float other_half(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);

@@ -1,8 +1,8 @@
 """Decode: a few bf16 queries over a long cache (mfma_attn_fwd_decode), with
 and without the device-held masks, at the edges of its blocks of 32 keys,
-steps of 128 and parts, against the float64 oracle.  The weights are carried
-in two bf16 parts (2^-17 relative), so what is left is the result's one
-rounding to bf16: at most 2^-9 of each element."""
+steps of 128 and parts, against the float64 oracle.  The weights are fp32's
+(three bf16 parts each), so what is left is the result's one rounding to bf16:
+at most 2^-9 of each element."""
 import numpy as np
 import pytest
 import torch
@@ -123,3 +123,43 @@ def test_decode_recorded_before_its_first_run(target):
         f()
         torch.cuda.synchronize()
         assert torch.equal(got, o)
+
+
+@pytest.mark.parametrize("D,H,KV,S,Sk", [(64, 2, 2, 1, 64), (128, 8, 2, 2, 1000)])
+def test_decode_weights_hold_fp32s_bits(target, D, H, KV, S, Sk):
+    """Keys in pairs, the second one bf16 step from the first in one feature,
+    its value the negative: the output is the difference of weights 2^-13
+    apart.  fp32's score, exponential and sums leave each weight within about
+    2^-22, so 2^-9 of that difference, and the result's rounding another 2^-9;
+    weights of 16 bits would leave 2^-5."""
+    announce("attn decode weights", D, H, KV, S, Sk)
+    q, k, v, o = _case(D, 2, H, KV, S, Sk)
+    q *= 0.25
+    k[:, 1::2], v[:, 1::2] = k[:, ::2], -v[:, ::2]
+    k[:, 1::2, :, 0] = torch.where(k[:, ::2, :, 0] == 0, 0.0, k[:, ::2, :, 0] * (1 + 2.0 ** -7))
+    lse = torch.empty(2, S, H, device="cuda")
+    lengths = torch.tensor([Sk, Sk // 4 * 2], dtype=torch.int32, device="cuda")
+    _launch(q, k, v, o, lse, lengths=lengths)()
+    torch.cuda.synchronize()
+    ro, _ = interpret.attention_fwd(_np(q), _np(k), _np(v), False, None, None, lengths.cpu().numpy())
+    assert np.linalg.norm(ro) < 2.0 ** -8 * np.linalg.norm(_np(v)) / Sk ** 0.5
+    assert relative(_np(o), ro) < 2.0 ** -7, relative(_np(o), ro)
+
+
+def test_decode_an_infinite_value_stays_one(target):
+    """A value of +-inf that a query sees makes its feature of the output that
+    infinity, as a weighted sum in fp32 does, and leaves the others as they are."""
+    announce("attn decode infinite")
+    q, k, v, o = _case(64, 1, 4, 2, 2, 500)
+    lse = torch.empty(1, 2, 4, device="cuda")
+    v[0, 3, 0, 5], v[0, 499, 1, 63] = float("inf"), -float("inf")
+    k[0, 3] = 0.0  # (a weight whose nearest bf16 it may well be)
+    q[0, 1] = 0.0  # every weight 1
+    _launch(q, k, v, o, lse)()
+    torch.cuda.synchronize()
+    assert torch.isposinf(o[0, :, :2, 5]).all() and torch.isneginf(o[0, :, 2:, 63]).all()
+    finite = v.nan_to_num(posinf=0.0, neginf=0.0)
+    _launch(q, k, finite, o2 := torch.empty_like(o), lse)()
+    torch.cuda.synchronize()
+    o[0, :, :2, 5], o[0, :, 2:, 63] = o2[0, :, :2, 5], o2[0, :, 2:, 63]
+    assert torch.equal(o, o2)
