@@ -20,7 +20,7 @@
 //     16 + 4 g + j - 4; V' comes from whole rows of V (16 lanes of one row a
 //     load) by an 8 x 8 transpose of halves inside each lane (v_perm_b32);
 //   - the weights are fp32's as in the general kernels: P in three bf16 parts
-//     (weights2), three products on V, whose values are bf16 already.
+//     (split2_towards0), three products on V, whose values are bf16 already.
 // Rows of q, k, v, o may start at any even address.  B16 H32 KV8, 4096 keys of
 // 128 features, lengths of 1/8 to all of it (151 MB on average): 3593 us on the
 // general kernels, 45 here (44 with weights of 16 bits), 40 of them this sweep (3.8 TB/s; the copy rate is
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256, 2) void mfma_attn_fwd_decode(DecodeArgs p) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       uint32_t x0, x1, x2;
-      weights2(w[2 * i], w[2 * i + 1], x0, x1, x2);
+      split2_towards0(w[2 * i], w[2 * i + 1], x0, x1, x2);
       w0[i] = x0, w1[i] = x1, w2[i] = x2;
     }
     const bool tail = key0 + kBlock > nk;  // keys past the length: V may hold anything there
@@ -195,15 +195,16 @@ __global__ __launch_bounds__(256, 2) void mfma_attn_fwd_decode(DecodeArgs p) {
     }
   };
   // Blocks that end before every row's first key see nothing.
-  int from = first;
+  int from = 0;
   if (p.starts) {
-    if (!live) from = 0x7fffffff;
+    from = live ? first : 0x7fffffff;
 #pragma unroll
     for (int x = 1; x < 16; x *= 2) from = min(from, __shfl_xor(from, x, 64));
-    from = from > k_lo ? (min(from, nk) - k_lo) / kStep * kStep : 0;
+    from = max(0, min(from, nk) - k_lo);
   }
   const int last = nk - 1;
-  int key0 = k_lo + from + kBlock * wave;
+  int key0 = k_lo + from / kStep * kStep + kBlock * wave;
+  if (key0 + kBlock <= k_lo + from) key0 += kStep;
   if (key0 < k_hi) {
     Block<D> even, odd;
     even.load(kb, vb, p.k_ss, key0, last);

@@ -603,16 +603,6 @@ __device__ __forceinline__ void dq_block(const FArgs& p, const int qb, const int
 
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
-// x = part 0 + part 1 + part 2 in bf16, two values a word (8 bits each, rounded
-// to nearest: what is left is at most 2^-27 of x).
-__device__ __forceinline__ void split2(float u, float v, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
-  w0 = pack2(u, v);
-  u -= __uint_as_float(w0 << 16), v -= __uint_as_float(w0 & 0xffff0000u);
-  w1 = pack2(u, v);
-  u -= __uint_as_float(w1 << 16), v -= __uint_as_float(w1 & 0xffff0000u);
-  w2 = pack2(u, v);
-}
-
 // An operand of eight values a lane, in its three parts.
 struct Parts {
   bf16x8 of[3];

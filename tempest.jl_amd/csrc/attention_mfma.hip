@@ -30,10 +30,10 @@
 // A forward or dQ workgroup starts at its queries' least first key, a dK/dV
 // workgroup finds the span of queries that see any of its keys, so packed
 // documents cost their own pairs and not the sequence's.  The general kernels hold P and dS
-// in fp32, so here each is hi + lo in bf16 (2^-17 relative) and takes two
+// in fp32, so here each is three bf16 parts (split2_towards0) and takes three
 // products, on operands that are bf16 already.  Rows may start at any element.
 // B2 H12 S2048 d64 in documents of about 256, forward + backward: 5981 us on
-// the general kernels, 96 here.
+// the general kernels, 111 here (99 with P and dS of 16 bits, beside it).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -95,6 +95,21 @@ __device__ __forceinline__ int most(int x) {
 #pragma unroll
   for (int i = 1; i < 64; i *= 2) x = max(x, __shfl_xor(x, i, 64));
   return __builtin_amdgcn_readfirstlane(x);
+}
+
+// The least of x over the wave's lanes.
+__device__ __forceinline__ int fewest(int x) {
+#pragma unroll
+  for (int i = 1; i < 64; i *= 2) x = min(x, __shfl_xor(x, i, 64));
+  return __builtin_amdgcn_readfirstlane(x);
+}
+
+// M: whether any of a wave's queries, from q0 on, may see any of the 32 keys from
+// k0: none before `first`, its least first key, nor, causal, after its last one.
+// Products over keys leave out those of no use, whose values may be anything (a
+// weight of 0 times an infinity or a NaN would be a NaN).
+__device__ __forceinline__ bool of_use(const MArgs& p, int k0, int first, int q0) {
+  return k0 + 32 > first && (!p.causal || k0 < q0 + 32);
 }
 
 // The least of x over the workgroup's 256 P threads, through 4 P ints of LDS; a
@@ -225,6 +240,7 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
     }
   }
   const int last_first = M ? most(first) : 0;  // tiles from here on see no first key
+  const int least_first = M ? fewest(first) : 0;
   const int k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
   const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
   Stage<D> sk, sv;
@@ -250,7 +266,8 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
     for (int ks = 0; ks < NS; ++ks)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) s[kb] = mfma(frag_rows<D>(K(cur), 32 * kb, ks), qf[ks], s[kb]);
-    if (k0 + 64 > nk || k0 < last_first || (p.causal && k0 + 63 > q0)) {
+    const bool edge = k0 + 64 > nk || k0 < last_first || (p.causal && k0 + 63 > q0);
+    if (edge) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -272,32 +289,54 @@ __device__ __forceinline__ void fwd_block(const MArgs& p, const int qb, const in
 #pragma unroll
     for (int i = 0; i < NB; ++i) o[i] *= alpha;
     m = mn;
-    bf16x8 pf[4], pl[4];
+    if constexpr (M) {
+      // O' (D x 32 queries) += V' P', the weights in three bf16 parts, 32 keys at a time.
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < 2; ++kb) {
+        if (edge && !of_use(p, k0 + 32 * kb, least_first, q0)) continue;
 #pragma unroll
-      for (int part = 0; part < 2; ++part) {
-        u32x4 w, r;
+        for (int part = 0; part < 2; ++part) {
+          u32x4 w, x, y;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float w0 = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * part + 2 * e], c, -shift));
-          const float w1 = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * part + 2 * e + 1], c, -shift));
-          l += w0 + w1;
-          w[e] = pack2(w0, w1);
-          if constexpr (M) r[e] = rest2(w0, w1, w[e]);
+          for (int e = 0; e < 4; ++e) {
+            const float w0 = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * part + 2 * e], c, -shift));
+            const float w1 = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * part + 2 * e + 1], c, -shift));
+            l += w0 + w1;
+            uint32_t x0, x1, x2;
+            split2_towards0(w0, w1, x0, x1, x2);
+            w[e] = x0, x[e] = x1, y[e] = x2;
+          }
+#pragma unroll
+          for (int db = 0; db < NB; ++db) {
+            const bf16x8 vt = frag_tr<D>(V(cur), 32 * db, 2 * kb + part);
+            o[db] = mfma(vt, (bf16x8)y, o[db]);
+            o[db] = mfma(vt, (bf16x8)x, o[db]);
+            o[db] = mfma(vt, (bf16x8)w, o[db]);
+          }
         }
-        pf[2 * kb + part] = (bf16x8)w;
-        if constexpr (M) pl[2 * kb + part] = (bf16x8)r;
       }
-    // O' (D x 32 queries) += V' P', the weights rounded to bf16 (M: in two parts).
+    } else {
+      bf16x8 pf[4];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int db = 0; db < NB; ++db) {
-        const bf16x8 vt = frag_tr<D>(V(cur), 32 * db, ks);
-        if constexpr (M) o[db] = mfma(vt, pl[ks], o[db]);
-        o[db] = mfma(vt, pf[ks], o[db]);
-      }
+        for (int part = 0; part < 2; ++part) {
+          u32x4 w;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float w0 = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * part + 2 * e], c, -shift));
+            const float w1 = __builtin_amdgcn_exp2f(fmaf(s[kb][8 * part + 2 * e + 1], c, -shift));
+            l += w0 + w1;
+            w[e] = pack2(w0, w1);
+          }
+          pf[2 * kb + part] = (bf16x8)w;
+        }
+      // O' (D x 32 queries) += V' P', the weights rounded to bf16.
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int db = 0; db < NB; ++db) o[db] = mfma(frag_tr<D>(V(cur), 32 * db, ks), pf[ks], o[db]);
+    }
     if (j + 1 < mine) {
       // The other stage was last read in step j - 1, before the barrier that ended it.
       sk.store(K(cur ^ 1));
@@ -511,6 +550,7 @@ __device__ __forceinline__ void dkdv_half(const MArgs& p, const uint16_t* Qt, co
     const int qi = 32 * jj + 8 * (i / 4) + 4 * lh + i % 4;
     s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c, -L[qi]));
     dp[i] = s[i] * (dp[i] - L[64 + qi]);
+    if constexpr (M) dp[i] += 0.0f;  // no -0 (split2_towards0)
   }
   if (edge) {
 #pragma unroll
@@ -524,12 +564,19 @@ __device__ __forceinline__ void dkdv_half(const MArgs& p, const uint16_t* Qt, co
   }
 #pragma unroll
   for (int part = 0; part < 2; ++part) {
-    u32x4 ph, pl, sh, sl;
+    u32x4 ph, pm, pl, sh, sm, sl;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int i = 8 * part + 2 * e;
-      ph[e] = pack2(s[i], s[i + 1]), sh[e] = pack2(dp[i], dp[i + 1]);
-      if constexpr (M) pl[e] = rest2(s[i], s[i + 1], ph[e]), sl[e] = rest2(dp[i], dp[i + 1], sh[e]);
+      if constexpr (M) {
+        uint32_t x0, x1, x2;
+        split2_towards0(s[i], s[i + 1], x0, x1, x2);
+        ph[e] = x0, pm[e] = x1, pl[e] = x2;
+        split2_towards0(dp[i], dp[i + 1], x0, x1, x2);
+        sh[e] = x0, sm[e] = x1, sl[e] = x2;
+      } else {
+        ph[e] = pack2(s[i], s[i + 1]), sh[e] = pack2(dp[i], dp[i + 1]);
+      }
     }
     // dV' (DO features x 32 keys) += dO' P;  dK' += Q' dS.
 #pragma unroll
@@ -538,6 +585,8 @@ __device__ __forceinline__ void dkdv_half(const MArgs& p, const uint16_t* Qt, co
       if constexpr (M) {
         dv[db] = mfma(g, (bf16x8)pl, dv[db]);
         dk[db] = mfma(q, (bf16x8)sl, dk[db]);
+        dv[db] = mfma(g, (bf16x8)pm, dv[db]);
+        dk[db] = mfma(q, (bf16x8)sm, dk[db]);
       }
       dv[db] = mfma(g, (bf16x8)ph, dv[db]);
       dk[db] = mfma(q, (bf16x8)sh, dk[db]);
@@ -626,7 +675,10 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
       bool edge = qq0 + 64 > p.seq || kw + 32 > nk || (p.causal && kw + 31 > qq0);
       if constexpr (M) edge = edge || kw < __builtin_amdgcn_readfirstlane(__float_as_int(L[192]));
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj) dkdv_half<D, DO, M>(p, Qt, Gt, L, jj, edge, qq0, key, nk, dh, kf, vf, dk, dv);
+      for (int jj = 0; jj < 2; ++jj) {
+        if (M && p.causal && qq0 + 32 * jj + 31 < kw) continue;  // queries before the wave's keys (as of_use)
+        dkdv_half<D, DO, M>(p, Qt, Gt, L, jj, edge, qq0, key, nk, dh, kf, vf, dk, dv);
+      }
       if (j + 1 < mine) store(cur ^ 1);
     };
     for (int j = 0; P * j < nsteps; ++j) {
@@ -652,6 +704,10 @@ __device__ __forceinline__ void dkdv_block(const MArgs& p, const int kblk, const
   int ko = key;
   if constexpr (D == 128) asm volatile("" : "+v"(ko));
   if (ko >= p.kv_seq) return;
+  if (M && ko >= nk) {  // past the sequence's length: zeros, whatever the gradients are
+#pragma unroll
+    for (int i = 0; i < NBO; ++i) dk[i] = f32x16{}, dv[i] = f32x16{};
+  }
   if (split >= 0) {
     const int64_t rows = (int64_t)p.batch * p.kv_seq * p.kv_heads;
     const int64_t row = (((int64_t)split * p.batch + b) * p.kv_seq + ko) * p.kv_heads + hk;
@@ -720,6 +776,7 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
     }
   }
   const int last_first = M ? most(first) : 0;  // tiles from here on see no first key
+  const int least_first = M ? fewest(first) : 0;
   const int k_hi = split < 0 ? kend : min(kend, k_lo + p.q_span);
   const int nsteps = k_hi > k_lo ? (k_hi - k_lo + 63) / 64 : 0;
   Stage<D> sk, sv;
@@ -739,52 +796,86 @@ __device__ __forceinline__ void dq_block(const MArgs& p, const int qb, const int
       sk.load(kbase, p.k_ss, k0 + 64 * P, nk);
       sv.load(vbase, p.k_ss, k0 + 64 * P, nk);
     }
-    f32x16 s[2] = {f32x16{}, f32x16{}}, dp[2] = {f32x16{}, f32x16{}};
-#pragma unroll
-    for (int ks = 0; ks < NS; ++ks)
+    if constexpr (M) {
+      // 32 keys at a time, dS in three bf16 parts.
+      const bool edge = k0 + 64 > nk || k0 < last_first || (p.causal && k0 + 63 > q0);
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
-        s[kb] = mfma(frag_rows<D>(K(cur), 32 * kb, ks), qf[ks], s[kb]);
-        dp[kb] = mfma(frag_rows<D>(V(cur), 32 * kb, ks), gf[ks], dp[kb]);
+        if (edge && !of_use(p, k0 + 32 * kb, least_first, q0)) continue;
+        f32x16 s = {}, dp = {};
+#pragma unroll
+        for (int ks = 0; ks < NS; ++ks) {
+          s = mfma(frag_rows<D>(K(cur), 32 * kb, ks), qf[ks], s);
+          dp = mfma(frag_rows<D>(V(cur), 32 * kb, ks), gf[ks], dp);
+        }
+        // dS' into dp, without a -0 (split2_towards0).
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          dp[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c, -l2)) * (dp[i] - dl) + 0.0f;
+        if (edge) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
+            dp[i] = key < nk && key >= first && (!p.causal || key <= query) ? dp[i] : 0.0f;
+          }
+        }
+#pragma unroll
+        for (int part = 0; part < 2; ++part) {
+          u32x4 w, x, y;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            uint32_t x0, x1, x2;
+            split2_towards0(dp[8 * part + 2 * e], dp[8 * part + 2 * e + 1], x0, x1, x2);
+            w[e] = x0, x[e] = x1, y[e] = x2;
+          }
+#pragma unroll
+          for (int db = 0; db < NB; ++db) {
+            const bf16x8 kt = frag_tr<D>(K(cur), 32 * db, 2 * kb + part);
+            dq[db] = mfma(kt, (bf16x8)y, dq[db]);
+            dq[db] = mfma(kt, (bf16x8)x, dq[db]);
+            dq[db] = mfma(kt, (bf16x8)w, dq[db]);
+          }
+        }
       }
-    // dS' into dp, masked where the tile needs it.
+    } else {
+      f32x16 s[2] = {f32x16{}, f32x16{}}, dp[2] = {f32x16{}, f32x16{}};
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+      for (int ks = 0; ks < NS; ++ks)
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        dp[kb][i] = __builtin_amdgcn_exp2f(fmaf(s[kb][i], c, -l2)) * (dp[kb][i] - dl);
-    if (k0 + 64 > nk || k0 < last_first || (p.causal && k0 + 63 > q0)) {
+        for (int kb = 0; kb < 2; ++kb) {
+          s[kb] = mfma(frag_rows<D>(K(cur), 32 * kb, ks), qf[ks], s[kb]);
+          dp[kb] = mfma(frag_rows<D>(V(cur), 32 * kb, ks), gf[ks], dp[kb]);
+        }
+      // dS' into dp, masked where the tile needs it.
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
-          dp[kb][i] = key < nk && (!M || key >= first) && (!p.causal || key <= query) ? dp[kb][i] : 0.0f;
+        for (int i = 0; i < 16; ++i)
+          dp[kb][i] = __builtin_amdgcn_exp2f(fmaf(s[kb][i], c, -l2)) * (dp[kb][i] - dl);
+      if (k0 + 64 > nk || (p.causal && k0 + 63 > q0)) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int key = k0 + 32 * kb + 8 * (i / 4) + 4 * lh + i % 4;
+            dp[kb][i] = key < nk && (!p.causal || key <= query) ? dp[kb][i] : 0.0f;
+          }
+      }
+      bf16x8 sf[4];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int part = 0; part < 2; ++part) {
+          u32x4 w;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[e] = pack2(dp[kb][8 * part + 2 * e], dp[kb][8 * part + 2 * e + 1]);
+          sf[2 * kb + part] = (bf16x8)w;
         }
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int db = 0; db < NB; ++db) dq[db] = mfma(frag_tr<D>(K(cur), 32 * db, ks), sf[ks], dq[db]);
     }
-    bf16x8 sf[4], sl[4];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int part = 0; part < 2; ++part) {
-        u32x4 w, r;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int i = 8 * part + 2 * e;
-          w[e] = pack2(dp[kb][i], dp[kb][i + 1]);
-          if constexpr (M) r[e] = rest2(dp[kb][i], dp[kb][i + 1], w[e]);
-        }
-        sf[2 * kb + part] = (bf16x8)w;
-        if constexpr (M) sl[2 * kb + part] = (bf16x8)r;
-      }
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int db = 0; db < NB; ++db) {
-        const bf16x8 kt = frag_tr<D>(K(cur), 32 * db, ks);
-        if constexpr (M) dq[db] = mfma(kt, sl[ks], dq[db]);
-        dq[db] = mfma(kt, sf[ks], dq[db]);
-      }
     if (j + 1 < mine) {
       sk.store(K(cur ^ 1));
       sv.store(V(cur ^ 1));

@@ -26,22 +26,28 @@ constexpr float kLn2 = 0.6931471805599453f;
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
-// What pack2 rounded away of each.
-__device__ __forceinline__ uint32_t rest2(float a, float b, uint32_t packed) {
-  return pack2(a - __uint_as_float(packed << 16), b - __uint_as_float(packed & 0xffff0000u));
+// x = part 0 + part 1 + part 2 in bf16, two values a word (8 bits each, rounded
+// to nearest: what is left is at most 2^-27 of x, or 2^-134, half of bf16's
+// least subnormal, which the matrix cores keep).
+__device__ __forceinline__ void split2(float u, float v, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
+  w0 = pack2(u, v);
+  u -= __uint_as_float(w0 << 16), v -= __uint_as_float(w0 & 0xffff0000u);
+  w1 = pack2(u, v);
+  u -= __uint_as_float(w1 << 16), v -= __uint_as_float(w1 & 0xffff0000u);
+  w2 = pack2(u, v);
 }
-// Two weights (>= 0) in three bf16 parts each, exactly for those from 2^-94 on,
-// every part of a positive weight positive: each is the top 8 bits of the number just below
-// what is left, and the last all of it.  An infinity among the values that the
-// weights multiply then stays one, as with the weight itself; nearest parts, which
-// are 0 or of both signs, would make it NaN.
-__device__ __forceinline__ void weights2(float u, float v, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
-  auto below = [](float x) { return __builtin_elementwise_sub_sat(__float_as_uint(x), 1u); };
+// The same (of anything but -0), exactly from 2^-94 on, and every part of x's sign
+// and not 0: each is the top 8 bits of the number next to what is left towards
+// 0, and the last all of it.  An infinity among the values that x multiplies, or in
+// x, then gives what it gives with x itself; nearest parts, which are 0 or of both
+// signs, would make it NaN.
+__device__ __forceinline__ void split2_towards0(float u, float v, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
+  auto next = [](float x) { return __builtin_elementwise_sub_sat(__float_as_uint(x), 1u); };
   auto high = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); };
-  uint32_t a = below(u), b = below(v);
+  uint32_t a = next(u), b = next(v);
   w0 = high(a, b);
   u -= __uint_as_float(a & 0xffff0000u), v -= __uint_as_float(b & 0xffff0000u);
-  a = below(u), b = below(v);
+  a = next(u), b = next(v);
   w1 = high(a, b);
   u -= __uint_as_float(a & 0xffff0000u), v -= __uint_as_float(b & 0xffff0000u);
   w2 = high(__float_as_uint(u), __float_as_uint(v));

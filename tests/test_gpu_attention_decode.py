@@ -163,3 +163,21 @@ def test_decode_an_infinite_value_stays_one(target):
     torch.cuda.synchronize()
     o[0, :, :2, 5], o[0, :, 2:, 63] = o2[0, :, :2, 5], o2[0, :, 2:, 63]
     assert torch.equal(o, o2)
+
+
+@pytest.mark.parametrize("lo", [32, 96, 128, 160, 544])
+def test_decode_reads_nothing_into_what_lies_before_the_first_key(target, lo):
+    """A cache padded on the left: what lies before the first key (a multiple
+    of 32, as far as the general kernels skip) may be anything."""
+    announce("attn decode left padding", lo)
+    q, k, v, o = _case(64, 1, 4, 2, 1, 700)
+    lse = torch.empty(1, 1, 4, device="cuda")
+    starts = torch.tensor([[lo + 1]], dtype=torch.int32, device="cuda")
+    _launch(q, k, v, o, lse, starts=starts)()
+    torch.cuda.synchronize()
+    _check(q, k, v, o, lse, starts=starts)
+    want = o.clone()
+    k[:, :lo], v[:, :lo] = float("nan"), float("nan")
+    _launch(q, k, v, o, lse, starts=starts)()
+    torch.cuda.synchronize()
+    assert torch.equal(o, want)
