@@ -17,9 +17,11 @@
 // registers, two barriers a step; bound by the vector work of the splits and
 // the wait at the barriers, the products being under half of the time.
 //
-// A block whose results are not finite, or all of whose staged values are under
-// 2^-90 (their lower parts fall under bf16's range), is computed again with fp32
-// products (v_mfma_f32_32x32x2_f32; *_block), forms of depth 2 instead of 16:
+// Q, K, V and dO are scaled by 2^24 as they are split (kUp; dS with them, and the
+// results back), so that a part of the least fp32 number is one of bf16's; a weight
+// under 2^-109 keeps what bits of it lie above 2^-134.  A block whose results are not finite
+// (also those of factors past 2^103) is computed again with fp32 products
+// (v_mfma_f32_32x32x2_f32; *_block), forms of depth 2 instead of 16:
 //   - products over d (S' = K Q', S = Q K', dP = dO V'): lane half h takes d
 //     in [h D/2, (h + 1) D/2), step s the d h D/2 + s, so a lane's operand
 //     of four steps is one 16-byte read of a tile row (rows of D + 4 floats:
@@ -601,7 +603,9 @@ __device__ __forceinline__ void dq_block(const FArgs& p, const int qb, const int
 
 // ---- the sweeps in bf16 parts -------------------------------------------------------
 
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+// The factors' scale, and what takes products of two and three of them back.
+constexpr float kUp = 0x1p24f, kDown = 0x1p-24f, kDown2 = 0x1p-48f, kDown3 = 0x1p-72f;
+constexpr float kUp2 = 0x1p48f;
 
 // An operand of eight values a lane, in its three parts.
 struct Parts {
@@ -643,8 +647,8 @@ __device__ __forceinline__ Parts tr3(const uint16_t* t, int d0, int ks) {
   return Parts{{frag_tr<D>(t, d0, ks), frag_tr<D>(t + kPart<D>, d0, ks), frag_tr<D>(t + 2 * kPart<D>, d0, ks)}};
 }
 
-// A position's row as the B operand of a product over d: d = 16 ks + 8 (lane /
-// 32) + (0..7); zeros for a position past the end.
+// A position's row, times kUp, as the B operand of a product over d: d = 16 ks
+// + 8 (lane / 32) + (0..7); zeros for a position past the end.
 template <int D>
 __device__ __forceinline__ void row_parts(const float* row, bool live, Parts (&f)[D / 16]) {
   const int lh = threadIdx.x % 64 / 32;
@@ -655,7 +659,7 @@ __device__ __forceinline__ void row_parts(const float* row, bool live, Parts (&f
     u32x4 w[3];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const f32x4& x = e < 2 ? lo : hi;
+      const f32x4 x = (e < 2 ? lo : hi) * kUp;
       uint32_t w0, w1, w2;
       split2(x[2 * (e % 2)], x[2 * (e % 2) + 1], w0, w1, w2);
       w[0][e] = w0, w[1][e] = w1, w[2][e] = w2;
@@ -664,33 +668,24 @@ __device__ __forceinline__ void row_parts(const float* row, bool live, Parts (&f
   }
 }
 
-// A tile loaded into registers (StageF) and stored in its parts; `most`: the
-// largest leading parts this thread has stored.
+// A tile loaded into registers (StageF) and stored, times kUp, in its parts.
 template <int D>
 struct StageP : StageF<D> {
-  u16x2 most = {0, 0};
-  __device__ void store(uint16_t* t) {
+  __device__ void store(uint16_t* t) const {
 #pragma unroll
     for (int i = 0; i < StageF<D>::kPer; ++i) {
       const int c = threadIdx.x + 256 * i, row = c / StageF<D>::kChunks, col = c % StageF<D>::kChunks;
-      const f32x4& x = this->r[i];
+      const f32x4 x = this->r[i] * kUp;
       u32x2 w[3];
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         uint32_t w0, w1, w2;
         split2(x[2 * e], x[2 * e + 1], w0, w1, w2);
         w[0][e] = w0, w[1][e] = w1, w[2][e] = w2;
-        most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, w0 & 0x7fff7fffu));
       }
 #pragma unroll
       for (int s = 0; s < 3; ++s) *reinterpret_cast<u32x2*>(t + s * kPart<D> + row * (D + 8) + 4 * col) = w[s];
     }
-  }
-  // Whether all it stored was under 2^-90, and not all zero: the lower parts
-  // then fall under bf16's normal range.
-  __device__ bool tiny() const {
-    const int x = max((int)most[0], (int)most[1]);
-    return x > 0 && x < (127 - 90) << 7;
   }
 };
 
@@ -735,7 +730,7 @@ __device__ __forceinline__ bool fwd_parts(const FArgs& p, const int qb, const in
 #pragma unroll
   for (int i = 0; i < NB; ++i) o[i] = f32x16{};
   float m = -INFINITY, l = 0.0f;
-  const float c = p.scale * kLog2e;
+  const float c = p.scale * kLog2e * kDown2;  // of scores times kUp2
   const int qlast = min(qb * 128 + 127, p.seq - 1);
   const int kend = p.causal ? min(p.kv_seq, qlast + 1) : p.kv_seq;
   const int k_lo = split < 0 ? 0 : split * p.span, k_hi = split < 0 ? kend : min(kend, k_lo + p.span);
@@ -801,15 +796,15 @@ __device__ __forceinline__ bool fwd_parts(const FArgs& p, const int qb, const in
   }
   l += other_half(l);
   const bool good = query >= p.seq || (finite(o) && fabsf(l) < INFINITY);
-  if (__syncthreads_or(!good || sk.tiny() || sv.tiny())) return false;
+  if (__syncthreads_or(!good)) return false;
   if (query >= p.seq) return true;
   if (split >= 0) {
     const int64_t row = (((int64_t)split * p.batch + b) * p.seq + query) * p.heads + h;
-    store_quads<D>(p.part + row * D, o, 1.0f);
+    store_quads<D>(p.part + row * D, o, kDown);
     if (lh == 0) reinterpret_cast<f32x2*>(p.part_ml)[row] = f32x2{m, l};
     return true;
   }
-  store_quads<D>(p.o + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)query * p.q_ss, o, 1.0f / l);
+  store_quads<D>(p.o + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)query * p.q_ss, o, kDown / l);
   if (lh == 0 && p.lse) p.lse[((int64_t)b * p.seq + query) * p.heads + h] = (m + log2f(l)) * kLn2;
   return true;
 }
@@ -821,7 +816,7 @@ __device__ __forceinline__ bool dkdv_parts(const FArgs& p, const int kblk, const
   extern __shared__ __attribute__((aligned(16))) float flds[];
   uint16_t* Q = reinterpret_cast<uint16_t*>(flds);
   uint16_t* G = Q + kTileP<D>;
-  float* L = reinterpret_cast<float*>(G + kTileP<D>);  // lse * log2e (64) | delta (64)
+  float* L = reinterpret_cast<float*>(G + kTileP<D>);  // lse * log2e (64) | delta times kUp2 (64)
   const int group = p.heads / p.kv_heads;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lh = lane / 32;
   const int kw = __builtin_amdgcn_readfirstlane(kblk * 128 + wave * 32), key = kw + lane % 32;
@@ -832,13 +827,13 @@ __device__ __forceinline__ bool dkdv_parts(const FArgs& p, const int kblk, const
   f32x16 dk[NB], dv[NB];
 #pragma unroll
   for (int i = 0; i < NB; ++i) dk[i] = f32x16{}, dv[i] = f32x16{};
-  const float c = p.scale * kLog2e;
+  const float c = p.scale * kLog2e * kDown2;  // of scores times kUp2
   const int qfirst = p.causal ? kblk * 128 : 0;
   const int qstart = split < 0 ? qfirst : qfirst + split * p.span;
   const int qstop = split < 0 ? p.seq : min(p.seq, qstart + p.span);
   const int nsteps = qstart < qstop ? (qstop - qstart + 63) / 64 : 0;
   StageP<D> sq, sg;
-  float st = 0.0f;  // threads 0..127: a query's lse * log2e or delta
+  float st = 0.0f;  // threads 0..127: a query's lse * log2e or delta, times kUp2
   auto load = [&](int h, int q0) {
     const int64_t qoff = (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
     sq.load(p.q + qoff, p.q_ss, q0, p.seq);
@@ -846,7 +841,7 @@ __device__ __forceinline__ bool dkdv_parts(const FArgs& p, const int kblk, const
     if (threadIdx.x < 128) {
       const int j = q0 + threadIdx.x % 64;
       const int64_t row = ((int64_t)b * p.seq + j) * p.heads + h;
-      st = j < p.seq ? (threadIdx.x < 64 ? p.lse[row] * kLog2e : p.delta[row]) : 0.0f;
+      st = j < p.seq ? (threadIdx.x < 64 ? p.lse[row] * kLog2e : p.delta[row] * kUp2) : 0.0f;
     }
   };
   const int total = nsteps * group;  // steps over the group's query heads
@@ -870,7 +865,7 @@ __device__ __forceinline__ bool dkdv_parts(const FArgs& p, const int kblk, const
         s = mfma6(rows3<D>(Q, 32 * jj, ks), kf[ks], s);
         dp = mfma6(rows3<D>(G, 32 * jj, ks), vf[ks], dp);
       }
-      // P into s, dS into dp.
+      // P into s, dS times kUp2 into dp.
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int qi = 32 * jj + 8 * (i / 4) + 4 * lh + i % 4;
@@ -899,18 +894,18 @@ __device__ __forceinline__ bool dkdv_parts(const FArgs& p, const int kblk, const
     }
   }
   const bool good = key >= p.kv_seq || (finite(dk) && finite(dv));
-  if (__syncthreads_or(!good || sq.tiny() || sg.tiny())) return false;
+  if (__syncthreads_or(!good)) return false;
   if (key >= p.kv_seq) return true;
   if (split >= 0) {
     const int64_t rows = (int64_t)p.batch * p.kv_seq * p.kv_heads;
     const int64_t row = (((int64_t)split * p.batch + b) * p.kv_seq + key) * p.kv_heads + hk;
-    store_quads<D>(p.part + row * D, dk, 1.0f);
-    store_quads<D>(p.part + ((int64_t)p.nsplit * rows + row) * D, dv, 1.0f);
+    store_quads<D>(p.part + row * D, dk, kDown3);
+    store_quads<D>(p.part + ((int64_t)p.nsplit * rows + row) * D, dv, kDown);
     return true;
   }
   const int64_t out = koff + (int64_t)key * p.k_ss;
-  store_quads<D>(p.dk + out, dk, p.scale);
-  store_quads<D>(p.dv + out, dv, 1.0f);
+  store_quads<D>(p.dk + out, dk, p.scale * kDown3);
+  store_quads<D>(p.dv + out, dv, kDown);
   return true;
 }
 
@@ -931,8 +926,8 @@ __device__ __forceinline__ bool dq_parts(const FArgs& p, const int qb, const int
   row_parts<D>(p.dout + qoff, live, gf);
   const int64_t srow = ((int64_t)b * p.seq + query) * p.heads + h;
   const float l2 = live ? p.lse[srow] * kLog2e : 0.0f;
-  const float dl = live ? p.delta[srow] : 0.0f;
-  const float c = p.scale * kLog2e;
+  const float dl = live ? p.delta[srow] * kUp2 : 0.0f;
+  const float c = p.scale * kLog2e * kDown2;  // of scores times kUp2
   const float* kbase = p.k + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
   const float* vbase = p.v + (int64_t)b * p.k_sb + (int64_t)hk * p.k_sh;
   f32x16 dq[NB];
@@ -966,7 +961,7 @@ __device__ __forceinline__ bool dq_parts(const FArgs& p, const int qb, const int
         s = mfma6(rows3<D>(K, 32 * kb, ks), qf[ks], s);
         dp = mfma6(rows3<D>(V, 32 * kb, ks), gf[ks], dp);
       }
-      // dS' into s.
+      // dS' times kUp2 into s.
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c, -l2)) * (dp[i] - dl);
       if (edge) {
@@ -984,12 +979,12 @@ __device__ __forceinline__ bool dq_parts(const FArgs& p, const int qb, const int
       }
     }
   }
-  if (__syncthreads_or((live && !finite(dq)) || sk.tiny() || sv.tiny())) return false;
+  if (__syncthreads_or(live && !finite(dq))) return false;
   if (!live) return true;
   if (split >= 0)
-    store_quads<D>(p.q_part + ((((int64_t)split * p.batch + b) * p.seq + query) * p.heads + h) * D, dq, 1.0f);
+    store_quads<D>(p.q_part + ((((int64_t)split * p.batch + b) * p.seq + query) * p.heads + h) * D, dq, kDown3);
   else
-    store_quads<D>(p.dq + qoff, dq, p.scale);
+    store_quads<D>(p.dq + qoff, dq, p.scale * kDown3);
   return true;
 }
 
@@ -1001,12 +996,15 @@ constexpr size_t kLdsF = (2 * kTileP<D> * sizeof(uint16_t) > 4 * kTileF<D> * siz
                                                                                            : 4 * kTileF<D> * sizeof(float)) +
                          2 * 128 * sizeof(float);
 
+// Scales under this, times kDown3, would lose bits: fp32 products alone.
+constexpr float kLeastScale = 0x1p-50f;
+
 template <int D>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void f32_attn_fwd(FArgs p) {
   const bool split = p.nsplit > 1;
   const int z = gridDim.z - 1 - blockIdx.z;  // the last queries first
   const int qb = split ? z / p.nsplit : z, part = split ? z % p.nsplit : -1;
-  if (!fwd_parts<D>(p, qb, blockIdx.y, part)) fwd_block<D>(p, qb, blockIdx.y, part);
+  if (p.scale < kLeastScale || !fwd_parts<D>(p, qb, blockIdx.y, part)) fwd_block<D>(p, qb, blockIdx.y, part);
 }
 
 // Both sweeps in one launch: neither needs the other, and alone each leaves
@@ -1017,7 +1015,9 @@ struct FBwdArgs {
   uint32_t n_dkdv;
 };
 
-// One wave a SIMD: with two, d = 64 spills around its sweeps.
+// One wave a SIMD: with two, d = 64 spills around its sweeps.  d = 128 spills 43
+// registers even so (K and V of a wave's keys take 192 in parts, dK' and dV'
+// 128, the next tile 64), 36 of them without the fp32 form beside it.
 template <int D>
 __global__ __launch_bounds__(256, 1) void f32_attn_bwd(FBwdArgs a) {
   const FArgs& p = a.p;
@@ -1025,14 +1025,14 @@ __global__ __launch_bounds__(256, 1) void f32_attn_bwd(FBwdArgs a) {
     const int hk = blockIdx.x % p.kv_heads, b = blockIdx.x / p.kv_heads % p.batch, z = blockIdx.x / p.kv_heads / p.batch;
     const bool split = p.nsplit > 1;
     const int kblk = split ? z / p.nsplit : z, part = split ? z % p.nsplit : -1;
-    if (!dkdv_parts<D>(p, kblk, hk, b, part)) dkdv_block<D>(p, kblk, hk, b, part);
+    if (p.scale < kLeastScale || !dkdv_parts<D>(p, kblk, hk, b, part)) dkdv_block<D>(p, kblk, hk, b, part);
     return;
   }
   const uint32_t i = gridDim.x - 1 - blockIdx.x;  // (from the end: the last queries first)
   const int h = i % p.heads, b = i / p.heads % p.batch, z = i / p.heads / p.batch;
   const bool split = p.q_nsplit > 1;
   const int qb = split ? z / p.q_nsplit : z, part = split ? z % p.q_nsplit : -1;
-  if (!dq_parts<D>(p, qb, h, b, part)) dq_block<D>(p, qb, h, b, part);
+  if (p.scale < kLeastScale || !dq_parts<D>(p, qb, h, b, part)) dq_block<D>(p, qb, h, b, part);
 }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }

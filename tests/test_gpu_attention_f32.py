@@ -69,8 +69,8 @@ def test_fp32_split_and_whole_sweeps(target, D, B, H, KV, S, causal, split):
                                         (128, 64, False), (64, 1, True)])
 def test_fp32_values_out_of_the_parts_reach(target, D, S, causal):
     """Tiles computed again with fp32 products: an infinity in V gives infinity
-    where it is seen and leaves the other features alone; gradients scaled far
-    under 2^-90 keep their relative accuracy, at the edges of tiles."""
+    where it is seen and leaves the other features alone; and gradients scaled far
+    down keep their relative accuracy, at the edges of tiles."""
     announce("attn fp32 parts", D, S, causal)
     gen = torch.Generator(device="cuda").manual_seed(D + S)
     r = lambda: torch.randn(2, S, 2, D, device="cuda", generator=gen) * 0.5  # noqa: E731
@@ -93,3 +93,29 @@ def test_fp32_values_out_of_the_parts_reach(target, D, S, causal):
     ro, _ = interpret.attention_fwd(_np(q), _np(k), _np(clean), False)
     keep = rest.cpu().numpy()
     assert relative(_np(o)[keep], ro[keep]) < TOL_F32
+
+
+@pytest.mark.parametrize("D,S", [(64, 1024), (128, 300)])
+@pytest.mark.parametrize("what,e", [("dout", -110), ("dout", -119), ("v", -119), ("features", 122)])
+def test_fp32_attention_over_fp32s_range(target, D, S, what, e):
+    """dO, or V, of about 2^e; and a quarter of the features 2^e in Q, 2^-e in K:
+    the same results as at ordinary sizes, scaled (a power of two, so exactly what
+    fp32 products of the scaled factors give), where the lower parts of a factor
+    lie under bf16's least subnormal."""
+    announce("attn fp32 range", D, S, what, e)
+    gen = torch.Generator(device="cuda").manual_seed(D + S + e)
+    q, k, v, g = (torch.randn(1, S, 2, D, device="cuda", generator=gen) * 0.5 for _ in range(4))
+    t = 2.0 ** e
+    up = torch.ones(D, device="cuda")
+    if what == "features":
+        up[::4] = t
+    scaled = [q * up, k / up, v * t if what == "v" else v, g * t if what == "dout" else g]
+    (o, _, dq, dk, dv), _ = _run(*scaled, True, True)
+    ro, _ = interpret.attention_fwd(_np(q), _np(k), _np(v), True)
+    want = interpret.attention_bwd(_np(q), _np(k), _np(v), _np(g), True)
+    u = _np(up).astype("f8")
+    so, sg, sv = t if what == "v" else 1.0, t if what in ("v", "dout") else 1.0, t if what == "dout" else 1.0
+    for name, got, ref in (("o", _np(o).astype("f8") / so, ro), ("dq", _np(dq).astype("f8") / sg * u, want[0]),
+                           ("dk", _np(dk).astype("f8") / sg / u, want[1]), ("dv", _np(dv).astype("f8") / sv, want[2])):
+        print("   ", name, relative(got, ref), flush=True)
+        assert relative(got, ref) < 4e-6, (name, relative(got, ref))
