@@ -191,8 +191,9 @@ __global__ __launch_bounds__(256) void gemm_general(GenGemmArgs p) {
 // 1030 5.7e-7 and 1.9e-7, 256 x 256 x 8192 2.5e-7 and 1.6e-7; time 1289 and 800
 // to 860 us, 156 and 66, 32 and 21.  What bounds it now: of a step's 1.0 us (one
 // workgroup on a CU; 1.56 two) the products take 0.43, the rest is LDS traffic
-// and the wait at its barrier.  A tile whose sums are not finite, or with a row of values all
-// under 2^-90, is computed again on the fp32 matrix cores
+// and the wait at its barrier.  The factors are scaled by 2^24 as they are split, and
+// the sums back, so that the parts reach as far down as fp32 does; a tile whose sums
+// are not finite is computed again on the fp32 matrix cores
 // (v_mfma_f32_32x32x2_f32), as every tile was before.
 // K moves 16 at a time through two LDS stages, the next two slices held in
 // registers (SplitOp).  K may be split over parts (grid.y), each writing its fp32 sums to the
@@ -223,10 +224,12 @@ typedef __bf16 bf16x8g __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4g __attribute__((ext_vector_type(4)));
 typedef f32x4 f32x4_any __attribute__((aligned(4)));
 typedef uint32_t u32x2g __attribute__((ext_vector_type(2)));
-typedef uint16_t u16x2g __attribute__((ext_vector_type(2)));
 // 16-byte pieces of a stage: operand, part, half of 16 k, row; the halves 128
 // bytes apart modulo the banks, so that quads of both halves write at once.
 constexpr int kSplitHalf = kFT + 8;
+// Both factors' scale as they are split: a part of the least fp32 number is then
+// one of bf16's, whose least subnormal is 2^-133.
+constexpr float kUp = 0x1p24f;
 constexpr int kSplitStage = 2 * 3 * 2 * kSplitHalf;
 
 // A's 128 x 16 slice at (m0, k0) into LDS As[k][m]: eight values a thread.
@@ -382,7 +385,6 @@ struct SplitOp {
   int k[2];
   bool unit;
   uint32_t to[2];   // the quads' places in a stage, in 8-byte units
-  u16x2g most[2];   // the largest leading parts of each quad so far, as bf16 bits
 
   __device__ __forceinline__ void init(const float* base, int64_t s_r, int64_t s_k_, int row0, int rows) {
     const int t = threadIdx.x;
@@ -393,7 +395,6 @@ struct SplitOp {
       k[q] = KC ? 4 * (t % 4) : 8 * (t / kFT) + 4 * q;
       at[q] = base + (int64_t)min(row0 + lr, rows - 1) * s_r + (int64_t)k[q] * s_k;
       to[q] = 2 * (k[q] / 8 * kSplitHalf + lr) + k[q] / 4 % 2;
-      most[q] = u16x2g{0, 0};
     }
   }
   // The slice at k0, whole (nothing but loads, so that none waits for
@@ -417,21 +418,20 @@ struct SplitOp {
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[q][i] = k0 + k[q] + i < kend ? at[q][(int64_t)(k0 + i) * s_k] : 0.0f;
   }
-  // x = part 0 + part 1 + part 2 in bf16 (8 bits each, rounded to nearest:
-  // what is left is at most 2^-27 of x).
-  __device__ __forceinline__ void split(const f32x4 (&x)[2], u32x2g (&w)[2][3]) {
+  // x kUp = part 0 + part 1 + part 2 in bf16 (8 bits each, rounded to nearest:
+  // what is left is at most 2^-27 of it).
+  __device__ __forceinline__ void split(const f32x4 (&x)[2], u32x2g (&w)[2][3]) const {
 #pragma unroll
     for (int q = 0; q < 2; ++q)
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        float u = x[q][2 * i], v = x[q][2 * i + 1];
+        float u = x[q][2 * i] * kUp, v = x[q][2 * i + 1] * kUp;
 #pragma unroll
         for (int s = 0; s < 3; ++s) {
           w[q][s][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2g{u, v}, bf16x2g));
           if (s == 2) break;
           u -= __uint_as_float(w[q][s][i] << 16), v -= __uint_as_float(w[q][s][i] & 0xffff0000u);
         }
-        most[q] = __builtin_elementwise_max(most[q], __builtin_bit_cast(u16x2g, w[q][0][i] & 0x7fff7fffu));
       }
   }
   __device__ __forceinline__ void store(u32x2g* stage, const u32x2g (&w)[2][3]) const {
@@ -439,17 +439,6 @@ struct SplitOp {
     for (int q = 0; q < 2; ++q)
 #pragma unroll
       for (int s = 0; s < 3; ++s) stage[to[q] + s * 4 * kSplitHalf] = w[q][s];
-  }
-  // Whether a quad's values were all under 2^-90, not all zero.
-  __device__ __forceinline__ bool tiny() const {
-    constexpr int limit = (127 - 90) << 7;
-    bool t = false;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int x = max((int)most[q][0], (int)most[q][1]);
-      t |= x > 0 && x < limit;
-    }
-    return t;
   }
 };
 
@@ -550,15 +539,14 @@ __global__ __launch_bounds__(256, 2) void gemm_f32(F32GemmArgs p) {
     if (st + 1 < steps) step(st + 1, a0, b0, a1, b1);
   }
   // Sums that are not finite (an infinity or a NaN among the factors, whose
-  // parts are NaN; or an overflow), and rows whose every value is so small
-  // that its lower parts fall under bf16's normal range: the tile again in
-  // full precision.
-  bool again = A.tiny() || B.tiny();
+  // parts are NaN; or an overflow, also of the scaled ones): the tile again in full
+  // precision.
+  bool again = false;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      acc[i][j] += low[i][j];
+      acc[i][j] = (acc[i][j] + low[i][j]) * (1.0f / (kUp * kUp));
 #pragma unroll
       for (int e = 0; e < 16; ++e) again |= !(fabsf(acc[i][j][e]) < INFINITY);
     }

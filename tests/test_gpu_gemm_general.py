@@ -403,8 +403,9 @@ def test_f32_split_factors_at_the_edges(target, a_kfast, b_kfast, k):
 
 def test_f32_split_factors_of_any_value(target):
     """Whole numbers are exact; infinities and NaN give what fp32 products
-    give; values near fp32's largest and rows of values under bf16's reach
-    (each computed again on the fp32 matrix cores) keep fp32's accuracy."""
+    give; values near fp32's largest (computed again on the fp32 matrix cores),
+    rows of values under bf16's reach, and a few such values among ordinary ones
+    where only they count, keep fp32's accuracy."""
     announce("fp32 split factors values")
     rng = np.random.default_rng(5)
 
@@ -441,3 +442,14 @@ def test_f32_split_factors_of_any_value(target):
         z[9] *= f32(s)
         want = z.astype(np.float64) @ y.astype(np.float64)
         assert relative(run(z, y)[9], want[9]) < TOL_F32, s
+    for e in (60, 100, 125):  # columns of the left factor against rows of the right one
+        z, w = x.copy(), y.copy()
+        z[:, 3::5] *= f32(2.0) ** -e
+        w[3::5] *= f32(2.0) ** (e - 1)  # (the largest under 2^128)
+        w[:, 7] = np.where(np.arange(40) % 5 == 3, w[:, 7], 0)  # only they count
+        want = z.astype(np.float64) @ w.astype(np.float64)
+        got = run(z, w)
+        bound = np.abs(z).astype(np.float64) @ np.abs(w).astype(np.float64) * 48 * 2.0 ** -24
+        assert np.all(np.abs(got - want) <= bound), (e, np.max(np.abs(got - want) / bound))
+        back = run(w.T.copy(), z.T.copy())
+        assert np.all(np.abs(back - want.T) <= bound.T), e
