@@ -645,8 +645,11 @@ int th_build_gemm(const th_gemm_desc* desc, th_launch** host_out);
  * th_time_launch measures).  The search runs in stages as the reference's
  * cover searches a product's tiles (ext/cuTileExt/contract.jl:12-27,171-200,
  * tinygrad's beam search at width one): every tile that takes the product at
- * its chosen split, then the other splits (1, 2, 4, ... 16, each part at
- * least 256 deep) of the best.  `desc`'s tile and splits are ignored; its
+ * its chosen split, and the library's own choice (TH_TILE_AUTO where a fused
+ * product runs on a middle tile, which only the library chooses), then the
+ * other splits (1, 2, 4, ... 16, each part at least 256 deep) of the best.  A
+ * descriptor with the tile and splits returned builds the launch measured (an
+ * fp32 product's splits are 0, the library's choice, where that is the fastest).  `desc`'s tile and splits are ignored; its
  * arrays are the ones measured on, and the product's outputs (c, and what
  * the epilogue writes) are overwritten; D + A B in place (d == c) is refused.
  * Results are kept for the process, keyed by the product's shape, layouts,

@@ -601,15 +601,12 @@ std::string tune_key(const th_gemm_desc* d) {
   return buf;
 }
 
-// The splits a build with `splits` asked (0: the builder's choice) ends up
-// with, as the builders round them.
-int splits_used(const th_gemm_desc* d, int tile, int splits) {
-  if (tile == TH_TILE_GENERAL) return 1;
-  int s = splits > 0 ? splits : auto_splits(d, tile);
-  if (s <= 1) return 1;
-  const int step = tile == TH_TILE_256 ? kDepth : kMidStep;
-  const int ks = ((d->k + s - 1) / s + step - 1) / step * step;
-  return (d->k + ks - 1) / ks;
+// The parts of K with which a build for `tile` is what one left to the
+// builder (splits 0) is: named, but for fp32 factors, whose builders choose among
+// kernels by them too (0 stays 0).
+int splits_of(const th_gemm_desc* d, int tile) {
+  if (d->flags & TH_GEMM_F32_FACTORS) return 0;
+  return tile == TH_TILE_GENERAL ? 1 : auto_splits(d, tile);
 }
 
 int measure(const th_gemm_desc* base, int tile, int splits, double* seconds) {
@@ -637,40 +634,47 @@ extern "C" int th_gemm_tune(const th_gemm_desc* desc, int32_t* tile_out, int32_t
     th_gemm_desc d = *desc;
     d.tile = TH_TILE_AUTO;
     d.splits = 0;
-    std::vector<int> tiles;
+    // Every choice is kept as it is measured (tile, splits), so that the launch
+    // built from the answer is the one measured.
+    std::vector<Tuned> choices;
     const bool x3 = (d.flags & TH_GEMM_BF16X3) != 0;
+    auto add = [&](int tile) { choices.push_back(Tuned{tile, splits_of(&d, tile), 0.0}); };
     if (x3) {
       // The bf16 tiles the tripled product may run on: those that build.
-      for (int t : {TH_TILE_256, TH_TILE_128X128, TH_TILE_128X64, TH_TILE_64X128, TH_TILE_64X64}) tiles.push_back(t);
+      for (int t : {TH_TILE_256, TH_TILE_128X128, TH_TILE_128X64, TH_TILE_64X128, TH_TILE_64X64}) add(t);
     } else {
-      if (tile_kernel_takes(&d)) tiles.push_back(TH_TILE_256);
+      if (tile_kernel_takes(&d)) add(TH_TILE_256);
       if (mid_takes(&d))
-        for (int t : {TH_TILE_128X128, TH_TILE_128X64, TH_TILE_64X128, TH_TILE_64X64}) tiles.push_back(t);
-      if (d.epilogue == TH_EPI_STORE && !d.bias) tiles.push_back(TH_TILE_GENERAL);
+        for (int t : {TH_TILE_128X128, TH_TILE_128X64, TH_TILE_64X128, TH_TILE_64X64}) add(t);
+      if (d.epilogue == TH_EPI_STORE && !d.bias) add(TH_TILE_GENERAL);
+      // The library's own choice where it is none of these: parts of K it takes
+      // by its estimate, or a fused product on a middle tile (which no caller names).
+      int s = 0;
+      const int t = choose_tile(&d, &s);
+      if (d.epilogue != TH_EPI_STORE && t != TH_TILE_256 && !choices.empty()) choices.push_back(Tuned{TH_TILE_AUTO, 0, 0.0});
+      else if (t != TH_TILE_256 && t != TH_TILE_GENERAL && s != splits_of(&d, t)) choices.push_back(Tuned{t, s, 0.0});
     }
-    TH_REQUIRE(!tiles.empty(), "th_gemm_tune: no kernel takes the product");
+    TH_REQUIRE(!choices.empty(), "th_gemm_tune: no kernel takes the product");
     // Stage one: every tile at the split the builder would choose.
-    Tuned best{0, 0, 0.0};
-    for (int t : tiles) {
-      double s = 0;
-      if (int r = measure(&d, t, 0, &s)) {
-        if (x3) continue;  // a tile the tripled product does not fit
-        return r;
-      }
-      if (best.tile == 0 || s < best.seconds) best = Tuned{t, splits_used(&d, t, 0), s};
-    }
-    TH_REQUIRE(best.tile != 0, "th_gemm_tune: no kernel takes the product");
+    Tuned best{-1, 0, 0.0};
+    auto consider = [&](Tuned c) -> int {
+      if (int r = measure(&d, c.tile, c.splits, &c.seconds)) return r;
+      if (best.tile < 0 || c.seconds < best.seconds) best = c;
+      return TH_OK;
+    };
+    for (const Tuned& c : choices)
+      if (int r = consider(c))
+        if (!x3) return r;  // (x3: a tile the tripled product does not fit)
+    TH_REQUIRE(best.tile >= 0, "th_gemm_tune: no kernel takes the product");
     // Stage two: the other splits of the best (plain products on the tile
     // kernels, and fp32 ones on the general kernel), each part at least 256 deep.
     const bool general_splits = d.flags & TH_GEMM_F32_FACTORS && d.c_dtype == TH_F32 && !d.bias;
     if ((best.tile != TH_TILE_GENERAL || general_splits) && d.epilogue == TH_EPI_STORE) {
+      const Tuned first = best;
       for (int sp : {1, 2, 4, 8, 16}) {
         if (sp > 1 && d.k / sp < 256) break;
-        const int used = splits_used(&d, best.tile, sp);
-        if (used == best.splits) continue;
-        double s = 0;
-        if (int r = measure(&d, best.tile, sp, &s)) return r;
-        if (s < best.seconds) best = Tuned{best.tile, used, s};
+        if (sp == first.splits) continue;
+        if (int r = consider(Tuned{first.tile, sp, 0.0})) return r;
       }
     }
     hit = g_tuned.emplace(key, best).first;

@@ -115,7 +115,7 @@ STORE, GELU, SQUARE_LOSS, GELU_BACKWARD = 0, 1, 2, 3
 F32_FACTORS, F16_FACTORS, ACCUMULATE, BF16X3 = 1, 2, 4, 8  # TH_GEMM_*
 # TH_TILE_*: which kernel and output tile a product runs on.
 TILE_AUTO, TILE_256, TILE_128X128, TILE_128X64, TILE_64X128, TILE_64X64, TILE_GENERAL = range(7)
-TILE_NAMES = {TILE_256: "256x256", TILE_128X128: "128x128", TILE_128X64: "128x64", TILE_64X128: "64x128",
+TILE_NAMES = {TILE_AUTO: "the library's choice", TILE_256: "256x256", TILE_128X128: "128x128", TILE_128X64: "128x64", TILE_64X128: "64x128",
               TILE_64X64: "64x64", TILE_GENERAL: "general 64x64 fp32"}
 
 
@@ -158,8 +158,9 @@ def gemm(m: int, n: int, k: int, a: int, a_m: int, a_k: int, b: int, b_k: int, b
 def gemm_tune(m: int, n: int, k: int, a: int, a_m: int, a_k: int, b: int, b_k: int, b_n: int, c: int, c_ld: int,
               **extra) -> tuple[int, int, float]:
     """(tile, splits, seconds): the product's fastest choice, measured on the
-    device on these arrays (th_gemm_tune: every tile that takes it, then the
-    splits of the best; kept for the process).  extra: gemm's keywords."""
+    device on these arrays (th_gemm_tune: every tile that takes it and the
+    library's own choice, then the splits of the best; kept for the process).
+    extra: gemm's keywords."""
     desc = _gemm_desc(m, n, k, a, a_m, a_k, b, b_k, b_n, c, c_ld, **extra)
     tile, splits, seconds = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_double()
     call("th_gemm_tune", ctypes.byref(desc), ctypes.byref(tile), ctypes.byref(splits), ctypes.byref(seconds))

@@ -128,7 +128,7 @@ def test_middle_tiles_half_result_batch_bias_and_added(target, tile):
 
 @pytest.mark.parametrize("tile", [2, 5])
 def test_middle_tiles_split_k(target, tile):
-    """K in 3 uneven parts (each a multiple of 32, the last shorter), summed
+    """K in 3 uneven parts (each a multiple of 64, the last shorter), summed
     by the second launch with the bias, into bf16 and fp32 results."""
     rng = np.random.default_rng(11)
     announce("gemm mid split", tile)
@@ -219,3 +219,45 @@ def test_environment_asks_for_measured_choices(target, monkeypatch):
     l()
     torch.cuda.synchronize()
     assert relative(c.double().cpu().numpy().T, interpret.product(A[0], B[0])) < TOL_F32
+
+
+@pytest.mark.parametrize("m,n,k", [(256, 256, 8192), (256, 384, 512)])
+def test_tuned_fp32_product_is_the_one_measured(target, m, n, k):
+    """An fp32 product's tuned choice builds what was measured: K in parts,
+    and the 32 x 32 kernel, where they are the fastest (at these sizes by far:
+    21 us in parts against over 200 in one, 12 against 27), not one part of it."""
+    import tempest_hip.launch as L
+    announce("gemm tune fp32", m, n, k)
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a, b = (torch.randn(*s, device="cuda", generator=gen) for s in ((m, k), (k, n)))
+    c = torch.empty(n, m, device="cuda")
+    args = (m, n, k, a.data_ptr(), k, 1, b.data_ptr(), n, 1, c.data_ptr(), m)
+    tile, splits, seconds = L.gemm_tune(*args, c_dtype=L.F32, factors=L.F32)
+    built = L.gemm(*args, c_dtype=L.F32, factors=L.F32, tile=tile, splits=splits)
+    assert ("gemm_f32_sum_parts" if k > 4096 else "gemm_f32_32x32") in built.describe(), (splits, built.describe())
+    again = target.time_launch(built)
+    assert again < 1.5 * seconds, (again, seconds)
+    built()
+    torch.cuda.synchronize()
+    assert relative(c.double().cpu().numpy().T, a.double().cpu().numpy() @ b.double().cpu().numpy()) < TOL_F32
+
+
+def test_tuned_fused_product_keeps_the_middle_tiles(target, monkeypatch):
+    """A fused product the library runs on a middle tile is measured there too
+    (a GELU layer of 12 tiles of 256 x 256, a third of the time on 64 x 64 ones),
+    and TEMPEST_HIP_TUNE=1 builds it so."""
+    import tempest_hip.launch as L
+    announce("gemm tune fused")
+    m, n, k = 3072, 256, 768
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    a, b, bias = (torch.randn(*s, device="cuda", generator=gen).to(torch.bfloat16) for s in ((m, k), (n, k), (m,)))
+    z, h = (torch.empty(n, m, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    args = (m, n, k, a.data_ptr(), k, 1, b.data_ptr(), 1, k, z.data_ptr(), m)
+    extra = {"epilogue": L.GELU, "bias": bias.data_ptr(), "aux_out": h.data_ptr()}
+    auto = L.gemm(*args, **extra)
+    assert "gemm_mid_gelu" in auto.describe()
+    tile, splits, seconds = L.gemm_tune(*args, **extra)
+    assert (tile, splits) == (L.TILE_AUTO, 0) and seconds < 0.7 * target.time_launch(
+        L.gemm(*args, tile=L.TILE_256, **extra))
+    monkeypatch.setenv("TEMPEST_HIP_TUNE", "1")
+    assert L.gemm(*args, **extra).describe() == auto.describe()
