@@ -577,7 +577,7 @@ enum { TH_EPI_STORE = 0, TH_EPI_GELU = 1, TH_EPI_SQUARE_LOSS = 2, TH_EPI_GELU_BA
  *   TH_TILE_GENERAL: anything with TH_EPI_STORE and no bias, any shape and
  *     strides: fp32 factors with an fp32 result on 128 x 128 tiles (each factor
  *     as three bf16 parts on the bf16 matrix cores, in fp32's precision; the fp32
- *     matrix cores where a part would leave bf16's range; K split like the
+ *     matrix cores where a tile's sums are not finite; K split like the
  *     others) or, few and short, 32 x 32 ones, half factors or a half
  *     result on 64 x 64 tiles of the fp32 matrix cores (unsplit).
  *     fp32 factors run only here unless TH_GEMM_BF16X3.

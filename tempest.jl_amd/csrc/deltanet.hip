@@ -890,15 +890,17 @@ __global__ __launch_bounds__(kScanThreads, 1) void dn_state_grad(DnArgs p) {
 // ---- backward: the chunk's products, WY form, decays and gates ---------------------
 // dQg = dO S', dW = -dU S', dKd = U dSn', dP = lower(dO U'), then everything
 // that follows from them: dT, dA = -T' dT T', the gate gradients and dQ, dK, dV.
-// Bound by memory: a chunk reads 336 KB of states, U, dU, T and arrays and
-// writes 48.  The products stay in the registers that the outputs sum in (dQg
+// Bound by instructions, the splits of fp32 operands and the elementwise work: split
+// once where they are written it took 889 us, at each read 1022, for the same
+// bytes (a chunk reads 336 KB of states, U, dU, T and arrays and writes 48, 3.3
+// TB/s of traffic).  The products stay in the registers that the outputs sum in (dQg
 // in dQ's, dKd and T' dW in dK's, dP in the lanes that form dQK), so none of
 // them goes through memory; as two kernels that passed dQg, dW, dKd and dP on
-// (224 KB a chunk, out and back) the same took 1293 us at B4 H16 T8192, now 889.
+// (224 KB a chunk, out and back) the same took 1293 us at B4 H16 T8192.
 //
 // Every product on the matrix cores, split bf16; dO, Q and K sit in LDS as
-// bf16 (their exact values) and are widened as they are read; U, dU and dW take
-// turns in one fp32 buffer, which M and N then share; V, T, S and dSn are
+// bf16 (their exact values); U, dU and dW take turns in one pair of bf16 planes (hi and
+// lo), whose LDS M and N then share; V, T, S and dSn are
 // read from memory by the products that use them (S and dSn by rows, each
 // wave's 32).  Under 80 KB, so two workgroups share a CU.
 // Wave w: columns 32 w .. 32 w + 31 of the 64 x 128 work, rows 16 w .. of the

@@ -188,10 +188,10 @@ __global__ __launch_bounds__(256) void gemm_general(GenGemmArgs p) {
 // from the others; what is left out is at most 2^-25 of each a b, under the
 // rounding of the sums.  Error against float64 (norm-wise, normal
 // factors), with fp32 products and so: 4096^3 1.1e-6 and 4.0e-7, 2000 x 1500 x
-// 1030 5.7e-7 and 1.9e-7, 256 x 256 x 8192 2.5e-7 and 1.6e-7; time 1289 and 800
-// to 860 us, 156 and 66, 32 and 21.  What bounds it now: of a step's 1.0 us (one
-// workgroup on a CU; 1.56 two) the products take 0.43, the rest is LDS traffic
-// and the wait at its barrier.  The factors are scaled by 2^24 as they are split, and
+// 1030 5.7e-7 and 1.3e-7, 256 x 256 x 8192 2.5e-7 and 1.6e-7; time 1289 and 730
+// to 760 us, 156 and 60, 32 and 21.  What bounds it now: the products keep the
+// matrix cores busy 28 % of the time at 2000 x 1500 x 1030 (54 % at 4096^3), the rest
+// is the splits' vector work, LDS traffic and the wait at its barrier.  The factors are scaled by 2^24 as they are split, and
 // the sums back, so that the parts reach as far down as fp32 does; a tile whose sums
 // are not finite is computed again on the fp32 matrix cores
 // (v_mfma_f32_32x32x2_f32), as every tile was before.
@@ -722,8 +722,8 @@ int build_gemm_general(const th_gemm_desc* d, th_launch** out) {
 // keep its workgroups within the 512 the device holds, where the tiles alone
 // are fewer than 256, each part at least 256 deep (128 where the tiles are under
 // a quarter of the device).  In one part and as chosen: 2000 x 1500 x 1030 (192
-// tiles) 72 us and, in two, 66; 3500 x 640 x 2600 (140) 148 and 91 in three;
-// 1100 x 1000 x 3000 (72) 172 and 63 to 73 in six or seven; 1500 x 1300 x 400
+// tiles) 69 us and, in two, 60; 3500 x 640 x 2600 (140) 146 and 89 in three;
+// 1100 x 1000 x 3000 (72) 172 and 61 to 66 in six or seven; 1500 x 1300 x 400
 // (132) 26 in one, 30 in two.
 static int f32_splits(const th_gemm_desc* d) {
   const int64_t tiles = (int64_t)((d->m + kFT - 1) / kFT) * ((d->n + kFT - 1) / kFT) * std::max(1, d->batch);

@@ -182,12 +182,11 @@ the cover, tried in order beside the floor; by default all of this
 extension's.
 
 - `precision`: the numerics policy for products of Float32 factors (as
-  CUDATarget's, target.jl:42-44): `:full` keeps them in Float32 on the fp32
-  matrix cores; `:bf16x3` splits each factor into two BFloat16 parts,
+  CUDATarget's, target.jl:42-44): `:full` keeps all of Float32's bits, as three
+  BFloat16 parts a factor on the bf16 matrix cores; `:bf16x3` splits each factor into two BFloat16 parts,
   `x = hi + lo`, and sums three bf16 products in Float32
   (`A_hi B_hi + A_hi B_lo + A_lo B_hi`, about 16 of Float32's 24 significant
-  bits), on matrix cores sixteen times faster: the MI355X counterpart of
-  `:tf32x3`, which this device has no TF32 for.
+  bits): the MI355X counterpart of `:tf32x3`, which this device has no TF32 for.
 - `deterministic = true` keeps every sum's rounding independent of the order
   blocks run in (target.jl:229-231): the floor's folds by key then add their
   elements one at a time in the order of the items instead of by atomics,

@@ -79,7 +79,8 @@ class HIPTarget:
     """Run on one MI355X (gfx950) through libtempest_hip.
 
     Options as CUDATarget's (target.jl:30-75): ``precision`` for products of
-    fp32 factors, ``"full"`` (fp32 on the fp32 matrix cores) or ``"bf16x3"``
+    fp32 factors, ``"full"`` (fp32's precision: three bf16 parts a factor
+    on the bf16 matrix cores) or ``"bf16x3"``
     (each factor split hi + lo in bf16 and three bf16 products summed in
     fp32, TH_GEMM_BF16X3: the counterpart of CUDA's ``:tf32x3``); half
     factors always accumulate in fp32.  ``online`` (permits the online
