@@ -347,18 +347,21 @@ def config1(target):
     comp = th.compile(th.programs.tanh_layer(), target, w, b, x)
     ex = comp.executable
     dispatch = graph_vs_direct(target, ex, reps=2000, warmup=20)
+    # The call as a program that only calls sees it (comp's launches have been
+    # looked into, so its results go through a copy).
+    comp = th.compile(th.programs.tanh_layer(), target, w, b, x)
     for _ in range(50):
         comp(w, b, x)
     torch.cuda.synchronize()
     n = 500
     t = time.perf_counter()
     for _ in range(n):
-        comp(w, b, x)  # point, replay, copy dw/db/dx, read the loss
+        comp(w, b, x)  # point, run into memory of the call's, read the loss
     call_s = (time.perf_counter() - t) / n
     return {"us_per_step_graph": dispatch["us_graph"], "us_per_step_execute": dispatch["us_direct"],
             "recording": dispatch["chosen"], "us_per_compiled_call_host": call_s * 1e6,
             "note": "graph/execute: device time per step from events around 2000 back-to-back replays/runs; "
-                    "compiled call: host wall time of c(w, b, x) incl. result copies and the loss read"}
+                    "compiled call: host wall time of c(w, b, x) incl. the loss read"}
 
 
 def config3(target, steps: int = 20, warmup: int = 10):
