@@ -1196,8 +1196,9 @@ bool f32_attention_takes(const th_attention_desc* d) {
                           (const void*)d->dout, (const void*)d->dq, (const void*)d->dk, (const void*)d->dv})
     if (!aligned16(ptr)) return false;
   const int64_t kv = d->kv_seq > 0 ? d->kv_seq : d->seq;
-  // (blocks of 128 positions along grid z, at most 8 parts each)
-  return (d->seq + 127) / 128 <= 8191 && (kv + 127) / 128 <= 8191 && d->heads <= 65535 && d->batch <= 65535;
+  // (Blocks of 128 positions along grid z; sweeps are split only where all the
+  // blocks are fewer than 256.)
+  return (d->seq + 127) / 128 <= 65535 && (kv + 127) / 128 <= 65535 && d->heads <= 65535 && d->batch <= 65535;
 }
 
 int build_attention_f32_fwd(const th_attention_desc* d, th_launch** out) {

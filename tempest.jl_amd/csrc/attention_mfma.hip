@@ -1165,8 +1165,9 @@ bool mfma_attention_takes(const th_attention_desc* d) {
   for (int64_t s : {d->q_strides[0], d->q_strides[1], d->q_strides[2], d->k_strides[0], d->k_strides[1], d->k_strides[2]})
     if (s <= 0 || s % 8) return false;
   const int64_t kv = d->kv_seq > 0 ? d->kv_seq : d->seq;
-  // (blocks of 128 positions along grid z, at most 8 parts or halves each)
-  return (d->seq + 127) / 128 <= 8191 && (kv + 127) / 128 <= 8191 && d->heads <= 65535 && d->batch <= 65535;
+  // (Blocks of 128 positions along grid z; sweeps are split only where all the
+  // blocks are fewer than 256.)
+  return (d->seq + 127) / 128 <= 65535 && (kv + 127) / 128 <= 65535 && d->heads <= 65535 && d->batch <= 65535;
 }
 
 int build_attention_mfma_fwd(const th_attention_desc* d, th_launch** out) {

@@ -132,3 +132,18 @@ def test_forward_sweeps_in_halves(target, D, B, H, KV, S, Sk, causal):
     ro, rl = interpret.attention_fwd(_np(q), _np(k), _np(v), causal)
     assert relative(_np(o), ro) < TOL_BF16, relative(_np(o), ro)
     assert np.max(np.abs(_np(lse) - rl)) < 1e-3 * max(1.0, np.abs(rl).max())
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("S", [1048449, 65535 * 128])
+def test_the_longest_sequences_are_the_matrix_cores(target, f32, S):
+    """Past 2^20 positions, and up to as many blocks of 128 as a grid has, a
+    forward and a backward are built on the matrix cores (not run here)."""
+    import tempest_hip.launch as L
+    announce("attn longest", f32, S)
+    p = [4096 * (i + 1) for i in range(9)]  # places that nothing reads
+    extra = {"causal": True, "head_dim": 64, "f32": f32}
+    fwd = L.attention_fwd(1, 1, 1, S, *p[:5], **extra)
+    bwd = L.attention_bwd(1, 1, S, *p, kv_heads=1, **extra)
+    kind = "f32_attn" if f32 else "mfma_attn"
+    assert f"{kind}_fwd_d64" in fwd.describe() and f"{kind}_dkdv_d64" in bwd.describe(), (fwd.describe(), bwd.describe())
