@@ -360,9 +360,9 @@ class Executable:
         None, and nothing run, where those are what the caller has to have
         (someone knows where they lie), where torch would not order the memory
         with the launches (another current stream than the library's), or
-        where the recording is a graph, whose every node with a result would
-        be retargeted."""
-        if self._seen or isinstance(self._graph, Graph):
+        where the recording is not the launches themselves (a graph's every
+        node with a result would be retargeted)."""
+        if self._seen or not (self._graph is None or isinstance(self._graph, Direct)):
             return None
         handle = ctypes.c_void_p()
         call("th_get_stream", ctypes.byref(handle))

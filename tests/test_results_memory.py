@@ -139,6 +139,19 @@ def test_a_run_leaves_returned_arrays_alone(compiled, run):
     assert torch.equal(ex.outputs()[0], want(x)) and ex.outputs()[1] == x.sum()
 
 
+def test_another_kind_of_recording_is_what_a_call_replays(compiled):
+    """What a target records that is not the launches themselves runs as it
+    replays it, into the executable's results."""
+    comp, lib = compiled.comp, compiled.lib
+    replayed = []
+    comp.executable._graph = object()
+    comp.executable.target.replay = lambda graph: replayed.append(graph) or lib.run()
+    y, s = comp(compiled.x(3))
+    assert len(replayed) == 1 and "th_launches_lend" not in lib.log
+    assert torch.equal(y, want(compiled.x(3))) and s == compiled.x(3).sum()
+    assert torch.equal(comp.executable._results.view(torch.float32)[:N], y) and y.data_ptr() != comp.executable._results.data_ptr()
+
+
 def test_outputs_show_the_last_call_and_follow_later_ones(compiled):
     """outputs(ex) are the buffers themselves: the last call's results right
     after it, whatever its caller has done to what it was given, and those of
