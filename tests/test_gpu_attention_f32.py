@@ -119,3 +119,27 @@ def test_fp32_attention_over_fp32s_range(target, D, S, what, e):
                            ("dk", _np(dk).astype("f8") / sg / u, want[1]), ("dv", _np(dv).astype("f8") / sv, want[2])):
         print("   ", name, relative(got, ref), flush=True)
         assert relative(got, ref) < 4e-6, (name, relative(got, ref))
+
+
+@pytest.mark.parametrize("e", [20, 30])
+def test_fp32_attention_at_small_scales(target, e):
+    """Q and K of 2^e under a scale of 2^-2e / 8: in three parts down to a scale
+    of 2^-50, in fp32 products under it, the same results as at e = 0 either way."""
+    import tempest_hip.launch as L
+    announce("attn fp32 scale", e)
+    gen = torch.Generator(device="cuda").manual_seed(e)
+    q, k, v, g = (torch.randn(1, 200, 2, 64, device="cuda", generator=gen) for _ in range(4))
+    t = 2.0 ** e
+    o, dq, dk, dv = (torch.empty_like(q) for _ in range(4))
+    lse = torch.empty(1, 200, 2, device="cuda")
+    qt, kt = q * t, k * t
+    p = [x.data_ptr() for x in (qt, kt, v, o, lse)]
+    extra = {"causal": True, "head_dim": 64, "f32": True, "scale": t ** -2 / 8}
+    L.attention_fwd(1, 2, 2, 200, *p, **extra)()
+    L.attention_bwd(1, 2, 200, *p, g.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), kv_heads=2, **extra)()
+    torch.cuda.synchronize()
+    ro, _ = interpret.attention_fwd(_np(q), _np(k), _np(v), True)
+    want = interpret.attention_bwd(_np(q), _np(k), _np(v), _np(g), True)
+    for name, got, ref in (("o", _np(o), ro), ("dq", _np(dq) * t, want[0]), ("dk", _np(dk) * t, want[1]),
+                           ("dv", _np(dv), want[2])):
+        assert relative(got, ref) < 4e-6, (name, relative(got, ref))
